@@ -177,6 +177,11 @@ bool gemm2_cfg_splittable(int cfg);  // false: the config always runs the whole 
 // v5: four-wave GEMM / implicit-GEMM conv (gemm_w4.hip), bn = 256: 256 x 256 tiles, bn = 320: 192 x 320 tiles
 bool gemm_w4_supported(const GemmArgs& a);
 void launch_gemm_w4(const GemmArgs& a, int bn, hipStream_t s);
+// small tiles with a deep ring of K-tiles in flight (gemm_deep.hip)
+constexpr int kDeepCfgs = 3;
+bool gemm_deep_supported(const GemmArgs& a);
+void gemm_deep_tile(int which, int* bm, int* bn);
+void launch_gemm_deep(const GemmArgs& a, int which, float* ws, int splits, hipStream_t s);
 // v6: W-stationary low-K GEMM (gemm_ws.hip): K = 320, N % 320 == 0, persistent over M, weights in VGPRs
 bool gemm_ws_supported(const GemmArgs& a);
 void launch_gemm_ws(const GemmArgs& a, hipStream_t s);
