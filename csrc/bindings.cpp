@@ -1504,6 +1504,14 @@ int64_t gemm_tuning_import(const std::vector<std::string>& entries) {
   return n;
 }
 
+void mean_tokens(const Tensor& x, const Tensor& out) {
+  check_bf16(x, "x");
+  check_f32(out, "out");
+  SHAI_CHECK(x.dim() == 3 && x.is_contiguous() && x.size(2) % 8 == 0 && x.size(1) > 0, "mean_tokens input [B, S, D], D % 8 == 0");
+  SHAI_CHECK(out.dim() == 2 && out.size(0) == x.size(0) && out.size(1) == x.size(2), "mean_tokens output [B, D]");
+  if (x.size(0) > 0) shai::launch_mean_tokens(cptr(x), out.data_ptr<float>(), x.size(0), x.size(1), x.size(2), stream());
+}
+
 void embedding(const Tensor& ids, const Tensor& table, const Tensor& out) {
   check_i32(ids, "ids");
   check_bf16(table, "table");
@@ -1662,6 +1670,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("sched_step(Tensor model_out, Tensor(a!) latents, bool cfg, float guidance, int pred_type, float a_t, float a_prev, float dt) -> ()");
   m.def("sched_step_rows(Tensor model_out, Tensor(a!) latents, bool cfg, float guidance, int pred_type, Tensor rows_params) -> ()");
   m.def("softmax_(Tensor(a!) x, float scale) -> ()");
+  m.def("mean_tokens(Tensor x, Tensor(a!) out) -> ()");
   m.def("embedding(Tensor ids, Tensor table, Tensor(a!) out) -> ()");
   m.def("decode_attn_rope(Tensor qkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, "
         "Tensor ctx_lens, Tensor positions, Tensor cos, Tensor sin, Tensor slots, Tensor(d!) ws, int h, int hk, "
@@ -1704,6 +1713,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("sched_step", &sched_step);
   m.impl("sched_step_rows", &sched_step_rows);
   m.impl("softmax_", &softmax_);
+  m.impl("mean_tokens", &mean_tokens);
   m.impl("embedding", &embedding);
   m.impl("decode_attn_rope", &decode_attn_rope);
   m.impl("gemm_partials", &gemm_partials);

@@ -283,6 +283,54 @@ void launch_cache_flush(const void* buf, size_t bytes, unsigned* sink, hipStream
   cache_flush_kernel<<<2048, 256, 0, s>>>(reinterpret_cast<const uint4_*>(buf), (long)(bytes / 16), sink);
 }
 
+// out[b, c] = mean over s of x[b, s, c]: a block is 512 columns (64 lanes x 8) of one b, its four waves take every fourth row and
+// meet in LDS.  One launch for a widening copy and a library reduction (which may clear its semaphores with a memset: not
+// for a captured graph).  32 x 128 x 1024: 16.5 us of two launches before, 5.6 us; 1 x 32 x 1024: 8.8 us, 3.1 us.
+__global__ void __launch_bounds__(256) mean_tokens_kernel(const bf16_t* __restrict__ x, float* __restrict__ out, int S, int D) {
+  __shared__ float4_ part[3][64][2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = (blockIdx.x * 64 + lane) * 8;
+  const bf16_t* src = x + (long)blockIdx.y * S * D + c;
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (c < D) {
+    constexpr int U = 8;  // rows in flight
+    for (int r = wave; r < S; r += 4 * U) {
+      uint4_ v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        v[u] = r + 4 * u < S ? *reinterpret_cast<const uint4_*>(src + (long)(r + 4 * u) * D) : uint4_{0, 0, 0, 0};
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float f[8];
+        unpack8(v[u], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += f[e];
+      }
+    }
+  }
+  if (wave > 0) {
+    part[wave - 1][lane][0] = float4_{s[0], s[1], s[2], s[3]};
+    part[wave - 1][lane][1] = float4_{s[4], s[5], s[6], s[7]};
+  }
+  __syncthreads();
+  if (wave == 0 && c < D) {
+    float4_ a = {s[0], s[1], s[2], s[3]}, b = {s[4], s[5], s[6], s[7]};
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+      a += part[w][lane][0];
+      b += part[w][lane][1];
+    }
+    float4_* dst = reinterpret_cast<float4_*>(out + (long)blockIdx.y * D + c);
+    const float n = (float)S;
+    dst[0] = a / n;
+    dst[1] = b / n;
+  }
+}
+
+void launch_mean_tokens(const bf16_t* x, float* out, int B, int S, int D, hipStream_t s) {
+  mean_tokens_kernel<<<dim3((D + 511) / 512, B), 256, 0, s>>>(x, out, S, D);
+}
+
 void launch_embedding(const int* ids, const bf16_t* table, bf16_t* out, long T, int D, hipStream_t s) {
   embedding_kernel<<<grid_for(T * (D / 8)), 256, 0, s>>>(ids, table, out, T, D);
 }

@@ -10,12 +10,14 @@ from __future__ import annotations
 import base64
 import io
 import os
+import threading
+from collections import OrderedDict
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
 
-from . import capture
+from . import capture, new_graph
 from ..tokenizers import load_tokenizer
 from ..weights import materialize
 
@@ -110,7 +112,7 @@ class ImageClassifierEngine:
                 for _ in range(2):  # warm-up: GEMM autotuning and allocator growth happen outside capture
                     self._forward_u8(static)
             torch.cuda.current_stream(self.device).wait_stream(side)
-            graph = torch.cuda.CUDAGraph()
+            graph = new_graph(self.device)
             with capture(graph):
                 out = self._forward_u8(static)
             g = self._graphs[B] = (graph, static, out)
@@ -171,9 +173,44 @@ class DetectorEngine:
         return out
 
 
+class _EmbeddingGraph:
+    """The encoder on a batch of one shape as a HIP graph: token ids and lengths of the rows in one buffer, filled by one copy."""
+
+    def __init__(self, model, B: int, L: int, device, pool):
+        self.host = torch.zeros(B * L + B, dtype=torch.int32, pin_memory=True)
+        self.rows = self.host.numpy()
+        self.dev = torch.zeros(B * L + B, dtype=torch.int32, device=device)
+        ids, lens = self.dev[:B * L].view(B, L), self.dev[B * L:]
+        lens.fill_(L)
+        side = torch.cuda.Stream(device=device)
+        side.wait_stream(torch.cuda.current_stream(device))
+        with torch.cuda.stream(side):      # GEMM autotuning, the position bias and allocator growth happen outside the capture
+            model.encode_mean(ids, lens=lens)
+        torch.cuda.current_stream(device).wait_stream(side)
+        self.graph = new_graph(device)
+        with capture(self.graph, pool=pool, capture_error_mode="thread_local"):
+            self.out = model.encode_mean(ids, lens=lens)
+
+    def run(self, ids: np.ndarray, mask: np.ndarray) -> np.ndarray:
+        n = ids.size
+        self.rows[:n] = ids.reshape(-1)
+        self.rows[n:] = mask.sum(-1)
+        self.dev.copy_(self.host, non_blocking=True)
+        self.graph.replay()
+        return self.out.cpu().numpy()      # waits: the host buffer is free again
+
+
 class TextEmbeddingEngine:
-    def __init__(self, cfg=None, device="cuda", model_path=None, seed=0):
+    """T5 sentence embeddings.  An encoder step is some 200 launches that the host takes longer to issue than a small batch to run,
+    so every batch shape runs as a HIP graph (the least recently used of ``MAX_GRAPHS`` goes); with tensor parallelism eagerly.
+    T5-v1.1-large: one 32-token text 2.24 ms eager, 1.23 ms; 32 texts of 128 tokens 6.0 ms either way (4.8 ms of kernels, then
+    tokenizing)."""
+
+    MAX_GRAPHS = 16
+
+    def __init__(self, cfg=None, device="cuda", model_path=None, seed=0, use_graphs=True):
         from ..models.t5 import T5Config, T5EncoderModel
+        from ..parallel.state import tp
         self.cfg = cfg or T5Config.v1_1_large()
         self.device = torch.device(device)
         with torch.device(self.device):
@@ -182,14 +219,26 @@ class TextEmbeddingEngine:
         self.tokenizer = load_tokenizer(model_path, vocab_size=self.cfg.vocab_size, bos_id=None,
                                         eos_id=self.cfg.eos_token_id, pad_id=self.cfg.pad_token_id,
                                         model_max_length=1024)
+        self.use_graphs = use_graphs and self.device.type == "cuda" and tp().size == 1
+        self._graphs: "OrderedDict[tuple, _EmbeddingGraph]" = OrderedDict()
+        self._pool = torch.cuda.graph_pool_handle() if self.use_graphs else None
+        self._lock = threading.Lock()      # the graphs share buffers: one replay at a time
 
     @torch.inference_mode()
     def embed(self, texts: Sequence[str], max_length: int) -> np.ndarray:
         enc = self.tokenizer(list(texts), max_length=max_length, padding="max_length", truncation=True,
                              return_tensors="pt")
-        ids = enc["input_ids"].to(self.device)
-        mask = enc["attention_mask"].to(self.device)
-        return self.model.encode_mean(ids, mask).cpu().numpy()
+        ids, mask = enc["input_ids"], enc["attention_mask"]
+        if not self.use_graphs or not ids.numel():
+            return self.model.encode_mean(ids.to(self.device), mask.to(self.device)).cpu().numpy()
+        with self._lock, torch.cuda.device(self.device):
+            g = self._graphs.get(tuple(ids.shape))
+            if g is None:
+                if len(self._graphs) >= self.MAX_GRAPHS:
+                    self._graphs.popitem(last=False)
+                g = self._graphs[tuple(ids.shape)] = _EmbeddingGraph(self.model, *ids.shape, self.device, self._pool)
+            self._graphs.move_to_end(tuple(ids.shape))
+            return g.run(ids.numpy(), mask.numpy())
 
 
 def _resize_u8(x: torch.Tensor, H: int, W: int) -> torch.Tensor:

@@ -118,10 +118,12 @@ class T5EncoderModel(nn.Module):
             self._bias_cache[key] = b
         return b
 
-    def forward(self, input_ids: torch.Tensor, attention_mask: torch.Tensor = None) -> torch.Tensor:
+    def forward(self, input_ids: torch.Tensor, attention_mask: torch.Tensor = None, lens: torch.Tensor = None) -> torch.Tensor:
+        """``lens``: int32 number of tokens of every row, instead of their mask."""
         B, S = input_ids.shape
-        lens = (attention_mask.sum(-1).to(torch.int32) if attention_mask is not None
-                else torch.full((B,), S, dtype=torch.int32, device=input_ids.device))
+        if lens is None:
+            lens = (attention_mask.sum(-1).to(torch.int32) if attention_mask is not None
+                    else torch.full((B,), S, dtype=torch.int32, device=input_ids.device))
         x = self.shared(input_ids)
         bias = self.position_bias(S, input_ids.device)
         for blk in self.blocks:
@@ -158,6 +160,6 @@ class T5EncoderModel(nn.Module):
                                                                         out[p + "1.DenseReluDense.wi_0.weight"])
         return res
 
-    def encode_mean(self, input_ids, attention_mask=None) -> torch.Tensor:
+    def encode_mean(self, input_ids, attention_mask=None, lens=None) -> torch.Tensor:
         """t5_model_api.py:35-46 semantics: mean over ALL (padded) positions, fp32."""
-        return self.forward(input_ids, attention_mask).float().mean(dim=1)
+        return ops.mean_tokens(self.forward(input_ids, attention_mask, lens))

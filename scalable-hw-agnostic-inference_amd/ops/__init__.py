@@ -755,6 +755,15 @@ def token_feedback(ids, rowmap, prev):
     return ids
 
 
+def mean_tokens(x):
+    """fp32 mean over the tokens of x [B, S, D] -> [B, D]."""
+    if not _gpu(x) or x.dtype != torch.bfloat16 or x.shape[-1] % 8 or not x.numel():
+        return x.float().mean(dim=1)
+    out = torch.empty(x.shape[0], x.shape[2], dtype=torch.float32, device=x.device)
+    _K().mean_tokens(x.contiguous(), out)
+    return out
+
+
 def embedding(ids, table):
     if not _gpu(table):
         return table[ids.long()]

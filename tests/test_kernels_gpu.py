@@ -652,3 +652,10 @@ def test_linear_weight_slices(cuda, S, R, N, K):
     want = torch.einsum("smk,snk->smn", x.float().view(S, R, K), w.float()) + b2.float()[:, None, :]
     close(y, want.reshape(S * R, N), 2e-2)
     torch.testing.assert_close(st, ref.row_moments(y, 1e-5), atol=2e-3, rtol=2e-3)
+
+
+@pytest.mark.parametrize("B,S,D", [(1, 1, 8), (3, 5, 520), (32, 128, 1024), (2, 333, 512), (1, 1024, 4096)])
+def test_mean_tokens(cuda, B, S, D):
+    """fp32 sums of at most 1024 bf16 values: 1e-6 of their spread."""
+    x = torch.randn(B, S, D, device=cuda).bfloat16()
+    assert (ops.mean_tokens(x).double() - x.double().mean(1)).abs().max().item() < 1e-6

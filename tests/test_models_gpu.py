@@ -250,3 +250,35 @@ def test_decode_splits_grow_with_long_context(cuda):
         want = [s.output for s in mk(False).generate(prompts, sp)]
     assert got == want
     assert any(k[0] == 32 and k[3] > e.decode_splits(32, 0) for k in e._graphs)
+
+
+def test_t5_graph_replay_matches_eager(cuda):
+    """Embeddings of replayed graphs equal the eager ones: shapes that take turns, more of them than graphs are kept, other work
+    between the replays, two threads."""
+    import threading
+    from shai_amd.engines.encoders import TextEmbeddingEngine
+    from shai_amd.models.t5 import T5Config
+    eng = TextEmbeddingEngine(cfg=T5Config.tiny())
+    eng.MAX_GRAPHS = 3
+    eager = TextEmbeddingEngine(cfg=T5Config.tiny(), use_graphs=False)
+    texts = ["a photo of a horse", "red", "the quick brown fox jumps over the lazy dog and more"]
+    shapes = [(1, 8), (3, 8), (2, 33), (3, 64), (1, 8)]
+    want = {s: eager.embed(texts[:s[0]], s[1]) for s in shapes}
+    for _ in range(3):
+        for s in shapes:
+            torch.randn(64, 64, device=cuda).sum().item()
+            assert np.array_equal(eng.embed(texts[:s[0]], s[1]), want[s]), s
+    assert len(eng._graphs) == 3
+    bad = []
+
+    def work(s):
+        for _ in range(10):
+            if not np.array_equal(eng.embed(texts[:s[0]], s[1]), want[s]):
+                bad.append(s)
+
+    ts = [threading.Thread(target=work, args=(s,)) for s in shapes[:2]]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
