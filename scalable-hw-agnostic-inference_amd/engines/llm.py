@@ -697,7 +697,15 @@ class LLMEngine:
             g = self._decode_program(rows, [s.n_cached for s in rows], logits=True)[0]
             self._enqueue(g, rows, [s.n_cached for s in rows], [s.prompt[-1] for s in rows], [-1] * len(rows),
                           [s.prompt[-2] if s.n_cached else -1 for s in rows], sampled=False)
-            out = g.logits.index_select(0, torch.from_numpy(want).to(self.device).long()) if len(want) else None
+            # a copy: the program's buffer takes the next step's logits.  Nothing here waits for the step, so the host prepares
+            # the next one meanwhile (a blocking copy of the row numbers cost 0.1 to 0.2 ms of idle GPU per step)
+            out = None
+            if len(want) == len(rows) and (want == np.arange(len(rows))).all():
+                out = g.logits[:len(rows)].clone()
+            elif len(want):
+                at = torch.from_numpy(want.astype(np.int64))
+                at = at.pin_memory().to(self.device, non_blocking=True) if self.device.type == "cuda" else at
+                out = g.logits.index_select(0, at)
         else:
             out = self.model(self._packed_batch(rows, news, want if len(want) else None), self.kv)
             out = out if len(want) else None
