@@ -173,7 +173,8 @@ static void stream(const GemmArgs& a, hipStream_t s) {
 
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t s) {
   const int ec = epi_class(a.epi);
-  if (f32) stream<float, float, EC_ANY>(a, s);
+  if (!f32 && gemm_ring_fits(a)) launch_gemm_ring(a, s);
+  else if (f32) stream<float, float, EC_ANY>(a, s);
   else if (a.out_f32 && ec == EC_PLAIN) stream<bf16_t, float, EC_PLAIN>(a, s);
   else if (a.out_f32) stream<bf16_t, float, EC_ANY>(a, s);
   else if (ec == EC_PLAIN) stream<bf16_t, bf16_t, EC_PLAIN>(a, s);

@@ -1,0 +1,179 @@
+// C = epi(A W^T) for 17 to 64 rows of A (decode steps of a batch) with bf16 weights.
+//
+// The streaming kernel (gemm.hip) reads both operands straight into registers, 16 rows x 16 bytes per quarter wave: 14 bytes per
+// clock and CU, of which A, the same for every workgroup, is as much as W at 64 rows.  DMA to LDS moves 30.  So here both
+// operands go through a ring in LDS, 128 k at a time, and one workgroup per CU owns as many columns as give every CU one
+// (16 NT; A is read once per CU): 17424 x 2048 on 64 rows is 228 workgroups of 80 columns (5 blocks of 16), 32768 x 2048 is 256 of 128.
+//
+// 8 waves: wave w takes the 32 k of sub-step w % 4 and the row blocks of half w / 4; the four k-groups' sums meet in LDS and are
+// added in their order.  Rows past M or N and values past K are out of the buffers' range: zeros, no traffic.
+// LDS rows are 256 bytes; chunk c (16 bytes) of row r is at c ^ (r & 15): no bank conflicts, and the DMA stays lane-linear because
+// the source address carries the permutation.
+//
+// Replays of a HIP graph over weights larger than the caches, us (streaming kernel -> here; N x K, 64 rows): 17424 x 2048
+// 24.0 -> 19.3, 32768 x 2048 40.7 -> 34.7, 24576 x 4096 63.7 -> 44.7, 8256 x 2048 17.5 -> 12.6, 4096 x 2048 10.3 -> 7.9, partial
+// sums of 2048 x 12544 21.6 (4 parts) -> 14.5 (8 parts).  17424 x 2048 is 71 MB: 3.7 TB/s.  What is left is the start (launch, the
+// first stage's latency) and the joining of the sums, about 5 us, and the memory's rate in between.
+#include "lm_device.h"
+#include "lm.h"
+
+#include <type_traits>
+
+namespace shai_lm {
+
+namespace {
+
+constexpr uint32_t kOob = 0x80000000u;
+constexpr int KS = 128;                       // k of one ring stage
+
+constexpr int ring_stages(int MT, int NT) {   // as many as fit in 160 KB, at most 5
+  const int n = 160 * 1024 / ((MT + NT) * 16 * KS * 2);
+  return n < 5 ? n : 5;
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <typename O, int EC, int MT, int NT>
+__global__ void __launch_bounds__(512) gemm_ring_kernel(const GemmArgs p) {
+  constexpr int S = ring_stages(MT, NT), STAGE = (MT + NT) * 16 * KS;  // elements
+  constexpr int PIECES = 4 * (MT + NT);       // DMA instructions of a stage (4 rows each): W's, then A's
+  constexpr int HI = (PIECES + 7) / 8, LO = PIECES / 8, MH = MT / 2;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4, kg = wid & 3, mh = wid >> 2;
+  const int n0 = blockIdx.x * 16 * NT;
+  const __amdgpu_buffer_rsrc_t rw = rsrc(p.W, (long)p.N * p.K * 2), ra = rsrc(p.A, ((long)(p.M - 1) * p.lda + p.K) * 2);
+  int first = 0, steps = (p.K + KS - 1) / KS;
+  O* C = static_cast<O*>(p.C);
+  if (p.splits > 1) {
+    const int all = steps;
+    first = (int)(blockIdx.y * (long)all / p.splits);
+    steps = (int)((blockIdx.y + 1L) * all / p.splits) - first;
+    C += (long)blockIdx.y * p.M * p.N;
+  }
+  uint32_t off[HI];
+  int col[HI];                                // first k of this lane's chunk within a stage
+#pragma unroll
+  for (int j = 0; j < HI; ++j) {
+    const int piece = wid + 8 * j, row = (piece < 4 * NT ? piece : piece - 4 * NT) * 4 + g;
+    col[j] = (r ^ (row & 15)) * 8;
+    if (piece < 4 * NT) off[j] = n0 + row < p.N ? (uint32_t)(((long)(n0 + row) * p.K + col[j]) * 2) : kOob;
+    else off[j] = row < p.M ? (uint32_t)(((long)row * p.lda + col[j]) * 2) : kOob;
+  }
+  auto stage = [&](int buf, int s) {          // step s of this workgroup; past its end: zeros
+    const int k = (first + s) * KS;
+#pragma unroll
+    for (int j = 0; j < HI; ++j) {
+      const int piece = wid + 8 * j;
+      if (j < LO || piece < PIECES) {
+        const uint32_t o = s < steps && k + col[j] < p.K ? off[j] + (uint32_t)(k * 2) : kOob;
+        dma16(piece < 4 * NT ? rw : ra, lds + buf * STAGE + piece * 512, o);
+      }
+    }
+  };
+  float4_ acc[NT][MH];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MH; ++j) acc[i][j] = float4_{0.f, 0.f, 0.f, 0.f};
+  auto frag = [&](const bf16_t* base, int block) {
+    return *reinterpret_cast<const bf16x8*>(base + (block * 16 + r) * KS + (((kg * 4 + g) ^ r) * 8));
+  };
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s) stage(s, s);
+  int buf = 0;
+  for (int s = 0; s < steps; ++s) {
+    if (wid < PIECES % 8) wait_vm<(S - 2) * HI>();
+    else wait_vm<(S - 2) * LO>();
+    __builtin_amdgcn_s_barrier();             // every wave's part of the step is there, and the buffer before it has been read
+    stage(buf == 0 ? S - 1 : buf - 1, s + S - 1);
+    const bf16_t *w = lds + buf * STAGE, *a = w + NT * 16 * KS;
+    bf16x8 fw[NT], fa[MH];
+#pragma unroll
+    for (int j = 0; j < MH; ++j) fa[j] = frag(a, mh * MH + j);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) fw[i] = frag(w, i);
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MH; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[i], fa[j], acc[i][j], 0, 0, 0);
+    buf = buf == S - 1 ? 0 : buf + 1;
+  }
+  wait_vm<0>();
+  __syncthreads();
+  static_assert(4 * NT * MT * 1024 <= S * STAGE * 2, "partial sums larger than the ring");
+  float4_* red = reinterpret_cast<float4_*>(lds);  // [k-group][block][lane]
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MH; ++j) red[((kg * NT + i) * MT + mh * MH + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  for (int t = wid; t < NT * MT; t += 8) {
+    float4_ c = red[t * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) c += red[(q * NT * MT + t) * 64 + lane];
+    const int m = t % MT * 16 + r;
+    if (m < p.M) store_cols<O, EC>(p, C, m, n0 + t / MT * 16 + 4 * g, c);
+  }
+}
+
+template <typename O, int EC, int MT>
+void launch_blocks(const GemmArgs& a, int nt, hipStream_t s) {
+  auto go = [&](auto kernel, int NT) {
+    const size_t bytes = (size_t)ring_stages(MT, NT) * (MT + NT) * 16 * KS * 2;
+    kernel<<<dim3((a.N + 16 * NT - 1) / (16 * NT), a.splits > 1 ? a.splits : 1), 512, bytes, s>>>(a);
+  };
+  switch (nt) {
+    case 2: go(gemm_ring_kernel<O, EC, MT, 2>, 2); break;
+    case 3: go(gemm_ring_kernel<O, EC, MT, 3>, 3); break;
+    case 4: go(gemm_ring_kernel<O, EC, MT, 4>, 4); break;
+    case 5: go(gemm_ring_kernel<O, EC, MT, 5>, 5); break;
+    case 6: go(gemm_ring_kernel<O, EC, MT, 6>, 6); break;
+    default: go(gemm_ring_kernel<O, EC, MT, 8>, 8); break;
+  }
+  SHAI_CHECK_LAUNCH();
+}
+
+}  // namespace
+
+// Columns of a workgroup, in blocks of 16: one workgroup per CU, or as few rounds of them as 128 columns allow.  Up to 32 rows a
+// stage is short, and beyond one round of 112 columns two workgroups of 48 per CU, each other's prologue and end hidden, are
+// faster (50176 x 4096, 32 rows: 91 us; one of 128: 95; 32768 x 2048: 32.9 and 34.1).
+static int ring_blocks(const GemmArgs& a) {
+  const long cols = (long)a.N * (a.splits > 1 ? a.splits : 1), rounds = (cols + 256 * 128 - 1) / (256 * 128);
+  if (a.M <= 32 && cols > 256 * 112) return 3;
+  const int nt = (int)((cols + 256 * 16 * rounds - 1) / (256 * 16 * rounds));
+  return nt < 2 ? 2 : nt > 6 ? 8 : nt;
+}
+
+// From 9 rows on (partial sums: from one).  Below, the streaming kernel's 16-column workgroups read their few rows of A from as
+// few cache lines and start faster: 17424 x 2048 takes 16.0 us (here 18.4) on one row, 18.7 (18.1) on 8, 21.6 (17.5) on 16.
+// Products per head, grouped by expert or longer than a buffer's range stay there.
+bool gemm_ring_fits(const GemmArgs& a) {
+  const long lim = 0x7fffffffL;
+  return !a.tiles && a.batch <= 1 && a.M <= 64 && (a.M > 8 || a.splits > 1) && a.K >= 512 && a.N >= 512 &&
+         (long)a.N * a.K * 2 < lim && (long)a.M * a.lda * 2 < lim;
+}
+
+void launch_gemm_ring(const GemmArgs& a, hipStream_t s) {
+  const int nt = ring_blocks(a), ec = epi_class(a.epi);
+  auto rows = [&](auto o, auto c) {
+    using O = decltype(o);
+    if (a.M <= 32) launch_blocks<O, decltype(c)::value, 2>(a, nt, s);
+    else launch_blocks<O, decltype(c)::value, 4>(a, nt, s);
+  };
+#define CLASS(EC_) std::integral_constant<int, EC_>()
+  if (a.out_f32 && ec == EC_PLAIN) rows(float(), CLASS(EC_PLAIN));
+  else if (a.out_f32) rows(float(), CLASS(EC_ANY));
+  else if (ec == EC_PLAIN) rows(bf16_t(), CLASS(EC_PLAIN));
+  else if (ec == EC_CLAMP) rows(bf16_t(), CLASS(EC_CLAMP));
+  else if (ec == EC_GELU) rows(bf16_t(), CLASS(EC_GELU));
+  else rows(bf16_t(), CLASS(EC_OTHER));
+#undef CLASS
+}
+
+}  // namespace shai_lm

@@ -137,6 +137,8 @@ struct GemmArgs {
   int table_rows;
   bool table_f32;
 };
+bool gemm_ring_fits(const GemmArgs& a);                                // bf16 products of few rows through a ring in LDS
+void launch_gemm_ring(const GemmArgs& a, hipStream_t s);
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t s);          // streaming kernel, any M
 void launch_gemm_tile(const GemmArgs& a, hipStream_t s);               // LDS-tiled bf16 kernel (gemm_tile.hip)
 

@@ -152,7 +152,14 @@ __global__ void __launch_bounds__(NT, conv_waves(TAPS, NT, NV)) residual_norm_ke
               s += p.wts[row * p.top + k] * load4(static_cast<const T*>(p.ye) + (long)p.slot_of[row * p.top + k] * p.Dp + c);
             q.d[i] = s;
           }
-          for (int k = 1; k < p.parts; k += 3) {           // three loads at a time, none of them waited for alone
+          for (int k = 1; p.parts > 4 && k < p.parts; k += 7) {   // 8 parts: seven loads at a time, none waited for alone
+            float4_ e[7];
+#pragma unroll
+            for (int j = 0; j < 7; ++j) e[j] = raw4(d + min(k + j, p.parts - 1) * p.part_stride + c);
+#pragma unroll
+            for (int j = 0; j < 7; ++j) q.d[i] += k + j < p.parts ? e[j] : zero;
+          }
+          for (int k = 1; p.parts <= 4 && k < p.parts; k += 3) {
             float4_ e[3];
 #pragma unroll
             for (int j = 0; j < 3; ++j) e[j] = raw4(d + min(k + j, p.parts - 1) * p.part_stride + c);
