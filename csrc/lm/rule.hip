@@ -46,7 +46,14 @@ __device__ __forceinline__ float gate_act(float z, int kind) {
 // ------------------------------------------------------------------------------------------------ row by row
 // Thread: 4 columns x DK / RG rows of S.  S^T k and S^T q are taken from the decayed state in one pass: with kq = k . q,
 // o = S^T q + kq u.
-template <typename T, int MODE, int DK, int DV, int NT>
+//
+// Decode: every workgroup of a step is resident at once, so whatever stands between the state's arrival and its way back is time
+// in which memory idles.  A wave's loads return in order; everything small is therefore loaded first, without branches (the
+// convolution's taps one after the other, each waited for, cost 10 us of a step), and the state after it: convolutions, norms and
+// decays are done when it arrives.  64 sequences x 16 heads of 128 x 128 (134 MB of state),
+// us: decay per head 37.6 -> 34.8, per channel 39.8 -> 35.1, retention 28.7 (the rate of a large copy: 27); one sequence 7.1 -> 6.6 and
+// 7.6 -> 6.8.  The one row of a step is compiled apart from prompts': 126 registers instead of 168, four workgroups per CU.
+template <typename T, int MODE, int DK, int DV, int NT, bool STEP>   // STEP: decode of the delta rule
 __global__ void __launch_bounds__(NT, NT > 256 ? 4 : 3) rule_rows_kernel(const RuleArgs p) {
   constexpr bool DELTA = MODE != kRetention;
   constexpr int NC = DV / 4, RG = NT / NC, R = DK / RG, NW = NT / 64, KW = DK / 64;
@@ -56,40 +63,91 @@ __global__ void __launch_bounds__(NT, NT > 256 ? 4 : 3) rule_rows_kernel(const R
   __shared__ float red[NW], skq[NW], rout[NW];
   const int tid = threadIdx.x, h = blockIdx.x, b = blockIdx.y;
   const int c = (tid % NC) * 4, r0 = (tid / NC) * R;
-  const int n = p.q_lens ? p.q_lens[b] : 1;
+  const int n = !STEP && p.q_lens ? p.q_lens[b] : 1;
   if (n < 1) return;
-  const long t0 = p.q_start ? p.q_start[b] : b;
+  const long t0 = !STEP && p.q_start ? p.q_start[b] : b;
   const int slot = p.slots[b], pos0 = p.pos[t0];
   const int g = h / (p.H / p.G), channels = 2 * p.G * DK + p.H * DV;
   float* st = p.state + (((long)max(slot, 0) * p.H + h) * DK + r0) * DV + c;
   const bool old = slot >= 0 && pos0 > 0;
-  float4_ S[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) S[i] = old ? load4(st + (long)i * DV) : float4_{0.f, 0.f, 0.f, 0.f};
   const T* x = static_cast<const T*>(p.x);
   T* ring = DELTA ? static_cast<T*>(p.ring) + (long)max(slot, 0) * p.taps * channels : nullptr;
   const int ring0 = DELTA ? pos0 % p.taps : 0;
+  // The newest inputs of a channel and their taps; the others are added by `conv`
+  constexpr int NEAR = 4;
+  struct Near {
+    T x[NEAR];
+    float w[NEAR];
+  };
+  auto source = [&](long t, int ch, int j, bool& valid) {    // input j rows before row t
+    const int row = STEP ? 0 : (int)(t - t0), m = ring0 + row - j;      // before the step's first row: its place in the ring
+    const bool here = row >= j;
+    valid = j < p.taps && (here || (pos0 + row >= j && slot >= 0));
+    return here || !valid ? x + (valid ? t - j : t) * p.ldx + ch : ring + (m < 0 ? m + p.taps : m) * channels + ch;
+  };
+  auto near = [&](long t, int ch) {
+    Near a;
+#pragma unroll
+    for (int j = 0; j < NEAR; ++j) {
+      bool valid;
+      a.x[j] = *source(t, ch, j, valid);
+      a.w[j] = p.conv[max(p.taps - 1 - j, 0) * channels + ch];
+    }
+    return a;
+  };
   // channel ch of row t after its convolution and silu
-  auto conv = [&](long t, int ch) {
-    const int row = (int)(t - t0);
-    float y = p.conv[(p.taps - 1) * channels + ch] * load1(x + t * p.ldx + ch);
-#pragma unroll 3
-    for (int j = 1; j < p.taps; ++j) {
-      const int m = ring0 + row - j;                         // before the step's first row: its place in the ring
-      const bool here = row >= j;
-      const T* src = here ? x + (t - j) * p.ldx + ch : ring + (m < 0 ? m + p.taps : m) * channels + ch;
-      if (here || (pos0 + row >= j && slot >= 0)) y += p.conv[(p.taps - 1 - j) * channels + ch] * load1(src);
+  auto conv = [&](long t, int ch, const Near& a) {
+    float y = a.w[0] * load1(&a.x[0]);
+#pragma unroll
+    for (int j = 1; j < NEAR; ++j) {
+      bool valid;
+      source(t, ch, j, valid);
+      if (valid) y += a.w[j] * load1(&a.x[j]);
+    }
+    for (int j = NEAR; j < p.taps; ++j) {
+      bool valid;
+      const T* src = source(t, ch, j, valid);
+      if (valid) y += p.conv[(p.taps - 1 - j) * channels + ch] * load1(src);
     }
     return silu_exact(y);
   };
+  const bool key = tid >= DK;
+  const int my_d = key ? tid - DK : tid, my_ch = (key ? p.G + g : g) * DK + my_d;   // delta rule: this thread's q or k channel
+  const int v_ch = 2 * p.G * DK + h * DV + tid;
+  struct Small {             // what a row needs besides the state
+    Near qk, v;
+    float decay, bias, beta;
+    T gate;
+  };
+  auto small = [&](long t) {
+    Small s{};
+    if constexpr (DELTA) {
+      if (tid < 2 * DK) s.qk = near(t, my_ch);
+      if (tid < DV) s.v = near(t, v_ch);
+      s.beta = p.beta[t * p.ldb + h];
+      const int d = MODE == kChannel ? h * DK + min(tid, DK - 1) : h;
+      s.decay = p.decay[t * p.ldd + d];
+      s.bias = p.bias[d];
+    }
+    if (tid < DV) s.gate = static_cast<const T*>(p.gate)[t * p.ldg + h * DV + tid];
+    return s;
+  };
+  Small in{};
+  if constexpr (STEP) in = small(t0);
+  const float rate = p.rate[h];
+  __builtin_amdgcn_sched_barrier(0);
+  float4_ S[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) S[i] = old ? load4(st + (long)i * DV) : float4_{0.f, 0.f, 0.f, 0.f};
+  __builtin_amdgcn_sched_barrier(0);
   for (long t = t0; t < t0 + n; ++t) {
     const T* row = x + t * p.ldx;
+    if constexpr (!STEP) in = small(t);
     float mine = 0.f;
     if (tid < 2 * DK) {
-      const bool key = tid >= DK;
-      const int d = key ? tid - DK : tid, first = DELTA ? (key ? p.G + g : g) * DK : (key ? p.H + h : h) * DK;
+      const int d = my_d, first = DELTA ? my_ch - my_d : (key ? p.H + h : h) * DK;
       if constexpr (DELTA) {
-        mine = conv(t, first + d);
+        mine = conv(t, my_ch, in.qk);
       } else {
         mine = load1(row + first + d);
         if (d < p.rot) {
@@ -107,15 +165,12 @@ __global__ void __launch_bounds__(NT, NT > 256 ? 4 : 3) rule_rows_kernel(const R
       if ((tid & 63) == 0) red[tid >> 6] = ss;
     }
     const int v0 = (DELTA ? 2 * p.G * DK : 2 * p.H * DK) + h * DV;
-    if (tid < DV) sv[tid] = DELTA ? conv(t, v0 + tid) : load1(row + v0 + tid);
+    if (tid < DV) sv[tid] = DELTA ? conv(t, v_ch, in.v) : load1(row + v0 + tid);
     if constexpr (MODE == kChannel) {
-      if (tid < DK) {
-        const int d = h * DK + tid;
-        sg[tid] = expf(-p.rate[h] * softplus_exact(p.decay[t * p.ldd + d] + p.bias[d]));
-      }
+      if (tid < DK) sg[tid] = expf(-rate * softplus_exact(in.decay + in.bias));
     }
     __syncthreads();
-    float rq = 1.f, rk = 1.f, gh = MODE == kRetention ? p.rate[h] : 1.f, beta = 1.f;
+    float rq = 1.f, rk = 1.f, gh = MODE == kRetention ? rate : 1.f, beta = 1.f;
     if constexpr (DELTA) {
       float s0 = 0.f, s1 = 0.f;
 #pragma unroll
@@ -125,8 +180,8 @@ __global__ void __launch_bounds__(NT, NT > 256 ? 4 : 3) rule_rows_kernel(const R
       }
       rq = 1.f / sqrtf(s0 + 1e-6f) * (1.f / sqrtf((float)p.dim));
       rk = 1.f / sqrtf(s1 + 1e-6f);
-      beta = sigmoid_f(p.beta[t * p.ldb + h]);
-      if constexpr (MODE == kHead) gh = expf(-p.rate[h] * softplus_exact(p.decay[t * p.ldd + h] + p.bias[h]));
+      beta = sigmoid_f(in.beta);
+      if constexpr (MODE == kHead) gh = expf(-rate * softplus_exact(in.decay + in.bias));
     } else {
       rk = 1.f / sqrtf((float)p.dim);
     }
@@ -199,7 +254,7 @@ __global__ void __launch_bounds__(NT, NT > 256 ? 4 : 3) rule_rows_kernel(const R
       float sum = 0.f;
 #pragma unroll
       for (int w = 0; w < DV / 64; ++w) sum += rout[w];
-      const float z = load1(static_cast<const T*>(p.gate) + t * p.ldg + h * DV + tid);
+      const float z = load1(&in.gate);
       const float r = 1.f / sqrtf(sum / (float)p.vdim + p.eps);
       store1(static_cast<T*>(p.out) + t * p.ldo + h * DV + tid, y * r * (DELTA ? p.gain[tid] : 1.f) * gate_act<false>(z, p.gate_kind));
     }
@@ -1199,7 +1254,13 @@ void launch_rule_chunks(const RuleArgs& a, hipStream_t s) {
 template <typename T, int MODE, int DK, int DV>
 static void rows(const RuleArgs& a, hipStream_t s) {
   constexpr int NT = DK > 128 ? 1024 : 256;
-  rule_rows_kernel<T, MODE, DK, DV, NT><<<dim3(a.H, a.B), NT, 0, s>>>(a);
+  if constexpr (MODE != kRetention) {       // (whose few loads are faster behind the state's: 28.7 and 29.8 us)
+    if (!a.q_lens) {
+      rule_rows_kernel<T, MODE, DK, DV, NT, true><<<dim3(a.H, a.B), NT, 0, s>>>(a);
+      return;
+    }
+  }
+  rule_rows_kernel<T, MODE, DK, DV, NT, false><<<dim3(a.H, a.B), NT, 0, s>>>(a);
 }
 
 template <typename T>
