@@ -435,7 +435,7 @@ class LLMEngine:
         cache through 1-2 workgroups per head).  Powers of two: each value is one captured graph."""
         span = self.model.attn_span or self.max_model_len
         max_ctx = min(max_ctx, span)
-        base = ops.decode_splits(Bc, self.model.kv_heads_local, min(self.max_model_len, span))
+        base = ops.decode_splits(Bc, self.model.kv_heads_local, min(self.max_model_len, span), *self.model.split_blocks)
         per = int(os.environ.get("SHAI_DECODE_SPLIT_TOKENS", "1024"))
         need = 1
         while need < 64 and need * per < max_ctx:

@@ -128,6 +128,7 @@ class FaledraForCausalLM(nn.Module):
     needs_prev_token = False
     has_state = True             # sequences hold a state slot (allocate_state); their prefixes cannot be shared by blocks
     attn_span: Optional[int] = None
+    split_blocks = (1, 0)
     dtypes = (torch.bfloat16, torch.float32)
 
     def __init__(self, cfg: FaledraConfig, dtype=torch.bfloat16):

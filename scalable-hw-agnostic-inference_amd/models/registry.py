@@ -2,7 +2,8 @@
 
 A model class offers the engine: ``forward(batch, kv_caches)`` -> logits, ``kv_heads_local``, ``fold_norms()``,
 ``allocate_cache(blocks, device)``, ``cache_bytes_per_block()``, and the attributes ``dtypes`` (weight formats it runs
-in), ``needs_prev_token`` (rows carry their preceding token), ``attn_span`` (most keys a position sees, or None) and
+in), ``needs_prev_token`` (rows carry their preceding token), ``attn_span`` (most keys a position sees, or None),
+``split_blocks`` (how decode attention is split, the last arguments of :func:`ops.decode_splits`) and
 ``has_state`` (sequences hold a slot of the state that ``allocate_state(slots, device)`` makes; ``Batch.states``).
 """
 from __future__ import annotations

@@ -302,3 +302,12 @@ def test_no_garbage_collection_during_a_capture(monkeypatch):
         assert gc.isenabled()
     finally:
         gc.set_threshold(*old)
+
+
+@pytest.mark.parametrize("batch,hkv,ctx,blocks,whole,want", [
+    (1, 8, 64, 1, 0, 1), (1, 8, 65, 1, 0, 2), (1, 8, 4096, 1, 0, 64), (64, 8, 4096, 1, 0, 1),      # a split per block
+    (1, 8, 512, 1, 8, 1), (1, 8, 513, 1, 8, 9), (16, 8, 512, 1, 8, 1), (16, 8, 513, 1, 8, 4),      # short contexts whole
+    (1, 4, 256, 4, 0, 1), (1, 4, 257, 4, 0, 2), (1, 4, 4096, 4, 0, 16), (64, 4, 4096, 4, 0, 2)])   # four blocks per split
+def test_decode_splits(batch, hkv, ctx, blocks, whole, want):
+    from shai_amd import ops
+    assert ops.decode_splits(batch, hkv, ctx, blocks, whole) == want
