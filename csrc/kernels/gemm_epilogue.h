@@ -101,4 +101,71 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& p, bf16_t* C, const bf
   }
 }
 
+// Whether rows and bases of everything epilogue8 touches are aligned for its accesses: 16 bytes, or 8 for the output side of a GLU.
+template <bool GLU>
+__device__ __forceinline__ bool epilogue8_aligned(const GemmArgs& p, const bf16_t* C, const bf16_t* R) {
+  constexpr int OUT = GLU ? 4 : 8;  // columns stored per call
+  long rows = p.ldc;
+  uintptr_t out = (uintptr_t)C, in = (uintptr_t)p.bias | (uintptr_t)p.bias2d;
+  if (R) rows |= p.ldr, out |= (uintptr_t)R;
+  if (p.gate) rows |= p.gate_stride, out |= (uintptr_t)p.gate;
+  return (rows & (OUT - 1)) == 0 && (out & (2 * OUT - 1)) == 0 && (in & 15) == 0 && (!p.bias2d || (p.N & 7) == 0);
+}
+
+template <int V>
+__device__ __forceinline__ void load_bf(const bf16_t* src, float (&x)[V]) {
+  if constexpr (V == 8) {
+    const uint4_ t = *reinterpret_cast<const uint4_*>(src);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = bf2f(e & 1 ? t[e >> 1] >> 16 : t[e >> 1] & 0xffff);
+  } else {
+    const uint2_ t = *reinterpret_cast<const uint2_*>(src);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = bf2f(e & 1 ? t[e >> 1] >> 16 : t[e >> 1] & 0xffff);
+  }
+}
+
+// epilogue4 for the 8 consecutive columns n .. n + 7 of row m, all below N, with epilogue8_aligned true: the same operations in
+// the same order, one 16-byte access (8 bytes on the output side of a GLU) instead of two.
+template <bool GLU, int ACT>
+__device__ __forceinline__ void epilogue8(const GemmArgs& p, bf16_t* C, const bf16_t* R, int m, int n, float (&v)[8], int b) {
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] *= p.alpha;
+  if (p.bias) {
+    load_bf<8>(p.bias + n, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += x[e];
+  }
+  if (p.bias2d) {
+    load_bf<8>(p.bias2d + (long)(m / p.rows_per_bias2d) * p.N + n, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += x[e];
+  }
+  constexpr int OUT = GLU ? 4 : 8;
+  const int nc = GLU ? n >> 1 : n;
+  float o[OUT], y[OUT];
+#pragma unroll
+  for (int e = 0; e < OUT; ++e) {
+    if constexpr (GLU) o[e] = v[2 * e] * apply_act<ACT>(v[2 * e + 1]);
+    else o[e] = apply_act<ACT>(v[e]);
+  }
+  if (p.gate) {
+    load_bf<OUT>(p.gate + ((long)b * p.M + m) / p.rows_per_gate * p.gate_stride + nc, y);
+#pragma unroll
+    for (int e = 0; e < OUT; ++e) o[e] *= y[e];
+  }
+  if (R) {
+    load_bf<OUT>(R + (long)m * p.ldr + nc, y);
+#pragma unroll
+    for (int e = 0; e < OUT; ++e) o[e] += y[e] * p.res_alpha;
+  }
+  if constexpr (GLU) {
+    *reinterpret_cast<uint2_*>(C + (long)m * p.ldc + nc) = uint2_{pack2(o[0], o[1]), pack2(o[2], o[3])};
+  } else {
+    *reinterpret_cast<uint4_*>(C + (long)m * p.ldc + nc) =
+        uint4_{pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7])};
+  }
+}
+
 }  // namespace shai

@@ -181,6 +181,12 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
 
   const int nk = k_end > k_begin ? (k_end - k_begin + BK2 - 1) / BK2 : 0;
   const int fr = lane & 31, fh = lane >> 5;
+  // W's fragment rows: in order where fp32 partials are stored (4 columns are 16 bytes); else with bits 2 and 3 of the row
+  // exchanged, so that a lane's register groups 2h and 2h + 1 are the 8 consecutive columns 16h + 8fh of the 32 and one 16-byte
+  // store takes them.  8-byte stores, 32 rows by 16 bytes an instruction, were most of a short K's time: 6304 x 3072, K = 64
+  // 21.5 -> 14.7 us at the 128 x 64 tile, K = 768 53.4 -> 48.4 (128 x 128: 51.2 -> 44.3), 8192 x 960, K = 320 14.5 -> 12.2,
+  // 6304 x 768, K = 768 17.8 -> 15.7.  (Whole lines by way of LDS: 1 .. 3 % more, not worth the second path.)
+  const int fw = SPLITK ? fr : (fr & 19) | (fr & 4) << 1 | (fr & 8) >> 1;
   auto compute = [&](int buf) {
     const bf16_t* sa = smem + buf * STAGE;
     const bf16_t* sw = sa + BM * BK2;
@@ -191,7 +197,7 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
 #pragma unroll
       for (int i = 0; i < IM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(sa + swz2(wm * TM + i * 32 + fr, 2 * s + fh));
 #pragma unroll
-      for (int j = 0; j < JN; ++j) wf[j] = *reinterpret_cast<const bf16x8*>(sw + swz2(wn * TN + j * 32 + fr, 2 * s + fh));
+      for (int j = 0; j < JN; ++j) wf[j] = *reinterpret_cast<const bf16x8*>(sw + swz2(wn * TN + j * 32 + fw, 2 * s + fh));
 #pragma unroll
       for (int i = 0; i < IM; ++i)
 #pragma unroll
@@ -234,7 +240,7 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
-  // ---- epilogue: lane owns row m, 4 groups of 4 consecutive n per 32x32 block.  WK > 1: the wave groups' sums meet in LDS
+  // ---- epilogue: lane owns row m, 4 groups of 4 consecutive n per 32x32 block (without split-K two of 8).  WK > 1: the wave groups' sums meet in LDS
   // (the ring is free by now) and are added in group order; each group finishes 4 / WK of the four column groups.
   if constexpr (WK > 1) {
     static_assert(NW * IM * JN * 4096 <= STAGES * STAGE * 2, "partial tiles larger than the ring");
@@ -263,6 +269,7 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
       }
   }
   constexpr int G1 = 4 / WK;
+  static_assert(G1 >= 2, "a lane's two column groups lie in one wave group");
   const int g0 = wk * G1;
   // In-launch split-K fixup (tiles with <= 4 32x32 blocks per wave; the skinny kernel's write-through hand-off, gemv.hip): every K group
   // stores its fp32 partial tile write-through (sc1), drains, joins the barrier and takes a ticket; the group
@@ -396,6 +403,7 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
   } else {
     bf16_t* C = p.C + (long)b * p.batch_c;
     const bf16_t* R = p.residual ? p.residual + (long)b * p.batch_r : nullptr;
+    const bool wide = epilogue8_aligned<GLU>(p, C, R);
 #pragma unroll
     for (int i = 0; i < IM; ++i) {
       const int m = m0 + wm * TM + i * 32 + fr;
@@ -403,11 +411,18 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
 #pragma unroll
       for (int j = 0; j < JN; ++j)
 #pragma unroll
-        for (int g = 0; g < G1; ++g) {
-          const int n = n0 + wn * TN + j * 32 + 8 * (g0 + g) + 4 * fh;
-          if (n >= p.N) continue;
-          float v[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-          epilogue4<GLU, ACT>(p, C, R, m, n, v, b);
+        for (int h = 0; h < G1 / 2; ++h) {
+          const int n = n0 + wn * TN + j * 32 + 16 * (g0 / 2 + h) + 8 * fh;
+          float v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = acc[i][j][8 * h + e];
+          if (wide && n + 7 < p.N) {
+            epilogue8<GLU, ACT>(p, C, R, m, n, v, b);
+          } else {
+#pragma unroll
+            for (int q = 0; q < 8; q += 4)
+              if (n + q < p.N) epilogue4<GLU, ACT>(p, C, R, m, n + q, v + q, b);
+          }
         }
     }
   }

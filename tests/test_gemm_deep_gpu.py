@@ -70,6 +70,25 @@ def test_batched_strided(cuda, cfg):
     assert _rel(j[:, 10:], a.float() @ w.float().t()) < TOL and j[:, :10].abs().sum().item() == 0
 
 
+# widths where a lane's 8 columns are whole, cut by 4 or by single ones, and rows whose stride allows 16-byte, 8-byte or 2-byte
+# accesses only: columns beside the output stay as they were
+@pytest.mark.parametrize("N,ld,glu", [(128, 136, False), (132, 136, False), (132, 132, False), (72, 76, False), (70, 72, False),
+                                      (330, 338, False), (128, 136, True), (132, 68, True), (140, 74, True), (68, 34, True)])
+@pytest.mark.parametrize("cfg", [3, 4] + CFGS)
+def test_epilogue_widths(cuda, cfg, N, ld, glu):
+    M, K, n = 131, 128, N // (2 if glu else 1)
+    a, w, b, _ = _problem(M, N, K, cuda)
+    r = torch.randn(M, ld, device=cuda).bfloat16()[:, :n]
+    gate = torch.randn(3, ld, device=cuda).bfloat16()[:, :n]
+    per_image = torch.randn(2, N, device=cuda).bfloat16()
+    out = torch.full((M, ld), 7.0, device=cuda, dtype=torch.bfloat16)
+    ops._K().gemm(a, w, out[:, :n], b, per_image, 100, r, 0.5, 2.0, ops.act_id("silu"), glu, gate, 50, cfg)
+    y = 0.5 * (a.float() @ w.float().t()) + b.float() + per_image.float().repeat_interleave(100, 0)[:M]
+    y = y[:, 0::2] * torch.nn.functional.silu(y[:, 1::2]) if glu else torch.nn.functional.silu(y)
+    assert _rel(out[:, :n], y * gate.float().repeat_interleave(50, 0)[:M] + 2.0 * r.float()) < TOL
+    assert bool((out[:, n:] == 7).all())
+
+
 CONV_SCRIPT = r"""
 import sys, torch
 sys.path.insert(0, {root!r})
