@@ -83,7 +83,7 @@ std::string gemm_key(const shai::GemmArgs& g) {
            g.Nimg, g.H, g.Wd, g.Cin, g.Cin1, g.KH, g.stride, g.upsample, g.A2 != nullptr);
   // library-eligible problems (plain GEMM, bias at most) race hipBLASLt in the tuner, so their winner must
   // not be reused by a same-shape problem with a fused epilogue (and vice versa): separate key class
-  // a folded-LayerNorm GEMM (row_mr) runs only unsplit on v4: it tunes and caches apart from the plain problem
+  // a folded-LayerNorm GEMM (row_mr) runs only unsplit: it tunes and caches apart from the plain problem
   return std::string(buf) + (g.rms ? "|rms" : "") + (g.w_scale ? "|fp8w" : "") + (g.row_mr ? "|ln" : "") +
          (g.w_slice_rows ? "|wslice" + std::to_string(g.w_slice_rows) : "") +
          (lib_supported(g) && !g.residual ? "|lib" : "");
@@ -166,7 +166,7 @@ bool lib_enabled() {  // off by default: every GEMM runs on the hand-written ker
 
 int max_splits_for(const shai::GemmArgs& g) {
   const int batch = g.batch > 0 ? g.batch : 1;
-  if (batch != 1 || g.row_mr != nullptr) return 1;  // folded LayerNorm: applied by the unsplit v4 epilogue only
+  if (batch != 1 || g.row_mr != nullptr) return 1;  // folded LayerNorm: applied by unsplit epilogues only
   const long kt = (g.K + 63) / 64;
   int s = 1;
   while (s < 16 && kt / (s * 2) >= 4) s *= 2;
@@ -187,8 +187,8 @@ inline bool is_skinny(int cfg) { return cfg == kSkinnyCfg || cfg == kSkinnyFixCf
 
 // Last resort when neither the tuner nor the planner produced a usable config: an explicit, directly tested
 // config, never "whichever kernel happens to be numbered highest".  The v2 128x64 tile (cfg 4) runs every
-// problem the v2 kernel accepts; folded-LayerNorm problems (row_mr) are applied only by the v4 epilogue
-// (cfg 9 / 10, 256 x 256 / 256 x 320).  tests/test_gemm3_gpu.py forces each of these.
+// problem the v2 kernel accepts; convolutions with a folded LayerNorm (row_mr) only v4 (cfg 9 / 10,
+// 256 x 256 / 256 x 320).  tests/test_gemm3_gpu.py forces each of these.
 Choice fallback_choice(const shai::GemmArgs& g) {
   for (int c : {4, 9, 10})
     if (shai::gemm2_cfg_supported(g, c)) return Choice{c, 1};

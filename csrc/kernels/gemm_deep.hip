@@ -80,7 +80,8 @@ void launch_which(const GemmArgs& a, int which, float* ws, int splits, hipStream
 }  // namespace
 
 bool gemm_deep_supported(const GemmArgs& a) {
-  if (a.rms || a.w_scale || a.row_mr || a.w_slice_rows || a.in_scale || a.upsample == 2) return false;
+  if (a.rms || a.w_scale || a.w_slice_rows || a.in_scale || a.upsample == 2) return false;
+  if (a.row_mr && (a.conv || a.batch > 1)) return false;
   // a convolution's K-tile lies in one filter tap and one source
   return !a.conv || (a.Cin % 64 == 0 && (a.A2 == nullptr || a.Cin1 % 64 == 0));
 }

@@ -408,6 +408,10 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
     for (int i = 0; i < IM; ++i) {
       const int m = m0 + wm * TM + i * 32 + fr;
       if (m >= p.M) continue;
+      float2 mr = make_float2(0.f, 1.f);
+      if constexpr (!CONV) {
+        if (p.row_mr != nullptr) mr = *reinterpret_cast<const float2*>(p.row_mr + 2 * (long)m);
+      }
 #pragma unroll
       for (int j = 0; j < JN; ++j)
 #pragma unroll
@@ -416,6 +420,23 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
           float v[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = acc[i][j][8 * h + e];
+          if constexpr (!CONV) {
+            if (p.row_mr != nullptr) {  // LayerNorm of A folded in: rstd[m] * (acc - mean[m] * s[n]), W carries the gain
+              float s[8];
+              if (n + 7 < p.N) {
+#pragma unroll
+                for (int q = 0; q < 8; q += 4) {
+                  const float4_ t = *reinterpret_cast<const float4_*>(p.col_s + n + q);
+                  s[q] = t[0]; s[q + 1] = t[1]; s[q + 2] = t[2]; s[q + 3] = t[3];
+                }
+              } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s[e] = n + e < p.N ? p.col_s[n + e] : 0.f;
+              }
+#pragma unroll
+              for (int e = 0; e < 8; ++e) v[e] = mr.y * fmaf(-mr.x, s[e], v[e]);
+            }
+          }
           if (wide && n + 7 < p.N) {
             epilogue8<GLU, ACT>(p, C, R, m, n, v, b);
           } else {

@@ -89,6 +89,20 @@ def test_epilogue_widths(cuda, cfg, N, ld, glu):
     assert bool((out[:, n:] == 7).all())
 
 
+# a folded LayerNorm at a cut row tile, column tails of 4 and fewer; the product of the normalised rows comes out as the
+# difference of two larger terms, in fp32
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (131, 132, 128), (197, 330, 776), (300, 768, 768)])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4] + CFGS)
+def test_folded_layernorm(cuda, cfg, M, N, K):
+    a, w, b, r = _problem(M, N, K, cuda)
+    mean, rstd, s = torch.randn(M, device=cuda), torch.rand(M, device=cuda) + 0.5, w.float().sum(1)
+    out = torch.empty_like(r)
+    ops._K().gemm(a, w, out, b, None, 1, r, 1.0, 1.0, ops.act_id("gelu"), False, None, 1, cfg, -1.0, None,
+                  torch.stack([mean, rstd], 1).contiguous(), s)
+    y = rstd[:, None] * (a.float() @ w.float().t() - mean[:, None] * s) + b.float()
+    assert _rel(out, torch.nn.functional.gelu(y) + r.float()) < TOL
+
+
 CONV_SCRIPT = r"""
 import sys, torch
 sys.path.insert(0, {root!r})
