@@ -26,7 +26,7 @@
 //   unchanged; if any lane's partial row sum of the tile exceeds 2^8 (or is not finite), or a row has no
 //   max yet, the wave takes the exact path for that tile (tile max, O / l rescale, recompute P).  P is
 //   therefore bounded by 2^8 in the fast path (bf16 P, fp32 O / l absorb it), as with v1's deferred max.
-// * Causal masking (with offset), per-batch q / kv lengths, GQA.  Additive bias and paged K/V stay on v1.
+// * Causal masking (with offset), per-batch q / kv lengths, GQA; paged K/V (PAGED).  Additive bias stays on v1.
 #include <cstdlib>
 #include <type_traits>
 
@@ -109,7 +109,7 @@ __device__ __forceinline__ void f2_glds(__amdgpu_buffer_rsrc_t r, bf16_t* lds, u
 // waves 0 and 4 of workgroup (0, 0, 0) at every segment boundary into g_f2_stamps.
 __device__ unsigned long long g_f2_stamps[2][2048];
 
-template <int D, bool CAUSAL, int EXP = 0>
+template <int D, bool CAUSAL, int EXP = 0, bool PAGED = false>
 __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   constexpr int KT = 64;                 // keys per tile
   constexpr int NS = D / 16;             // k-steps of QK^T
@@ -122,13 +122,17 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   // D = 64 (softmax-issue-bound): Q is pre-multiplied by scale * log2(e) and the score accumulators start at
   // -m (the running max they are computed against), so the fast path's exponent is the raw accumulator --
   // one v_exp per score, no v_fma.  Costs one bf16 rounding of the scaled Q (|rel| <= 2^-9 per element).
-  constexpr bool PRE = !(EXP & 16);  // EXP & 16: the unscaled form (A/B: SHAI_FLASH2_PRE=0)
+  constexpr bool PRE = !PAGED && !(EXP & 16);  // EXP & 16: the unscaled form (A/B: SHAI_FLASH2_PRE=0)
   // D = 64 M segment (EXP & 32 restores the previous form for A/B): (a) every LDS fragment read is an immediate
   // offset from one of six per-tile base addresses (was one v_add per read: 29 VALU per tile); (b) the score
   // accumulators start at zero (inline constant) and -m enters through one extra MFMA per 32-key block,
   // A = a ones column, B = -m on the bf16 grid (was 32 v_mov per tile).  VALU issue, not the matrix pipe,
   // bounds this loop at D = 64 (profiles/flash_attn_v2_round2.md), so 2 MFMAs buy back ~60 VALU.
   constexpr bool NEWM = PRE && !(EXP & 32);  // D = 64 and D = 128
+  // Paged K/V: a 64-key tile is one block of the pool, 64 x D contiguous, found through the block table.  Q stays as it is
+  // stored (scores scaled in fp32, one v_fma each), as in the kernel this form took the long prompts from.
+  constexpr bool IMM = NEWM || PAGED;  // fragment reads at immediate offsets
+  static_assert(!PAGED || D == 128, "paged: D = 128");
   static_assert(NPW >= 1 && (2 * NPI) % 8 == 0, "bad D");
   extern __shared__ __attribute__((aligned(16))) bf16_t f2_smem[];
 
@@ -136,12 +140,24 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wid >> 2;
   const int fr = lane & 31, fh = lane >> 5;
-  const int b = blockIdx.z, hq = blockIdx.y;
+  int b = blockIdx.z, hq = blockIdx.y, qb = blockIdx.x;
+  if constexpr (PAGED && CAUSAL) {
+    // The queries of one K/V head go to one XCD (its L2 then reads those K/V once), the longest rows of them first: in launch
+    // order the XCD that gets every eighth block of rows has up to a fifth more work than the mean.
+    const int gx = gridDim.x, grp_q = p.Hq / p.Hkv, total = gx * gridDim.y * gridDim.z;
+    int id = blockIdx.x + gx * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int xcd = id & 7, q = total >> 3, r = total & 7;
+    id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
+    const int per = gx * grp_q, head = id / per, in = id - head * per;
+    qb = gx - 1 - in / grp_q;
+    b = head / p.Hkv;
+    hq = (head - b * p.Hkv) * grp_q + in % grp_q;
+  }
   const int hk = hq / (p.Hq / p.Hkv);
   const int q_len = p.q_lens ? p.q_lens[b] : p.Sq;
   const int kv_len = p.kv_lens ? p.kv_lens[b] : p.Skv;
   const int c_off = p.q_lens ? kv_len - q_len : p.causal_offset;
-  const int q0 = blockIdx.x * 256;
+  const int q0 = qb * 256;
   if (q0 >= q_len) return;  // whole workgroup, before any barrier
   const int qi = q0 + wid * 32 + fr;
 
@@ -184,10 +200,23 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
     const int op = gi / NPI, piece = gi % NPI;
     const int row = piece * RPI + lane / CPR, ch = lane % CPR;
     const int src = op ? f2_vch<D>(row, ch) : f2_kch<D>(row, ch);
-    soff[j] = (uint32_t)(((long)row * (op ? p.v_ts : p.k_ts) + src * 8) * 2);
+    soff[j] = (uint32_t)(((long)row * (PAGED ? (long)D : op ? p.v_ts : p.k_ts) + src * 8) * 2);
   }
-  auto stage = [&](int t) {  // always issued (tiles past the end read as zeros) so vmcnt counts are fixed
+  // PAGED: the pool block of the tile that is staged next, read a segment ahead (0 and no rows past the last tile)
+  const __attribute__((address_space(4))) int* table =
+      PAGED ? (const __attribute__((address_space(4))) int*)(uintptr_t)(p.block_table + (long)b * p.max_blocks) : nullptr;
+  auto block_of = [&](int t) { return PAGED && t < nt ? table[t] : 0; };
+  auto stage = [&](int t, int phys) {  // always issued (tiles past the end read as zeros) so vmcnt counts are fixed
     bf16_t* slot = f2_smem + (t & 3) * TILE;
+    if constexpr (PAGED) {
+      constexpr int W = NPI / NPW;  // waves per operand
+      const bf16_t* base = (wid < W ? p.k : p.v) + (long)phys * p.kc_bs + (long)hk * p.kc_hs;
+      const int rows = t < nt ? min(kv_len - t * KT, KT) : 0;
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), (short)0, rows * D * 2, 0x00020000);
+#pragma unroll
+      for (int j = 0; j < NPW; ++j) f2_glds(r, slot + (wid * NPW + j) * RPI * D, soff[j]);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < NPW; ++j) {
       const int gi = wid * NPW + j;
@@ -351,9 +380,10 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   }
 
   // ---- prologue: tiles 0..2 in flight, 0 and 1 landed; S(0), P(0) by every wave
-  stage(0);
-  stage(1);
-  stage(2);
+  stage(0, block_of(0));
+  stage(1, block_of(1));
+  stage(2, block_of(2));
+  int phys = block_of(3);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NPW) : "memory");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
@@ -379,7 +409,7 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   for (int t = 0; t < nt; ++t) {
     // ---- M segment: S(t+1) = K(t+1) Q^T, O += V(t)^T P(t); DMA of tile t+3
     stamp();
-    stage(t + 3);
+    stage(t + 3, phys);
     s4a vr0[ND][2][2], vr1[ND][2][2];
     if constexpr (NEWM && D == 64) {
       const bool more = t + 1 < nt;
@@ -433,7 +463,7 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // V^T kb1
       __builtin_amdgcn_sched_barrier(0);
       if (!(EXP & 2)) pv_mfma(1, vr1);
-    } else if constexpr (NEWM) {  // D = 128
+    } else if constexpr (IMM) {  // D = 128
       // Same scheme at D = 128 (8 K fragments and 16 transposed V reads per 32-key block): reads issued in
       // consumption order in groups of 8 so that at most 16 are outstanding (lgkmcnt counts to 15), each group
       // waited for by a counted lgkmcnt before the MFMAs that consume it.  Row = 256 B: key block 8192 B,
@@ -459,8 +489,8 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   VR[D_][1][1] = f2_tr_read_o<(KB) * 8192 + 6144>(va[D_]);
 #define F2_QK(KB)                                                                                               \
   if (!(EXP & 2) && more) {                                                                                     \
-    const float16_ z = {};                                                                                      \
-    sacc[KB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_one, b_negm, z, 0, 0, 0);                              \
+    sacc[KB] = float16_{};                                                                                      \
+    if constexpr (NEWM) sacc[KB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_one, b_negm, sacc[KB], 0, 0, 0);   \
     _Pragma("unroll") for (int s2 = 0; s2 < NS; ++s2)                                                           \
       sacc[KB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s2], qf[s2], sacc[KB], 0, 0, 0);                   \
   }
@@ -547,6 +577,7 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
     __builtin_amdgcn_sched_barrier(0);
     // ---- V segment: softmax of S(t+1)
     stamp();
+    phys = block_of(t + 4);
     if (!(EXP & 1) && t + 1 < nt) softmax(t + 1);
     if (grp == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NPW) : "memory");  // tile t+2 landed
     __builtin_amdgcn_sched_barrier(0);
@@ -579,7 +610,11 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
 }
 
 bool flash2_supported(const AttnArgs& a) {
-  if (a.bias != nullptr || a.block_table != nullptr) return false;
+  if (a.bias != nullptr) return false;
+  // Paged K/V (blocks of 64 x D, 16-byte aligned heads), D = 128, from 2048 rows on.  Causal, 32 / 8 heads, us (4-wave kernel
+  // -> this one): 1 x 8000 805 -> 575 (911 TF/s), 1 x 4096 319 -> 162, 1 x 2048 95 -> 72, 1 x 1024 41 -> 40; below, the last
+  // 256 rows' padding costs more than the pipeline gives: 7 x 1100 138 -> 151, 1 x 512 23 -> 26.
+  if (a.block_table != nullptr) return a.D == 128 && a.Sq >= 2048 && ((a.q_ts | a.kc_bs | a.kc_hs) & 7) == 0;
   if (a.D != 64 && a.D != 128) return false;
   if (a.Sq < 512) return false;  // 256-query workgroups; v1's 128-query blocks waste less on short rows
   if (a.Skv < 512) return false;  // a few key tiles: v1 has less per-workgroup setup (cross-attention to 77 tokens)
@@ -594,7 +629,10 @@ bool flash2_supported(const AttnArgs& a) {
 void launch_flash2(const AttnArgs& a, hipStream_t s) {
   dim3 grid((a.Sq + 255) / 256, a.Hq, a.B);
   const size_t lds = (size_t)4 * 2 * 64 * a.D * sizeof(bf16_t);
-  if (a.D == 128) {
+  if (a.block_table != nullptr) {
+    if (a.causal) flash2_kernel<128, true, 0, true><<<grid, 512, lds, s>>>(a);
+    else flash2_kernel<128, false, 0, true><<<grid, 512, lds, s>>>(a);
+  } else if (a.D == 128) {
     if (a.causal) flash2_kernel<128, true><<<grid, 512, lds, s>>>(a);
     else flash2_kernel<128, false><<<grid, 512, lds, s>>>(a);
   } else {

@@ -45,6 +45,43 @@ def test_paged_attention_varlen_kernel(cuda, D):
         assert rel < 2e-2, (b, rel)
 
 
+# the 8-wave kernel over paged K/V: whole and cut 256-row blocks and 64-key tiles, sequences of one row and of none beside the
+# long one, a cached context, head groups of 1 .. 8.  What lies behind a sequence's last key is NaN and must not be read as a value.
+# Tolerance: bf16 results (2^-8 / sqrt(3) rms) and bf16 probabilities (half of that, by the same bound on each).
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,n_cached,n_new", [(8, 2, [0, 70, 0], [2048, 1, 130]), (4, 4, [5, 0, 64], [2049, 0, 255]),
+                                                  (8, 1, [1000], [2111]), (9, 3, [0, 0], [2300, 2048])])
+def test_paged_attention_varlen_long(cuda, Hq, Hkv, n_cached, n_new, causal):
+    torch.manual_seed(1)
+    D, B = 128, len(n_new)
+    per = [(c + n + 63) // 64 for c, n in zip(n_cached, n_new)]
+    kc = torch.randn(sum(per) + 1, Hkv, 64, D, device=cuda).bfloat16()
+    vc = torch.randn_like(kc)
+    order = (torch.randperm(sum(per)) + 1).tolist()
+    bt = torch.zeros(B, max(per) + 1, dtype=torch.int32)
+    for b in range(B):
+        bt[b, :per[b]] = torch.tensor([order.pop() for _ in range(per[b])], dtype=torch.int32)
+        left = (n_cached[b] + n_new[b]) % 64
+        if left:
+            kc[bt[b, per[b] - 1].long(), :, left:] = float("nan")
+            vc[bt[b, per[b] - 1].long(), :, left:] = float("nan")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda)
+    q_start = [sum(n_new[:b]) for b in range(B)]
+    q = torch.randn(sum(n_new), Hq, D, device=cuda).bfloat16()
+    got = ops.paged_attention_varlen(q, kc, vc, bt.to(cuda), i32([c + n for c, n in zip(n_cached, n_new)]), i32(n_new), i32(q_start),
+                                     max(n_new), causal=causal)
+    for b in range(B):
+        n, s0, L = n_new[b], q_start[b], n_cached[b] + n_new[b]
+        rows = bt[b, :per[b]].long().to(cuda)
+        for h in range(Hq):
+            k, v = (c[rows, h // (Hq // Hkv)].reshape(-1, D)[:L].float() for c in (kc, vc))
+            s = q[s0:s0 + n, h].float() @ k.t() / D ** 0.5
+            if causal:
+                s = s.masked_fill(torch.arange(L, device=cuda)[None] > torch.arange(n, device=cuda)[:, None] + L - n, float("-inf"))
+            want = torch.softmax(s, -1) @ v
+            assert not n or ((got[s0:s0 + n, h].float() - want).norm() / want.norm()).item() < 4e-3, (b, h)
+
+
 def test_engine_packed_prefill_matches_padded(cuda):
     from shai_amd.engines.llm import LLMEngine, SamplingParams
     from shai_amd.models.llama import LlamaConfig
