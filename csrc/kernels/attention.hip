@@ -130,6 +130,11 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
   float m_run = -INFINITY, l_run = 0.f;
   const float sl2 = p.scale * kLog2e;
   const bf16_t* bias_row = p.bias ? p.bias + ((long)hq * p.Sq + min(qi, q_len - 1)) * p.Skv : nullptr;
+  // A lane's bias: 8 groups of 4 consecutive keys of its query's row.  One 8-byte load each, issued before the tile's scores, where
+  // rows allow it; 32 loads of 2 bytes and a division per score bounded short sequences (T5, 32 x 128 tokens, 16 heads of 64:
+  // 28.0 -> 16.7 us).
+  const bool bias4 = (p.Skv & 3) == 0 && ((uintptr_t)p.bias & 7) == 0;
+  const float inv_scale = 1.f / p.scale;
 
   if (ntiles > 0) {
     load_tile(0);
@@ -146,6 +151,14 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
     if (t + 1 < ntiles) load_tile(t + 1);
     const bf16_t* ks = sK + cur * KT * D;
     const bf16_t* vs = sV + cur * KT * D;
+    uint2_ bias[8];
+    if (bias_row && bias4) {
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const int key = t * KT + 8 * g + 4 * fh;
+        bias[g] = key < p.Skv ? *reinterpret_cast<const uint2_*>(bias_row + key) : uint2_{0u, 0u};
+      }
+    }
 
     // ---- S^T = K Q^T for two 32-key blocks
     float16_ sacc[2];
@@ -169,7 +182,9 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = key0 + kb * 32 + (r & 3) + 8 * (r >> 2) + 4 * fh;
-          sacc[kb][r] += (key < p.Skv ? bf2f(bias_row[key]) : 0.f) / p.scale;
+          const uint32_t two = bias[4 * kb + (r >> 2)][(r >> 1) & 1];
+          const float x = bias4 ? bf2f(r & 1 ? two >> 16 : two & 0xffff) : key < p.Skv ? bf2f(bias_row[key]) : 0.f;
+          sacc[kb][r] += x * inv_scale;
         }
     }
     if (need_mask) {

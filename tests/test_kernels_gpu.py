@@ -242,6 +242,24 @@ def test_flash_attn_bias(cuda):
     close(ops.attention(q, k, v, scale=1.0, bias=bias), ref.attention(q, k, v, 1.0, bias=bias), 3e-2)
 
 
+# bias rows of 4 keys at a time and, where their stride does not allow that, key by key; cut key tiles, a scale that is not one.
+# Tolerance: bf16 results (2^-8 / sqrt(3) rms) and bf16 probabilities (half of that, by the same bound on each).
+@pytest.mark.parametrize("Sq,Skv,lens", [(1, 1, None), (5, 4, None), (33, 60, [60, 33]), (32, 62, None), (128, 128, [128, 65]),
+                                         (130, 132, [129, 1]), (64, 257, [257, 130])])
+@pytest.mark.parametrize("D,scale", [(64, 1.0), (128, 0.3)])
+def test_flash_attn_bias_rows(cuda, Sq, Skv, lens, D, scale):
+    torch.manual_seed(11)
+    q, k, v = rnd(2, Sq, 3, D, scale=0.5), rnd(2, Skv, 3, D), rnd(2, Skv, 3, D)
+    bias = rnd(3, Sq, Skv, scale=2.0)
+    kv = None if lens is None else torch.tensor(lens, device="cuda", dtype=torch.int32)
+    got = ops.attention(q, k, v, scale=scale, bias=bias, kv_lens=kv).float()
+    s = torch.matmul(q.float().transpose(1, 2), k.float().permute(0, 2, 3, 1).contiguous()) * scale + bias.float()
+    if lens is not None:
+        s = s.masked_fill(torch.arange(Skv, device="cuda") >= kv[:, None, None, None], float("-inf"))
+    want = torch.matmul(torch.softmax(s, -1), v.float().transpose(1, 2).contiguous()).transpose(1, 2)
+    assert ((got - want).norm() / want.norm()).item() < 4e-3
+
+
 @pytest.mark.parametrize("S,D", [(256, 128), (700, 64)])
 def test_flash_attn_spike_forces_rescale(cuda, S, D):
     """Late keys with huge scores force the online-softmax rescale branch; a moderate one exercises the
