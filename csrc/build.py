@@ -46,13 +46,14 @@ KERNEL_SRCS = ["kernels/norm.hip", "kernels/gemm.hip", "kernels/gemm_lds.hip", "
 EXTRA_KFLAGS = {"kernels/attention3.hip": "-mllvm -amdgpu-mfma-vgpr-form -fno-slp-vectorize",
                 # flash2 (d128): +0.5-1.2 % at the Flux / LLM-prefill shapes with the same flags (attention lab A/B)
                 "kernels/attention2.hip": "-mllvm -amdgpu-mfma-vgpr-form -fno-slp-vectorize",
+                "lm/gemm_wide.hip": "-mllvm -pragma-unroll-threshold=100000",
                 "kernels/gemm_w4.hip": "-mllvm -pragma-unroll-threshold=100000",
                 "kernels/gemm_ws.hip": "-mllvm -pragma-unroll-threshold=100000 -fno-slp-vectorize",
                 "kernels/conv_halo.hip": "-mllvm -pragma-unroll-threshold=100000 -fno-slp-vectorize"}
 BINDING_SRCS = ["bindings.cpp"]
 # the decoder-block kernels and the token-level ops of every language model's step (their own library: a model that
 # runs on them alone needs nothing else compiled)
-LM_SRCS = ["lm/norm.hip", "lm/gemm.hip", "lm/gemm_ring.hip", "lm/gemm_tile.hip", "lm/moe.hip", "lm/attn.hip", "lm/latent.hip", "lm/scan.hip",
+LM_SRCS = ["lm/norm.hip", "lm/gemm.hip", "lm/gemm_ring.hip", "lm/gemm_tile.hip", "lm/gemm_wide.hip", "lm/moe.hip", "lm/attn.hip", "lm/latent.hip", "lm/scan.hip",
            "lm/hgrn2.hip", "lm/rule.hip", "kernels/sampling.hip"]
 LM_BINDING_SRCS = ["lm/bindings.cpp"]
 RUNTIME_SRCS = ["runtime/block_manager.cpp", "runtime/scheduler.cpp"]

@@ -182,7 +182,8 @@ void launch_gemm_tile(const GemmArgs& a, hipStream_t s) {
   const long m128 = (a.M + 127) / 128, n128 = (a.N + 127) / 128;
   const bool fills = a.N > 128 && a.K > 1536 && (long)((a.M + 255) / 256) * ((a.N + 255) / 256) >= 192;
   const bool big = a.tiles ? a.bm == 256 : a.splits <= 1 && fills;
-  if (big) tile<256, 256, 2, 4>(a, s);
+  if (big && !a.out_f32 && epi_class(a.epi) == EC_PLAIN) launch_gemm_wide(a, s);
+  else if (big) tile<256, 256, 2, 4>(a, s);
   else if (!a.tiles && a.splits <= 1 && m128 * n128 < 256 && a.K <= 2048) tile<64, 64, 2, 2>(a, s);
   else tile<128, 128, 2, 2>(a, s);
 }
