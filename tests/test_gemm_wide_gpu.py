@@ -20,8 +20,10 @@ def _problem(M, N, K, dev, spare=0):
     return a, (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).bfloat16()
 
 
-# at least 192 tiles: whole ones, a last row, a row missing; columns cut by 4, by 8 and by 252; odd and even counts of k-tiles
-@pytest.mark.parametrize("M,N", [(4096, 3072), (3073, 3588), (3327, 3336), (257, 24580), (5120, 2820)])
+# at least 192 tiles: whole ones, a last row, a row missing; columns cut by 4, by 8 and by 252; odd and even counts of k-tiles;
+# 258, 288, 351 and 375 tiles, whose last 2, 32, 95 and 119 are cut in quarters, and 391 whose last 135 are not
+@pytest.mark.parametrize("M,N", [(4096, 3072), (3073, 3588), (3327, 3336), (257, 24580), (5120, 2820), (257, 32900), (4096, 4608),
+                                 (4100, 5636), (3840, 6400), (9900, 2300)])
 @pytest.mark.parametrize("K", [1600, 1664])
 def test_plain(cuda, M, N, K):
     a, w = _problem(M, N, K, cuda, spare=8)
