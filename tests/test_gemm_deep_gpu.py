@@ -112,6 +112,7 @@ torch.manual_seed(0)
 # images, side, channels, outputs, kernel, stride, padding, upsampled, channels of a second source
 cases = [(2, 8, 1280, 1280, 3, 1, 1, False, 0), (1, 16, 64, 96, 3, 2, 1, False, 0), (2, 8, 128, 64, 3, 1, 1, True, 0),
          (2, 7, 64, 64, 1, 1, 0, False, 0), (1, 9, 64, 128, 3, 1, 1, False, 192), (2, 8, 640, 320, 3, 1, 1, True, 640),
+         (1, 9, 64, 64, 5, 2, 2, False, 64), (1, 10, 64, 64, 6, 1, 0, False, 0), (2, 7, 128, 32, 3, 1, 3, False, 0),
          (2, 16, 96, 64, 3, 1, 1, False, 0)]  # the last: 96 channels, which these configs do not take
 worst = 0.0
 for N, H, C, Co, k, stride, pad, up, c2 in cases:
@@ -128,7 +129,7 @@ assert worst < {tol}, worst
 
 
 @pytest.mark.parametrize("splits", [1, 4])
-@pytest.mark.parametrize("cfg", CFGS)
+@pytest.mark.parametrize("cfg", [0, 2, 3, 4] + CFGS)    # 6 x 6 taps are more than a lane's mask holds
 def test_conv(cuda, cfg, splits):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     env = dict(os.environ, SHAI_GEMM_FORCE=str(cfg), SHAI_GEMM_FORCE_SPLITS=str(splits))
