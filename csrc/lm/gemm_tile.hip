@@ -1,6 +1,6 @@
 // C = epi(A W^T), LDS-tiled bf16 form for many rows (prefill): 64 x 64 or 128 x 128 tiles of 4 waves or 256 x 256 tiles of
-// 8, 64-wide k-tiles moved global -> LDS by DMA (buffer_load ... lds, 16 bytes per lane) into two stages; the load of
-// k-tile t + 1 is issued before the MFMAs of t.  The bank swizzle is applied to the per-lane source chunk.  Buffer range checks zero-fill
+// 8, 64-wide k-tiles moved global -> LDS by DMA (buffer_load ... lds, 16 bytes per lane) into a ring of two or four
+// stages; the loads of the next one or three k-tiles are in flight during the MFMAs of t.  The bank swizzle is applied to the per-lane source chunk.  Buffer range checks zero-fill
 // rows past the ends.  Dense or grouped by expert: the row tiles of a grouped product come from the tile list, each with
 // its own W and with A rows gathered per lane.  Tiles are walked XCD by XCD in groups of 8 row tiles that share their W
 // columns.
@@ -13,7 +13,7 @@ constexpr uint32_t kOob = 0x80000000u;
 
 __device__ __forceinline__ int swz(int row, int ch) { return row * 64 + ((ch ^ ((row >> 1) & 7)) << 3); }
 
-template <typename O, int EC, int BM, int BN, int WM, int WN>
+template <typename O, int EC, int BM, int BN, int WM, int WN, int ST>
 __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1) gemm_tile_kernel(const GemmArgs p) {
   constexpr int NW = WM * WN, TM = BM / WM, TN = BN / WN, IM = TM / 32, JN = TN / 32;
   constexpr int JA = BM / 8 / NW, JB = BN / 8 / NW, STAGE = (BM + BN) * 64;
@@ -58,16 +58,16 @@ __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1) gemm_tile_
     const int r = (wid * JB + j) * 8 + lrow, n = n0 + r;
     offW[j] = n < p.N ? (uint32_t)(((long)n * p.K + (lpos ^ ((r >> 1) & 7)) * 8) * 2) : kOob;
   }
-  auto stage = [&](int buf, int kt) {
+  auto stage = [&](int buf, int kt, bool live) {
     bf16_t* sa = smem + buf * STAGE;
     bf16_t* sw = sa + BM * 64;
-    const uint32_t kb = (uint32_t)kt * 128u;
+    const uint32_t kb = (uint32_t)kt * 128u, none = live ? 0u : kOob;   // kOob stays out of range with a k added
 #pragma unroll
     for (int j = 0; j < JB; ++j)
-      dma16(rW, sw + (wid * JB + j) * 512, offW[j] == kOob ? kOob : offW[j] + kb);
+      dma16(rW, sw + (wid * JB + j) * 512, (offW[j] + kb) | none);
 #pragma unroll
     for (int j = 0; j < JA; ++j)
-      dma16(rA, sa + (wid * JA + j) * 512, offA[j] == kOob ? kOob : offA[j] + kb);
+      dma16(rA, sa + (wid * JA + j) * 512, (offA[j] + kb) | none);
   };
 
   float16_ acc[IM][JN];
@@ -86,13 +86,17 @@ __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1) gemm_tile_
     C += (long)blockIdx.y * p.M * p.N;
   }
   const int fr = lane & 31, fh = lane >> 5;
-  stage(0, k0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  // k-tile t; past the end zeros without traffic, so that the count before every tile is the same
+  auto load = [&](int t) { stage(t & (ST - 1), k0 + t, t < nk); };
+  static_assert((ST & (ST - 1)) == 0 && (ST - 2) * (JA + JB) < 64, "a ring of 2, 4 or 8; vmcnt has six bits");
+#pragma unroll
+  for (int t = 0; t < ST - 1; ++t) load(t);
   for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) stage(cur ^ 1, k0 + kt + 1);
-    const bf16_t* sa = smem + cur * STAGE;
+    // tile kt has landed for every wave, and every wave is done with tile kt - 1, whose place tile kt + ST - 1 takes
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 2) * (JA + JB)) : "memory");
+    __builtin_amdgcn_s_barrier();
+    load(kt + ST - 1);
+    const bf16_t* sa = smem + (kt & (ST - 1)) * STAGE;
     const bf16_t* sw = sa + BM * 64;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -109,9 +113,8 @@ __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1) gemm_tile_
         for (int j = 0; j < JN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // bf16 results go through LDS, so that rows are stored 16 bytes a lane, whole lines at a time
   const bool glu = glu_class(EC) && glu_epi(p.epi);
   if (sizeof(O) == 2 && p.ldc % 8 == 0 && (glu || p.n_main % 8 == 0) && (p.n_main == p.N || n0 + BN <= p.n_main)) {
@@ -156,22 +159,22 @@ __global__ void __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1) gemm_tile_
   }
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, int ST>
 static void tile(const GemmArgs& a, hipStream_t s) {
   const int tiles_m = a.tiles ? a.n_tiles : (a.M + BM - 1) / BM;
   const int grid = tiles_m * ((a.N + BN - 1) / BN);
-  constexpr int lds = 2 * (BM + BN) * 64 * 2 > BM * (BN + 8) * 2 ? 2 * (BM + BN) * 64 * 2 : BM * (BN + 8) * 2;
+  constexpr int lds = ST * (BM + BN) * 64 * 2 > BM * (BN + 8) * 2 ? ST * (BM + BN) * 64 * 2 : BM * (BN + 8) * 2;
   auto go = [&](auto k) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     k<<<dim3(grid, a.splits > 1 ? a.splits : 1), WM * WN * 64, lds, s>>>(a);
   };
   const int ec = epi_class(a.epi);
-  if (a.out_f32 && ec == EC_PLAIN) go(gemm_tile_kernel<float, EC_PLAIN, BM, BN, WM, WN>);
-  else if (a.out_f32) go(gemm_tile_kernel<float, EC_ANY, BM, BN, WM, WN>);
-  else if (ec == EC_PLAIN) go(gemm_tile_kernel<bf16_t, EC_PLAIN, BM, BN, WM, WN>);
-  else if (ec == EC_CLAMP) go(gemm_tile_kernel<bf16_t, EC_CLAMP, BM, BN, WM, WN>);
-  else if (ec == EC_GELU) go(gemm_tile_kernel<bf16_t, EC_GELU, BM, BN, WM, WN>);
-  else go(gemm_tile_kernel<bf16_t, EC_OTHER, BM, BN, WM, WN>);
+  if (a.out_f32 && ec == EC_PLAIN) go(gemm_tile_kernel<float, EC_PLAIN, BM, BN, WM, WN, ST>);
+  else if (a.out_f32) go(gemm_tile_kernel<float, EC_ANY, BM, BN, WM, WN, ST>);
+  else if (ec == EC_PLAIN) go(gemm_tile_kernel<bf16_t, EC_PLAIN, BM, BN, WM, WN, ST>);
+  else if (ec == EC_CLAMP) go(gemm_tile_kernel<bf16_t, EC_CLAMP, BM, BN, WM, WN, ST>);
+  else if (ec == EC_GELU) go(gemm_tile_kernel<bf16_t, EC_GELU, BM, BN, WM, WN, ST>);
+  else go(gemm_tile_kernel<bf16_t, EC_OTHER, BM, BN, WM, WN, ST>);
   SHAI_CHECK_LAUNCH();
 }
 
@@ -179,13 +182,20 @@ void launch_gemm_tile(const GemmArgs& a, hipStream_t s) {
   // 256 x 256 tiles (8 waves) once they fill the chip, 128 x 128 (4 waves, two workgroups per CU) below and for narrow
   // outputs and short K (a second workgroup computes while the first one stores), 64 x 64 where those would leave most of
   // the chip idle
+  //
+  // Four stages where a CU holds one workgroup, which has nothing else to hide its loads behind: 64 x 64 tiles, and 128 x 128
+  // up to one for each CU.  With two workgroups a CU each hides the other's, and four stages would take its LDS.
+  // Two stages that drain at every k-tile -> two of the ring -> four, us, weights from memory: 155 x 2048 x 8192 110 -> 100 -> 71,
+  // in 8 parts of K 34.4 -> 32.5 -> 24.4; 600 in 4 parts (320 workgroups) 41 -> 37 -> 49; 155 x 17664 x 2048 (276) 38.6 -> 35.7 ->
+  // 45.2; 64 x 64 tiles: 155 x 2048 x 1024 10.4 -> 7.2 (four), 1000 x 1024 x 2048 17.8 -> 12.2.
   const long m128 = (a.M + 127) / 128, n128 = (a.N + 127) / 128;
   const bool fills = a.N > 128 && a.K > 1536 && (long)((a.M + 255) / 256) * ((a.N + 255) / 256) >= 192;
   const bool big = a.tiles ? a.bm == 256 : a.splits <= 1 && fills;
   if (big && !a.out_f32 && epi_class(a.epi) == EC_PLAIN) launch_gemm_wide(a, s);
-  else if (big) tile<256, 256, 2, 4>(a, s);
-  else if (!a.tiles && a.splits <= 1 && m128 * n128 < 256 && a.K <= 2048) tile<64, 64, 2, 2>(a, s);
-  else tile<128, 128, 2, 2>(a, s);
+  else if (big) tile<256, 256, 2, 4, 2>(a, s);
+  else if (!a.tiles && a.splits <= 1 && m128 * n128 < 256 && a.K <= 2048) tile<64, 64, 2, 2, 4>(a, s);
+  else if (!a.tiles && m128 * n128 * (a.splits > 1 ? a.splits : 1) <= 256) tile<128, 128, 2, 2, 4>(a, s);
+  else tile<128, 128, 2, 2, 2>(a, s);
 }
 
 }  // namespace shai_lm

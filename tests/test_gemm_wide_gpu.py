@@ -1,4 +1,4 @@
-"""The four-wave 256 x 256 products (csrc/lm/gemm_wide.hip) against fp64.
+"""The tiled products (csrc/lm/gemm_wide.hip: four waves of 256 x 256; gemm_tile.hip: rings of smaller tiles) against fp64.
 
 Tolerances, relative 2-norms: fp32 sums of bf16 products 1e-5; one rounding to bf16 (an error spread evenly over half a unit in
 the last of 8 bits) at most 2^-8 / sqrt(3) = 2.3e-3."""
@@ -33,6 +33,17 @@ def test_plain(cuda, M, N, K):
     lm.matmul_joint(a, w, out[:, 8:N + 8], 0, 0)
     assert _rel(out[:, 8:N + 8], want) < 2.3e-3
     assert bool((out[:, :8] == 3).all()) and bool((out[:, N + 8:] == 3).all())
+
+
+# smaller tiles: fewer k-tiles than the ring holds, one more, many; 64 x 64, one 128 x 128 tile per CU and more than one
+@pytest.mark.parametrize("M,N", [(65, 64), (129, 452), (300, 2052), (1030, 4100), (2100, 4100)])
+@pytest.mark.parametrize("K", [64, 192, 256, 320, 2112])
+def test_small_tiles(cuda, M, N, K):
+    a, w = _problem(M, N, K, cuda, spare=8)
+    want = a.double() @ w.double().T
+    assert _rel(lm.matmul(a, w, torch.float32), want) < 1e-5
+    assert _rel(lm.matmul(a, w), want) < 2.3e-3
+    assert _rel(lm.matmul_parts(a, w, torch.float32).double().reshape(-1, M, N).sum(0), want) < 1e-5
 
 
 # fp32 side columns inside the last tile and over the border of two, of a count that allows 16-byte stores and of one that does not
