@@ -13,6 +13,7 @@
 // split of K; M x N x K): 197 x 768 x 768 8.4 -> 6.2, 197 x 3072 x 768 12.3 -> 6.8, 197 x 768 x 3072 12.4 -> 10.3 (4 splits),
 // 154 x 4096 x 1024 13.7 -> 7.6, 512 x 1280 x 1280 14.4 -> 8.5, 2048 x 640 x 2560 22.7 -> 17.9, 8192 x 320 x 1280 19.4 -> 17.6
 // (128 x 128: 14.3), 4096 x 1024 x 2816 35.1 -> 29.9.  Which one runs is the autotuner's choice, like that of every tile.
+// (Both with 8-byte stores; 16-byte ones, gemm_lds_kernel.h, take about a tenth off either.)
 // (Operands straight into registers, with the waves splitting K, were tried too: 16 rows x 64 bytes per load instruction reach
 // 14 bytes per clock and CU, LDS-DMA 30.)
 #include "gemm_lds_kernel.h"
