@@ -268,6 +268,7 @@ void launch_choice(const shai::GemmArgs& g, const Tensor& like, Choice c) {
   }
   // a choice reused from another row count of the same bucket must still fit this problem
   if (!shai::gemm2_cfg_supported(g, c.cfg)) c = fallback_choice(g);
+  if (g.row_mr != nullptr) c.splits = 1;  // the planner's or a cached choice; K parts and their fold know no LayerNorm
   Tensor ws;
   float* wsp = nullptr;
   if (c.splits > 1) {
@@ -475,7 +476,7 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
       }
     }
   }
-  if (g.row_mr != nullptr) c.splits = 1;  // a cached choice of the plain problem with this key may be split
+  if (g.row_mr != nullptr) c.splits = 1;  // before the statistics' rule looks at the choice; launch_choice does the same
   launch_final(g, like, c, st);
 }
 
@@ -912,7 +913,9 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
     attach_norm_io(g, ln_mr, ln_s, gn_part, ln_stats, ln_eps, &st);
     if (force_cfg >= 3000) {  // tests: a split-K tile choice (the fold writes the GroupNorm partials)
       const int cfg = (int)((force_cfg - 3000) % 100), splits = (int)((force_cfg - 3000) / 100);
-      SHAI_CHECK(cfg < shai::gemm2_num_cfgs() && shai::gemm2_cfg_supported(g, cfg) && splits >= 1, "bad forced split");
+      SHAI_CHECK(cfg < shai::gemm2_num_cfgs() && shai::gemm2_cfg_supported(g, cfg) && splits >= 1 &&
+                     (g.row_mr == nullptr || splits == 1 || !shai::gemm2_cfg_splittable(cfg)),
+                 "bad forced split (a folded LayerNorm runs unsplit)");
       launch_final(g, a, Choice{cfg, splits}, &st);
     } else if (force_cfg >= 0) {
       SHAI_CHECK(shai::gemm2_cfg_supported(g, force_cfg), "bad force_cfg");

@@ -103,6 +103,22 @@ def test_folded_layernorm(cuda, cfg, M, N, K):
     assert _rel(out, torch.nn.functional.gelu(y) + r.float()) < TOL
 
 
+# K parts and their fold do not know a LayerNorm: a forced split is refused; the W-stationary kernel runs whole whatever is asked
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 9, 10] + CFGS)
+def test_folded_layernorm_is_not_split(cuda, cfg):
+    a, w, b, _ = _problem(300, 640, 320, cuda)
+    mr = torch.stack([torch.randn(300, device=cuda), torch.rand(300, device=cuda) + 0.5], 1)
+    s, y = w.float().sum(1), torch.empty(300, 640, device=cuda, dtype=torch.bfloat16)
+    run = lambda force: ops._K().gemm(a, w, y, b, None, 1, None, 1.0, 1.0, 0, False, None, 1, force, -1.0, None, mr, s)
+    with pytest.raises(RuntimeError, match="runs unsplit"):
+        run(3200 + cfg)
+    want = mr[:, 1:] * (a.float() @ w.float().t() - mr[:, :1] * s) + b.float()
+    for force in (3100 + cfg, 3215):
+        y.zero_()
+        run(force)
+        assert _rel(y, want) < TOL
+
+
 CONV_SCRIPT = r"""
 import sys, torch
 sys.path.insert(0, {root!r})
