@@ -109,6 +109,15 @@ __device__ __forceinline__ void f2_glds(__amdgpu_buffer_rsrc_t r, bf16_t* lds, u
 // waves 0 and 4 of workgroup (0, 0, 0) at every segment boundary into g_f2_stamps.
 __device__ unsigned long long g_f2_stamps[2][2048];
 
+// Paged: the 8 XCDs form gcd(8, K/V heads) sets.  The queries of one K/V head stay on the XCDs of one set (whose L2 then read those
+// K/V once), and every set has its part of every sequence.  Sequence by sequence, the last rows of all heads of a set come first, which
+// see the most keys, to and fro over the set's XCDs.  Parts by whole (sequence, head) pairs instead gave the longest sequence of a
+// batch to a few XCDs; and sequences side by side are worse than one by one: consecutive workgroups of an XCD go to its shader
+// engines in turn, so that one engine got all of the longest.  us, 32 / 8 heads (4-wave kernel, pairs to XCDs -> now): 4096 rows and
+// 8 of 500 573, 1133 -> 214; 2048 and 16 of 300 277, 373 -> 136; 6000 and 7 of 1, 6000 keys cached, 1200, 6289 -> 1025; 4 of 2048
+// 307, 200 -> 176; 1 of 2048, 40 / 10 heads, 133, 93 -> 73.
+__host__ __device__ inline int f2_sets(int hkv) { return hkv % 8 == 0 ? 8 : hkv % 4 == 0 ? 4 : hkv % 2 == 0 ? 2 : 1; }
+
 template <int D, bool CAUSAL, int EXP = 0, bool PAGED = false>
 __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   constexpr int KT = 64;                 // keys per tile
@@ -141,17 +150,16 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
   const int grp = wid >> 2;
   const int fr = lane & 31, fh = lane >> 5;
   int b = blockIdx.z, hq = blockIdx.y, qb = blockIdx.x;
-  if constexpr (PAGED && CAUSAL) {
-    // The queries of one K/V head go to one XCD (its L2 then reads those K/V once), the longest rows of them first: in launch
-    // order the XCD that gets every eighth block of rows has up to a fifth more work than the mean.
-    const int gx = gridDim.x, grp_q = p.Hq / p.Hkv, total = gx * gridDim.y * gridDim.z;
-    int id = blockIdx.x + gx * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = id & 7, q = total >> 3, r = total & 7;
-    id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
-    const int per = gx * grp_q, head = id / per, in = id - head * per;
-    qb = gx - 1 - in / grp_q;
-    b = head / p.Hkv;
-    hq = (head - b * p.Hkv) * grp_q + in % grp_q;
+  if constexpr (PAGED) {  // 1-D grid (launch_flash2)
+    const int gx = (p.Sq + 255) / 256, grp_q = p.Hq / p.Hkv, sets = f2_sets(p.Hkv), span = 8 / sets;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, sub = xcd % span;
+    int i = slot * span + (slot & 1 ? span - 1 - sub : sub);
+    const int per = p.Hkv / sets * grp_q, row = i / per;
+    b = row / gx;
+    if (b >= p.B) return;
+    i -= row * per;
+    qb = gx - 1 - (row - b * gx);
+    hq = (i / grp_q * sets + xcd / span) * grp_q + i % grp_q;
   }
   const int hk = hq / (p.Hq / p.Hkv);
   const int q_len = p.q_lens ? p.q_lens[b] : p.Sq;
@@ -612,8 +620,9 @@ __global__ void __launch_bounds__(512) flash2_kernel(const AttnArgs p) {
 bool flash2_supported(const AttnArgs& a) {
   if (a.bias != nullptr) return false;
   // Paged K/V (blocks of 64 x D, 16-byte aligned heads), D = 128, from 2048 rows on.  Causal, 32 / 8 heads, us (4-wave kernel
-  // -> this one): 1 x 8000 805 -> 575 (911 TF/s), 1 x 4096 319 -> 162, 1 x 2048 95 -> 72, 1 x 1024 41 -> 40; below, the last
-  // 256 rows' padding costs more than the pipeline gives: 7 x 1100 138 -> 151, 1 x 512 23 -> 26.
+  // -> this one): 1 x 8000 805 -> 565 (926 TF/s), 1 x 2048 95 -> 74, 1 x 1024 41 -> 40; below, the last 256 rows' padding costs
+  // more than the pipeline gives: 1 x 512 23 -> 26.  It is the longest sequence that counts: beside one of 2048 rows, shorter ones of
+  // any number and length (64 of one row, over cached keys) were faster here too.
   if (a.block_table != nullptr) return a.D == 128 && a.Sq >= 2048 && ((a.q_ts | a.kc_bs | a.kc_hs) & 7) == 0;
   if (a.D != 64 && a.D != 128) return false;
   if (a.Sq < 512) return false;  // 256-query workgroups; v1's 128-query blocks waste less on short rows
@@ -630,8 +639,10 @@ void launch_flash2(const AttnArgs& a, hipStream_t s) {
   dim3 grid((a.Sq + 255) / 256, a.Hq, a.B);
   const size_t lds = (size_t)4 * 2 * 64 * a.D * sizeof(bf16_t);
   if (a.block_table != nullptr) {
-    if (a.causal) flash2_kernel<128, true, 0, true><<<grid, 512, lds, s>>>(a);
-    else flash2_kernel<128, false, 0, true><<<grid, 512, lds, s>>>(a);
+    const long sets = f2_sets(a.Hkv), span = 8 / sets, items = a.Hkv / sets * a.B * grid.x * (a.Hq / a.Hkv);
+    const unsigned n = (unsigned)(8 * ((items + span - 1) / span));
+    if (a.causal) flash2_kernel<128, true, 0, true><<<n, 512, lds, s>>>(a);
+    else flash2_kernel<128, false, 0, true><<<n, 512, lds, s>>>(a);
   } else if (a.D == 128) {
     if (a.causal) flash2_kernel<128, true><<<grid, 512, lds, s>>>(a);
     else flash2_kernel<128, false><<<grid, 512, lds, s>>>(a);

@@ -50,7 +50,8 @@ def test_paged_attention_varlen_kernel(cuda, D):
 # Tolerance: bf16 results (2^-8 / sqrt(3) rms) and bf16 probabilities (half of that, by the same bound on each).
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("Hq,Hkv,n_cached,n_new", [(8, 2, [0, 70, 0], [2048, 1, 130]), (4, 4, [5, 0, 64], [2049, 0, 255]),
-                                                  (8, 1, [1000], [2111]), (9, 3, [0, 0], [2300, 2048])])
+                                                  (8, 1, [1000], [2111]), (9, 3, [0, 0], [2300, 2048]),
+                                                  (16, 8, [0, 64], [1, 2050]), (12, 12, [0, 0, 0, 0], [300, 2049, 256, 40])])
 def test_paged_attention_varlen_long(cuda, Hq, Hkv, n_cached, n_new, causal):
     torch.manual_seed(1)
     D, B = 128, len(n_new)
@@ -80,6 +81,39 @@ def test_paged_attention_varlen_long(cuda, Hq, Hkv, n_cached, n_new, causal):
                 s = s.masked_fill(torch.arange(L, device=cuda)[None] > torch.arange(n, device=cuda)[:, None] + L - n, float("-inf"))
             want = torch.softmax(s, -1) @ v
             assert not n or ((got[s0:s0 + n, h].float() - want).norm() / want.norm()).item() < 4e-3, (b, h)
+
+
+# A long sequence with company costs no more than the sequences one after the other.  Dealt to the XCDs by whole sequences, the
+# long one ran on one or two of them: 2 to 6 times that.  (It takes about 0.6 of it; the margin is for other timings.)
+@pytest.mark.parametrize("Hq,Hkv,cached,news", [(32, 8, 0, [4096] + [500] * 8), (32, 8, 6000, [6000] + [1] * 7), (32, 32, 0, [5000] + [1000] * 3)])
+def test_paged_attention_varlen_mixed_time(cuda, Hq, Hkv, cached, news):
+    D, per = 128, [(cached + n + 63) // 64 for n in news]
+    kc = torch.randn(sum(per), Hkv, 64, D, device=cuda).bfloat16()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda)
+    bt = torch.zeros(len(news), max(per), dtype=torch.int32, device=cuda)
+    for b, n in enumerate(per):
+        bt[b, :n] = torch.arange(sum(per[:b]), sum(per[:b + 1]), device=cuda)
+    q = torch.randn(sum(news), Hq, D, device=cuda).bfloat16()
+
+    def call(bs):
+        at, rows = [sum(news[:b]) for b in bs], [news[b] for b in bs]
+        args = (bt[bs].contiguous(), i32([cached + n for n in rows]), i32(rows), i32([a - at[0] for a in at]), max(rows))
+        return lambda: ops.paged_attention_varlen(q[at[0]:at[-1] + rows[-1]], kc, kc, *args, causal=True)
+
+    def best(fns):
+        ts = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for f in fns:
+                f()
+            b.record()
+            torch.cuda.synchronize()
+            ts.append(a.elapsed_time(b))
+        return min(ts)
+
+    together, alone = best([call(list(range(len(news))))]), best([call([b]) for b in range(len(news))])
+    assert together < 1.25 * alone, (together, alone)
 
 
 def test_engine_packed_prefill_matches_padded(cuda):
