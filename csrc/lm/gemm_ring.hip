@@ -1,4 +1,4 @@
-// C = epi(A W^T) for 17 to 64 rows of A (decode steps of a batch) with bf16 weights.
+// C = epi(A W^T) for few rows of A (decode steps of a batch: up to 64) with bf16 weights; gemm_ring_fits says from how many on.
 //
 // The streaming kernel (gemm.hip) reads both operands straight into registers, 16 rows x 16 bytes per quarter wave: 14 bytes per
 // clock and CU, of which A, the same for every workgroup, is as much as W at 64 rows.  DMA to LDS moves 30.  So here both
@@ -143,20 +143,34 @@ void launch_blocks(const GemmArgs& a, int nt, hipStream_t s) {
 // Columns of a workgroup, in blocks of 16: one workgroup per CU, or as few rounds of them as 128 columns allow.  Up to 32 rows a
 // stage is short, and beyond one round of 112 columns two workgroups of 48 per CU, each other's prologue and end hidden, are
 // faster (50176 x 4096, 32 rows: 91 us; one of 128: 95; 32768 x 2048: 32.9 and 34.1).
+constexpr long kRound = 256 * 112;
 static int ring_blocks(const GemmArgs& a) {
   const long cols = (long)a.N * (a.splits > 1 ? a.splits : 1), rounds = (cols + 256 * 128 - 1) / (256 * 128);
-  if (a.M <= 32 && cols > 256 * 112) return 3;
+  if (a.M <= 32 && cols > kRound) return 3;
   const int nt = (int)((cols + 256 * 16 * rounds - 1) / (256 * 16 * rounds));
   return nt < 2 ? 2 : nt > 6 ? 8 : nt;
 }
 
-// From 9 rows on (partial sums: from one).  Below, the streaming kernel's 16-column workgroups read their few rows of A from as
-// few cache lines and start faster: 17424 x 2048 takes 16.0 us (here 18.4) on one row, 18.7 (18.1) on 8, 21.6 (17.5) on 16.
-// Products per head, grouped by expert or longer than a buffer's range stay there.
+// Where the ring is no slower than the streaming kernel, whose 16-column workgroups read few rows of A from few cache lines, start
+// faster, and have no sums to join.  Replays of a HIP graph, cold weights, N x K (streaming -> ring, us):
+//   from 4097 columns on, which are more 16-column workgroups than CUs: 9 rows (5120 x 2048: 0.87 of the time), from 7169 on 12 (8192 x
+//     8192: 9 rows 1.05, 12 1.04, 16 0.94; 17424 x 2048: 9 rows 0.96, 16 0.86);
+//   below: 33 rows from 2049 columns on (2304 x 4096, 64 rows: 24.2 -> 15.5; 2048 x 2048 8.5 -> 9.4), and 17 to 32 rows where M K >=
+//     24 * 1024 (2048 x 2048, 32 rows: 8.4 -> 7.5; 4096 x 1024: 17 rows 1.03 of the time, 24 rows 0.99);
+//   partial sums: more than 16 rows, or a K of 8192; of a K of 4096 from 2049 columns on, and in 8 parts from 9 rows on: 1024 x 4096 in
+//     4 parts, 8 rows 8.1 -> 8.7, 32 rows 10.5 -> 9.3; 2048 x 4096 in 8, 1 row 9.8 -> 10.2, 16 rows 11.7 -> 11.0; x 12544, 1 row 16.5
+//     either way, 16 rows 20.7 -> 16.8.
+//   Up to 32 rows more columns than one round of 112 (ring_blocks) take a K, or part of one, of 3072: 32768 x 1024, 32 rows 1.09 of
+//     the time, x 4096 0.98; 8192 x 2048 in 4 parts, 8 rows 15.6 -> 19.0.
+// Products per head, grouped by expert or longer than a buffer's range stay with the streaming kernel.
 bool gemm_ring_fits(const GemmArgs& a) {
-  const long lim = 0x7fffffffL;
-  return !a.tiles && a.batch <= 1 && a.M <= 64 && (a.M > 8 || a.splits > 1) && a.K >= 512 && a.N >= 512 &&
-         (long)a.N * a.K * 2 < lim && (long)a.M * a.lda * 2 < lim;
+  const long lim = 0x7fffffffL, splits = a.splits > 1 ? a.splits : 1;
+  if (a.tiles || a.batch > 1 || a.M > 64 || a.K < 512 || a.N < 512 || (long)a.N * a.K * 2 >= lim || (long)a.M * a.lda * 2 >= lim)
+    return false;
+  if (a.M <= 32 && a.N * splits > kRound && a.K / splits < 3072) return false;
+  if (splits > 1) return a.M > 16 || a.K >= 8192 || (a.K >= 4096 && (a.N > 2048 || (splits >= 8 && a.M > 8)));
+  if (a.N > 4096) return a.M >= (a.N <= 7168 ? 9 : 12);
+  return a.M > 32 ? a.N > 2048 : a.M > 16 && a.M * a.K >= 24 * 1024;
 }
 
 void launch_gemm_ring(const GemmArgs& a, hipStream_t s) {

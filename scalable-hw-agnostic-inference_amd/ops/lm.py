@@ -32,7 +32,7 @@ MAX_TAPS = 16                # convolution taps
 MAX_LATENT = 1024            # columns of a cached latent
 LATENT_SHORT = 16            # portions up to this many rows attend in latent space, longer ones expand keys and values
 LATENT_GROUP_ROWS = 1 << 18  # context rows that are expanded at a time
-PARTS, PARTS_COLUMNS = 4, 8192   # partial sums: so many, of products up to so wide in a decode step
+PARTS, PARTS_COLUMNS = 4, 8192   # partial sums: so many (of long K twice as many), of products up to so wide in a decode step
 SCAN_CHUNK, SCAN_MAX_CHUNKS = 64, 64
 STATE_SEGMENT, STATE_MAX_SEGMENTS = 128, 32      # rows of a matrix-state segment at least; segments at most
 WHOLE = 1 << 30              # window that holds any sequence
@@ -162,8 +162,12 @@ def matmul_parts(a, w, out_dtype=None):
     """a w^T for a consumer that adds partial sums (:func:`residual_norm`, :func:`latent_prep`): [parts, M, N] fp32
     where the product needs K cut up to fill the chip (few rows, few columns); else :func:`matmul`."""
     M, K, N = a.shape[0], a.shape[1], w.shape[0]
-    if M <= 64:     # twice as many where that makes 64-column workgroups out of 32-column ones (2048 x 12544: 17.4 -> 14.5 us)
-        parts = (PARTS if N > 2048 or K < 4096 else 2 * PARTS) if N <= PARTS_COLUMNS and K >= PARTS * 128 else 1
+    if M <= 64:
+        # Twice as many of a long K, up to 2048 columns: more of the streaming kernel's narrow workgroups (64 x 4096, 32 rows, with
+        # the norm that adds them: 9.6 -> 7.9 us), wider ones of the ring's (2048 x 12544, 16 rows: 17.1 -> 16.8; 4 parts before the
+        # ring: 21.7).  Not where that is slower: 768 x 4096, 8 rows 7.8 -> 8.1.
+        deep = N <= 2048 and K >= 4096 and not (512 < N <= 1024 and K < 5120 and M <= 16)
+        parts = (2 * PARTS if deep else PARTS) if N <= PARTS_COLUMNS and K >= PARTS * 128 else 1
     else:   # tiles of 128 x 128: two for each of the 256 CUs
         tiles = -(-M // 128) * (-(-N // 128))
         parts = min(PARTS, 512 // tiles, K // 512) if tiles < 256 else 1
