@@ -1,0 +1,30 @@
+"""Which kernel a product of a decoder block runs on, at the borders of the rules in csrc/lm: those sizes were measured on both sides."""
+import os
+
+import pytest
+
+from shai_amd import native
+
+if not os.path.exists(native.LM_LIB):
+    pytest.skip("the native library is not built", allow_module_level=True)
+
+
+def form(*args):
+    return native.lm_ops().lm_gemm_form(*args)
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    (8, 8192, 2048, "stream"), (9, 5120, 2048, "ring"), (9, 7232, 2048, "stream"), (12, 17424, 2048, "ring"),      # many columns
+    (16, 2048, 2048, "stream"), (17, 2048, 2048, "ring"), (17, 4096, 1024, "stream"), (24, 4096, 1024, "ring"),    # few columns
+    (32, 512, 768, "ring"), (33, 2048, 8192, "stream"), (33, 2304, 512, "ring"), (64, 508, 4096, "stream"), (64, 4096, 448, "stream"),
+    (32, 32768, 2048, "stream"), (32, 32768, 3072, "ring"), (33, 32768, 512, "ring")])                             # more than a round
+def test_few_rows(M, N, K, want):
+    assert form(M, N, K) == want
+
+
+@pytest.mark.parametrize("M,N,K,splits,want", [
+    (16, 1024, 2048, 4, "stream"), (17, 1024, 2048, 4, "ring"), (1, 2048, 8192, 8, "ring"), (8, 2048, 4096, 8, "stream"),
+    (9, 2048, 4096, 8, "ring"), (1, 2304, 4096, 4, "ring"), (1, 3072, 4032, 4, "stream"), (16, 1024, 4096, 4, "stream"),
+    (1, 8192, 4096, 4, "stream"), (32, 8192, 512, 4, "stream"), (33, 8192, 512, 4, "ring")])
+def test_parts(M, N, K, splits, want):
+    assert form(M, N, K, splits) == want

@@ -25,7 +25,7 @@ def _problem(M, N, K, dev, spare=0):
 # K of a few stages, with half a stage at the end
 @pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(512, 512), (516, 576), (8256, 640), (14628, 1088), (17424, 512), (24576, 512), (28676, 576),
-                                 (32768, 512), (50180, 576)])
+                                 (32768, 512), (50180, 576), (512, 1536), (2052, 1472), (4100, 512), (32772, 3072)])
 def test_plain(cuda, M, N, K):
     a, w = _problem(M, N, K, cuda, spare=8)
     want = a.double() @ w.double().T
@@ -43,12 +43,14 @@ def test_parts(cuda, M, N, K):
     a, w = _problem(M, N, K, cuda, spare=64)
     y = lm.matmul_parts(a, w)
     assert y.shape == (8 if N <= 2048 and K >= 4096 else 4, M, N)
+    if K == 4160:                                          # where eight are slower
+        assert lm.matmul_parts(a, w[:768]).shape[0] == (8 if M > 16 else 4)
     assert _rel(y.sum(0), a.double() @ w.double().T) < 1e-5
 
 
-@pytest.mark.parametrize("M", [12, 40])
-def test_epilogues(cuda, M):
-    N, K = 1036, 704
+@pytest.mark.parametrize("M,N", [(12, 1036), (40, 1036), (12, 5132), (40, 2060)])      # streaming kernel, ring
+def test_epilogues(cuda, M, N):
+    K = 704
     a, w = _problem(M, N, K, cuda)
     c = a.double() @ w.double().T
     gate, up = c[:, 0::2], c[:, 1::2]
