@@ -310,15 +310,18 @@ void lm_gemm_parts(const Tensor& A, const Tensor& W, const Tensor& C) {
   else shai_lm::launch_gemm(g, f32, stream());
 }
 
-// Which kernel a plain bf16 product of up to 64 rows runs on (for tests and tools)
-std::string lm_gemm_form(int64_t M, int64_t N, int64_t K, int64_t splits) {
+// Which kernel a plain bf16 product runs on (for tests and tools); n_tiles > 0: grouped, in that many tiles of up to 256 rows
+std::string lm_gemm_form(int64_t M, int64_t N, int64_t K, int64_t splits, int64_t n_tiles) {
   shai_lm::GemmArgs g{};
+  const int none = 0;
   g.M = g.a_rows = M;
   g.N = g.n_main = g.n_act = N;
   g.K = g.lda = K;
   g.splits = splits;
   g.out_f32 = splits > 1;
   g.batch = 1;
+  if (n_tiles > 0) g.tiles = &none, g.n_tiles = n_tiles, g.bm = 256;
+  if (n_tiles > 0 || M > 64) return shai_lm::gemm_tile_name(g);
   return shai_lm::gemm_ring_fits(g) ? "ring" : "stream";
 }
 
@@ -1193,7 +1196,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("rule_rows(Tensor x, Tensor gate, Tensor(a!) state, Tensor(b!) out, Tensor pos, Tensor slots, int kv_heads, int dim, int vdim, int gate_kind, float eps, Tensor rate, Tensor? decay=None, Tensor? beta=None, Tensor? conv=None, Tensor? bias=None, Tensor? gain=None, Tensor(c!)? ring=None, Tensor? rope=None, Tensor? q_start=None, Tensor? q_lens=None) -> ()");
   m.def("rule_chunks(Tensor x, Tensor gate, Tensor(a!) state, Tensor(b!) out, Tensor pos, Tensor slots, int kv_heads, int dim, int vdim, int gate_kind, float eps, Tensor rate, Tensor? decay=None, Tensor? beta=None, Tensor? conv=None, Tensor? bias=None, Tensor? gain=None, Tensor? ring=None, Tensor? rope=None, *, Tensor q_start, Tensor q_lens, Tensor(c!) ws, int max_q, int head0, int heads, int seg=0, Tensor(d!)? seg_ws=None) -> ()");
   m.def("rule_segment_bytes(int dk, int dv, int heads, bool retention) -> int", &rule_segment_bytes);
-  m.def("lm_gemm_form(int M, int N, int K, int splits=1) -> str", &lm_gemm_form);
+  m.def("lm_gemm_form(int M, int N, int K, int splits=1, int n_tiles=0) -> str", &lm_gemm_form);
   m.def("rule_chunk_bytes(int dk, int dv, int heads, int keys, bool channel) -> int", &rule_chunk_bytes);
   m.def("ring_commit(Tensor x, Tensor(a!) ring, Tensor pos, Tensor q_start, Tensor q_lens, Tensor slots) -> ()");
   m.def("gated_attn_prefill(Tensor qkvg, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor ctx_lens, Tensor q_lens, Tensor q_start, int max_q, int heads, int chunk, float scale, bool window=False, bool per_element=False, bool own_kv=True, Tensor? temp=None, Tensor? sink=None, float out_scale=1.) -> ()");

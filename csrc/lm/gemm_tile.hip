@@ -178,24 +178,42 @@ static void tile(const GemmArgs& a, hipStream_t s) {
   SHAI_CHECK_LAUNCH();
 }
 
+// 256 x 256 tiles once they fill the chip (without an epilogue: gemm_wide.hip), 128 x 128 (4 waves, two workgroups per CU) below and
+// for narrow outputs and short K (a second workgroup computes while the first one stores), 64 x 64 where those would leave most of the
+// chip idle.  Grouped: the caller's tile; the wide form from a K of 1600 on, as for dense products (us, 8 waves -> wide: 32 experts,
+// 18000 rows, 1536 x 512 60 -> 69; 8, 7000, 1024 x 1024 33.9 -> 36.1; 8, 5000, 1024 x 2048 55.4 -> 55.7, x 4096 97 -> 93; 8, 16000,
+// 2816 x 4096 428 -> 403).
+//
+// Four stages where a CU holds one workgroup, which has nothing else to hide its loads behind: 128 x 128 tiles up to one for each CU,
+// and 64 x 64 up to two, or beyond with a K of 2048.  Otherwise the workgroups of a CU hide each other's, and four stages would take
+// their LDS.  Two stages that drain at every k-tile -> two of the ring -> four, us, weights from memory: 155 x 2048 x 8192 110 -> 100 ->
+// 71, in 8 parts of K 34.4 -> 32.5 -> 24.4; 600 in 4 parts (320 workgroups) 41 -> 37 -> 49; 155 x 17664 x 2048 (276) 38.6 -> 35.7 ->
+// 45.2; 64 x 64 tiles: 155 x 2048 x 1024 10.4 -> 7.2 (four), 1000 x 1024 x 2048 17.8 -> 12.2; 600 x 4096 (640 workgroups), K = 512
+// 8.5 -> 10.6 (four), 1024 16.0 -> 17.0, 2048 27.8 -> 27.2.
+enum class Tile { wide, big, mid4, mid2, small4, small2 };
+static Tile tile_of(const GemmArgs& a) {
+  const long m128 = (a.M + 127) / 128, n128 = (a.N + 127) / 128, m64 = (a.M + 63) / 64, n64 = (a.N + 63) / 64;
+  const bool deep = a.K > 1536;
+  if (a.tiles ? a.bm == 256 : a.splits <= 1 && a.N > 128 && deep && (long)((a.M + 255) / 256) * ((a.N + 255) / 256) >= 192)
+    return deep && !a.out_f32 && epi_class(a.epi) == EC_PLAIN ? Tile::wide : Tile::big;
+  if (!a.tiles && a.splits <= 1 && m128 * n128 < 256 && a.K <= 2048) return m64 * n64 <= 512 || a.K == 2048 ? Tile::small4 : Tile::small2;
+  return !a.tiles && m128 * n128 * (a.splits > 1 ? a.splits : 1) <= 256 ? Tile::mid4 : Tile::mid2;
+}
+
+const char* gemm_tile_name(const GemmArgs& a) {
+  const char* const names[] = {"wide", "256x256", "128x128 of 4", "128x128", "64x64 of 4", "64x64"};
+  return names[(int)tile_of(a)];
+}
+
 void launch_gemm_tile(const GemmArgs& a, hipStream_t s) {
-  // 256 x 256 tiles (8 waves) once they fill the chip, 128 x 128 (4 waves, two workgroups per CU) below and for narrow
-  // outputs and short K (a second workgroup computes while the first one stores), 64 x 64 where those would leave most of
-  // the chip idle
-  //
-  // Four stages where a CU holds one workgroup, which has nothing else to hide its loads behind: 64 x 64 tiles, and 128 x 128
-  // up to one for each CU.  With two workgroups a CU each hides the other's, and four stages would take its LDS.
-  // Two stages that drain at every k-tile -> two of the ring -> four, us, weights from memory: 155 x 2048 x 8192 110 -> 100 -> 71,
-  // in 8 parts of K 34.4 -> 32.5 -> 24.4; 600 in 4 parts (320 workgroups) 41 -> 37 -> 49; 155 x 17664 x 2048 (276) 38.6 -> 35.7 ->
-  // 45.2; 64 x 64 tiles: 155 x 2048 x 1024 10.4 -> 7.2 (four), 1000 x 1024 x 2048 17.8 -> 12.2.
-  const long m128 = (a.M + 127) / 128, n128 = (a.N + 127) / 128;
-  const bool fills = a.N > 128 && a.K > 1536 && (long)((a.M + 255) / 256) * ((a.N + 255) / 256) >= 192;
-  const bool big = a.tiles ? a.bm == 256 : a.splits <= 1 && fills;
-  if (big && !a.out_f32 && epi_class(a.epi) == EC_PLAIN) launch_gemm_wide(a, s);
-  else if (big) tile<256, 256, 2, 4, 2>(a, s);
-  else if (!a.tiles && a.splits <= 1 && m128 * n128 < 256 && a.K <= 2048) tile<64, 64, 2, 2, 4>(a, s);
-  else if (!a.tiles && m128 * n128 * (a.splits > 1 ? a.splits : 1) <= 256) tile<128, 128, 2, 2, 4>(a, s);
-  else tile<128, 128, 2, 2, 2>(a, s);
+  switch (tile_of(a)) {
+    case Tile::wide: return launch_gemm_wide(a, s);
+    case Tile::big: return tile<256, 256, 2, 4, 2>(a, s);
+    case Tile::mid4: return tile<128, 128, 2, 2, 4>(a, s);
+    case Tile::mid2: return tile<128, 128, 2, 2, 2>(a, s);
+    case Tile::small4: return tile<64, 64, 2, 2, 4>(a, s);
+    case Tile::small2: return tile<64, 64, 2, 2, 2>(a, s);
+  }
 }
 
 }  // namespace shai_lm

@@ -141,6 +141,7 @@ bool gemm_ring_fits(const GemmArgs& a);                                // bf16 p
 void launch_gemm_ring(const GemmArgs& a, hipStream_t s);
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t s);          // streaming kernel, any M
 void launch_gemm_tile(const GemmArgs& a, hipStream_t s);               // LDS-tiled bf16 kernel (gemm_tile.hip)
+const char* gemm_tile_name(const GemmArgs& a);                         // which of its forms that is
 void launch_gemm_wide(const GemmArgs& a, hipStream_t s);               // its 256 x 256 tiles without an epilogue (gemm_wide.hip)
 
 struct RouteArgs {

@@ -28,3 +28,19 @@ def test_few_rows(M, N, K, want):
     (1, 8192, 4096, 4, "stream"), (32, 8192, 512, 4, "stream"), (33, 8192, 512, 4, "ring")])
 def test_parts(M, N, K, splits, want):
     assert form(M, N, K, splits) == want
+
+
+# 64 x 64 tiles up to two for each CU, more with a K of 2048; 128 x 128 up to one; 256 x 256 from 192 on
+@pytest.mark.parametrize("M,N,K,splits,want", [
+    (512, 4096, 512, 1, "64x64 of 4"), (600, 4096, 1984, 1, "64x64"), (600, 4096, 2048, 1, "64x64 of 4"), (600, 4096, 2112, 1, "128x128 of 4"),
+    (1024, 4096, 512, 1, "128x128 of 4"), (1025, 4096, 512, 1, "128x128"), (600, 2048, 8192, 3, "128x128 of 4"),
+    (600, 2048, 8192, 4, "128x128"), (4096, 3072, 1600, 1, "wide"), (4096, 3072, 1536, 1, "128x128"), (4096, 3008, 1600, 1, "wide"),
+    (4096, 2816, 1600, 1, "128x128"), (8192, 128, 4096, 1, "128x128 of 4")])
+def test_tiles(M, N, K, splits, want):
+    assert form(M, N, K, splits) == want
+
+
+# grouped rows in tiles of 256: the wide form from a K of 1600 on
+@pytest.mark.parametrize("N,K,want", [(1024, 1600, "wide"), (1024, 4096, "wide"), (1536, 512, "256x256"), (1536, 1536, "256x256")])
+def test_grouped(N, K, want):
+    assert form(5000, N, K, 1, 27) == want
