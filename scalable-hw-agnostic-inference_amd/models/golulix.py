@@ -142,7 +142,7 @@ class GolulixForCausalLM(nn.Module):
     def kv_heads_local(self) -> int:
         return max(layer.mix.c.kv_heads for layer in self.layers)
 
-    split_blocks = (4, 0)        # a block for each wave of an attention workgroup
+    split_blocks = lm.ATTENTION_SPLIT_BLOCKS
 
     @property
     def attn_span(self) -> int:

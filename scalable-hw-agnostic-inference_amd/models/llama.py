@@ -249,7 +249,8 @@ class LlamaForCausalLM(nn.Module):
     def split_blocks(self) -> tuple:
         """(64-token blocks of a decode split, at least; of a context that is not split) for :func:`ops.decode_splits`.  With 4
         query heads of 128 per KV head an unsplit context's blocks go to the waves of one workgroup at a time
-        (decode_attn_wb_kernel), and the launch that joins splits is saved: Mistral-7B's 8 layers, one step at 254 cached tokens
+        (decode_attn_wb_kernel), and the launch that joins splits is saved, in an engine whose longest context is that short
+        (``LLMEngine.decode_splits`` goes by ``max_model_len``): Mistral-7B, 8 layers, one step at 254 cached tokens
         932 -> 893 us (batch 1), 967 -> 910 (16), 989 -> 943 (32); at 504 tokens 965 -> 936; at 724 no longer faster."""
         a = self.layers[0].self_attn
         return 1, 8 if a.hd == 128 and a.h == 4 * a.hk else 0

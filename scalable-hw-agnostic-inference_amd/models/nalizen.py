@@ -168,7 +168,7 @@ class NalizenForCausalLM(nn.Module):
     def kv_heads_local(self) -> int:
         return max((m.c.kv_heads for m in self._attention()), default=1)
 
-    split_blocks = (4, 0)        # a block for each wave of an attention workgroup
+    split_blocks = lm.ATTENTION_SPLIT_BLOCKS
 
     @property
     def attn_span(self) -> int:

@@ -152,7 +152,7 @@ class PugozenForCausalLM(nn.Module):
     needs_prev_token = False
     has_state = True             # sequences hold a state slot (allocate_state); their prefixes cannot be shared by blocks
     attn_span: Optional[int] = None
-    split_blocks = (4, 0)        # a block for each wave of an attention workgroup
+    split_blocks = lm.ATTENTION_SPLIT_BLOCKS
     dtypes = (torch.bfloat16, torch.float32)
 
     def __init__(self, cfg: PugozenConfig, dtype=torch.bfloat16):

@@ -571,16 +571,17 @@ def paged_attention_varlen(q, k_cache, v_cache, block_table, kv_lens, q_lens, q_
 SAMPLER_MAX_K = 1024
 
 
-def decode_splits(batch: int, hkv: int, max_ctx: int, blocks: int = 1, whole: int = 0) -> int:
+def decode_splits(batch: int, hkv: int, max_ctx: int, blocks: int = 1, whole: int = 0, many: int = 0) -> int:
     """Split-K factor of the paged decode attention: enough (sequence, KV head, split) workgroups to fill
-    the chip (``SHAI_DECODE_WG`` of them, default 512 = two per CU), at most one split per ``blocks`` 64-token blocks (a
-    workgroup's waves take a block each), and one in all for contexts of up to ``whole`` blocks."""
+    the chip (``SHAI_DECODE_WG`` of them, default 512 = two per CU), at most one split per 64-token block, or per ``blocks`` of
+    them from ``many`` on (a workgroup's waves take a block each), and one in all up to ``whole`` blocks.  ``max_ctx``: the longest
+    context of any step that the factor is for."""
     nblk = max(1, (max_ctx + 63) // 64)
     if nblk <= whole:
         return 1
     target = int(os.environ.get("SHAI_DECODE_WG", "512"))
     want = max(1, target // max(1, batch * hkv))
-    return int(min(-(-nblk // blocks), want, 64))
+    return int(min(-(-nblk // (blocks if nblk >= many else 1)), want, 64))
 
 
 def decode_attention(q, k_cache, v_cache, block_table, ctx_lens, scale=None, num_splits: Optional[int] = None,

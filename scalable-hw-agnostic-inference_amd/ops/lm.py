@@ -32,6 +32,11 @@ MAX_TAPS = 16                # convolution taps
 MAX_LATENT = 1024            # columns of a cached latent
 LATENT_SHORT = 16            # portions up to this many rows attend in latent space, longer ones expand keys and values
 LATENT_GROUP_ROWS = 1 << 18  # context rows that are expanded at a time
+# Decode attention (:func:`ops.decode_splits`): up to 4 blocks, one for each wave, unsplit, which saves the launch that joins the splits;
+# from 64 blocks on 4 per split; between, where a wave's second block is waited for, one.  16 query / 4 KV heads of 128, one
+# sequence, us, splits by one block -> by four: 124 tokens 11.0 -> 8.8, 256 11.5 -> 9.8, 512 10.8 -> 12.5, 1024 11.6 -> 13.5, 2048
+# 12.6 -> 12.9, 4096 14.0 -> 13.3, 8192 14.9 -> 14.2; 16 / 8 heads of 64, 32 / 8 and 8 / 8 of 128 and 4 sequences lie alike.
+ATTENTION_SPLIT_BLOCKS = (4, 4, 64)
 PARTS, PARTS_COLUMNS = 4, 8192   # partial sums: so many (of long K twice as many), of products up to so wide in a decode step
 SCAN_CHUNK, SCAN_MAX_CHUNKS = 64, 64
 STATE_SEGMENT, STATE_MAX_SEGMENTS = 128, 32      # rows of a matrix-state segment at least; segments at most

@@ -311,3 +311,16 @@ def test_no_garbage_collection_during_a_capture(monkeypatch):
 def test_decode_splits(batch, hkv, ctx, blocks, whole, want):
     from shai_amd import ops
     assert ops.decode_splits(batch, hkv, ctx, blocks, whole) == want
+
+
+@pytest.mark.parametrize("batch,hkv,ctx,want", [
+    (1, 4, 256, 1), (1, 4, 257, 5), (1, 8, 512, 8), (1, 4, 2048, 32), (1, 4, 4032, 63), (1, 4, 4033, 16), (1, 8, 8192, 32),
+    (16, 4, 256, 1), (16, 4, 512, 8), (64, 4, 512, 2)])
+def test_decode_splits_of_layer_lists(batch, hkv, ctx, want):
+    """Short contexts whole, four blocks a split only of long ones: between, one block a split is faster."""
+    from shai_amd import ops
+    from shai_amd.models.golulix import GolulixForCausalLM
+    from shai_amd.models.nalizen import NalizenForCausalLM
+    from shai_amd.models.pugozen import PugozenForCausalLM
+    for m in (GolulixForCausalLM, NalizenForCausalLM, PugozenForCausalLM):
+        assert ops.decode_splits(batch, hkv, ctx, *m.split_blocks) == want
