@@ -21,6 +21,7 @@
 #include "launchers.h"
 
 #include <algorithm>
+#include <cmath>
 
 #include <cstdlib>
 #include <type_traits>
@@ -44,7 +45,8 @@ __device__ __forceinline__ int v_swz(int row, int ch) {
   else return row * 64 + ((ch ^ (((row >> 1) & 1) << 2)) << 3);
 }
 
-template <int D>
+enum { kBiasAny, kBiasDiv, kBiasMul };  // see bias_form
+template <int D, int BIAS>
 __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
   constexpr int KT = 64;                 // keys per tile
   constexpr int CPR = D / 8;             // 16-byte chunks per row
@@ -130,10 +132,6 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
   float m_run = -INFINITY, l_run = 0.f;
   const float sl2 = p.scale * kLog2e;
   const bf16_t* bias_row = p.bias ? p.bias + ((long)hq * p.Sq + min(qi, q_len - 1)) * p.Skv : nullptr;
-  // A lane's bias: 8 groups of 4 consecutive keys of its query's row.  One 8-byte load each, issued before the tile's scores, where
-  // rows allow it; 32 loads of 2 bytes and a division per score bounded short sequences (T5, 32 x 128 tokens, 16 heads of 64:
-  // 28.0 -> 16.7 us).
-  const bool bias4 = (p.Skv & 3) == 0 && ((uintptr_t)p.bias & 7) == 0;
   const float inv_scale = 1.f / p.scale;
 
   if (ntiles > 0) {
@@ -151,8 +149,8 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
     if (t + 1 < ntiles) load_tile(t + 1);
     const bf16_t* ks = sK + cur * KT * D;
     const bf16_t* vs = sV + cur * KT * D;
-    uint2_ bias[8];
-    if (bias_row && bias4) {
+    [[maybe_unused]] uint2_ bias[8];  // 8 groups of 4 consecutive keys of the lane's query
+    if constexpr (BIAS != kBiasAny) {
 #pragma unroll
       for (int g = 0; g < 8; ++g) {
         const int key = t * KT + 8 * g + 4 * fh;
@@ -176,15 +174,19 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const AttnArgs p) {
     const int key0 = t * KT;
     const bool need_mask = (key0 + KT > kv_len) || (p.causal && key0 + KT - 1 > q0 + c_off);
     float mloc = -INFINITY;
-    if (bias_row) {  // T5 relative-position bias: additive in the natural-log domain
+    if (BIAS != kBiasAny || bias_row) {  // T5 relative-position bias: additive in the natural-log domain
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = key0 + kb * 32 + (r & 3) + 8 * (r >> 2) + 4 * fh;
-          const uint32_t two = bias[4 * kb + (r >> 2)][(r >> 1) & 1];
-          const float x = bias4 ? bf2f(r & 1 ? two >> 16 : two & 0xffff) : key < p.Skv ? bf2f(bias_row[key]) : 0.f;
-          sacc[kb][r] += x * inv_scale;
+          if constexpr (BIAS != kBiasAny) {
+            const uint32_t two = bias[4 * kb + (r >> 2)][(r >> 1) & 1];
+            const float x = bf2f(r & 1 ? two >> 16 : two & 0xffff);
+            sacc[kb][r] += BIAS == kBiasMul ? x * inv_scale : x / p.scale;
+          } else {
+            const int key = key0 + kb * 32 + (r & 3) + 8 * (r >> 2) + 4 * fh;
+            sacc[kb][r] += (key < p.Skv ? bf2f(bias_row[key]) : 0.f) / p.scale;
+          }
         }
     }
     if (need_mask) {
@@ -569,6 +571,28 @@ int set_flash128x2(int mode) {
   return prev;
 }
 
+// An additive bias in 8-byte loads, issued before the tile's scores, for rows of whole groups of 4 keys, 8-byte aligned; times 1 / scale
+// for a scale that is a power of two (the product is then the quotient), which saves a division per score.  32 loads of 2 bytes and 32
+// divisions bound short sequences: T5, 16 heads of 64, 32 x 128 tokens 25.0 -> 12.2 us, 32 x 512 297 -> 102; 8 heads of 128, scale 0.3,
+// 32 x 512 173 -> 91.  Forms of their own: in one kernel with the key-by-key form, that one took 344 us for 32 x 511 tokens (269),
+// and attention without a bias 10.6 for 2 x 100 tokens, 32 heads of 128 (9.9).
+static int bias_form(const AttnArgs& a) {
+  if (a.bias == nullptr || a.Skv % 4 != 0 || ((uintptr_t)a.bias & 7) != 0) return kBiasAny;
+  int e;
+  return std::isnormal(a.scale) && std::isnormal(1.f / a.scale) && std::fabs(std::frexp(a.scale, &e)) == 0.5f ? kBiasMul : kBiasDiv;
+}
+
+template <int D>
+static void launch_flash_fwd(const AttnArgs& a, hipStream_t s) {
+  const dim3 grid((a.Sq + 127) / 128, a.Hq, a.B);
+  const size_t lds = (size_t)4 * 64 * D * sizeof(bf16_t);
+  switch (bias_form(a)) {
+    case kBiasMul: flash_fwd_kernel<D, kBiasMul><<<grid, 256, lds, s>>>(a); break;
+    case kBiasDiv: flash_fwd_kernel<D, kBiasDiv><<<grid, 256, lds, s>>>(a); break;
+    default: flash_fwd_kernel<D, kBiasAny><<<grid, 256, lds, s>>>(a); break;
+  }
+}
+
 void launch_flash_attn(const AttnArgs& a, hipStream_t s) {
   static const bool v1_only = getenv("SHAI_FLASH_V1") != nullptr;  // A/B and tests: pin the v1 kernel
   if (!v1_only && flash64_supported(a)) {  // D = 64 (every SD2.1 / ViT / BERT attention)
@@ -583,10 +607,8 @@ void launch_flash_attn(const AttnArgs& a, hipStream_t s) {
     launch_flash2(a, s);
     return;
   }
-  dim3 grid((a.Sq + 127) / 128, a.Hq, a.B);
-  const size_t lds = (size_t)4 * 64 * a.D * sizeof(bf16_t);
-  if (a.D == 128) flash_fwd_kernel<128><<<grid, 256, lds, s>>>(a);
-  else flash_fwd_kernel<64><<<grid, 256, lds, s>>>(a);
+  if (a.D == 128) launch_flash_fwd<128>(a, s);
+  else launch_flash_fwd<64>(a, s);
 }
 
 // ----------------------------------------------------------------------------

@@ -246,7 +246,7 @@ def test_flash_attn_bias(cuda):
 # Tolerance: bf16 results (2^-8 / sqrt(3) rms) and bf16 probabilities (half of that, by the same bound on each).
 @pytest.mark.parametrize("Sq,Skv,lens", [(1, 1, None), (5, 4, None), (33, 60, [60, 33]), (32, 62, None), (128, 128, [128, 65]),
                                          (130, 132, [129, 1]), (64, 257, [257, 130])])
-@pytest.mark.parametrize("D,scale", [(64, 1.0), (128, 0.3)])
+@pytest.mark.parametrize("D,scale", [(64, 1.0), (128, 0.3), (128, 0.25), (64, 0.7)])
 def test_flash_attn_bias_rows(cuda, Sq, Skv, lens, D, scale):
     torch.manual_seed(11)
     q, k, v = rnd(2, Sq, 3, D, scale=0.5), rnd(2, Skv, 3, D), rnd(2, Skv, 3, D)
@@ -258,6 +258,16 @@ def test_flash_attn_bias_rows(cuda, Sq, Skv, lens, D, scale):
         s = s.masked_fill(torch.arange(Skv, device="cuda") >= kv[:, None, None, None], float("-inf"))
     want = torch.matmul(torch.softmax(s, -1), v.float().transpose(1, 2).contiguous()).transpose(1, 2)
     assert ((got - want).norm() / want.norm()).item() < 4e-3
+
+
+@pytest.mark.parametrize("D,scale", [(64, 1.0), (128, 0.25), (128, 0.3), (64, 3.7)])
+def test_flash_attn_bias_forms_agree(cuda, D, scale):
+    """Rows of 4 keys at a time and key by key give the same bits, whatever the scale."""
+    torch.manual_seed(12)
+    q, k, v, bias = rnd(4, 150, 5, D), rnd(4, 512, 5, D), rnd(4, 512, 5, D), rnd(5, 150, 512, scale=9.0)
+    n = torch.full((4,), 509, device="cuda", dtype=torch.int32)
+    got = ops.attention(q, k, v, scale=scale, bias=bias, kv_lens=n)
+    assert torch.equal(got, ops.attention(q, k[:, :509], v[:, :509], scale=scale, bias=bias[:, :, :509].contiguous()))
 
 
 @pytest.mark.parametrize("S,D", [(256, 128), (700, 64)])
