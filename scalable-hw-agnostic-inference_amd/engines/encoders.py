@@ -11,7 +11,6 @@ import base64
 import io
 import os
 import threading
-from collections import OrderedDict
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -173,20 +172,46 @@ class DetectorEngine:
         return out
 
 
+class ShapeGraphs:
+    """Graphs by input shape for a service whose clients choose shapes.  A capture takes as long as several eager calls, so a shape is
+    captured when it comes again within ``RECENT`` calls, while there is room; where there is none, in place of a graph that has not
+    been used for ``IDLE`` calls.  Shapes that take turns in larger numbers therefore stay eager, and captures are at most ``most``
+    per ``IDLE`` calls once there are so many.  Not thread-safe."""
+
+    RECENT, IDLE = 64, 1024
+
+    def __init__(self, make):
+        self.make, self.graphs, self.seen, self.calls = make, {}, {}, 0
+
+    def __len__(self):
+        return len(self.graphs)
+
+    def get(self, shape: tuple, most: int):
+        """The graph of ``shape`` for one call, or None: this call runs eagerly."""
+        self.calls += 1
+        last = self.seen.get(shape, -self.RECENT)
+        self.seen[shape] = self.calls
+        if shape not in self.graphs and self.calls - last <= self.RECENT:
+            if len(self.graphs) >= most:
+                old = min(self.graphs, key=self.seen.get)
+                if self.calls - self.seen[old] > self.IDLE:
+                    del self.graphs[old]
+            if len(self.graphs) < most:
+                self.graphs[shape] = self.make(*shape)
+        if len(self.seen) > 2 * (self.RECENT + most):
+            self.seen = {s: n for s, n in self.seen.items() if s in self.graphs or self.calls - n < self.RECENT}
+        return self.graphs.get(shape)
+
+
 class _EmbeddingGraph:
-    """The encoder on a batch of one shape as a HIP graph: token ids and lengths of the rows in one buffer, filled by one copy."""
+    """The encoder on a batch of one shape, which has run eagerly before, as a HIP graph: token ids and lengths of the rows in one
+    buffer, filled by one copy."""
 
     def __init__(self, model, B: int, L: int, device, pool):
         self.host = torch.zeros(B * L + B, dtype=torch.int32, pin_memory=True)
         self.rows = self.host.numpy()
         self.dev = torch.zeros(B * L + B, dtype=torch.int32, device=device)
         ids, lens = self.dev[:B * L].view(B, L), self.dev[B * L:]
-        lens.fill_(L)
-        side = torch.cuda.Stream(device=device)
-        side.wait_stream(torch.cuda.current_stream(device))
-        with torch.cuda.stream(side):      # GEMM autotuning, the position bias and allocator growth happen outside the capture
-            model.encode_mean(ids, lens=lens)
-        torch.cuda.current_stream(device).wait_stream(side)
         self.graph = new_graph(device)
         with capture(self.graph, pool=pool, capture_error_mode="thread_local"):
             self.out = model.encode_mean(ids, lens=lens)
@@ -201,12 +226,12 @@ class _EmbeddingGraph:
 
 
 class TextEmbeddingEngine:
-    """T5 sentence embeddings.  An encoder step is some 200 launches that the host takes longer to issue than a small batch to run,
-    so every batch shape runs as a HIP graph (the least recently used of ``MAX_GRAPHS`` goes); with tensor parallelism eagerly.
-    T5-v1.1-large: one 32-token text 2.24 ms eager, 1.23 ms; 32 texts of 128 tokens 6.0 ms either way (4.8 ms of kernels, then
-    tokenizing)."""
+    """T5 sentence embeddings.  An encoder step is some 200 launches that the host takes longer to issue than a small batch to run, so
+    batch shapes of up to ``GRAPH_TOKENS`` tokens that come again run as HIP graphs (:class:`ShapeGraphs`, up to ``MAX_GRAPHS``);
+    with tensor parallelism eagerly.  T5-v1.1-large, ms eager -> graph: 1 text of 32 tokens 2.25 -> 1.16, 8 of 32 2.29 -> 1.50, 16 of 32
+    2.33 -> 1.87, 8 of 128 2.46 -> 2.38, 32 of 128 6.1 either way; the call that captures 3.8."""
 
-    MAX_GRAPHS = 16
+    MAX_GRAPHS, GRAPH_TOKENS = 16, 512
 
     def __init__(self, cfg=None, device="cuda", model_path=None, seed=0, use_graphs=True):
         from ..models.t5 import T5Config, T5EncoderModel
@@ -220,9 +245,9 @@ class TextEmbeddingEngine:
                                         eos_id=self.cfg.eos_token_id, pad_id=self.cfg.pad_token_id,
                                         model_max_length=1024)
         self.use_graphs = use_graphs and self.device.type == "cuda" and tp().size == 1
-        self._graphs: "OrderedDict[tuple, _EmbeddingGraph]" = OrderedDict()
         self._pool = torch.cuda.graph_pool_handle() if self.use_graphs else None
-        self._lock = threading.Lock()      # the graphs share buffers: one replay at a time
+        self._graphs = ShapeGraphs(lambda B, L: _EmbeddingGraph(self.model, B, L, self.device, self._pool))
+        self._lock = threading.Lock()      # the graphs share buffers: one replay at a time, and none beside a capture
 
     @torch.inference_mode()
     def embed(self, texts: Sequence[str], max_length: int) -> np.ndarray:
@@ -232,13 +257,11 @@ class TextEmbeddingEngine:
         if not self.use_graphs or not ids.numel():
             return self.model.encode_mean(ids.to(self.device), mask.to(self.device)).cpu().numpy()
         with self._lock, torch.cuda.device(self.device):
-            g = self._graphs.get(tuple(ids.shape))
-            if g is None:
-                if len(self._graphs) >= self.MAX_GRAPHS:
-                    self._graphs.popitem(last=False)
-                g = self._graphs[tuple(ids.shape)] = _EmbeddingGraph(self.model, *ids.shape, self.device, self._pool)
-            self._graphs.move_to_end(tuple(ids.shape))
-            return g.run(ids.numpy(), mask.numpy())
+            g = self._graphs.get(tuple(ids.shape), self.MAX_GRAPHS) if ids.numel() <= self.GRAPH_TOKENS else None
+            if g is not None:
+                return g.run(ids.numpy(), mask.numpy())
+            out = self.model.encode_mean(ids.to(self.device), mask.to(self.device))
+        return out.cpu().numpy()           # waits, while another thread may launch
 
 
 def _resize_u8(x: torch.Tensor, H: int, W: int) -> torch.Tensor:

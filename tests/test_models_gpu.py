@@ -282,3 +282,30 @@ def test_t5_graph_replay_matches_eager(cuda):
     for t in ts:
         t.join()
     assert not bad
+
+
+def test_t5_graphs_that_give_way(cuda):
+    """Graphs dropped while other threads wait for theirs: values stay those of the eager encoder; a first call captures nothing."""
+    import threading
+    from shai_amd.engines.encoders import TextEmbeddingEngine
+    from shai_amd.models.t5 import T5Config
+    eng = TextEmbeddingEngine(cfg=T5Config.tiny())
+    eager = TextEmbeddingEngine(cfg=T5Config.tiny(), use_graphs=False)
+    eng.MAX_GRAPHS, eng._graphs.IDLE = 1, 1
+    texts = ["a photo of a horse", "red", "the quick brown fox jumps over the lazy dog and more"]
+    shapes = [(1, 8), (3, 8), (2, 33)]
+    want = {s: eager.embed(texts[:s[0]], s[1]) for s in shapes}
+    assert np.array_equal(eng.embed(texts[:1], 8), want[1, 8]) and len(eng._graphs) == 0
+    bad = []
+
+    def work(s):
+        for _ in range(12):
+            if not np.array_equal(eng.embed(texts[:s[0]], s[1]), want[s]):
+                bad.append(s)
+
+    ts = [threading.Thread(target=work, args=(s,)) for s in shapes]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad and len(eng._graphs) == 1
