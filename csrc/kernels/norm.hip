@@ -237,12 +237,10 @@ void launch_layernorm(const RowNormArgs& a, hipStream_t s) { launch_row_norm<tru
 //         y = x * scale + shift  ==  (x - mean) * rstd * gamma + beta.
 // Pass 3 (optional): apply (+ SiLU) elementwise.
 // ----------------------------------------------------------------------------
-// Per-(image, group) finalize shared by the fused path (last stats block of an image) and the
-// standalone kernel: reduce the NB partials of image n, emit scale/shift [C].
+// Finalize of the fused path (the last stats block of an image): reduce the NB partials of image n, emit scale/shift [C].
 __device__ void gn_finalize_image(const float* __restrict__ part, const bf16_t* __restrict__ gamma,
                                   const bf16_t* __restrict__ beta, float* __restrict__ scale,
-                                  float* __restrict__ shift, int n, int HW, int C, int G, int NB, float eps,
-                                  bool coherent) {
+                                  float* __restrict__ shift, int n, int HW, int C, int G, int NB, float eps) {
   __shared__ float mean_s[128], rstd_s[128];
   __shared__ float red[2][256];
   const int Cg = C / G;
@@ -253,14 +251,9 @@ __device__ void gn_finalize_image(const float* __restrict__ part, const bf16_t* 
   if (lane_k < L) {
     for (int k = lane_k; k < NB; k += L) {
       const float* src = part + (((long)n * NB + k) * G + g0) * 2;
-      if (coherent) {  // written by other workgroups (possibly other XCDs) of this launch
-        a += __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        b += __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      } else {
-        const float2 v = *reinterpret_cast<const float2*>(src);
-        a += v.x;
-        b += v.y;
-      }
+      // written by other workgroups (possibly other XCDs) of this launch
+      a += __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      b += __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   red[0][threadIdx.x] = a;
@@ -463,7 +456,7 @@ __global__ void __launch_bounds__(256) gn_stats_kernel(const bf16_t* __restrict_
   }
   __syncthreads();
   if (!s_last) return;
-  gn_finalize_image(part, gamma, beta, scale, shift, n, HW, C, G, NB, eps, true);
+  gn_finalize_image(part, gamma, beta, scale, shift, n, HW, C, G, NB, eps);
 }
 
 // The same as a launch of its own: one wave per (image, group), its partials (at most 256) summed in double with all loads in

@@ -135,7 +135,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs p) 
 }
 
 // Workgroup shapes (16 MT rows of A x 16 NT rows of W, NW waves along K, D k-steps in flight), from a sweep at decode
-// sizes: enough workgroups to fill the chip come first, then fewer passes over W (MT), then fewer re-reads of A (NT).
+// sizes: enough workgroups to fill the chip come first, then fewer passes over W (MT), then fewer re-reads of A (NT).  Dense bf16
+// products reach the shapes of more than 32 rows up to 2048 columns, with a K below 512, and past a buffer's range; the others run in
+// gemm_ring.hip.
 template <typename T, typename O, int EC>
 static void stream(const GemmArgs& a, hipStream_t s) {
   auto go = [&](auto kernel, int mt, int nt, int nw) {
