@@ -18,6 +18,8 @@
 // 14 bytes per clock and CU, LDS-DMA 30.)
 #include "gemm_lds_kernel.h"
 
+#include <type_traits>
+
 namespace shai {
 
 namespace {
@@ -36,8 +38,21 @@ void launch_one(const GemmArgs& a, float* ws, int splits, int kps, hipStream_t s
   constexpr size_t lds = (size_t)ST * (BM + BN) * BK2 * sizeof(bf16_t);
   static_assert(lds <= 160 * 1024, "ring larger than a CU's LDS");
   const dim3 grid(tiles, SPLITK ? splits : (a.batch > 0 ? a.batch : 1));
-  gemm2_kernel<BM, BN, D.wm, D.wn, CONV, CONV, GLU, ACT, SPLITK, ST, D.wk>
-      <<<grid, D.wm * D.wn * D.wk * 64, lds, s>>>(a, ws, kps, nullptr);
+  auto run = [&](auto epi) {
+    gemm2_kernel<BM, BN, D.wm, D.wn, CONV, CONV, GLU, ACT, SPLITK, ST, D.wk, decltype(epi)::value>
+        <<<grid, D.wm * D.wn * D.wk * 64, lds, s>>>(a, ws, kps, nullptr);
+  };
+#define SHAI_EPI(E) run(std::integral_constant<int, E>())
+  if constexpr (SPLITK) {
+    SHAI_EPI(0);
+  } else {
+    const bool eight = epilogue8_fits<GLU>(a);
+    if constexpr (!CONV) {
+      if (a.row_mr != nullptr) return eight ? SHAI_EPI(kEpi8 | kEpiLn) : SHAI_EPI(kEpiLn);
+    }
+    eight ? SHAI_EPI(kEpi8) : SHAI_EPI(0);
+  }
+#undef SHAI_EPI
 }
 
 template <int W, bool CONV>

@@ -101,15 +101,16 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& p, bf16_t* C, const bf
   }
 }
 
-// Whether rows and bases of everything epilogue8 touches are aligned for its accesses: 16 bytes, or 8 for the output side of a GLU.
+// Whether the width, and rows and bases of everything epilogue8 touches, allow its accesses: 16 bytes, or 8 for the output side of a GLU.
 template <bool GLU>
-__device__ __forceinline__ bool epilogue8_aligned(const GemmArgs& p, const bf16_t* C, const bf16_t* R) {
+inline bool epilogue8_fits(const GemmArgs& a) {
   constexpr int OUT = GLU ? 4 : 8;  // columns stored per call
-  long rows = p.ldc;
-  uintptr_t out = (uintptr_t)C, in = (uintptr_t)p.bias | (uintptr_t)p.bias2d;
-  if (R) rows |= p.ldr, out |= (uintptr_t)R;
-  if (p.gate) rows |= p.gate_stride, out |= (uintptr_t)p.gate;
-  return (rows & (OUT - 1)) == 0 && (out & (2 * OUT - 1)) == 0 && (in & 15) == 0 && (!p.bias2d || (p.N & 7) == 0);
+  long rows = a.ldc;
+  uintptr_t out = (uintptr_t)a.C;
+  if (a.residual) rows |= a.ldr, out |= (uintptr_t)a.residual;
+  if (a.gate) rows |= a.gate_stride, out |= (uintptr_t)a.gate;
+  if (a.batch > 1) rows |= a.batch_c | (a.residual ? a.batch_r : 0);
+  return a.N % 8 == 0 && (rows & (OUT - 1)) == 0 && (out & (2 * OUT - 1)) == 0 && (((uintptr_t)a.bias | (uintptr_t)a.bias2d) & 15) == 0;
 }
 
 template <int V>
@@ -125,7 +126,7 @@ __device__ __forceinline__ void load_bf(const bf16_t* src, float (&x)[V]) {
   }
 }
 
-// epilogue4 for the 8 consecutive columns n .. n + 7 of row m, all below N, with epilogue8_aligned true: the same operations in
+// epilogue4 for the 8 consecutive columns n .. n + 7 of row m, all below N, with epilogue8_fits true: the same operations in
 // the same order, one 16-byte access (8 bytes on the output side of a GLU) instead of two.
 template <bool GLU, int ACT>
 __device__ __forceinline__ void epilogue8(const GemmArgs& p, bf16_t* C, const bf16_t* R, int m, int n, float (&v)[8], int b) {

@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace shai {
 
@@ -84,12 +85,30 @@ template <int BM, int BN, int WM, int WN, bool CONV, bool FAST, bool GLU, int AC
 static void launch_cfg(const GemmArgs& a, float* ws, int splits, int kps, hipStream_t s, unsigned* cnt) {
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   dim3 grid(tiles, SPLITK ? splits : (a.batch > 0 ? a.batch : 1));
-  if (g_stages() == 3 && (size_t)3 * (BM + BN) * BK2 * sizeof(bf16_t) <= 160 * 1024) {
-    const size_t lds = (size_t)3 * (BM + BN) * BK2 * sizeof(bf16_t);
-    gemm2_kernel<BM, BN, WM, WN, CONV, FAST, GLU, ACT, SPLITK, 3><<<grid, WM * WN * 64, lds, s>>>(a, ws, kps, cnt);
+  auto go = [&](auto kernel, int stages) {
+    kernel<<<grid, WM * WN * 64, (size_t)stages * (BM + BN) * BK2 * sizeof(bf16_t), s>>>(a, ws, kps, cnt);
+  };
+  auto run = [&](auto epi) {
+    constexpr int E = decltype(epi)::value;
+    if constexpr (3 * (BM + BN) * BK2 * sizeof(bf16_t) <= 160 * 1024 && !(E & kEpiLn)) {
+      if (g_stages() == 3) return go(gemm2_kernel<BM, BN, WM, WN, CONV, FAST, GLU, ACT, SPLITK, 3, 1, E>, 3);
+    }
+    go(gemm2_kernel<BM, BN, WM, WN, CONV, FAST, GLU, ACT, SPLITK, 2, 1, E>, 2);
+  };
+  if constexpr (SPLITK) {
+    run(std::integral_constant<int, 0>());
   } else {
-    const size_t lds = (size_t)2 * (BM + BN) * BK2 * sizeof(bf16_t);
-    gemm2_kernel<BM, BN, WM, WN, CONV, FAST, GLU, ACT, SPLITK, 2><<<grid, WM * WN * 64, lds, s>>>(a, ws, kps, cnt);
+    const bool eight = epilogue8_fits<GLU>(a);
+    if constexpr (!CONV) {
+      if (a.row_mr != nullptr) {
+        if (eight) return run(std::integral_constant<int, kEpi8 | kEpiLn>());
+        // 10 blocks of accumulators a wave, 4 columns at a time and a GELU spill: 256 x 256 then
+        if constexpr (BM * BN / (WM * WN) > 8 * 1024) return launch_cfg<256, 256, 4, 2, CONV, FAST, GLU, ACT, false>(a, ws, splits, kps, s, cnt);
+        else return run(std::integral_constant<int, kEpiLn>());
+      }
+    }
+    if (eight) run(std::integral_constant<int, kEpi8>());
+    else run(std::integral_constant<int, 0>());
   }
 }
 

@@ -23,8 +23,13 @@ __device__ __forceinline__ void glds16(__amdgpu_buffer_rsrc_t r, bf16_t* lds_wav
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds_wave_base, 16, voff, 0, 0, 0);
 }
 
+// Epilogue of an unsplit kernel: 8 columns a lane (epilogue8) instead of 4, and a folded LayerNorm.  Kernels of their own: all of it in
+// one costs the large tiles their registers (256 x 320: 220, in one kernel 256 and spills, 8192 x 4096 x 4096 330 -> 1790 us) and
+// widths that 16 bytes do not fit a tenth (8192 x 330 x 1024 at 128 x 128: 37.5 -> 40.8).
+enum { kEpi8 = 1, kEpiLn = 2 };
+
 // WK > 1: that many groups of WM x WN waves, each taking 4 / WK of a K-tile's MFMA steps of the whole tile.
-template <int BM, int BN, int WM, int WN, bool CONV, bool FAST, bool GLU, int ACT, bool SPLITK, int STAGES, int WK = 1>
+template <int BM, int BN, int WM, int WN, bool CONV, bool FAST, bool GLU, int ACT, bool SPLITK, int STAGES, int WK = 1, int EPI = 0>
 __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs p, float* __restrict__ ws, int k_per_split,
                                                              unsigned* __restrict__ cnt) {
   constexpr int NW = WM * WN * WK;
@@ -225,12 +230,12 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
 
   const int nk = k_end > k_begin ? (k_end - k_begin + BK2 - 1) / BK2 : 0;
   const int fr = lane & 31, fh = lane >> 5;
-  // W's fragment rows: in order where fp32 partials are stored (4 columns are 16 bytes); else with bits 2 and 3 of the row
-  // exchanged, so that a lane's register groups 2h and 2h + 1 are the 8 consecutive columns 16h + 8fh of the 32 and one 16-byte
-  // store takes them.  8-byte stores, 32 rows by 16 bytes an instruction, were most of a short K's time: 6304 x 3072, K = 64
-  // 21.5 -> 14.7 us at the 128 x 64 tile, K = 768 53.4 -> 48.4 (128 x 128: 51.2 -> 44.3), 8192 x 960, K = 320 14.5 -> 12.2,
-  // 6304 x 768, K = 768 17.8 -> 15.7.  (Whole lines by way of LDS: 1 .. 3 % more, not worth the second path.)
-  const int fw = SPLITK ? fr : (fr & 19) | (fr & 4) << 1 | (fr & 8) >> 1;
+  // W's fragment rows: in order, or, for 8 columns a lane, with bits 2 and 3 of the row exchanged, so that a lane's register groups 2h
+  // and 2h + 1 are the 8 consecutive columns 16h + 8fh of the 32 and one 16-byte store takes them.  8-byte stores, 32 rows by 16 bytes
+  // an instruction, were most of a short K's time: 6304 x 3072, K = 64 21.5 -> 14.7 us at the 128 x 64 tile, K = 768 53.4 -> 48.4 (128 x
+  // 128: 51.2 -> 44.3), 8192 x 960, K = 320 14.5 -> 12.2, 6304 x 768, K = 768 17.8 -> 15.7.  (Whole lines by way of LDS: 1 .. 3 % more,
+  // not worth the second path.)
+  const int fw = EPI & kEpi8 ? (fr & 19) | (fr & 4) << 1 | (fr & 8) >> 1 : fr;
   auto compute = [&](int buf) {
     const bf16_t* sa = smem + buf * STAGE;
     const bf16_t* sw = sa + BM * BK2;
@@ -284,8 +289,8 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
-  // ---- epilogue: lane owns row m, 4 groups of 4 consecutive n per 32x32 block (without split-K two of 8).  WK > 1: the wave groups' sums meet in LDS
-  // (the ring is free by now) and are added in group order; each group finishes 4 / WK of the four column groups.
+  // ---- epilogue: lane owns row m, 4 groups of 4 consecutive n (2 of 8 with kEpi8) per 32x32 block.  WK > 1: the wave groups' sums meet in
+  // LDS (the ring is free by now) and are added in group order; each group finishes 4 / WK of the four column groups.
   if constexpr (WK > 1) {
     static_assert(NW * IM * JN * 4096 <= STAGES * STAGE * 2, "partial tiles larger than the ring");
     float4_* part = reinterpret_cast<float4_*>(smem);
@@ -313,7 +318,6 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
       }
   }
   constexpr int G1 = 4 / WK;
-  static_assert(G1 >= 2, "a lane's two column groups lie in one wave group");
   const int g0 = wk * G1;
   // In-launch split-K fixup (tiles with <= 4 32x32 blocks per wave; the skinny kernel's write-through hand-off, gemv.hip): every K group
   // stores its fp32 partial tile write-through (sc1), drains, joins the barrier and takes a ticket; the group
@@ -447,47 +451,36 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
   } else {
     bf16_t* C = p.C + (long)b * p.batch_c;
     const bf16_t* R = p.residual ? p.residual + (long)b * p.batch_r : nullptr;
-    const bool wide = epilogue8_aligned<GLU>(p, C, R);
+    constexpr int V = EPI & kEpi8 ? 8 : 4;
+    static_assert(G1 * 4 % V == 0, "a lane's columns lie in one wave group");
 #pragma unroll
     for (int i = 0; i < IM; ++i) {
       const int m = m0 + wm * TM + i * 32 + fr;
       if (m >= p.M) continue;
-      float2 mr = make_float2(0.f, 1.f);
-      if constexpr (!CONV) {
-        if (p.row_mr != nullptr) mr = *reinterpret_cast<const float2*>(p.row_mr + 2 * (long)m);
-      }
+      [[maybe_unused]] float2 mr;
+      if constexpr (EPI & kEpiLn) mr = *reinterpret_cast<const float2*>(p.row_mr + 2 * (long)m);
 #pragma unroll
       for (int j = 0; j < JN; ++j)
 #pragma unroll
-        for (int h = 0; h < G1 / 2; ++h) {
-          const int n = n0 + wn * TN + j * 32 + 16 * (g0 / 2 + h) + 8 * fh;
-          float v[8];
+        for (int g = 0; g < G1 * 4 / V; ++g) {
+          const int n = n0 + wn * TN + j * 32 + 8 * g0 + 2 * V * g + V * fh;
+          if (n >= p.N) continue;
+          float v[V];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = acc[i][j][8 * h + e];
-          if constexpr (!CONV) {
-            if (p.row_mr != nullptr) {  // LayerNorm of A folded in: rstd[m] * (acc - mean[m] * s[n]), W carries the gain
-              float s[8];
-              if (n + 7 < p.N) {
+          for (int e = 0; e < V; ++e) v[e] = acc[i][j][V * g + e];
+          if constexpr (EPI & kEpiLn) {  // LayerNorm of A folded in: rstd[m] * (acc - mean[m] * s[n]), W carries the gain
 #pragma unroll
-                for (int q = 0; q < 8; q += 4) {
-                  const float4_ t = *reinterpret_cast<const float4_*>(p.col_s + n + q);
-                  s[q] = t[0]; s[q + 1] = t[1]; s[q + 2] = t[2]; s[q + 3] = t[3];
-                }
-              } else {
+            for (int q = 0; q < V; q += 4) {
+              float4_ s = {0.f, 0.f, 0.f, 0.f};
+              if (V == 8 || n + 3 < p.N) s = *reinterpret_cast<const float4_*>(p.col_s + n + q);
+              else
+                for (int e = 0; e < 4 && n + e < p.N; ++e) s[e] = p.col_s[n + e];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) s[e] = n + e < p.N ? p.col_s[n + e] : 0.f;
-              }
-#pragma unroll
-              for (int e = 0; e < 8; ++e) v[e] = mr.y * fmaf(-mr.x, s[e], v[e]);
+              for (int e = 0; e < 4; ++e) v[q + e] = mr.y * fmaf(-mr.x, s[e], v[q + e]);
             }
           }
-          if (wide && n + 7 < p.N) {
-            epilogue8<GLU, ACT>(p, C, R, m, n, v, b);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 8; q += 4)
-              if (n + q < p.N) epilogue4<GLU, ACT>(p, C, R, m, n + q, v + q, b);
-          }
+          if constexpr (V == 8) epilogue8<GLU, ACT>(p, C, R, m, n, v, b);
+          else epilogue4<GLU, ACT>(p, C, R, m, n, v, b);
         }
     }
   }
