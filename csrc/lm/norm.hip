@@ -114,9 +114,11 @@ __device__ __forceinline__ float4_ wide4(uint2_ v) {
 // workgroup walks `run` consecutive rows, two of them loaded ahead, and keeps the last taps - 1 inputs in registers; the ones before its first row are recomputed from their
 // residual rows (which is why x_out is not x then) or, before the step's first row of a sequence, come from the sequence's
 // state.  Whatever the rows share (gains, taps, the rows' places) is read before the first row: a load inside the loop
-// would wait for the rows ahead of it.  TD: the type of delta.
+// would wait for the rows ahead of it.  TD: the type of delta.  MANY: partial sums and no convolution, up to seven loads at a time
+// (16 rows of 2048, 8 parts 6.2 -> 5.2 us, 4 parts 5.3 -> 5.0).  In the one kernel they took registers from all: with 4 taps and 4 parts 7.6
+// -> 8.8, with 8 taps 11 -> 23, and 2048 fp32 rows without either 11.7 -> 13.0.
 constexpr int conv_waves(int taps, int nt, int nv) { return taps > 0 && taps <= 4 && nt <= 512 && nv <= 2 ? 4 : 1; }   // per SIMD
-template <typename T, typename TD, int NT, int NV, int TAPS>
+template <typename T, typename TD, int NT, int NV, int TAPS, bool MANY = false>
 __global__ void __launch_bounds__(NT, conv_waves(TAPS, NT, NV)) residual_norm_kernel(const ResidualNormArgs p) {
   constexpr bool CONV = TAPS > 0, KEEP = CONV && TAPS <= 4 && NV <= 2;   // KEEP: taps in registers
   constexpr int KN = KEEP ? NV : 1, KT = KEEP ? TAPS : 1;
@@ -152,14 +154,14 @@ __global__ void __launch_bounds__(NT, conv_waves(TAPS, NT, NV)) residual_norm_ke
               s += p.wts[row * p.top + k] * load4(static_cast<const T*>(p.ye) + (long)p.slot_of[row * p.top + k] * p.Dp + c);
             q.d[i] = s;
           }
-          for (int k = 1; p.parts > 4 && k < p.parts; k += 7) {   // 8 parts: seven loads at a time, none waited for alone
+          for (int k = 1; MANY && p.parts > 4 && k < p.parts; k += 7) {   // 8 parts: seven loads at a time, none waited for alone
             float4_ e[7];
 #pragma unroll
             for (int j = 0; j < 7; ++j) e[j] = raw4(d + min(k + j, p.parts - 1) * p.part_stride + c);
 #pragma unroll
             for (int j = 0; j < 7; ++j) q.d[i] += k + j < p.parts ? e[j] : zero;
           }
-          for (int k = 1; p.parts <= 4 && k < p.parts; k += 3) {
+          for (int k = 1; !(MANY && p.parts > 4) && k < p.parts; k += 3) {   // three loads at a time
             float4_ e[3];
 #pragma unroll
             for (int j = 0; j < 3; ++j) e[j] = raw4(d + min(k + j, p.parts - 1) * p.part_stride + c);
@@ -394,6 +396,9 @@ void launch_add_norm(const AddNormArgs& a, bool f32, hipStream_t s) { SHAI_LM_RO
 template <typename T, typename TD, int NT, int NV>
 static void residual_norm(const ResidualNormArgs& a, hipStream_t s) {
   const int grid = a.cw ? (a.T + a.run - 1) / a.run : a.T;
+  if constexpr (sizeof(TD) == 4) {
+    if (!a.cw && a.parts > 1) return residual_norm_kernel<T, TD, NT, NV, 0, true><<<grid, NT, 0, s>>>(a);
+  }
   if (!a.cw) residual_norm_kernel<T, TD, NT, NV, 0><<<grid, NT, 0, s>>>(a);
   else if (a.taps <= 2) residual_norm_kernel<T, TD, NT, NV, 2><<<grid, NT, 0, s>>>(a);
   else if (a.taps <= 4) residual_norm_kernel<T, TD, NT, NV, 4><<<grid, NT, 0, s>>>(a);

@@ -1,5 +1,5 @@
-"""Tiles of csrc/kernels/gemm_lds_kernel.h keep their accumulators in registers: a tile that spills took five times its time, with the
-right results.  Read from the kernels' metadata in the built library."""
+"""Kernels that must keep their values in registers: a GEMM tile that spilled took five times its time, a norm with a convolution twice,
+with the right results.  Read from the kernels' metadata in the built libraries."""
 import os
 import re
 import shutil
@@ -10,13 +10,13 @@ import pytest
 from shai_amd import native
 
 READELF = shutil.which("llvm-readelf", path="/opt/rocm/llvm/bin")
-if READELF is None or not os.path.exists(native.KERNELS_LIB):
-    pytest.skip("needs the native library and llvm-readelf", allow_module_level=True)
+if READELF is None or not os.path.exists(native.KERNELS_LIB) or not os.path.exists(native.LM_LIB):
+    pytest.skip("needs the native libraries and llvm-readelf", allow_module_level=True)
 
 
-def spills(tmp_path):
-    """{kernel: registers spilled} over the device objects of the library."""
-    data, out = open(native.KERNELS_LIB, "rb").read(), {}
+def spills(lib, tmp_path):
+    """{kernel: registers spilled} over the device objects of a library."""
+    data, out = open(lib, "rb").read(), {}
     at = [m.start() for m in re.finditer(b"\x7fELF", data)][1:]     # behind the library's own header
     for i, (a, b) in enumerate(zip(at, at[1:] + [len(data)])):
         f = tmp_path / f"{i}.o"
@@ -28,6 +28,15 @@ def spills(tmp_path):
 
 
 def test_gemm_tiles_do_not_spill(tmp_path):
-    tiles = {k: n for k, n in spills(tmp_path).items() if "gemm2_kernel" in k}
+    tiles = {k: n for k, n in spills(native.KERNELS_LIB, tmp_path).items() if "gemm2_kernel" in k}
     assert len(tiles) > 100
     assert not {k: n for k, n in tiles.items() if n}
+
+
+def test_norms_do_not_spill(tmp_path):
+    """Without a convolution; with one of two taps, rows up to 4096 columns."""
+    norms = {k: n for k, n in spills(native.LM_LIB, tmp_path).items() if "residual_norm_kernel" in k}
+    plain = [k for k in norms if "ELi0ELb" in k]
+    conv = [k for k in norms if re.search(r"Li(256|512)ELi[12]ELi2ELb", k)]
+    assert len(plain) >= 15 and len(conv) >= 9
+    assert not {k: norms[k] for k in plain + conv if norms[k]}
