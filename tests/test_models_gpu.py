@@ -309,3 +309,26 @@ def test_t5_graphs_that_give_way(cuda):
     for t in ts:
         t.join()
     assert not bad and len(eng._graphs) == 1
+
+
+def test_extend_returns_copies(cuda):
+    """Logits of single-token steps: of all rows in order, of some of them in another; the next step leaves them alone."""
+    from shai_amd.engines.llm import LLMEngine
+    from shai_amd.models.llama import LlamaConfig
+    c = LlamaConfig(vocab_size=1024, hidden_size=512, intermediate_size=512, num_hidden_layers=2,
+                    num_attention_heads=8, num_key_value_heads=8, head_dim=64, max_position_embeddings=512)
+    toks = np.random.default_rng(0).integers(3, 1000, (3, 12)).tolist()
+    whole = LLMEngine(c, device="cuda", max_num_seqs=4, max_model_len=64, seed=2, use_graphs=False)
+    want = [whole.extend([(whole.open_request(), t, list(range(12)))]).float().cpu() for t in toks]
+    eng = LLMEngine(c, device="cuda", max_num_seqs=4, max_model_len=64, seed=2)
+    rs = [eng.open_request() for _ in toks]
+    eng.extend([(r, t[:4], []) for r, t in zip(rs, toks)])
+    steps = []                                             # read after the last step only
+    for i in range(4, 12):
+        order = [0, 1, 2] if i % 2 else [2, 0, 1]
+        wanted = order if i % 4 < 2 else [b for b in order if b != 1]
+        steps.append((i, wanted, eng.extend([(rs[b], [toks[b][i]], [0] if b in wanted else []) for b in order])))
+    for i, wanted, got in steps:
+        assert got.shape == (len(wanted), 1024)
+        for b, row in zip(wanted, got.float().cpu()):
+            assert ((row - want[b][i]).norm() / want[b][i].norm()).item() < 2e-2, (i, b)
