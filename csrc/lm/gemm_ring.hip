@@ -157,9 +157,10 @@ static int ring_blocks(const GemmArgs& a) {
 //     8192: 9 rows 1.05, 12 1.04, 16 0.94; 17424 x 2048: 9 rows 0.96, 16 0.86);
 //   below: 33 rows from 2049 columns on (2304 x 4096, 64 rows: 24.2 -> 15.5; 2048 x 2048 8.5 -> 9.4), and 17 to 32 rows where M K >=
 //     24 * 1024 (2048 x 2048, 32 rows: 8.4 -> 7.5; 4096 x 1024: 17 rows 1.03 of the time, 24 rows 0.99);
-//   partial sums: more than 16 rows, or a K of 8192; of a K of 4096 from 2049 columns on, and in 8 parts from 9 rows on: 1024 x 4096 in
-//     4 parts, 8 rows 8.1 -> 8.7, 32 rows 10.5 -> 9.3; 2048 x 4096 in 8, 1 row 9.8 -> 10.2, 16 rows 11.7 -> 11.0; x 12544, 1 row 16.5
-//     either way, 16 rows 20.7 -> 16.8.
+//   partial sums: more than 16 rows (512 x 8448 in 8 parts, 17 rows: 6.8 -> 5.8); up to 16 of a K of 4096, from 2049 columns on, or
+//     where 32-column workgroups of all parts fill 7 of 8 CUs and either 9 rows or a K of 8192 are there: 2048 x 8448 in 4 parts,
+//     1 row 10.2 -> 9.4, 16 rows 11.4 -> 9.3; x 6144, 9 rows 8.1 -> 7.5; 1024 x 12544 in 8, 1 row 8.0 ->
+//     7.9, 16 rows 9.1 -> 7.8; with half of the CUs the streaming kernel's 16 columns are faster: 512 x 8448 in 8, 1 row 4.8 -> 5.3.
 //   Up to 32 rows more columns than one round of 112 (ring_blocks) take a K, or part of one, of 3072: 32768 x 1024, 32 rows 1.09 of
 //     the time, x 4096 0.98; 8192 x 2048 in 4 parts, 8 rows 15.6 -> 19.0.
 // Products per head, grouped by expert or longer than a buffer's range stay with the streaming kernel.
@@ -168,7 +169,7 @@ bool gemm_ring_fits(const GemmArgs& a) {
   if (a.tiles || a.batch > 1 || a.M > 64 || a.K < 512 || a.N < 512 || (long)a.N * a.K * 2 >= lim || (long)a.M * a.lda * 2 >= lim)
     return false;
   if (a.M <= 32 && a.N * splits > kRound && a.K / splits < 3072) return false;
-  if (splits > 1) return a.M > 16 || a.K >= 8192 || (a.K >= 4096 && (a.N > 2048 || (splits >= 8 && a.M > 8)));
+  if (splits > 1) return a.M > 16 || (a.K >= 4096 && (a.N > 2048 || (a.N * splits >= 224 * 32 && (a.M > 8 || a.K >= 8192))));
   if (a.N > 4096) return a.M >= (a.N <= 7168 ? 9 : 12);
   return a.M > 32 ? a.N > 2048 : a.M > 16 && a.M * a.K >= 24 * 1024;
 }

@@ -163,22 +163,32 @@ def matmul_joint(a, w, out, act: int, side: int):
     return s
 
 
+def parts(M: int, N: int, K: int) -> int:
+    """How many partial sums :func:`matmul_parts` makes of a bf16 product of M rows, N columns and K."""
+    if M <= 64:
+        if N > PARTS_COLUMNS or K < PARTS * 128:
+            return 1
+        # Twice as many of a long K where four leave CUs without one of the ring's 32-column workgroups: 1536 x 8448, 1 row 9.5 -> 7.8 us,
+        # 16 rows 11.1 -> 7.9; not 1024 x 4096, up to 16 rows 4.4 to 4.8 either way.  From 1792 columns on the product gains nothing, and the
+        # norm that adds them loses 0.3 us, 0.8 with a convolution: 2048 x 8448 with it, 1 row 15.6 in four parts, 16.4 in eight.  But for
+        # more rows with a K from 9216 on: 2048 x 12544, 16 rows 12.8 and 12.7, 32 rows 13.8 and 13.2, 64 rows 15.9 and 15.0.
+        if N < 1792:
+            deep = K >= 4096 and not (512 < N <= 1024 and K < 5120 and M <= 16)
+        else:
+            deep = N <= 2048 and M > 24 and K >= 9216
+        return 2 * PARTS if deep else PARTS
+    tiles = -(-M // 128) * (-(-N // 128))       # tiles of 128 x 128: two for each of the 256 CUs
+    return min(PARTS, 512 // tiles, K // 512) if tiles < 256 else 1
+
+
 def matmul_parts(a, w, out_dtype=None):
     """a w^T for a consumer that adds partial sums (:func:`residual_norm`, :func:`latent_prep`): [parts, M, N] fp32
     where the product needs K cut up to fill the chip (few rows, few columns); else :func:`matmul`."""
     M, K, N = a.shape[0], a.shape[1], w.shape[0]
-    if M <= 64:
-        # Twice as many of a long K, up to 2048 columns: more of the streaming kernel's narrow workgroups (64 x 4096, 32 rows, with
-        # the norm that adds them: 9.6 -> 7.9 us), wider ones of the ring's (2048 x 12544, 16 rows: 17.1 -> 16.8; 4 parts before the
-        # ring: 21.7).  Not where that is slower: 768 x 4096, 8 rows 7.8 -> 8.1.
-        deep = N <= 2048 and K >= 4096 and not (512 < N <= 1024 and K < 5120 and M <= 16)
-        parts = (2 * PARTS if deep else PARTS) if N <= PARTS_COLUMNS and K >= PARTS * 128 else 1
-    else:   # tiles of 128 x 128: two for each of the 256 CUs
-        tiles = -(-M // 128) * (-(-N // 128))
-        parts = min(PARTS, 512 // tiles, K // 512) if tiles < 256 else 1
-    if not a.is_cuda or a.dtype != torch.bfloat16 or parts <= 1:
+    n = parts(M, N, K) if a.is_cuda and a.dtype == torch.bfloat16 else 1
+    if n <= 1:
         return matmul(a, w, out_dtype)
-    c = torch.empty(parts, M, N, dtype=torch.float32, device=a.device)
+    c = torch.empty(n, M, N, dtype=torch.float32, device=a.device)
     _K().lm_gemm_parts(a, w, c)
     return c
 

@@ -4,6 +4,7 @@ import os
 import pytest
 
 from shai_amd import native
+from shai_amd.ops import lm
 
 if not os.path.exists(native.LM_LIB):
     pytest.skip("the native library is not built", allow_module_level=True)
@@ -25,9 +26,20 @@ def test_few_rows(M, N, K, want):
 @pytest.mark.parametrize("M,N,K,splits,want", [
     (16, 1024, 2048, 4, "stream"), (17, 1024, 2048, 4, "ring"), (1, 2048, 8192, 8, "ring"), (8, 2048, 4096, 8, "stream"),
     (9, 2048, 4096, 8, "ring"), (1, 2304, 4096, 4, "ring"), (1, 3072, 4032, 4, "stream"), (16, 1024, 4096, 4, "stream"),
-    (1, 8192, 4096, 4, "stream"), (32, 8192, 512, 4, "stream"), (33, 8192, 512, 4, "ring")])
+    (1, 8192, 4096, 4, "stream"), (32, 8192, 512, 4, "stream"), (33, 8192, 512, 4, "ring"),
+    (9, 2048, 4096, 4, "ring"), (8, 2048, 8128, 4, "stream"), (1, 1792, 8192, 4, "ring"), (16, 1728, 8192, 4, "stream"),
+    (16, 512, 8192, 8, "stream"), (17, 512, 8192, 8, "ring"), (16, 832, 8192, 8, "stream"), (1, 896, 8192, 8, "ring")])
 def test_parts(M, N, K, splits, want):
     assert form(M, N, K, splits) == want
+
+
+# partial sums: eight where four would leave CUs idle, and of many rows and a long K; a norm pays for every one of them
+@pytest.mark.parametrize("M,N,K,want", [
+    (1, 2048, 8448, 4), (24, 2048, 12544, 4), (25, 2048, 9216, 8), (64, 2048, 9152, 4), (64, 2056, 12544, 4), (1, 1792, 8448, 4),
+    (1, 1784, 4096, 8), (1, 1784, 4032, 4), (16, 1024, 5056, 4), (16, 1024, 5120, 8), (17, 1024, 4096, 8), (1, 512, 4096, 8), (1, 8192, 512, 4),
+    (1, 8193, 512, 1), (1, 2048, 448, 1), (65, 2048, 8448, 4), (600, 8192, 4096, 1)])
+def test_number_of_parts(M, N, K, want):
+    assert lm.parts(M, N, K) == want
 
 
 # 64 x 64 tiles up to two for each CU, more with a K of 2048; 128 x 128 up to one; 256 x 256 from 192 on
