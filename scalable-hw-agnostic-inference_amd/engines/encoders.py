@@ -229,7 +229,8 @@ class TextEmbeddingEngine:
     """T5 sentence embeddings.  An encoder step is some 200 launches that the host takes longer to issue than a small batch to run, so
     batch shapes of up to ``GRAPH_TOKENS`` tokens that come again run as HIP graphs (:class:`ShapeGraphs`, up to ``MAX_GRAPHS``);
     with tensor parallelism eagerly.  T5-v1.1-large, ms eager -> graph: 1 text of 32 tokens 2.25 -> 1.16, 8 of 32 2.29 -> 1.50, 16 of 32
-    2.33 -> 1.87, 8 of 128 2.46 -> 2.38, 32 of 128 6.1 either way; the call that captures 3.8."""
+    2.33 -> 1.87, 8 of 128 2.46 -> 2.38, 32 of 128 6.1 either way; the call that captures 3.5 to 4.5, and up to 20 more where the
+    allocator holds much unused memory, as after loading weights: a capture gives that back first."""
 
     MAX_GRAPHS, GRAPH_TOKENS = 16, 512
 
