@@ -395,10 +395,42 @@ struct OutStats {
   float* gn_part = nullptr;
   float* ln_mr = nullptr;
   float ln_eps = 1e-5f;
+  // GroupNorm of the output in one launch (groupnorm.hip), behind a split-K choice the fold with it; keep: the output itself is wanted
+  const shai::GnOneArgs* one = nullptr;
+  bool keep = true;
   bool any() const { return gn_part != nullptr || ln_mr != nullptr; }
 };
 
+// The convolution with its output's GroupNorm (st->one).
+void launch_with_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, const OutStats& st) {
+  shai::GnOneArgs n = *st.one;
+  const bool fold = c.cfg >= 0 && c.cfg < shai::gemm2_num_cfgs() && c.splits > 1 && shai::gemm2_cfg_supported(g, c.cfg) &&
+                    shai::gemm2_cfg_splittable(c.cfg) && g.act == 0 && g.upsample != 2 && shai::gn_one_supported(n.HW, n.C, n.G, true);
+  if (!fold) {
+    launch_choice(g, like, c);
+    n.x = g.C;
+    shai::launch_gn_one(n, stream());
+    return;
+  }
+  Tensor ws = at::empty({(long)c.splits * g.M * g.N}, like.options().dtype(at::kFloat));
+  g.no_fold = 1;
+  shai::launch_gemm2_cfg(g, ws.data_ptr<float>(), c.cfg, c.splits, stream());
+  n.parts = ws.data_ptr<float>();
+  n.splits = c.splits;
+  n.bias = g.bias;
+  n.bias2d = g.bias2d;
+  n.bias2d_ld = g.bias2d_ld;
+  n.residual = g.residual;
+  n.res_alpha = g.res_alpha;
+  n.raw = st.keep ? g.C : nullptr;
+  shai::launch_gn_one(n, stream());
+}
+
 void launch_final(shai::GemmArgs g, const Tensor& like, const Choice& c, const OutStats* st) {
+  if (st != nullptr && st->one != nullptr) {
+    launch_with_norm(g, like, c, *st);
+    return;
+  }
   if (st == nullptr || !st->any()) {
     launch_choice(g, like, c);
     return;
@@ -443,6 +475,11 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
                  " is not implemented for this input layout");
     }
     shai::launch_gemm(g, stream());
+    if (st && st->one) {
+      shai::GnOneArgs n = *st->one;
+      n.x = g.C;
+      shai::launch_gn_one(n, stream());
+    }
     if (st && st->any()) {  // v1 writes no statistics
       if (st->gn_part) shai::launch_col_partials(g.C, g.M, g.N, g.ldc, st->gn_part, stream());
       if (st->ln_mr) shai::launch_row_moments(g.C, g.M, g.N, g.ldc, st->ln_eps, st->ln_mr, stream());
@@ -739,6 +776,49 @@ void groupnorm_apply(const Tensor& x, const optional<Tensor>& x2, const Tensor& 
   shai::launch_groupnorm_apply(a, stream());
 }
 
+shai::GnOneArgs gn_one_args(const optional<Tensor>& gamma, const optional<Tensor>& beta, const Tensor& out, int64_t N, int64_t HW,
+                            int64_t C, int64_t G, double eps, bool silu) {
+  shai::GnOneArgs n{};
+  for (const optional<Tensor>* t : {&gamma, &beta})
+    if (*t) {
+      check_bf16(**t, "groupnorm weight");
+      SHAI_CHECK((*t)->is_contiguous() && (*t)->numel() == C && ((uintptr_t)(*t)->data_ptr() & 7) == 0, "groupnorm weight / bias [C], 8-byte aligned");
+    }
+  SHAI_CHECK(((uintptr_t)out.data_ptr() & 7) == 0, "groupnorm output must be 8-byte aligned");
+  n.gamma = optr(gamma);
+  n.beta = optr(beta);
+  n.out = mptr(out);
+  n.N = N;
+  n.HW = HW;
+  n.C = n.C1 = C;
+  n.G = G;
+  n.eps = eps;
+  n.silu = silu;
+  return n;
+}
+
+bool groupnorm_one_supported(int64_t HW, int64_t C, int64_t G, bool fold) {
+  return HW < (1 << 20) && C <= 8192 && shai::gn_one_supported(HW, C, G, fold);
+}
+
+// GroupNorm (+ SiLU) of a small image in one launch
+void groupnorm_one(const Tensor& x, const optional<Tensor>& x2, const optional<Tensor>& gamma, const optional<Tensor>& beta,
+                   const Tensor& out, int64_t G, double eps, bool silu) {
+  shai::GroupNormArgs src{};
+  int C;
+  gn_sources(x, x2, src, &C);
+  check_bf16(out, "out");
+  SHAI_CHECK(out.is_contiguous() && out.numel() == x.size(0) * x.size(1) * (long)C, "groupnorm_one out must be [N, HW, C]");
+  SHAI_CHECK(groupnorm_one_supported(x.size(1), C, G, false), "groupnorm_one: image too large, or groups of an odd or too small width");
+  SHAI_CHECK(x.size(2) % 4 == 0 && ((uintptr_t)x.data_ptr() & 7) == 0 && (!x2 || ((uintptr_t)x2->data_ptr() & 7) == 0),
+             "groupnorm_one: 8-byte aligned pixels");
+  shai::GnOneArgs n = gn_one_args(gamma, beta, out, x.size(0), x.size(1), C, G, eps, silu);
+  n.x = cptr(x);
+  n.x2 = src.x2;
+  n.C1 = src.C1;
+  shai::launch_gn_one(n, stream());
+}
+
 // ---------------------------------------------------------------- GEMM
 // Norm hand-off tensors of a GEMM / conv: ln_mr [M, 2] + ln_s [N] (LayerNorm of A folded in), gn_part
 // [M / 128, N, 2] (GroupNorm partials of the output), ln_stats [M, 2] (LayerNorm moments of the output).
@@ -825,6 +905,7 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
     check_bf16(*bias2d, "bias2d");
     SHAI_CHECK(bias2d->is_contiguous() && bias2d->size(-1) == g.N && rows_per_bias2d > 0, "bias2d shape");
     g.bias2d = cptr(*bias2d);
+    g.bias2d_ld = g.N;
     g.rows_per_bias2d = rows_per_bias2d;
   }
   if (residual) {
@@ -958,7 +1039,9 @@ void conv2d(const Tensor& x, const optional<Tensor>& x2, const Tensor& w, const 
             const optional<Tensor>& in_scale, const optional<Tensor>& in_shift, int64_t in_act, int64_t kh,
             int64_t kw, int64_t stride, int64_t pad, bool upsample, int64_t act, double res_alpha,
             const optional<Tensor>& ln_mr, const optional<Tensor>& ln_s, const optional<Tensor>& gn_part,
-            const optional<Tensor>& ln_stats, double ln_eps, bool up_phases) {
+            const optional<Tensor>& ln_stats, double ln_eps, bool up_phases, const optional<Tensor>& gn_gamma,
+            const optional<Tensor>& gn_beta, const optional<Tensor>& gn_out, int64_t gn_groups, double gn_eps, bool gn_silu,
+            bool keep_out) {
   check_bf16(x, "x");
   check_bf16(w, "w");
   check_bf16(out, "out");
@@ -1028,8 +1111,11 @@ void conv2d(const Tensor& x, const optional<Tensor>& x2, const Tensor& w, const 
   }
   if (bias2d) {
     check_bf16(*bias2d, "bias2d");
-    SHAI_CHECK(bias2d->is_contiguous() && bias2d->size(0) == g.Nimg && bias2d->size(-1) == g.N, "bias2d [N, Cout]");
+    // contiguous, or columns of a wider tensor that 16 bytes fit (all of a UNet's time embeddings are one product)
+    const bool columns = bias2d->dim() == 2 && bias2d->stride(1) == 1 && bias2d->stride(0) % 8 == 0 && ((uintptr_t)bias2d->data_ptr() & 15) == 0;
+    SHAI_CHECK((bias2d->is_contiguous() || columns) && bias2d->size(0) == g.Nimg && bias2d->size(-1) == g.N, "bias2d [N, Cout]");
     g.bias2d = cptr(*bias2d);
+    g.bias2d_ld = bias2d->is_contiguous() ? g.N : bias2d->stride(0);
     g.rows_per_bias2d = g.OH * g.OW;
   }
   if (residual) {
@@ -1050,12 +1136,21 @@ void conv2d(const Tensor& x, const optional<Tensor>& x2, const Tensor& w, const 
   }
   OutStats st;
   attach_norm_io(g, ln_mr, ln_s, gn_part, ln_stats, ln_eps, &st);
+  shai::GnOneArgs one{};
+  if (gn_out) {  // the GroupNorm of the output as well; keep_out false: out may be left unwritten
+    check_bf16(*gn_out, "gn_out");
+    SHAI_CHECK(gn_out->is_contiguous() && gn_out->sizes() == out.sizes(), "gn_out must be shaped as out");
+    SHAI_CHECK(!st.any() && shai::gn_one_supported(g.OH * g.OW, g.N, gn_groups, false), "conv2d: GroupNorm of this output is not supported");
+    one = gn_one_args(gn_gamma, gn_beta, *gn_out, g.Nimg, g.OH * g.OW, g.N, gn_groups, gn_eps, gn_silu);
+    st.one = &one;
+    st.keep = keep_out;
+  }
   SHAI_CHECK(g.upsample != 2 || (shai::gemm4_supported(g) && use_v2(g, x.numel() * 2, w.numel() * 2, 0)),
              "up_phases: shape not supported by the phase conv (needs Cin % 64 == 0, H W % 256 == 0, v2 GEMM path)");
   // Halo-tiled conv (conv_halo.hip): GroupNorm(+SiLU) convs (SHAI_HALO_CONV >= 1) and, at mode 2, every 3x3
   // stride-1 conv it supports; the output's GroupNorm partials come from its epilogue.
   const int hmode = halo_conv_mode();
-  if (hmode > 0 && g.row_mr == nullptr && st.ln_mr == nullptr && (g.in_scale != nullptr || hmode >= 2) &&
+  if (hmode > 0 && g.row_mr == nullptr && st.ln_mr == nullptr && st.one == nullptr && (g.in_scale != nullptr || hmode >= 2) &&
       shai::conv_halo_supported(g)) {
     g.col_part = st.gn_part;
     shai::launch_conv_halo(g, stream(), g_halo_waves);
@@ -1660,7 +1755,9 @@ TORCH_LIBRARY(shai, m) {
   m.def("dequant_fp8(Tensor w8, Tensor scale, Tensor(a!) out) -> ()");
   m.def("layernorm_mod(Tensor x, Tensor scale, Tensor shift, Tensor(a!) out, int rows_per_mod, float eps) -> ()");
   m.def("qk_norm_rope(Tensor(a!) x, Tensor? q_w, Tensor? k_w, Tensor? cos, Tensor? sin, int H, int D, int S, float eps) -> ()");
-  m.def("conv2d(Tensor x, Tensor? x2, Tensor w, Tensor(a!) out, Tensor? bias, Tensor? bias2d, Tensor? residual, Tensor? in_scale, Tensor? in_shift, int in_act, int kh, int kw, int stride, int pad, bool upsample, int act, float res_alpha, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, bool up_phases=False) -> ()");
+  m.def("conv2d(Tensor x, Tensor? x2, Tensor w, Tensor(a!) out, Tensor? bias, Tensor? bias2d, Tensor? residual, Tensor? in_scale, Tensor? in_shift, int in_act, int kh, int kw, int stride, int pad, bool upsample, int act, float res_alpha, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, bool up_phases=False, Tensor? gn_gamma=None, Tensor? gn_beta=None, Tensor(d!)? gn_out=None, int gn_groups=0, float gn_eps=1e-5, bool gn_silu=False, bool keep_out=True) -> ()");
+  m.def("groupnorm_one(Tensor x, Tensor? x2, Tensor? gamma, Tensor? beta, Tensor(a!) out, int G, float eps, bool silu) -> ()");
+  m.def("groupnorm_one_supported(int HW, int C, int G, bool fold) -> bool", &groupnorm_one_supported);
   m.def("flash_attn(Tensor q, Tensor k, Tensor v, Tensor(a!) o, float scale, bool causal, int causal_offset, Tensor? kv_lens, Tensor? q_lens, Tensor? bias, Tensor? block_table) -> ()");
   m.def("paged_attn_varlen(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor kv_lens, Tensor q_lens, Tensor q_start, int max_q, float scale, bool causal) -> ()");
   m.def("decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor ctx_lens, Tensor(b!) ws, int num_splits, float scale) -> ()");
@@ -1696,6 +1793,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("col_partials", &col_partials);
   m.impl("row_moments", &row_moments);
   m.impl("groupnorm_apply", &groupnorm_apply);
+  m.impl("groupnorm_one", &groupnorm_one);
   m.impl("gemm", &gemm);
   m.impl("dequant_fp8", &dequant_fp8);
   m.impl("gemm_f8", &gemm_f8);

@@ -463,7 +463,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
         }
         // per-image bias (time embedding) in the wide path: each wave's 128 rows lie inside one image
         const bool b2ok = p.bias2d == nullptr ||
-                          (WIDE && (p.rows_per_bias2d & 127) == 0 && (p.N & 7) == 0 && ((uintptr_t)p.bias2d & 15) == 0);
+                          (WIDE && (p.rows_per_bias2d & 127) == 0 && (p.bias2d_ld & 7) == 0 && ((uintptr_t)p.bias2d & 15) == 0);
         const bool fast = m0 + G4_BM <= p.M && n0 + BN <= p.N && b2ok && p.gate == nullptr &&
                           (p.ldc & 3) == 0 && (R == nullptr || (p.ldr & 3) == 0);
         if constexpr (WIDE) {
@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
               bt[2] = bf2f(bb[1] & 0xffff); bt[3] = bf2f(bb[1] >> 16);
             }
             if (p.bias2d != nullptr) {  // b2ok: the wave's 128 rows share one bias2d row
-              const bf16_t* b2 = p.bias2d + (long)((m0 + wm * 128) / p.rows_per_bias2d) * p.N;
+              const bf16_t* b2 = p.bias2d + (long)((m0 + wm * 128) / p.rows_per_bias2d) * p.bias2d_ld;
 #pragma unroll
               for (int q = 0; q < NP; ++q) {
                 float t8[8];
@@ -820,7 +820,7 @@ bool gemm4_stats_ok(const GemmArgs& a, int bn) {
   if (a.M % G4_BM != 0 || a.N % bn != 0 || a.ldc % 8 != 0 || !al16(a.C)) return false;
   if (a.residual != nullptr && (a.ldr % 8 != 0 || !al16(a.residual))) return false;
   if (a.bias != nullptr && !al16(a.bias)) return false;
-  if (a.bias2d != nullptr && (a.rows_per_bias2d % 128 != 0 || a.N % 8 != 0 || !al16(a.bias2d))) return false;
+  if (a.bias2d != nullptr && (a.rows_per_bias2d % 128 != 0 || a.N % 8 != 0 || a.bias2d_ld % 8 != 0 || !al16(a.bias2d))) return false;
   // phase conv over image groups (H W < 256): the GEMM's 128-row blocks interleave the group's images, and the partials'
   // consumer maps block b to image b * 128 / (OH OW) -- statistics from a pass over the output instead
   if (a.upsample == 2 && a.H * a.Wd < G4_BM) return false;
@@ -872,7 +872,7 @@ void launch_gemm4(const GemmArgs& a, float* ws, int splits, int bn, hipStream_t 
   // persistent: + VAR bit 5 (the epilogue's stores stay in flight into the next tile; lab +0-4 %)
   if (persist && splits <= 1) g4_dispatch<60>(a, ws, splits, kps, bn, s);
   else g4_dispatch<20>(a, ws, splits, kps, bn, s);
-  if (splits > 1) launch_splitk_epilogue(a, ws, splits, s);
+  if (splits > 1 && !a.no_fold) launch_splitk_epilogue(a, ws, splits, s);
 }
 
 template <int VAR>

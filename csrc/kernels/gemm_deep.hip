@@ -60,7 +60,7 @@ void launch_tile(const GemmArgs& a, float* ws, int splits, hipStream_t s) {
   const int kt = (a.K + BK2 - 1) / BK2, kps = (kt + splits - 1) / splits * BK2;
   if (splits > 1) {
     launch_one<W, CONV, false, ACT_NONE, true>(a, ws, splits, kps, s);
-    launch_splitk_epilogue(a, ws, splits, s);
+    if (!a.no_fold) launch_splitk_epilogue(a, ws, splits, s);
     return;
   }
 #define SHAI_DEEP(GLU_, ACT_) launch_one<W, CONV, GLU_, ACT_, false>(a, nullptr, 1, kps, s)

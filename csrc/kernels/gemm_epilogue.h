@@ -46,8 +46,8 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& p, bf16_t* C, const bf
     }
   }
   if (p.bias2d) {
-    const bf16_t* b2 = p.bias2d + (long)(m / p.rows_per_bias2d) * p.N;
-    if (full && (p.N & 3) == 0) {
+    const bf16_t* b2 = p.bias2d + (long)(m / p.rows_per_bias2d) * p.bias2d_ld;
+    if (full && (p.bias2d_ld & 3) == 0) {
       const uint2_ bb = *reinterpret_cast<const uint2_*>(b2 + n);
       v[0] += bf2f(bb[0] & 0xffff); v[1] += bf2f(bb[0] >> 16);
       v[2] += bf2f(bb[1] & 0xffff); v[3] += bf2f(bb[1] >> 16);
@@ -109,6 +109,7 @@ inline bool epilogue8_fits(const GemmArgs& a) {
   uintptr_t out = (uintptr_t)a.C;
   if (a.residual) rows |= a.ldr, out |= (uintptr_t)a.residual;
   if (a.gate) rows |= a.gate_stride, out |= (uintptr_t)a.gate;
+  if (a.bias2d && (a.bias2d_ld & 7)) return false;
   if (a.batch > 1) rows |= a.batch_c | (a.residual ? a.batch_r : 0);
   return a.N % 8 == 0 && (rows & (OUT - 1)) == 0 && (out & (2 * OUT - 1)) == 0 && (((uintptr_t)a.bias | (uintptr_t)a.bias2d) & 15) == 0;
 }
@@ -139,7 +140,7 @@ __device__ __forceinline__ void epilogue8(const GemmArgs& p, bf16_t* C, const bf
     for (int e = 0; e < 8; ++e) v[e] += x[e];
   }
   if (p.bias2d) {
-    load_bf<8>(p.bias2d + (long)(m / p.rows_per_bias2d) * p.N + n, x);
+    load_bf<8>(p.bias2d + (long)(m / p.rows_per_bias2d) * p.bias2d_ld + n, x);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] += x[e];
   }

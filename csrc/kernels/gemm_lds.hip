@@ -228,7 +228,7 @@ static void launch_all(const GemmArgs& a, float* ws, int cfg, int splits, hipStr
   }();
   unsigned* cnt = nullptr;
   // (not at 128 x 128: the fixup's registers would halve that config's occupancy)
-  if (splits > 1 && (cfg == 2 || cfg == 4) && fixup_on && !a.rms && (long)splits * a.M * a.N * 4 < 0x7fffffffL) {
+  if (splits > 1 && (cfg == 2 || cfg == 4) && fixup_on && !a.rms && !a.no_fold && (long)splits * a.M * a.N * 4 < 0x7fffffffL) {
     const int bm = cfg == 2 ? 256 : 128, bn = cfg == 4 ? 64 : 128;
     const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
     if (tiles <= 4096) cnt = skinny_ticket_slice(s, (int)tiles);
@@ -236,7 +236,7 @@ static void launch_all(const GemmArgs& a, float* ws, int cfg, int splits, hipStr
 #define SHAI_G2(GLU_, ACT_)                                                   \
   do {                                                                        \
     launch_tiles<CONV, FAST, GLU_, ACT_>(a, cfg, ws, splits, kps, s, cnt);    \
-    if (splits > 1 && cnt == nullptr) launch_reduce<GLU_, ACT_>(a, ws, splits, s); \
+    if (splits > 1 && cnt == nullptr && !a.no_fold) launch_reduce<GLU_, ACT_>(a, ws, splits, s); \
   } while (0)
   if constexpr (CONV) {  // convs: no GLU, activation none / silu
     if (a.act == ACT_SILU) SHAI_G2(false, ACT_SILU);

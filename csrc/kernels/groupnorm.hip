@@ -1,0 +1,228 @@
+// GroupNorm (+ SiLU) of small images in one launch: statistics, normalisation and, behind a split-K convolution, the fold of
+// its partial sums.
+//
+// What bounds a small norm is launches, not bytes: at 4 x 16 x 16 x 1280 the column sums, the finalize and the apply pass took
+// 11.2 us in a graph for 5.2 MB, now 5.3 (4 x 8 x 8 x 1280 9.9 -> 3.9, 16 x 16 x 16 x 1280 14.4 -> 8.1, 4 x 32 x 32 x 640 12.0 -> 7.2),
+// and the fold of a split convolution is another launch less.  A workgroup owns one image's channels of one group (of two where a
+// group's width is no multiple of 4), holds them in registers as bf16, and takes mean and variance in two passes over the registers.
+#include "common.h"
+#include "launchers.h"
+
+namespace shai {
+
+namespace {
+
+// Registers allow 16 vectors of 4 channels a thread; with a fold's loads in flight beside them 8.  Two groups a workgroup leave half
+// as many workgroups, and with 16 vectors it was the slower way (4 x 32 x 32 x 960: 14.8 us, statistics and apply 12.8; 4 x 48 x 48 x
+// 320: 12.1 and 11.6; with 8, 4 x 16 x 16 x 960: 7.3 and 9.8).
+constexpr int kMaxVec = 16, kMaxVecTwo = 8, kMaxVecFold = 8;
+
+struct GnOneGeom {
+  int u;        // groups per workgroup
+  int vp;       // 4-channel vectors per pixel
+  int nv;       // vectors per thread: 1, 2, 4, 8 or 16
+  int active;   // threads with vectors, a multiple of vp: a thread's vectors are of the same channels
+};
+
+bool geometry(int HW, int C, int G, int max_vec, GnOneGeom* q) {
+  if (G <= 0 || C % G != 0) return false;
+  const int cg = C / G;
+  if (cg < 4 || cg % 2 != 0) return false;
+  q->u = cg % 4 == 0 ? 1 : 2;
+  if (G % q->u != 0) return false;
+  q->vp = q->u * cg / 4;
+  if (q->vp > 1024) return false;
+  const long items = (long)HW * q->vp;
+  if (q->u == 2 && max_vec > kMaxVecTwo) max_vec = kMaxVecTwo;
+  for (q->nv = 1; q->nv <= max_vec; q->nv *= 2) {
+    const long need = (items + q->nv - 1) / q->nv;
+    const long active = (need + q->vp - 1) / q->vp * q->vp;
+    if (active <= 1024) {
+      q->active = (int)active;
+      return true;
+    }
+  }
+  return false;
+}
+
+// Sums of lo and hi over the workgroup, the same value in every thread.
+template <bool TWO>
+__device__ __forceinline__ void block_sums(float& lo, float& hi, float2* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo += __shfl_xor(lo, o, 64);
+    if constexpr (TWO) hi += __shfl_xor(hi, o, 64);
+  }
+  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  __syncthreads();                     // the last call's reads
+  if ((threadIdx.x & 63) == 0) red[w] = make_float2(lo, hi);
+  __syncthreads();
+  lo = hi = 0.f;
+  for (int i = 0; i < nw; ++i) {
+    const float2 v = red[i];
+    lo += v.x;
+    if constexpr (TWO) hi += v.y;
+  }
+}
+
+template <int NV, bool TWO, bool FOLD>
+__global__ void __launch_bounds__(1024) gn_one_kernel(const GnOneArgs a, int units, int vp, int active) {
+  __shared__ float2 red[16];
+  // neighbouring channels share cache lines: consecutive units of an image on one XCD
+  int bid = blockIdx.x;
+  if ((gridDim.x & 7) == 0) bid = (bid & 7) * (gridDim.x >> 3) + (bid >> 3);
+  const int n = bid / units, unit = bid - n * units;
+  const int t = threadIdx.x, cg = a.C / a.G;
+  const bool live = t < active;
+  const int pix0 = t / vp, cv = t - pix0 * vp, step = active / vp;
+  const int c = unit * vp * 4 + cv * 4;                       // first of the thread's 4 channels
+  const int first = TWO ? min(4, max(0, cg - cv * 4)) : 4;    // how many of them are in the workgroup's first group
+
+  uint2_ gm{}, bt{};
+  if (live) {
+    if (a.gamma) gm = *reinterpret_cast<const uint2_*>(a.gamma + c);
+    if (a.beta) bt = *reinterpret_cast<const uint2_*>(a.beta + c);
+  }
+  uint2_ v[NV];
+  if constexpr (!FOLD) {
+    const bool one = c < a.C1;
+    const int ld = one ? a.C1 : a.C - a.C1;
+    const bf16_t* src = (one ? a.x + c : a.x2 + (c - a.C1)) + (long)n * a.HW * ld;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int p = pix0 + j * step;
+      v[j] = live && p < a.HW ? *reinterpret_cast<const uint2_*>(src + (long)p * ld) : uint2_{0, 0};
+    }
+  } else {
+    // the split-K fold: parts in order, then bias, the image's bias, residual, as gemm_splitk_reduce does it
+    constexpr int U = NV <= 2 ? 4 : NV <= 4 ? 2 : 1;          // parts whose loads are in flight together
+    const long slab = (long)a.N * a.HW * a.C;
+    const float* src = a.parts + (long)n * a.HW * a.C + c;
+    uint2_ rs[NV], bi{}, b2{};
+    if (live) {
+      if (a.bias) bi = *reinterpret_cast<const uint2_*>(a.bias + c);
+      if (a.bias2d) b2 = *reinterpret_cast<const uint2_*>(a.bias2d + (long)n * a.bias2d_ld + c);
+    }
+    float4_ acc[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      acc[j] = float4_{0.f, 0.f, 0.f, 0.f};
+      const int p = pix0 + j * step;
+      rs[j] = a.residual && live && p < a.HW ? *reinterpret_cast<const uint2_*>(a.residual + ((long)n * a.HW + p) * a.C + c) : uint2_{0, 0};
+    }
+    for (int s0 = 0; s0 < a.splits; s0 += U) {
+      float4_ x[U][NV];
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          const int p = pix0 + j * step;
+          x[q][j] = live && p < a.HW && s0 + q < a.splits ? *reinterpret_cast<const float4_*>(src + (s0 + q) * slab + (long)p * a.C)
+                                                          : float4_{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) acc[j] += x[q][j];
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int p = pix0 + j * step;
+      const bool in = live && p < a.HW;
+      float f[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int sh = e & 1 ? 0 : 16;
+        auto part = [&](const uint2_& w) { return __uint_as_float(sh ? w[e >> 1] << 16 : w[e >> 1] & 0xffff0000u); };
+        f[e] = acc[j][e];
+        if (a.bias) f[e] += part(bi);
+        if (a.bias2d) f[e] += part(b2);
+        if (a.residual) f[e] += part(rs[j]) * a.res_alpha;
+        if (!in) f[e] = 0.f;
+      }
+      v[j] = uint2_{pack2(f[0], f[1]), pack2(f[2], f[3])};
+      if (a.raw && in) *reinterpret_cast<uint2_*>(a.raw + ((long)n * a.HW + p) * a.C + c) = v[j];
+    }
+  }
+
+  auto at = [&](const uint2_& w, int e) { return __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16); };
+  const float inv = 1.f / ((float)a.HW * (float)cg);
+  float lo = 0.f, hi = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float f = at(v[j], e);
+      if (!TWO || e < first) lo += f;
+      else hi += f;
+    }
+  block_sums<TWO>(lo, hi, red);
+  const float mlo = lo * inv, mhi = hi * inv;
+  lo = hi = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    if (!live || pix0 + j * step >= a.HW) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool l = !TWO || e < first;
+      const float d = at(v[j], e) - (l ? mlo : mhi);
+      if (l) lo = fmaf(d, d, lo);
+      else hi = fmaf(d, d, hi);
+    }
+  }
+  block_sums<TWO>(lo, hi, red);
+  if (!live) return;
+  const float rlo = rsqrtf(lo * inv + a.eps), rhi = rsqrtf(hi * inv + a.eps);
+  float sc[4], sf[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool l = !TWO || e < first;
+    sc[e] = (l ? rlo : rhi) * (a.gamma ? at(gm, e) : 1.f);
+    sf[e] = (a.beta ? at(bt, e) : 0.f) - (l ? mlo : mhi) * sc[e];
+  }
+  bf16_t* dst = a.out + (long)n * a.HW * a.C + c;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int p = pix0 + j * step;
+    if (p >= a.HW) continue;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = fmaf(at(v[j], e), sc[e], sf[e]);
+      if (a.silu) y[e] = silu_f(y[e]);
+    }
+    *reinterpret_cast<uint2_*>(dst + (long)p * a.C) = uint2_{pack2(y[0], y[1]), pack2(y[2], y[3])};
+  }
+}
+
+}  // namespace
+
+bool gn_one_supported(int HW, int C, int G, bool fold) {
+  GnOneGeom q;
+  return HW > 0 && geometry(HW, C, G, fold ? kMaxVecFold : kMaxVec, &q);
+}
+
+void launch_gn_one(const GnOneArgs& a, hipStream_t s) {
+  GnOneGeom q;
+  const bool fold = a.parts != nullptr;
+  if (a.N <= 0 || !geometry(a.HW, a.C, a.G, fold ? kMaxVecFold : kMaxVec, &q)) return;   // the bindings refuse such a call
+  const int units = a.G / q.u, threads = (q.active + 63) / 64 * 64;
+  auto go = [&](auto kernel) { kernel<<<a.N * units, threads, 0, s>>>(a, units, q.vp, q.active); };
+#define SHAI_GN1(NV)                                                                    \
+  case NV:                                                                              \
+    if (q.u == 2) fold ? go(gn_one_kernel<NV, true, true>) : go(gn_one_kernel<NV, true, false>);  \
+    else fold ? go(gn_one_kernel<NV, false, true>) : go(gn_one_kernel<NV, false, false>);         \
+    break;
+  switch (q.nv) {
+    SHAI_GN1(1)
+    SHAI_GN1(2)
+    SHAI_GN1(4)
+    SHAI_GN1(8)
+    case 16:  // of one group, never behind a fold
+      go(gn_one_kernel<16, false, false>);
+      break;
+  }
+#undef SHAI_GN1
+}
+
+}  // namespace shai

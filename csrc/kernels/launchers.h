@@ -44,6 +44,29 @@ struct GroupNormArgs {
 int gn_num_blocks(int N, int HW, int C);
 void launch_groupnorm_stats(const GroupNormArgs& a, hipStream_t s);
 void launch_groupnorm_apply(const GroupNormArgs& a, hipStream_t s);
+// GroupNorm (+ SiLU) in one launch (groupnorm.hip), of x (and x2: channels [C1, C)), or of the fp32 partial sums
+// [splits][N HW][C] of a split-K convolution with what its fold adds.
+struct GnOneArgs {
+  const bf16_t* x;         // [N, HW, C1]
+  const bf16_t* x2;        // optional [N, HW, C - C1]
+  int C1;
+  const float* parts;      // not null: the input is the fold of these
+  int splits;
+  const bf16_t* bias;      // [C] optional
+  const bf16_t* bias2d;    // [N, C] optional, rows bias2d_ld apart
+  long bias2d_ld;
+  const bf16_t* residual;  // [N, HW, C] optional
+  float res_alpha;
+  bf16_t* raw;             // optional [N, HW, C]: receives the folded convolution
+  const bf16_t* gamma;
+  const bf16_t* beta;
+  bf16_t* out;             // [N, HW, C]
+  int N, HW, C, G;
+  float eps;
+  int silu;
+};
+bool gn_one_supported(int HW, int C, int G, bool fold);
+void launch_gn_one(const GnOneArgs& a, hipStream_t s);
 // Norm statistics produced by a GEMM epilogue (GemmArgs::col_part / row_part) and their fallback passes:
 //   col partials [M / 128, N, 2] (sum, sum of squares per 128-row block and column) of x [M, N] (row stride ldx)
 void launch_col_partials(const bf16_t* x, long M, int N, long ldx, float* part, hipStream_t s);
@@ -102,13 +125,14 @@ struct GemmArgs {
   const bf16_t* W;
   bf16_t* C;
   const bf16_t* bias;      // [N] optional
-  const bf16_t* bias2d;    // [M / rows_per_bias2d, N] optional (e.g. time-embedding per image)
+  const bf16_t* bias2d;    // [M / rows_per_bias2d, N] optional, rows bias2d_ld apart (e.g. time-embedding per image)
   const bf16_t* residual;  // [M, N] optional (same layout as C)
   int M, N, K;
   long lda, ldw, ldc, ldr;  // row strides (elements)
   long batch_a, batch_w, batch_c, batch_r;  // batch strides (elements)
   int batch;
   int rows_per_bias2d;
+  long bias2d_ld;           // row stride of bias2d
   float alpha;
   float res_alpha;          // C = epi + res_alpha * residual
   int act;                  // Act enum
@@ -147,6 +171,7 @@ struct GemmArgs {
   // > 0: rows [s w_slice_rows, (s + 1) w_slice_rows) multiply weight slice s (W is [M / w_slice_rows][N][ldw]; v4
   // kernel only, w_slice_rows % 256 == 0): a per-image weight, e.g. a GroupNorm's per-image scale folded into W
   int w_slice_rows;
+  int no_fold;              // split-K: leave the partial sums to the caller's consumer, launch no fold
 };
 // (conv, GLU, activation) epilogue variants the tile kernels (v2 / v4 / four-wave / W-stationary / halo conv)
 // instantiate: convolutions NONE / SILU, GLU SILU / GELU / GELU_TANH, plain GEMMs every activation.  Any other

@@ -139,12 +139,14 @@ class Conv2d(nn.Module):
         return x
 
     def forward(self, x, norm=None, temb=None, residual=None, upsample: bool = False, x2=None, act=None,
-                stats=None, eps: float = 1e-5):
-        """stats="gn" / "ln": returns (out, statistics of out for the next norm), see ``ops.conv2d``."""
+                stats=None, eps: float = 1e-5, gn=None, keep: bool = True):
+        """stats="gn" / "ln": returns (out, statistics of out for the next norm); ``gn``: (out, its GroupNorm); see ``ops.conv2d``."""
         if x2 is None:
             x = self._pad_in(x)
         extra = {} if stats is None else {"stats": stats, "eps": eps}
-        if upsample and ops.up2_phases_ok(x, self.k, self.k, self.stride, self.padding, x2, norm, residual, self.cout,
+        if gn is not None:
+            extra.update(gn=gn, keep=keep)
+        elif upsample and ops.up2_phases_ok(x, self.k, self.k, self.stride, self.padding, x2, norm, residual, self.cout,
                                           temb):
             w_up2 = self._phase_weight()
             if w_up2 is not None:
@@ -173,10 +175,20 @@ class GroupNorm(nn.Module):
                                                      part2=part2 if x2 is not None else None)
         return self.stats(x, x2)
 
+    def spec(self, silu: bool):
+        """This norm for ``ops.conv2d(gn=...)`` of the convolution before it."""
+        return self.weight, self.bias, self.groups, self.eps, silu
+
+    def one_ok(self, x, hw: int, channels: int) -> bool:
+        return ops.groupnorm_one_ok(x, hw, channels, self.groups)
+
     def forward(self, x, silu: bool = False, x2=None, part=None, part2=None):
         """GroupNorm of x, or of cat([x, x2], -1) without materialising the concat.  ``part`` / ``part2``:
         partials of x / x2 handed over by their producing GEMM (``conv2d(stats="gn")``), which replace the
         statistics pass over the input."""
+        C = x.shape[-1] + (x2.shape[-1] if x2 is not None else 0)
+        if part is None and self.one_ok(x, x[0, ..., 0].numel(), C):
+            return ops.groupnorm_one(x, self.weight, self.bias, self.groups, self.eps, silu, x2)
         sc, sh = self.scale_shift(x, x2, part, part2)
         return ops.groupnorm_apply(x, sc, sh, silu, x2=x2)
 

@@ -68,6 +68,13 @@ class UNetConfig:
                           cross_attention_dim=64, down_attn=(True, False), time_embed_dim=128)
 
 
+class Normed:
+    """In place of GroupNorm partials: the consuming norm's output."""
+
+    def __init__(self, y):
+        self.y = y
+
+
 class ResnetBlock2D(nn.Module):
     def __init__(self, cin: int, cout: int, temb: Optional[int], groups: int, eps: float):
         super().__init__()
@@ -84,12 +91,22 @@ class ResnetBlock2D(nn.Module):
         sources by GroupNorm and by the 1x1 shortcut conv (fused concat), never materialised."""
         return self.forward_parts(x, temb_proj, x2)[0]
 
-    def forward_parts(self, x, temb_proj=None, x2=None, xp=None, x2p=None, stats: bool = False):
+    def forward_parts(self, x, temb_proj=None, x2=None, xp=None, x2p=None, stats: bool = False, follow=None):
         """forward with the GroupNorm hand-off: ``xp`` / ``x2p`` are GroupNorm partials of x / x2 written by their
-        producers' epilogues (they replace the statistics pass of norm1); with ``stats`` conv1 and conv2 write
-        the partials of their outputs (norm2's input, and the next norm's).  Returns (out, partials or None)."""
-        st = {"stats": "gn"} if stats else {}
-        if FUSED_GN_CONV and x.shape[-1] % 8 == 0 and (x2 is None or x2.shape[-1] % 8 == 0):
+        producers' epilogues (they replace the statistics pass of norm1), or ``xp`` is norm1's output itself (:class:`Normed`);
+        with ``stats`` conv1 and conv2 write the partials of their outputs (norm2's input, and the next norm's).  Small images
+        (``GroupNorm.one_ok``) have no partials: a norm is one launch, conv1's and ``follow`` = (norm, silu), the one that reads
+        the output next, the launch that folds their convolution.  Returns (out, partials, Normed or None)."""
+        small = stats and self.norm2.one_ok(x, x.shape[1] * x.shape[2], self.cout)
+        st = {"stats": "gn"} if stats and not small else {}
+        if isinstance(xp, Normed) or (small and (xp is None or (x2 is not None and x2p is None))
+                                      and self.norm1.one_ok(x, x.shape[1] * x.shape[2], self.cin)):
+            n1 = xp.y if isinstance(xp, Normed) else self.norm1(x, silu=True, x2=x2)
+            if small:
+                _, n2 = self.conv1(n1, temb=temb_proj, gn=self.norm2.spec(True), keep=False)
+                return self._finish(n2, x, x2, follow)
+            out1 = self.conv1(n1, temb=temb_proj, **st)
+        elif FUSED_GN_CONV and x.shape[-1] % 8 == 0 and (x2 is None or x2.shape[-1] % 8 == 0):
             # GroupNorm + SiLU as the convs' prologue: (scale, shift) from the producers' partials, applied once per
             # staged element inside the halo-tiled conv (one apply pass + the tuned conv where it does not fit)
             sc, sh = self.norm1.scale_shift(x, x2, part=xp, part2=x2p)
@@ -98,17 +115,29 @@ class ResnetBlock2D(nn.Module):
             # the separate pass: GroupNorm + SiLU written out, then the conv
             n1 = self.norm1(x, silu=True, x2=x2, part=xp, part2=x2p)
             out1 = self.conv1(n1, temb=temb_proj, **st)
-        h, hp = out1 if stats else (out1, None)
-        if self.conv_shortcut is not None:
-            skip = self.conv_shortcut(x, x2=x2) if x2 is not None else self.conv_shortcut(x)
-        else:
-            skip = x if x2 is None else torch.cat([x, x2], dim=-1)
+        h, hp = out1 if st else (out1, None)
+        if small:
+            return self._finish(self.norm2(h, silu=True), x, x2, follow)
+        skip = self._skip(x, x2)
         if FUSED_GN_CONV and h.shape[-1] % 8 == 0:
             sc, sh = self.norm2.scale_shift(h, part=hp)
             out = self.conv2(h, norm=(sc, sh, "silu"), residual=skip, **st)
         else:
             out = self.conv2(self.norm2(h, silu=True, part=hp), residual=skip, **st)
         return out if stats else (out, None)
+
+    def _skip(self, x, x2):
+        if self.conv_shortcut is not None:
+            return self.conv_shortcut(x, x2=x2) if x2 is not None else self.conv_shortcut(x)
+        return x if x2 is None else torch.cat([x, x2], dim=-1)
+
+    def _finish(self, n2, x, x2, follow):
+        """conv2 of a small image, and the norm that follows."""
+        skip = self._skip(x, x2)
+        if follow is None:
+            return self.conv2(n2, residual=skip), None
+        out, y = self.conv2(n2, residual=skip, gn=follow[0].spec(follow[1]))
+        return out, Normed(y)
 
 
 class GEGLU(nn.Module):
@@ -211,7 +240,11 @@ class Transformer2DModel(nn.Module):
         output out.  Returns (out, partials or None)."""
         B, H, W, C = x.shape
         blocks = list(self.transformer_blocks)
-        if ops.fold_profitable(B * H * W, C):  # the Q projection (N = C) has the fewest tiles of the consumers
+        if isinstance(xp, Normed):
+            h = self.proj_in(xp.y).view(B, H * W, C)
+            for blk in blocks:
+                h = blk(h, ctx_kv)
+        elif ops.fold_profitable(B * H * W, C):  # the Q projection (N = C) has the fewest tiles of the consumers
             if self._gn_fold_ok(x):
                 h, mr = self._proj_in_gn_folded(x, xp, blocks[0].norm1.eps)
             else:
@@ -230,7 +263,7 @@ class Transformer2DModel(nn.Module):
             for blk in blocks:
                 h = blk(h, ctx_kv)
         res = x.view(B, H * W, C)
-        if stats and ops.stats_supported(B * H * W, C, "gn", H * W):
+        if stats and ops.stats_supported(B * H * W, C, "gn", H * W) and not self.norm.one_ok(x, H * W, C):
             out, op = self.proj_out.forward_stats(h, residual=res, stats="gn")
             return out.view(B, H, W, C), op
         return self.proj_out(h, residual=res).view(B, H, W, C), None
@@ -295,7 +328,10 @@ class Downsample2D(nn.Module):
     def forward(self, x):
         return self.conv(x)
 
-    def forward_parts(self, x, stats: bool = False):
+    def forward_parts(self, x, stats: bool = False, groups: int = 0):
+        """``groups`` of the next norm: the output of a small image is left without partials (``ResnetBlock2D.forward_parts``)."""
+        if stats and groups and ops.groupnorm_one_ok(x, ((x.shape[1] + 1) // 2) * ((x.shape[2] + 1) // 2), self.conv.cout, groups):
+            stats = False
         return self.conv(x, stats="gn") if stats else (self.conv(x), None)
 
 
@@ -307,7 +343,9 @@ class Upsample2D(nn.Module):
     def forward(self, x):
         return self.conv(x, upsample=True)
 
-    def forward_parts(self, x, stats: bool = False):
+    def forward_parts(self, x, stats: bool = False, groups: int = 0):
+        if stats and groups and ops.groupnorm_one_ok(x, 4 * x.shape[1] * x.shape[2], self.conv.cout, groups):
+            stats = False
         return self.conv(x, upsample=True, stats="gn") if stats else (self.conv(x, upsample=True), None)
 
 
@@ -426,7 +464,9 @@ class UNet2DConditionModel(nn.Module):
         # silu(emb) then one GEMM for all ResNets
         semb = ops.bias_act(emb, None, None, "silu")
         tall = ops.linear(semb, w, b)
-        tprojs = [tall[:, o:o + n].contiguous() for (o, n) in offs]
+        # a ResNet's columns as they lie, where 16 bytes fit (``ops.conv2d``'s temb)
+        tprojs = [tall[:, o:o + n] if tall.is_cuda and o % 8 == 0 and tall.shape[1] % 8 == 0 else tall[:, o:o + n].contiguous()
+                  for (o, n) in offs]
         ti = iter(tprojs)
         kvi = iter(ctx_kv)
 
@@ -434,28 +474,37 @@ class UNet2DConditionModel(nn.Module):
         # partial sums from its epilogue (no statistics pass over the activation), and the transformer blocks'
         # LayerNorms are folded into the projections that consume them (no normalised activation written).
         st = NORM_HANDOFF
-        x, xp = self.conv_in(sample, stats="gn") if st else (self.conv_in(sample), None)
+        small = ops.groupnorm_one_ok(sample, sample.shape[1] * sample.shape[2], cfg.block_out_channels[0], cfg.norm_num_groups)
+        x, xp = self.conv_in(sample, stats="gn") if st and not small else (self.conv_in(sample), None)
         skips = [(x, xp)]
+        g = cfg.norm_num_groups
         for blk in self.down_blocks:
             for i, r in enumerate(blk.resnets):
-                x, xp = r.forward_parts(x, next(ti), xp=xp, stats=st)
+                if blk.attentions is not None:
+                    follow = (blk.attentions[i].norm, False)
+                elif i + 1 < len(blk.resnets):
+                    follow = (blk.resnets[i + 1].norm1, True)
+                else:
+                    follow = (self.mid_block.resnets[0].norm1, True) if blk.downsamplers is None else None
+                x, xp = r.forward_parts(x, next(ti), xp=xp, stats=st, follow=follow)
                 if blk.attentions is not None:
                     x, xp = self._attn(blk.attentions[i], x, next(kvi), xp, st)
-                skips.append((x, xp))
+                skips.append((x, None if isinstance(xp, Normed) else xp))
             if blk.downsamplers is not None:
-                x, xp = blk.downsamplers[0].forward_parts(x, st)
+                x, xp = blk.downsamplers[0].forward_parts(x, st, g)
                 skips.append((x, xp))
-        x, xp = self.mid_block.resnets[0].forward_parts(x, next(ti), xp=xp, stats=st)
+        x, xp = self.mid_block.resnets[0].forward_parts(x, next(ti), xp=xp, stats=st, follow=(self.mid_block.attentions[0].norm, False))
         x, xp = self._attn(self.mid_block.attentions[0], x, next(kvi), xp, st)
         x, xp = self.mid_block.resnets[1].forward_parts(x, next(ti), xp=xp, stats=st)
         for blk in self.up_blocks:
             for i, r in enumerate(blk.resnets):
                 s, sp = skips.pop()
-                x, xp = r.forward_parts(x, next(ti), x2=s, xp=xp, x2p=sp, stats=st)
+                follow = (blk.attentions[i].norm, False) if blk.attentions is not None else None
+                x, xp = r.forward_parts(x, next(ti), x2=s, xp=xp, x2p=sp, stats=st, follow=follow)
                 if blk.attentions is not None:
                     x, xp = self._attn(blk.attentions[i], x, next(kvi), xp, st)
             if blk.upsamplers is not None:
-                x, xp = blk.upsamplers[0].forward_parts(x, st)
+                x, xp = blk.upsamplers[0].forward_parts(x, st, g)
         return self.conv_out(self.conv_norm_out(x, silu=True, part=xp))
 
     @staticmethod

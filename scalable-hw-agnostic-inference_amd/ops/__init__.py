@@ -10,6 +10,7 @@ captured into HIP graphs (``torch.cuda.CUDAGraph`` is hipGraph on ROCm).
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 from typing import Optional, Tuple
@@ -123,6 +124,35 @@ def groupnorm_apply(x: torch.Tensor, scale, shift, silu: bool = False, x2: Optio
     out = torch.empty(*x.shape[:-1], C, dtype=x.dtype, device=x.device)
     _K().groupnorm_apply(x.reshape(N, -1, x.shape[-1]), x2.reshape(N, -1, x2.shape[-1]) if x2 is not None else None,
                          scale, shift, out.view(N, -1, C), bool(silu))
+    return out
+
+
+# images whose GroupNorm runs as one launch: up to this many elements of all images together.  Beyond, a pass costs bytes, and the
+# statistics that a large product's epilogue leaves are worth more: us one launch / finalize and apply of given statistics / with the
+# column sums before them, at 16 x 32 x 32 x 320 9.1 / 8.9 / 14.2, 8 x 32 x 32 x 1280 12.7 / 13.2 / 19.7, 16 x 32 x 32 x 1280 24.2 / 19.3 / 28.0
+GN_ONE_MAX = 8 << 20
+
+
+@functools.lru_cache(maxsize=None)
+def _gn_one_fits(hw: int, c: int, groups: int) -> bool:
+    return bool(_K().groupnorm_one_supported(hw, c, groups, False))
+
+
+def groupnorm_one_ok(x: torch.Tensor, hw: int, c: int, groups: int) -> bool:
+    """Whether the GroupNorm of [N, hw, c] with the batch and the device of ``x`` runs as one launch (``groupnorm_one``,
+    ``conv2d(gn=...)``): on the GPU, what fits in a workgroup's registers and is small enough for launches to count."""
+    return x.is_cuda and x.shape[0] * hw * c <= GN_ONE_MAX and _gn_one_fits(hw, c, groups)
+
+
+def groupnorm_one(x, gamma, beta, groups: int, eps: float, silu: bool = False, x2=None) -> torch.Tensor:
+    """``groupnorm`` in one launch, for what ``groupnorm_one_ok`` says."""
+    if not _gpu(x):
+        return groupnorm(x, gamma, beta, groups, eps, silu, x2)
+    N = x.shape[0]
+    C = x.shape[-1] + (x2.shape[-1] if x2 is not None else 0)
+    out = torch.empty(*x.shape[:-1], C, dtype=x.dtype, device=x.device)
+    _K().groupnorm_one(x.reshape(N, -1, x.shape[-1]), x2.reshape(N, -1, x2.shape[-1]) if x2 is not None else None, gamma, beta,
+                       out.view(N, -1, C), int(groups), float(eps), bool(silu))
     return out
 
 
@@ -480,7 +510,7 @@ def conv2d(x: torch.Tensor, w_packed: torch.Tensor, bias: Optional[torch.Tensor]
            pad: int = 0, upsample: bool = False, x2: Optional[torch.Tensor] = None, norm=None,
            temb: Optional[torch.Tensor] = None, residual: Optional[torch.Tensor] = None, act=None,
            res_alpha: float = 1.0, stats: Optional[str] = None, eps: float = 1e-5,
-           w_up2: Optional[torch.Tensor] = None):
+           w_up2: Optional[torch.Tensor] = None, gn=None, keep: bool = True):
     """NHWC implicit-GEMM convolution with fused prologue/epilogue.
 
     norm = (scale [N,Cin] f32, shift [N,Cin] f32, act) applies GroupNorm(+act) to
@@ -491,9 +521,13 @@ def conv2d(x: torch.Tensor, w_packed: torch.Tensor, bias: Optional[torch.Tensor]
     (``pack_up2_phase_weight``) of an upsample conv -- used when ``up2_phases_ok``.
     stats="gn" / "ln": also return statistics of the output for the next norm, as ``linear_stats`` -- (out, st);
     st is None when the output shape cannot carry them (``stats_supported``).
+    gn = (gamma, beta, groups, eps, silu): returns (out, GroupNorm(+SiLU) of out) for an output that ``groupnorm_one_ok`` allows,
+    normalised in the launch that folds a split-K convolution; without ``keep`` out may be left unwritten and is None.
     """
     if not _gpu(x):
         y = ref.conv2d(x, w_packed, bias, kh, kw, stride, pad, upsample, x2, norm, temb, residual, act, res_alpha)
+        if gn is not None:
+            return (y if keep else None), groupnorm(y, *gn)
         if stats is None:
             return y
         y2 = y.reshape(-1, y.shape[-1])
@@ -514,6 +548,13 @@ def conv2d(x: torch.Tensor, w_packed: torch.Tensor, bias: Optional[torch.Tensor]
         want = stats
     gp = torch.empty(M // 128, cout, 2, dtype=torch.float32, device=x.device) if want == "gn" else None
     ls = torch.empty(M, 2, dtype=torch.float32, device=x.device) if want == "ln" else None
+    if gn is not None:
+        y = torch.empty_like(out)
+        gamma, beta, groups, geps, silu = gn
+        _K().conv2d(x, x2, w_packed, out, bias, temb, residual, sc, sh, act_id(nact), kh, kw, stride, pad, bool(upsample),
+                    act_id(act), float(res_alpha), gn_gamma=gamma, gn_beta=beta, gn_out=y, gn_groups=int(groups),
+                    gn_eps=float(geps), gn_silu=bool(silu), keep_out=bool(keep))
+        return (out if keep else None), y
     if upsample and w_up2 is not None and up2_phases_ok(x, kh, kw, stride, pad, x2, norm, residual, temb=temb):
         _K().conv2d(x, None, w_up2, out, bias, temb, None, None, None, 0, 2, 2, 1, 0, True, act_id(act), 1.0, None,
                     None, gp, ls, float(eps), True)

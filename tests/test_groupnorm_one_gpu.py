@@ -1,0 +1,80 @@
+"""GroupNorm in one launch (csrc/kernels/groupnorm.hip) against 64 bits: alone, of two sources, and behind a split-K convolution."""
+import pytest
+import torch
+
+from shai_amd import native, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def rnd(*shape, scale=1.0):
+    return (torch.randn(*shape, device="cuda") * scale).to(torch.bfloat16)
+
+
+def norm64(x, gamma, beta, groups, eps, silu):
+    N, C = x.shape[0], x.shape[-1]
+    g = x.double().reshape(N, -1, groups, C // groups)
+    g = g - g.mean((1, 3), keepdim=True)
+    y = (g * torch.rsqrt((g * g).mean((1, 3), keepdim=True) + eps)).reshape(x.shape) * gamma.double() + beta.double()
+    return y * torch.sigmoid(y) if silu else y
+
+
+def off(y, want):
+    """bf16 outputs: half a unit in the last place of 8 bits is 2^-9 of a value; the mean over them is below that."""
+    return ((y.double() - want).norm() / want.norm()).item()
+
+
+# pixels and channels (32 groups): groups of 4, 6, 10, 12, 20, 30, 40, 60 and 80 channels, one workgroup each or two groups together;
+# 1, 2, 4, 8 and 16 vectors a thread, whole and with a remainder; one pixel
+@pytest.mark.parametrize("hw,C", [(1, 1280), (3, 128), (64, 1280), (63, 192), (81, 320), (144, 960), (256, 960), (256, 384), (256, 2560), (576, 640),
+                                  (1024, 640), (1024, 1920), (2304, 640), (4096, 512), (1023, 1920)])
+def test_alone(cuda, hw, C):
+    torch.manual_seed(hw + C)
+    for N, silu, mean in ((1, True, 0.0), (3, False, 8.0)):
+        x, gamma, beta = (rnd(N, hw, C) + mean).bfloat16(), rnd(C), rnd(C)
+        assert ops.groupnorm_one_ok(x, hw, C, 32)
+        assert off(ops.groupnorm_one(x, gamma, beta, 32, 1e-5, silu), norm64(x, gamma, beta, 32, 1e-5, silu)) < 2 ** -8
+    assert off(ops.groupnorm_one(x, None, None, 32, 1e-5), norm64(x, torch.ones(C, device="cuda"), torch.zeros(C, device="cuda"), 32, 1e-5, False)) < 2 ** -8
+
+
+@pytest.mark.parametrize("hw,C1,C2", [(64, 1280, 640), (256, 640, 320), (1000, 320, 640), (16, 8, 120)])
+def test_two_sources(cuda, hw, C1, C2):
+    """The border lies inside a group (1920 / 32 = 60 channels) or between two."""
+    torch.manual_seed(C1)
+    x, x2, gamma, beta = rnd(2, hw, C1), (rnd(2, hw, C2) - 3).bfloat16(), rnd(C1 + C2), rnd(C1 + C2)
+    y = ops.groupnorm_one(x, gamma, beta, 32, 1e-5, True, x2=x2)
+    assert off(y, norm64(torch.cat([x, x2], -1), gamma, beta, 32, 1e-5, True)) < 2 ** -8
+
+
+def test_refused(cuda):
+    """Odd and narrow groups, and images that registers do not hold, keep the other kernels."""
+    x = rnd(1, 64, 96)
+    for hw, C, groups in ((64, 96, 32), (64, 224, 32), (1024, 960, 32), (64, 2 * 4, 2 * 2), (70000, 128, 32), (64, 100, 32)):
+        assert not ops.groupnorm_one_ok(x, hw, C, groups)
+    with pytest.raises(RuntimeError):
+        ops.groupnorm_one(x, None, None, 32, 1e-5)
+
+
+# a split-K choice is folded by the norm's launch, an unsplit one is not; the residual, the image's bias as columns of a wider tensor
+@pytest.mark.parametrize("cfg,splits", [(3, 4), (4, 3), (18, 8), (9, 2), (16, 1), (4, 1)])
+@pytest.mark.parametrize("side,cin,cout", [(16, 128, 640), (8, 192, 1280), (12, 64, 320)])
+def test_after_convolution(cuda, cfg, splits, side, cin, cout):
+    torch.manual_seed(side + splits)
+    N = 2
+    x, b, res = rnd(N, side, side, cin), rnd(cout), rnd(N, side, side, cout)
+    w4 = (torch.randn(cout, cin, 3, 3, device="cuda") * (9 * cin) ** -0.5).bfloat16()
+    w, temb, gamma, beta = ops.pack_conv_weight(w4), rnd(N, cout + 64)[:, 16:16 + cout], rnd(cout), rnd(cout)
+    M, K = N * side * side, 9 * cin
+    native.ops().gemm_tuning_import([f"1:{M},{cout},{K},b1,g0|{N},{side},{side},{cin},{cin},3,1,0,0={cfg},{splits}"])
+    want = torch.nn.functional.conv2d(x.double().permute(0, 3, 1, 2).cpu(), w4.double().cpu(), b.double().cpu(), padding=1).permute(0, 2, 3, 1).cuda()
+    want = want + temb.double()[:, None, None, :]
+    for keep in (True, False):
+        out, y = ops.conv2d(x, w, b, 3, 3, 1, 1, temb=temb, residual=res if keep else None, gn=(gamma, beta, 32, 1e-5, True), keep=keep)
+        raw = want + res.double() if keep else want
+        # the norm is of the rounded convolution: 2^-9 of a value, and 2^-9 of its own result
+        assert off(y, norm64(raw, gamma, beta, 32, 1e-5, True)) < 2 ** -7
+        assert out is None if not keep else off(out, raw) < 2 ** -8
+        if keep:
+            assert off(y, norm64(out, gamma, beta, 32, 1e-5, True)) < 2 ** -8
+            plain = ops.conv2d(x, w, b, 3, 3, 1, 1, temb=temb, residual=res)
+            assert torch.equal(out, plain)      # the fold's sums in its order
