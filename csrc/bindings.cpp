@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "kernels/launchers.h"
+#include "kernels/vision.h"
 
 using at::Tensor;
 using c10::optional;
@@ -1602,6 +1603,56 @@ int64_t gemm_tuning_import(const std::vector<std::string>& entries) {
   return n;
 }
 
+void patches_u8(const Tensor& x, const Tensor& out, int64_t P, at::ArrayRef<double> mean, at::ArrayRef<double> inv_std) {
+  SHAI_CHECK(x.is_cuda() && x.scalar_type() == at::kByte && x.is_contiguous() && x.dim() == 4 && x.size(3) == 3, "patches_u8: uint8 [B, H, W, 3]");
+  check_bf16(out, "out");
+  SHAI_CHECK(P > 0 && P % 8 == 0 && x.size(1) % P == 0 && x.size(2) % P == 0 && mean.size() == 3 && inv_std.size() == 3,
+             "patches_u8: patch a multiple of 8 that divides the image; three means and scales");
+  SHAI_CHECK(((uintptr_t)x.data_ptr() & 7) == 0 && ((uintptr_t)out.data_ptr() & 15) == 0 && out.is_contiguous() && out.numel() == x.numel(),
+             "patches_u8: aligned images, out [patches, P P 3]");
+  shai::PatchArgs a{};
+  a.x = x.data_ptr<uint8_t>();
+  a.out = mptr(out);
+  a.B = x.size(0);
+  a.H = x.size(1);
+  a.W = x.size(2);
+  a.P = P;
+  for (int c = 0; c < 3; ++c) a.mean[c] = mean[c], a.inv_std[c] = inv_std[c];
+  shai::launch_patches_u8(a, stream());
+}
+
+void tokens(const Tensor& patches, const Tensor& cls, const optional<Tensor>& det, const Tensor& pos, const Tensor& out,
+            const optional<Tensor>& mr, double eps) {
+  shai::TokenArgs a{};
+  for (const Tensor* t : {&patches, &cls, &pos, &out}) {
+    check_bf16(*t, "tokens");
+    SHAI_CHECK(t->is_contiguous() && ((uintptr_t)t->data_ptr() & 15) == 0, "tokens: contiguous, 16-byte aligned");
+  }
+  SHAI_CHECK(patches.dim() == 3 && out.dim() == 3 && out.size(0) == patches.size(0) && out.size(2) == patches.size(2), "tokens: [B, n, D] -> [B, T, D]");
+  a.B = patches.size(0);
+  a.n = patches.size(1);
+  a.D = patches.size(2);
+  if (det) {
+    check_bf16(*det, "det");
+    SHAI_CHECK(det->dim() == 2 && det->size(1) == a.D && det->is_contiguous() && ((uintptr_t)det->data_ptr() & 15) == 0, "det [nd, D]");
+    a.det = cptr(*det);
+    a.nd = det->size(0);
+  }
+  const long T = 1 + a.n + a.nd;
+  SHAI_CHECK(a.D % 8 == 0 && a.D <= 2048 && out.size(1) == T && cls.numel() == a.D && pos.numel() == T * a.D, "tokens: shapes");
+  if (mr) {
+    check_f32(*mr, "mr");
+    SHAI_CHECK(mr->is_contiguous() && mr->numel() == 2 * a.B * T, "mr [B T, 2]");
+    a.mr = mr->data_ptr<float>();
+  }
+  a.patches = cptr(patches);
+  a.cls = cptr(cls);
+  a.pos = cptr(pos);
+  a.out = mptr(out);
+  a.eps = eps;
+  shai::launch_tokens(a, stream());
+}
+
 void mean_tokens(const Tensor& x, const Tensor& out) {
   check_bf16(x, "x");
   check_f32(out, "out");
@@ -1770,6 +1821,8 @@ TORCH_LIBRARY(shai, m) {
   m.def("sched_step(Tensor model_out, Tensor(a!) latents, bool cfg, float guidance, int pred_type, float a_t, float a_prev, float dt) -> ()");
   m.def("sched_step_rows(Tensor model_out, Tensor(a!) latents, bool cfg, float guidance, int pred_type, Tensor rows_params) -> ()");
   m.def("softmax_(Tensor(a!) x, float scale) -> ()");
+  m.def("patches_u8(Tensor x, Tensor(a!) out, int P, float[] mean, float[] inv_std) -> ()");
+  m.def("tokens(Tensor patches, Tensor cls, Tensor? det, Tensor pos, Tensor(a!) out, Tensor(b!)? mr, float eps) -> ()");
   m.def("mean_tokens(Tensor x, Tensor(a!) out) -> ()");
   m.def("embedding(Tensor ids, Tensor table, Tensor(a!) out) -> ()");
   m.def("decode_attn_rope(Tensor qkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, "
@@ -1814,6 +1867,8 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("sched_step", &sched_step);
   m.impl("sched_step_rows", &sched_step_rows);
   m.impl("softmax_", &softmax_);
+  m.impl("patches_u8", &patches_u8);
+  m.impl("tokens", &tokens);
   m.impl("mean_tokens", &mean_tokens);
   m.impl("embedding", &embedding);
   m.impl("decode_attn_rope", &decode_attn_rope);

@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .attention import FusedSelfAttention, merge_linear_keys
-from .layers import Conv2d, LayerNorm, Linear
+from .layers import Conv2d, LayerNorm, Linear, _wkey
 
 
 # LayerNorms folded into the GEMMs that consume them, moments handed over by the producing GEMM (unet2d.py);
@@ -149,23 +149,47 @@ class ViTEncoderModel(nn.Module):
         patch = patch.flatten(2).transpose(1, 2).to(pe.dtype)
         return torch.cat([cls_pe, patch, det_pe], dim=1)
 
+    def _patch_weight(self):
+        """The patch convolution's weight without the channels that pad 3 to 8, [d, P P 3]; rebuilt when the weight changes.  None
+        when first needed inside a graph capture."""
+        key = _wkey(self.patch.weight)
+        cached = getattr(self, "_w_patch", None)
+        if cached is None or cached[0] != key:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            w = self.patch.weight.data
+            cached = (key, w.view(w.shape[0], -1, self.patch.cin_p)[..., :3].reshape(w.shape[0], -1).contiguous())
+            self._w_patch = cached
+        return cached[1]
+
+    def forward_u8(self, images: torch.Tensor, mean, std, cls_only: bool = False):
+        """``forward`` of uint8 images [B, H, W, 3] at the model's resolution, normalised with the channels' ``mean`` and ``std``
+        on the way into the patches; None where their sizes or address do not fit that kernel."""
+        P = self.cfg.patch_size
+        if not ops.patches_u8_ok(images, P):
+            return None
+        w = self._patch_weight()
+        if w is None:
+            return None
+        B, H, W, _ = images.shape
+        x = ops.linear(ops.patches_u8(images, P, mean, std), w, self.patch.bias)
+        return self._encode(x.view(B, H // P, W // P, -1), cls_only, False)
+
     def forward(self, pixels: torch.Tensor, cls_only: bool = False, det_only: bool = False) -> torch.Tensor:
         """pixels NHWC [B, H, W, 3] normalised bf16 -> hidden states [B, T, d]; ``cls_only``: [B, 1, d] of token 0,
         ``det_only``: [B, nd, d] of the detection tokens -- the last layer then runs its query side for those tokens
         only (``ViTLayer.forward_cls``)."""
-        B, H, W, _ = pixels.shape
-        x = self.patch(pixels)  # [B, gh, gw, d]
-        gh, gw = x.shape[1], x.shape[2]
-        toks = [self.cls_token.expand(B, -1, -1), x.reshape(B, gh * gw, -1)]
-        if self.det_tokens is not None:
-            toks.append(self.det_tokens.expand(B, -1, -1))
-        x = torch.cat(toks, dim=1)
-        pe = self.pos_embed(gh, gw).expand(B, -1, -1).contiguous()
-        x = ops.bias_act(x.contiguous(), None, pe)
-        c = self.cfg
-        if NORM_HANDOFF and ops.fold_profitable(x.shape[0] * x.shape[1], min(3 * c.hidden_size, c.intermediate_size)):
-            layers = list(self.layers)
-            mr = ops.row_moments(x, layers[0].layernorm_before.eps)
+        return self._encode(self.patch(pixels), cls_only, det_only)
+
+    def _encode(self, x, cls_only: bool, det_only: bool):
+        """The encoder on patch embeddings x [B, gh, gw, d]."""
+        B, gh, gw, d = x.shape
+        nd = self.det_tokens.shape[1] if self.det_tokens is not None else 0
+        pe, layers, c = self.pos_embed(gh, gw), list(self.layers), self.cfg
+        fold = NORM_HANDOFF and ops.fold_profitable(B * (1 + gh * gw + nd), min(3 * c.hidden_size, c.intermediate_size))
+        x, mr = ops.tokens(x.reshape(B, gh * gw, d), self.cls_token, self.det_tokens, pe,
+                           layers[0].layernorm_before.eps if fold else None)
+        if fold:
             for i, layer in enumerate(layers):
                 if (cls_only or det_only) and i + 1 == len(layers):
                     return self.layernorm(layer.forward_cls(x, mr, *self._kept(cls_only)))
@@ -223,6 +247,11 @@ class ViTForImageClassification(nn.Module):
     def forward(self, pixels):
         h = self.vit(pixels, cls_only=True)  # the logits read token 0 only
         return self.classifier(h[:, 0].contiguous())
+
+    def forward_u8(self, images, mean, std):
+        """``forward`` of uint8 images, or None (``ViTEncoderModel.forward_u8``)."""
+        h = self.vit.forward_u8(images, mean, std, cls_only=True)
+        return None if h is None else self.classifier(h[:, 0].contiguous())
 
     def convert_hf_state_dict(self, sd: dict) -> dict:
         out = {}

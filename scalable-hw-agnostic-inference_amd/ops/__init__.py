@@ -800,6 +800,41 @@ def token_feedback(ids, rowmap, prev):
     return ids
 
 
+def patches_u8_ok(images: torch.Tensor, patch: int) -> bool:
+    """Whether ``patches_u8`` takes these images as they are."""
+    return (images.is_cuda and images.dtype == torch.uint8 and images.dim() == 4 and images.shape[-1] == 3 and images.is_contiguous()
+            and patch % 8 == 0 and images.shape[1] % patch == 0 and images.shape[2] % patch == 0 and images.data_ptr() % 8 == 0)
+
+
+def patches_u8(images: torch.Tensor, patch: int, mean, std) -> torch.Tensor:
+    """uint8 images [B, H, W, 3] -> [B (H / patch) (W / patch), patch patch 3] bf16: the patches' pixels in the order (row, column,
+    channel), normalised (u8 / 255 - mean) / std."""
+    B, H, W, _ = images.shape
+    if not _gpu(images):
+        m, r = torch.tensor(mean, dtype=torch.float32), 1.0 / torch.tensor(std, dtype=torch.float32)
+        x = ((images.float() * (1.0 / 255.0) - m) * r).to(torch.bfloat16)
+        return x.view(B, H // patch, patch, W // patch, patch, 3).transpose(2, 3).reshape(-1, patch * patch * 3)
+    out = torch.empty(B * (H // patch) * (W // patch), patch * patch * 3, dtype=torch.bfloat16, device=images.device)
+    _K().patches_u8(images, out, int(patch), [float(m) for m in mean], [1.0 / float(v) for v in std])
+    return out
+
+
+def tokens(patches: torch.Tensor, cls: torch.Tensor, det: Optional[torch.Tensor], pos: torch.Tensor, eps: Optional[float] = None):
+    """(x, row moments of x or None): x [B, T, D] = cat(class token, patches, detection tokens) + position embeddings [1, T, D], and
+    with ``eps`` the (mean, rstd) [B T, 2] that the first layer's folded LayerNorm consumes."""
+    B, n, D = patches.shape
+    if not _gpu(patches) or D % 8 or D > 2048:
+        x = torch.cat([cls.expand(B, -1, -1), patches] + ([det.expand(B, -1, -1)] if det is not None else []), 1)
+        x = bias_act(x.contiguous(), None, pos.expand(B, -1, -1).contiguous())
+        return x, (row_moments(x, eps) if eps is not None else None)
+    nd = det.shape[1] if det is not None else 0
+    x = torch.empty(B, 1 + n + nd, D, dtype=patches.dtype, device=patches.device)
+    mr = torch.empty(B * (1 + n + nd), 2, dtype=torch.float32, device=x.device) if eps is not None else None
+    _K().tokens(patches.contiguous(), cls.reshape(-1).contiguous(), det.reshape(nd, D).contiguous() if nd else None, pos.contiguous(), x, mr,
+                float(eps) if eps is not None else 0.0)
+    return x, mr
+
+
 def mean_tokens(x):
     """fp32 mean over the tokens of x [B, S, D] -> [B, D]."""
     if not _gpu(x) or x.dtype != torch.bfloat16 or x.shape[-1] % 8 or not x.numel():
