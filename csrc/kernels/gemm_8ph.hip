@@ -40,6 +40,7 @@
 #include "gemm_epilogue.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace shai {
 
@@ -464,13 +465,18 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
         // per-image bias (time embedding) in the wide path: each wave's 128 rows lie inside one image
         const bool b2ok = p.bias2d == nullptr ||
                           (WIDE && (p.rows_per_bias2d & 127) == 0 && (p.bias2d_ld & 7) == 0 && ((uintptr_t)p.bias2d & 15) == 0);
-        const bool fast = m0 + G4_BM <= p.M && n0 + BN <= p.N && b2ok && p.gate == nullptr &&
-                          (p.ldc & 3) == 0 && (R == nullptr || (p.ldr & 3) == 0);
+        const bool inside = m0 + G4_BM <= p.M;
+        const bool fast = n0 + BN <= p.N && b2ok && p.gate == nullptr && (p.ldc & 3) == 0 && (R == nullptr || (p.ldr & 3) == 0);
         if constexpr (WIDE) {
           // 16-byte C / residual / bias accesses: 8-element aligned rows and bases
           const bool wide = fast && (((p.ldc | (R ? p.ldr : 0)) & 7) == 0) &&
                             ((((uintptr_t)C) | (uintptr_t)R | (uintptr_t)p.bias) & 15) == 0;
-          if (wide) {
+          // LAST: rows end inside the tile.  It reads clamped rows, guards its stores and has no statistics (gemm4_stats_ok).  Taken
+          // through epilogue4 below, such a tile held up the others of its round: 6304 x 2304 x 768 with a folded LayerNorm 45.4 ->
+          // 28.3 us, 3700 x 5632 x 1024 gated 73.6 -> 60.4.
+          auto rows = [&](auto last) {
+            constexpr bool LAST = decltype(last)::value;
+            const auto row_of = [&](int m) { return LAST ? min(m, p.M - 1) : m; };
             const bf16_t* __restrict__ bias = p.bias;
             float bq[NP][8];
 #pragma unroll
@@ -490,7 +496,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
               bt[2] = bf2f(bb[1] & 0xffff); bt[3] = bf2f(bb[1] >> 16);
             }
             if (p.bias2d != nullptr) {  // b2ok: the wave's 128 rows share one bias2d row
-              const bf16_t* b2 = p.bias2d + (long)((m0 + wm * 128) / p.rows_per_bias2d) * p.bias2d_ld;
+              const bf16_t* b2 = p.bias2d + (long)(row_of(m0 + wm * 128) / p.rows_per_bias2d) * p.bias2d_ld;
 #pragma unroll
               for (int q = 0; q < NP; ++q) {
                 float t8[8];
@@ -511,8 +517,8 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
             // the next tile restages buffer 1 only after the loop-top barrier) and summed down the rows by lanes
             // owning a column pair: 4 registers per lane.
             constexpr int IG = NJ == 4 ? 4 : 2;
-            float* __restrict__ colp = GLU ? nullptr : p.col_part;
-            float* __restrict__ rowp = GLU ? nullptr : p.row_part;
+            float* __restrict__ colp = GLU || LAST ? nullptr : p.col_part;
+            float* __restrict__ rowp = GLU || LAST ? nullptr : p.row_part;
             bf16_t* cst = g4_smem + G4_STAGE + wid * (IG * 16 * WC);  // [IG * 16][WC] bf16
             float c0 = 0.f, c1 = 0.f, d0 = 0.f, d1 = 0.f;              // column pair (2 lane, 2 lane + 1)
 #pragma unroll
@@ -523,7 +529,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
                 if (R) {
 #pragma unroll
                   for (int ii = 0; ii < IG; ++ii) {
-                    const bf16_t* rrow = R + (long)(m0 + wm * 128 + (i0 + ii) * 16 + fr) * p.ldr + n0 + wn * WC;
+                    const bf16_t* rrow = R + (long)row_of(m0 + wm * 128 + (i0 + ii) * 16 + fr) * p.ldr + n0 + wn * WC;
 #pragma unroll
                     for (int q = 0; q < NP; ++q) rr[ii][q] = *reinterpret_cast<const uint4_*>(rrow + q * 32 + 8 * fq);
                     if (TAIL) rt[ii] = *reinterpret_cast<const uint2_*>(rrow + 2 * NP * 16 + 4 * fq);
@@ -532,7 +538,9 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
 #pragma unroll
                 for (int ii = 0; ii < IG; ++ii) {
                   const int i = i0 + ii;
-                  bf16_t* crow = C + orow(m0 + wm * 128 + i * 16 + fr) * p.ldc + n0 + wn * WC;
+                  const int m = m0 + wm * 128 + i * 16 + fr;
+                  const bool keep = !LAST || m < p.M;
+                  bf16_t* crow = C + orow(row_of(m)) * p.ldc + n0 + wn * WC;
                   // row statistics of this lane's columns, shifted by the row's first stored value in this
                   // slot (lane fq = 0, column 0): (mean, M2) per slot, combined exactly by the finalizer
                   float rs = 0.f, rq = 0.f, rk = 0.f;
@@ -551,7 +559,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
                       for (int e = 0; e < 8; ++e) v[e] += r8[e] * p.res_alpha;
                     }
                     const uint4_ pv = pack8(v);
-                    *reinterpret_cast<uint4_*>(crow + q * 32 + 8 * fq) = pv;
+                    if (keep) *reinterpret_cast<uint4_*>(crow + q * 32 + 8 * fq) = pv;
                     if (colp) *reinterpret_cast<uint4_*>(cst + (ii * 16 + fr) * WC + q * 32 + 8 * fq) = pv;
                     if (rowp) {  // moments of the stored (bf16-rounded) values: what the consumer reads
                       float f[8];
@@ -576,7 +584,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
                     uint2_ o;
                     o[0] = pack2(v[0], v[1]);
                     o[1] = pack2(v[2], v[3]);
-                    *reinterpret_cast<uint2_*>(crow + 2 * NP * 16 + 4 * fq) = o;
+                    if (keep) *reinterpret_cast<uint2_*>(crow + 2 * NP * 16 + 4 * fq) = o;
                     if (colp) *reinterpret_cast<uint2_*>(cst + (ii * 16 + fr) * WC + 2 * NP * 16 + 4 * fq) = o;
                     if (rowp) {
                       const float f[4] = {bf2f(o[0] & 0xffff), bf2f(o[0] >> 16), bf2f(o[1] & 0xffff), bf2f(o[1] >> 16)};
@@ -624,7 +632,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
                 if (R) {
 #pragma unroll
                   for (int ii = 0; ii < IG; ++ii) {
-                    const bf16_t* rrow = R + (long)(m0 + wm * 128 + (i0 + ii) * 16 + fr) * p.ldr + ((n0 + wn * WC) >> 1);
+                    const bf16_t* rrow = R + (long)row_of(m0 + wm * 128 + (i0 + ii) * 16 + fr) * p.ldr + ((n0 + wn * WC) >> 1);
 #pragma unroll
                     for (int q = 0; q < NP; ++q) rr[ii][q] = *reinterpret_cast<const uint2_*>(rrow + q * 16 + 4 * fq);
                     if (TAIL) rt[ii] = *reinterpret_cast<const uint32_t*>(rrow + NP * 16 + 2 * fq);
@@ -633,7 +641,9 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
 #pragma unroll
                 for (int ii = 0; ii < IG; ++ii) {
                   const int i = i0 + ii;
-                  bf16_t* crow = C + (long)(m0 + wm * 128 + i * 16 + fr) * p.ldc + ((n0 + wn * WC) >> 1);
+                  const int m = m0 + wm * 128 + i * 16 + fr;
+                  const bool keep = !LAST || m < p.M;
+                  bf16_t* crow = C + (long)row_of(m) * p.ldc + ((n0 + wn * WC) >> 1);
                   uint32_t wq[NP][2];
 #pragma unroll
                   for (int q = 0; q < NP; ++q) {
@@ -662,14 +672,15 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
                       wq[q][e] = r[0];
                       wq[q + 1][e] = r[1];
                     }
-                    *reinterpret_cast<uint4_*>(crow + q * 16 + 16 * (fq & 1) + 8 * (fq >> 1)) =
-                        uint4_{wq[q][0], wq[q][1], wq[q + 1][0], wq[q + 1][1]};
+                    if (keep)
+                      *reinterpret_cast<uint4_*>(crow + q * 16 + 16 * (fq & 1) + 8 * (fq >> 1)) =
+                          uint4_{wq[q][0], wq[q][1], wq[q + 1][0], wq[q + 1][1]};
                   }
                   if constexpr ((NP & 1) != 0) {
                     uint2_ w;
                     w[0] = wq[NP - 1][0];
                     w[1] = wq[NP - 1][1];
-                    *reinterpret_cast<uint2_*>(crow + (NP - 1) * 16 + 4 * fq) = w;
+                    if (keep) *reinterpret_cast<uint2_*>(crow + (NP - 1) * 16 + 4 * fq) = w;
                   }
                   if constexpr (TAIL) {
                     float o0 = (acc[i][NJ - 1][0] * p.alpha + bt[0]) * apply_act<ACT>(acc[i][NJ - 1][1] * p.alpha + bt[1]);
@@ -678,7 +689,7 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
                       o0 += bf2f(rt[ii] & 0xffff) * p.res_alpha;
                       o1 += bf2f(rt[ii] >> 16) * p.res_alpha;
                     }
-                    *reinterpret_cast<uint32_t*>(crow + NP * 16 + 2 * fq) = pack2(o0, o1);
+                    if (keep) *reinterpret_cast<uint32_t*>(crow + NP * 16 + 2 * fq) = pack2(o0, o1);
                   }
                 }
               }
@@ -686,11 +697,16 @@ __global__ void __launch_bounds__(512) gemm4_kernel(const GemmArgs p, float* __r
             if (colp && lane < WC / 2)  // column totals over the wave's 128 rows -> partial block (m0 + 128 wm) / 128
               *reinterpret_cast<float4_*>(colp + ((long)((m0 + wm * 128) >> 7) * p.N + n0 + wn * WC + 2 * lane) * 2) =
                   float4_{c0, d0, c1, d1};
-            wide_done = true;
-            return;
+            wide_done = !LAST;
+          };
+          // (256 columns: guards or a second copy cost the persistent 320-wide kernel registers that it lacks, 16384 x 640 x 2560 77 ->
+          // 89 and 100 us)
+          if constexpr (BN == 256 && CONV != 3) {
+            if (wide && !inside) return rows(std::true_type{});
           }
+          if (wide && inside) return rows(std::false_type{});
         }
-        if (fast && !WIDE) {
+        if (fast && inside && !WIDE) {
           // interior tile: per-column bias hoisted, residual rows prefetched in groups of IG row blocks (all 8
           // at NJ = 4; 2 at NJ = 5, where 160 accumulator registers leave no room for 80 more)
           const bf16_t* __restrict__ bias = p.bias;

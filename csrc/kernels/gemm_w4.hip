@@ -304,10 +304,14 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
   bf16_t* C = p.C + (long)b * p.batch_c;
   const bf16_t* R = p.residual ? p.residual + (long)b * p.batch_r : nullptr;
   const uintptr_t ptrs = (uintptr_t)C | (uintptr_t)R | (uintptr_t)p.bias | (uintptr_t)p.bias2d | (uintptr_t)p.gate;
-  const bool full = m0 + BM <= p.M && n0 + BN <= p.N && ((p.ldc | (R ? p.ldr : 0)) & 7) == 0 && (ptrs & 15) == 0 &&
+  const bool full = n0 + BN <= p.N && ((p.ldc | (R ? p.ldr : 0)) & 7) == 0 && (ptrs & 15) == 0 &&
                     (p.bias2d == nullptr || (p.bias2d_ld & 7) == 0) && (p.gate == nullptr || (p.gate_stride & 7) == 0);
   constexpr int NQ = BNB / 2;
   if (full) {
+    // Rows may end inside the tile: it reads clamped rows and guards its stores.  Taken through the element-wise form below, such a
+    // tile took several times the others' time: 8000 x 4096 x 4096 275 -> 224 us, 8000 x 28672 x 4096 gated 1575 -> 1429, 1600 x
+    // 4096 x 14336 339 -> 307; whole tiles as before (8192 x 28672 x 4096 1440 and 1435; a second copy of the epilogue for them: 3 %
+    // slower on gated products).
     float bq[NQ][8];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -318,7 +322,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < BMB; ++i) {
-      const int m = m0 + wr * WM + 16 * i + fr;
+      const int row = m0 + wr * WM + 16 * i + fr, m = min(row, p.M - 1);
       const bf16_t* b2 = p.bias2d ? p.bias2d + (long)(m / p.rows_per_bias2d) * p.bias2d_ld : nullptr;
       const bf16_t* gr = p.gate ? p.gate + ((long)b * p.M + m) / p.rows_per_gate * p.gate_stride : nullptr;
 #pragma unroll
@@ -353,7 +357,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
           uint2_ w;
           w[0] = pack2(o[0], o[1]);
           w[1] = pack2(o[2], o[3]);
-          *reinterpret_cast<uint2_*>(C + (long)m * p.ldc + (n >> 1)) = w;
+          if (row < p.M) *reinterpret_cast<uint2_*>(C + (long)m * p.ldc + (n >> 1)) = w;
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = apply_act<ACT>(v[e]);
@@ -369,13 +373,14 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] += r8[e] * p.res_alpha;
           }
-          *reinterpret_cast<uint4_*>(C + (long)m * p.ldc + n) = pack8(v);
+          const uint4_ w = pack8(v);
+          if (row < p.M) *reinterpret_cast<uint4_*>(C + (long)m * p.ldc + n) = w;
         }
       }
     }
   } else {
-    // edge tiles: element-wise, guarded (no array indexed at run time: every index is unrolled, no early loop
-    // exits -- a run-time-bounded loop over the accumulators sends all of them to scratch)
+    // columns that end inside the tile, odd strides and bases: element-wise, guarded (no array indexed at run time: every index is
+    // unrolled, no early loop exits -- a run-time-bounded loop over the accumulators sends all of them to scratch)
 #pragma unroll
     for (int i = 0; i < BMB; ++i) {
       const int m = m0 + wr * WM + 16 * i + fr;

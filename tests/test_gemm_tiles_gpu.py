@@ -1,0 +1,99 @@
+"""Rings of K-tiles (gemm_deep.hip), and tiles that the rows end in (gemm_8ph.hip, gemm_w4.hip), against fp32
+PyTorch, each config forced.
+
+Tolerance: inputs are bf16, sums fp32, outputs rounded to bf16 once: a relative error of at most 2^-8 / sqrt(3) rms = 2.3e-3; 4e-3
+leaves room for the activations' approximations and the residual's cancellation."""
+import os
+import subprocess
+import sys
+
+import pytest
+import torch
+
+from shai_amd import ops
+from test_gemm_deep_gpu import CONV_SCRIPT
+
+pytestmark = pytest.mark.gpu
+GROUPS = [16, 17, 18]                    # the tiles with waves along K and the deep ring
+WHOLE = [9, 10, 11, 12, 13]              # eight phases (256 and 320 wide, persistent), four waves
+ACTS = {None: lambda t: t, "silu": torch.nn.functional.silu, "gelu": torch.nn.functional.gelu,
+        "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}
+TOL = 4e-3
+
+
+def _close(a, b):
+    a, b = a.float().cpu(), b.float().cpu()
+    return ((a - b).norm() / b.norm()).item() < TOL
+
+
+def _problem(M, N, K, dev):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    make = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    return make(M, K).bfloat16(), (make(N, K) / K ** 0.5).bfloat16(), make(N).bfloat16(), make(M, N).bfloat16()
+
+
+# M: one row, a tile's edges, a second tile of one row; N: inside a tile, and whole tiles; K: fewer K-tiles than the ring holds
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (129, 63, 72), (192, 128, 64), (193, 256, 192), (257, 330, 776), (511, 640, 1280)])
+@pytest.mark.parametrize("cfg", GROUPS + WHOLE)
+def test_in_place_residual(cuda, M, N, K, cfg):
+    a, w, b, r = _problem(M, N, K, cuda)
+    want = a.float() @ w.float().t() + b.float() + r.float()
+    out = torch.full((M + 1, N), 7.0, device=cuda, dtype=torch.bfloat16)
+    out[:M] = r
+    ops.gemm_into(a, w, out[:M], b, residual=out[:M], force_cfg=cfg)
+    assert _close(out[:M], want)
+    assert bool((out[M] == 7).all())
+
+
+@pytest.mark.parametrize("M", [100, 300, 513])
+@pytest.mark.parametrize("act", ["silu", "gelu", "gelu_tanh"])
+@pytest.mark.parametrize("cfg", GROUPS + WHOLE)
+def test_glu(cuda, M, act, cfg):
+    a, w, b, _ = _problem(M, 1280, 320, cuda)
+    out = torch.full((M + 1, 640), 7.0, device=cuda, dtype=torch.bfloat16)
+    ops.gemm_into(a, w, out[:M], b, act=act, glu=True, force_cfg=cfg)
+    y = a.float() @ w.float().t() + b.float()
+    assert _close(out[:M], y[:, 0::2] * ACTS[act](y[:, 1::2]))
+    assert bool((out[M] == 7).all())
+
+
+@pytest.mark.parametrize("cfg", GROUPS + WHOLE[:4])
+def test_folded_layernorm(cuda, cfg):
+    M, N, K = 300, 640, 768
+    a, w, b, _ = _problem(M, N, K, cuda)
+    mean, rstd, s = torch.randn(M, device=cuda), torch.rand(M, device=cuda) + 0.5, w.float().sum(1)
+    out = torch.empty(M, N, device=cuda, dtype=torch.bfloat16)
+    ops._K().gemm(a, w, out, b, None, 1, None, 1.0, 1.0, ops.act_id("gelu"), False, None, 1, cfg, -1.0, None,
+                  torch.stack([mean, rstd], 1).contiguous(), s)
+    assert _close(out, ACTS["gelu"](rstd[:, None] * (a.float() @ w.float().t() - mean[:, None] * s) + b.float()))
+
+
+# rows of a time embedding: the last tile's rows lie in the last image, whose row is the last there is
+@pytest.mark.parametrize("cfg", WHOLE)
+def test_rows_of_images(cuda, cfg):
+    M, N, K = 384, 1280, 128
+    a, w, b, r = _problem(M, N, K, cuda)
+    per_image = torch.randn(3, N, device=cuda).bfloat16()
+    out = torch.empty_like(r)
+    ops._K().gemm(a, w, out, b, per_image, 128, r, 0.5, 2.0, ops.act_id("silu"), False, None, 1, cfg)
+    y = 0.5 * (a.float() @ w.float().t()) + b.float() + per_image.float().repeat_interleave(128, 0)
+    assert _close(out, ACTS["silu"](y) + 2.0 * r.float())
+
+
+@pytest.mark.parametrize("splits", [2, 5])
+@pytest.mark.parametrize("cfg", GROUPS)
+def test_split_k(cuda, splits, cfg):
+    a, w, b, r = _problem(197, 330, 1544, cuda)
+    out = torch.empty_like(r)
+    ops.gemm_into(a, w, out, b, act="gelu", residual=r, force_cfg=3000 + 100 * splits + cfg)
+    assert _close(out, ACTS["gelu"](a.float() @ w.float().t() + b.float()) + r.float())
+
+
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("cfg", GROUPS)
+def test_convolution(cuda, cfg, splits):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, SHAI_GEMM_FORCE=str(cfg), SHAI_GEMM_FORCE_SPLITS=str(splits))
+    r = subprocess.run([sys.executable, "-c", CONV_SCRIPT.format(root=root, tol=TOL)], env=env, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-3000:]
