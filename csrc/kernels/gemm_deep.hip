@@ -13,7 +13,17 @@
 // split of K; M x N x K): 197 x 768 x 768 8.4 -> 6.2, 197 x 3072 x 768 12.3 -> 6.8, 197 x 768 x 3072 12.4 -> 10.3 (4 splits),
 // 154 x 4096 x 1024 13.7 -> 7.6, 512 x 1280 x 1280 14.4 -> 8.5, 2048 x 640 x 2560 22.7 -> 17.9, 8192 x 320 x 1280 19.4 -> 17.6
 // (128 x 128: 14.3), 4096 x 1024 x 2816 35.1 -> 29.9.  Which one runs is the autotuner's choice, like that of every tile.
-// (Both with 8-byte stores; 16-byte ones, gemm_lds_kernel.h, take about a tenth off either.)
+//   192 x 128, two groups along K of four waves (96 x 64 each), 3 tiles in flight: a row count between, one round of the chip where
+//     128 x 128 takes two (6304 x 768 x 3072: 198 workgroups of 300) and, as K is split inside the workgroup, without a fold:
+//     47.2 -> 37.2, 4096 x 1280 x 5120 74.5 (256 x 320, four parts) -> 58.5, 512 x 9216 x 3072 56.2 -> 41.4, a convolution of 512 x
+//     1280 x 23040 63.0 -> 49.6.  Its sums meet in two passes: all of them are larger than the ring.
+//   128 x 128 in that form: LDS gives 64 KB of fragments per K-tile instead of 96.  4096 x 1024 x 2816 28.5 -> 27.9, 1024 x 3072 x 12288
+//     100.2 (256 x 256, four parts) -> 83.5.
+//   192 x 128, four waves, 1 tile in flight, two workgroups to a CU: the end of one beside the other's loop.  1024 x 9216 x 3072 83.6 ->
+//     74.0, 3700 x 5632 x 1024 gated 60.4 -> 56.6, 16384 x 640 x 2560 65.9 -> 64.0.
+// Their LDS DMA runs at half the 118 to 130 GB/s a CU that it reaches alone (any pitch, one line or eight an instruction): what bounds
+// them is the MFMA pipe (52 % busy), a third of the waves' time at the barrier or waiting for loads.
+// (The first two with 8-byte stores; 16-byte ones, gemm_lds_kernel.h, take about a tenth off either.)
 // (Operands straight into registers, with the waves splitting K, were tried too: 16 rows x 64 bytes per load instruction reach
 // 14 bytes per clock and CU, LDS-DMA 30.)
 #include "gemm_lds_kernel.h"
@@ -28,7 +38,8 @@ namespace {
 struct Deep {
   int bm, bn, wm, wn, wk, stages;
 };
-constexpr Deep kDeep[kDeepCfgs] = {{64, 64, 2, 2, 2, 4}, {128, 64, 2, 2, 2, 3}, {128, 128, 2, 4, 1, 4}};
+constexpr Deep kDeep[kDeepCfgs] = {{64, 64, 2, 2, 2, 4}, {128, 64, 2, 2, 2, 3}, {128, 128, 2, 4, 1, 4},
+                                   {192, 128, 2, 2, 2, 4}, {128, 128, 2, 2, 2, 4}, {192, 128, 2, 2, 1, 2}};
 
 template <int W, bool CONV, bool GLU, int ACT, bool SPLITK>
 void launch_one(const GemmArgs& a, float* ws, int splits, int kps, hipStream_t s) {
@@ -89,7 +100,10 @@ void launch_which(const GemmArgs& a, int which, float* ws, int splits, hipStream
   switch (which) {
     case 0: launch_tile<0, CONV>(a, ws, splits, s); break;
     case 1: launch_tile<1, CONV>(a, ws, splits, s); break;
-    default: launch_tile<2, CONV>(a, ws, splits, s); break;
+    case 2: launch_tile<2, CONV>(a, ws, splits, s); break;
+    case 3: launch_tile<3, CONV>(a, ws, splits, s); break;
+    case 4: launch_tile<4, CONV>(a, ws, splits, s); break;
+    default: launch_tile<5, CONV>(a, ws, splits, s); break;
   }
 }
 

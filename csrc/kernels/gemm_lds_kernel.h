@@ -236,30 +236,35 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
   // 128: 51.2 -> 44.3), 8192 x 960, K = 320 14.5 -> 12.2, 6304 x 768, K = 768 17.8 -> 15.7.  (Whole lines by way of LDS: 1 .. 3 % more,
   // not worth the second path.)
   const int fw = EPI & kEpi8 ? (fr & 19) | (fr & 4) << 1 | (fr & 8) >> 1 : fr;
-  auto compute = [&](int buf) {
-    const bf16_t* sa = smem + buf * STAGE;
-    const bf16_t* sw = sa + BM * BK2;
-#pragma unroll
-    for (int t = 0; t < 4 / WK; ++t) {
-      const int s = wk * (4 / WK) + t;
-      bf16x8 af[IM], wf[JN];
-#pragma unroll
-      for (int i = 0; i < IM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(sa + swz2(wm * TM + i * 32 + fr, 2 * s + fh));
-#pragma unroll
-      for (int j = 0; j < JN; ++j) wf[j] = *reinterpret_cast<const bf16x8*>(sw + swz2(wn * TN + j * 32 + fw, 2 * s + fh));
-#pragma unroll
-      for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
-    }
-  };
-
-  if constexpr (STAGES == 2) {
+  // AHEAD: fragments of the next MFMA step are read beside the MFMAs of this one, across the barrier between K-tiles too.  One after
+  // the other, by all waves at once behind each barrier, LDS idled beside the MFMAs and they beside it: us before -> after, 4096 x 1024 x
+  // 2816 31.0 -> 28.5 (128 x 128, four stages), 512 x 1280 x 5120 21.3 -> 19.6 (64 x 64), 6304 x 768 x 3072 39.8 -> 36.8 (192 x 128), 2048 x
+  // 640 x 2560 37.1 -> 35.5 (128 x 128, two stages).  The 128 x 64 tile of two stages, three to a CU, lost (46.9 -> 49.5); the larger
+  // eight-wave ones have no registers for it.
+  constexpr bool AHEAD = STAGES > 2 || (WM * WN == 4 && IM * JN >= 4);
+  if constexpr (!AHEAD) {
     if (nk > 0) {
       stage(0, k_begin);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
+    auto compute = [&](int buf) {
+      const bf16_t* sa = smem + buf * STAGE;
+      const bf16_t* sw = sa + BM * BK2;
+#pragma unroll
+      for (int t = 0; t < 4 / WK; ++t) {
+        const int s = wk * (4 / WK) + t;
+        bf16x8 af[IM], wf[JN];
+#pragma unroll
+        for (int i = 0; i < IM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(sa + swz2(wm * TM + i * 32 + fr, 2 * s + fh));
+#pragma unroll
+        for (int j = 0; j < JN; ++j) wf[j] = *reinterpret_cast<const bf16x8*>(sw + swz2(wn * TN + j * 32 + fw, 2 * s + fh));
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+          for (int j = 0; j < JN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+      }
+    };
     for (int kt = 0; kt < nk; ++kt) {
       const int cur = kt & 1;
       if (kt + 1 < nk) stage(cur ^ 1, k_begin + (kt + 1) * BK2);
@@ -268,23 +273,66 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
       __syncthreads();
     }
   } else {
-    // A ring of STAGES tiles: t+1 .. t+STAGES-1 stay in flight while tile t is consumed.
-    // Per iteration: counted vmcnt retires this wave's DMA of tile t (FIFO), a raw
-    // s_barrier makes every wave's part visible AND proves all waves finished reading
-    // the buffer of tile t-1, which is then refilled with tile t+STAGES-1.  Tiles past the
-    // end are issued too (every lane out of range: zeros, no traffic), so that the count
-    // before each tile is the same; the last wait drains them.
+    // A ring of STAGES tiles.  In the last step of tile t a counted vmcnt retires this wave's DMA of tile t + 1 (FIFO), its reads of
+    // tile t have arrived, and a raw s_barrier makes both true of every wave: tile t's buffer takes tile t + STAGES, and tile t + 1
+    // is read.  Tiles past the end are issued too (every lane out of range: zeros, no traffic), so that the count before each tile
+    // is the same; the last wait drains them.
     constexpr int PER = JA + JB;  // DMA instructions per wave per tile
-    static_assert((STAGES - 2) * PER < 64, "vmcnt has six bits");
+    constexpr int KS = 4 / WK;
+    static_assert((STAGES - 1) * PER < 64, "vmcnt has six bits");
+    static_assert(KS % 2 == 0, "two sets of fragments take turns");
+    // fragments of this wave group's MFMA step t of the K-tile in buffer buf
+    struct Frags {
+      bf16x8 a[IM], w[JN];
+    };
+    auto read = [&](int buf, int t, Frags& f) {
+      const bf16_t* sa = smem + buf * STAGE;
+      const bf16_t* sw = sa + BM * BK2;
+      const int s = wk * (4 / WK) + t;
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) stage(s, k_begin + s * BK2);
+      for (int i = 0; i < IM; ++i) f.a[i] = *reinterpret_cast<const bf16x8*>(sa + swz2(wm * TM + i * 32 + fr, 2 * s + fh));
+#pragma unroll
+      for (int j = 0; j < JN; ++j) f.w[j] = *reinterpret_cast<const bf16x8*>(sw + swz2(wn * TN + j * 32 + fw, 2 * s + fh));
+    };
+    auto multiply = [&](const Frags& f) {
+#pragma unroll
+      for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[j], f.a[i], acc[i][j], 0, 0, 0);
+    };
+    Frags x[2];
+    auto meet = [] {
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) stage(s, k_begin + s * BK2);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * PER) : "memory");
+    meet();
+    read(0, 0, x[0]);
     int buf = 0;
     for (int kt = 0; kt < nk; ++kt) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * PER) : "memory");
-      __builtin_amdgcn_s_barrier();
-      stage(buf == 0 ? STAGES - 1 : buf - 1, k_begin + (kt + STAGES - 1) * BK2);
-      compute(buf);
-      buf = buf == STAGES - 1 ? 0 : buf + 1;
+      const int next = buf == STAGES - 1 ? 0 : buf + 1;
+#pragma unroll
+      for (int t = 0; t < KS; ++t) {
+        if (t < KS - 1) {
+          read(buf, t + 1, x[(t + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        } else {
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * PER) : "memory");
+#pragma unroll
+          for (int i = 0; i < IM; ++i) asm volatile("" : "+v"(x[t & 1].a[i]));
+#pragma unroll
+          for (int j = 0; j < JN; ++j) asm volatile("" : "+v"(x[t & 1].w[j]));
+          meet();
+          read(next, 0, x[(t + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+          stage(buf, k_begin + (kt + STAGES) * BK2);
+        }
+        multiply(x[t & 1]);
+      }
+      buf = next;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
@@ -292,30 +340,34 @@ __global__ void __launch_bounds__(WM * WN * WK * 64) gemm2_kernel(const GemmArgs
   // ---- epilogue: lane owns row m, 4 groups of 4 consecutive n (2 of 8 with kEpi8) per 32x32 block.  WK > 1: the wave groups' sums meet in
   // LDS (the ring is free by now) and are added in group order; each group finishes 4 / WK of the four column groups.
   if constexpr (WK > 1) {
-    static_assert(NW * IM * JN * 4096 <= STAGES * STAGE * 2, "partial tiles larger than the ring");
+    constexpr int BLOCKS = IM * JN, PASS = NW * BLOCKS * 4096 <= STAGES * STAGE * 2 ? BLOCKS : BLOCKS / 2;   // blocks of a wave at a time
+    static_assert(BLOCKS % PASS == 0 && NW * PASS * 4096 <= STAGES * STAGE * 2, "partial tiles larger than the ring");
     float4_* part = reinterpret_cast<float4_*>(smem);
-    __syncthreads();
 #pragma unroll
-    for (int b = 0; b < IM * JN; ++b)
+    for (int b0 = 0; b0 < BLOCKS; b0 += PASS) {
+      __syncthreads();
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float16_& a = acc[b / JN][b % JN];
-        part[((wid * IM * JN + b) * 4 + g) * 64 + lane] = float4_{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
-      }
-    __syncthreads();
+      for (int b = 0; b < PASS; ++b)
 #pragma unroll
-    for (int b = 0; b < IM * JN; ++b)
+        for (int g = 0; g < 4; ++g) {
+          const float16_& a = acc[(b0 + b) / JN][(b0 + b) % JN];
+          part[((wid * PASS + b) * 4 + g) * 64 + lane] = float4_{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+        }
+      __syncthreads();
 #pragma unroll
-      for (int g = 0; g < 4 / WK; ++g) {
-        const int at = (wid % (WM * WN) * IM * JN + b) * 4 + wk * (4 / WK) + g;
-        float4_ t[WK];
+      for (int b = 0; b < PASS; ++b)
 #pragma unroll
-        for (int q = 0; q < WK; ++q) t[q] = part[(at + q * WM * WN * IM * JN * 4) * 64 + lane];
+        for (int g = 0; g < 4 / WK; ++g) {
+          const int at = (wid % (WM * WN) * PASS + b) * 4 + wk * (4 / WK) + g;
+          float4_ t[WK];
 #pragma unroll
-        for (int q = 1; q < WK; ++q) t[0] += t[q];
+          for (int q = 0; q < WK; ++q) t[q] = part[(at + q * WM * WN * PASS * 4) * 64 + lane];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[b / JN][b % JN][4 * g + e] = t[0][e];
-      }
+          for (int q = 1; q < WK; ++q) t[0] += t[q];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[(b0 + b) / JN][(b0 + b) % JN][4 * g + e] = t[0][e];
+        }
+    }
   }
   constexpr int G1 = 4 / WK;
   const int g0 = wk * G1;

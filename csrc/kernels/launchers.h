@@ -205,7 +205,7 @@ bool gemm2_cfg_splittable(int cfg);  // false: the config always runs the whole 
 bool gemm_w4_supported(const GemmArgs& a);
 void launch_gemm_w4(const GemmArgs& a, int bn, hipStream_t s);
 // small tiles with a deep ring of K-tiles in flight (gemm_deep.hip)
-constexpr int kDeepCfgs = 3;
+constexpr int kDeepCfgs = 6;
 bool gemm_deep_supported(const GemmArgs& a);
 void gemm_deep_tile(int which, int* bm, int* bn);
 void launch_gemm_deep(const GemmArgs& a, int which, float* ws, int splits, hipStream_t s);

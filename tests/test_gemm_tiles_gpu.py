@@ -1,4 +1,4 @@
-"""Rings of K-tiles (gemm_deep.hip), and tiles that the rows end in (gemm_8ph.hip, gemm_w4.hip), against fp32
+"""Tiles with two groups of waves along K (gemm_deep.hip), and tiles that the rows end in (gemm_8ph.hip, gemm_w4.hip), against fp32
 PyTorch, each config forced.
 
 Tolerance: inputs are bf16, sums fp32, outputs rounded to bf16 once: a relative error of at most 2^-8 / sqrt(3) rms = 2.3e-3; 4e-3
@@ -14,7 +14,7 @@ from shai_amd import ops
 from test_gemm_deep_gpu import CONV_SCRIPT
 
 pytestmark = pytest.mark.gpu
-GROUPS = [16, 17, 18]                    # the tiles with waves along K and the deep ring
+GROUPS = [16, 17, 18, 19, 20, 21]        # 64 x 64, 128 x 64, 128 x 128; 192 x 128 and 128 x 128 with two wave groups, 192 x 128 two to a CU
 WHOLE = [9, 10, 11, 12, 13]              # eight phases (256 and 320 wide, persistent), four waves
 ACTS = {None: lambda t: t, "silu": torch.nn.functional.silu, "gelu": torch.nn.functional.gelu,
         "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}
