@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "kernels/fold_norm.h"
 #include "kernels/launchers.h"
 #include "kernels/vision.h"
 
@@ -115,7 +116,7 @@ std::string gemm_bucket_key(const shai::GemmArgs& g) {
 bool lib_enabled();
 constexpr int kLibCfgId = 2000;  // = kLibCfg (below)
 
-bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out) {
+bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out, const char* suffix = "") {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   // a cached library choice counts as untuned while the library path is off (the tuner races it afresh)
   auto usable = [](const Choice& c) { return c.cfg != kLibCfgId || lib_enabled(); };
@@ -124,8 +125,9 @@ bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out)
     *out = it->second;
     return true;
   }
-  const std::string bk = gemm_bucket_key(g);
+  std::string bk = gemm_bucket_key(g);
   if (bk.empty()) return false;
+  bk += suffix;
   it = g_tuned.find(bk);
   if (it == g_tuned.end() || !usable(it->second)) return false;
   *out = it->second;
@@ -133,11 +135,11 @@ bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out)
   return true;
 }
 
-void store_choice(const shai::GemmArgs& g, const std::string& key, const Choice& c) {
+void store_choice(const shai::GemmArgs& g, const std::string& key, const Choice& c, const char* suffix = "") {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tuned[key] = c;
   const std::string bk = gemm_bucket_key(g);
-  if (!bk.empty() && !g_tuned.count(bk)) g_tuned[bk] = c;
+  if (!bk.empty() && !g_tuned.count(bk + suffix)) g_tuned[bk + suffix] = c;
 }
 
 bool skinny2_enabled() {  // SHAI_SKINNY2=0 keeps the wide skinny kernel out of the tuner (A/B)
@@ -295,11 +297,52 @@ void flush_device_caches(hipStream_t st) {
   shai::launch_cache_flush(buf, kBytes, reinterpret_cast<unsigned*>(static_cast<char*>(buf) + kBytes), st);
 }
 
+// The row norm of the product's output, beside y = g.C.
+void launch_norm(const shai::GemmArgs& g, const shai::FoldNormArgs& n) {
+  shai::RowNormArgs r{};
+  r.x = g.C;
+  r.w = n.gamma;
+  r.b = n.beta;
+  r.out = n.out;
+  r.rows = g.M;
+  r.D = g.N;
+  r.x_stride = g.ldc;
+  r.out_stride = g.N;
+  r.eps = n.eps;
+  if (n.rms) shai::launch_rmsnorm(r, stream());
+  else shai::launch_layernorm(r, stream());
+}
+
+// A product with the row norm of its output: a split choice's fold and the norm are one launch.
+void launch_then_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, shai::FoldNormArgs n) {
+  n.y = g.C;
+  const bool skinny = (c.cfg == kSkinnyCfg || c.cfg == kSkinnyFixCfg) && shai::skinny_supported(g);
+  const bool tile = c.cfg >= 0 && c.cfg < shai::gemm2_num_cfgs() && shai::gemm2_cfg_supported(g, c.cfg) && shai::gemm2_cfg_splittable(c.cfg);
+  const int splits = skinny ? std::min(c.splits, shai::skinny_max_kgroups(g)) : c.splits;
+  if ((!skinny && !tile) || splits <= 1 || g.act != 0 || g.glu || g.alpha != 1.f || g.ldc != g.N || !shai::fold_norm_supported(n)) {
+    launch_choice(g, like, c);
+    launch_norm(g, n);
+    return;
+  }
+  Tensor ws;
+  if (skinny) {
+    ws = at::empty({(long)(shai::skinny_workspace_bytes_kg(g, splits) / sizeof(float))}, like.options().dtype(at::kFloat));
+    shai::launch_skinny_kg(g, ws.data_ptr<float>(), splits, stream(), false, false);
+  } else {
+    ws = at::empty({(long)splits * g.M * g.N}, like.options().dtype(at::kFloat));
+    g.no_fold = 1;
+    shai::launch_gemm2_cfg(g, ws.data_ptr<float>(), c.cfg, splits, stream());
+  }
+  n.parts = ws.data_ptr<float>();
+  n.splits = splits;
+  shai::launch_fold_norm(n, stream());
+}
+
 // Candidates are timed into a scratch output so that in-place epilogues (C aliasing
 // the residual, e.g. x = x + gate * f(x)) are applied exactly once, by the caller's
 // final launch.  skinny_only: the problem has an epilogue only the skinny kernel implements
 // (folded RMSNorm), so only its K-group counts are candidates.
-Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only = false) {
+Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only = false, const shai::FoldNormArgs* norm = nullptr) {
   shai::GemmArgs g = g_real;
   const long n_out = g.glu ? g.N / 2 : g.N;
   const int nb = g.batch > 0 ? g.batch : 1;
@@ -320,7 +363,7 @@ Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only =
   if (shai::skinny_supported(g))
     for (int kg = 1; kg <= shai::skinny_max_kgroups(g); kg *= 2) {
       cands.push_back({kSkinnyCfg, kg});
-      if (kg > 1) cands.push_back({kSkinnyFixCfg, kg});
+      if (kg > 1 && norm == nullptr) cands.push_back({kSkinnyFixCfg, kg});
     }
   if (shai::skinny2_supported(g) && skinny2_enabled())
     for (int kg = 1; kg <= shai::skinny2_max_kgroups(g); kg *= 2) {
@@ -330,6 +373,10 @@ Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only =
   // residual epilogues are in place (C aliases the residual): timing them into the scratch output is not
   // equivalent, so only bias-or-nothing problems race the library
   if (!skinny_only && lib_enabled() && lib_supported(g_real) && !g_real.residual) cands.push_back({kLibCfg, 1});
+  auto launch = [&](const Choice& c) {
+    if (norm) launch_then_norm(g, like, c, *norm);
+    else launch_choice(g, like, c);
+  };
   hipStream_t st = stream();
   hipEvent_t e0, e1;
   hipEventCreate(&e0);
@@ -341,14 +388,14 @@ Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only =
   // Infinity Cache so the candidates are ranked by their HBM-streaming speed, not by a warm-cache replay.
   const bool cold = g.M <= 64 && (long)g.N * g.K * (g.w_scale ? 1 : 2) >= (4L << 20);
   for (const Choice& c : cands) {
-    launch_choice(g, like, c);  // warm (also instantiates caches)
+    launch(c);  // warm (also instantiates caches)
     float ms = 0.f;
     if (cold) {  // median of 5 single cold launches
       float ts[5];
       for (int r = 0; r < 5; ++r) {
         flush_device_caches(st);
         hipEventRecord(e0, st);
-        launch_choice(g, like, c);
+        launch(c);
         hipEventRecord(e1, st);
         hipEventSynchronize(e1);
         ts[r] = 0.f;
@@ -358,7 +405,7 @@ Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only =
       ms = ts[2];
     } else {
       hipEventRecord(e0, st);
-      for (int r = 0; r < 3; ++r) launch_choice(g, like, c);
+      for (int r = 0; r < 3; ++r) launch(c);
       hipEventRecord(e1, st);
       hipEventSynchronize(e1);
       hipEventElapsedTime(&ms, e0, e1);
@@ -399,6 +446,8 @@ struct OutStats {
   // GroupNorm of the output in one launch (groupnorm.hip), behind a split-K choice the fold with it; keep: the output itself is wanted
   const shai::GnOneArgs* one = nullptr;
   bool keep = true;
+  // the row norm of the output, behind a split-K choice in one launch with its fold
+  const shai::FoldNormArgs* norm = nullptr;
   bool any() const { return gn_part != nullptr || ln_mr != nullptr; }
 };
 
@@ -430,6 +479,10 @@ void launch_with_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, con
 void launch_final(shai::GemmArgs g, const Tensor& like, const Choice& c, const OutStats* st) {
   if (st != nullptr && st->one != nullptr) {
     launch_with_norm(g, like, c, *st);
+    return;
+  }
+  if (st != nullptr && st->norm != nullptr) {
+    launch_then_norm(g, like, c, *st->norm);
     return;
   }
   if (st == nullptr || !st->any()) {
@@ -481,6 +534,7 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
       n.x = g.C;
       shai::launch_gn_one(n, stream());
     }
+    if (st && st->norm) launch_norm(g, *st->norm);
     if (st && st->any()) {  // v1 writes no statistics
       if (st->gn_part) shai::launch_col_partials(g.C, g.M, g.N, g.ldc, st->gn_part, stream());
       if (st->ln_mr) shai::launch_row_moments(g.C, g.M, g.N, g.ldc, st->ln_eps, st->ln_mr, stream());
@@ -496,16 +550,19 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
     launch_final(g, like, Choice{forced, sp}, st);
     return;
   }
-  const std::string key = gemm_key(g);
+  // with the row norm behind it a product has a choice of its own: splitting K costs no launch then
+  const shai::FoldNormArgs* norm = st ? st->norm : nullptr;
+  const char* suffix = norm ? "|norm" : "";
+  const std::string key = gemm_key(g) + suffix;
   Choice c{-1, 1};
-  if (!lookup_choice(g, key, &c)) c = Choice{-1, 1};
+  if (!lookup_choice(g, key, &c, suffix)) c = Choice{-1, 1};
   if (c.cfg < 0) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hipStreamIsCapturing(stream(), &cs);
     if (cs == hipStreamCaptureStatusNone && autotune_enabled()) {
-      c = tune(g, like);
-      store_choice(g, key, c);
-    } else {
+      c = tune(g, like, false, norm);
+      store_choice(g, key, c, suffix);
+    } else if (norm == nullptr || !lookup_choice(g, gemm_key(g), &c)) {
       if (shai::skinny_supported(g)) {
         c = Choice{kSkinnyCfg, shai::skinny_kgroups(g)};
       } else {
@@ -851,6 +908,68 @@ void attach_norm_io(shai::GemmArgs& g, const optional<Tensor>& ln_mr, const opti
 }
 
 // a: [M, K] or [B, M, K]; w: [N, K] or [B, N, K]; c: [M, N'] or [B, M, N'] (N' = N or N/2 for glu)
+// y = a w^T + bias + residual and out = RMS norm or LayerNorm of y's rows.  force_cfg, for tests: 3000 + 100 * parts + tile config,
+// 1000 + parts for the skinny kernel.
+void gemm_norm(const Tensor& a, const Tensor& w, const Tensor& y, const optional<Tensor>& bias, const optional<Tensor>& residual,
+               const optional<Tensor>& gamma, const optional<Tensor>& beta, const Tensor& out, double eps, bool rms, int64_t force_cfg) {
+  check_bf16(a, "a");
+  check_bf16(w, "w");
+  check_bf16(y, "y");
+  check_bf16(out, "out");
+  SHAI_CHECK(a.dim() == 2 && w.dim() == 2 && y.dim() == 2 && a.stride(1) == 1 && w.stride(1) == 1, "gemm_norm: rows");
+  shai::GemmArgs g{};
+  g.A = cptr(a);
+  g.W = cptr(w);
+  g.C = mptr(y);
+  g.M = a.size(0);
+  g.K = a.size(1);
+  g.N = w.size(0);
+  SHAI_CHECK(w.size(1) == g.K && g.K % 8 == 0 && g.N % 8 == 0 && g.N <= 8192, "gemm_norm: K and N are multiples of 8, N at most 8192");
+  SHAI_CHECK(y.size(0) == g.M && y.size(1) == g.N && y.is_contiguous() && out.sizes() == y.sizes() && out.is_contiguous(), "gemm_norm: outputs");
+  SHAI_CHECK(!rms || !beta, "gemm_norm: an RMS norm has no shift");
+  g.lda = a.stride(0);
+  g.ldw = w.stride(0);
+  g.ldc = g.N;
+  g.batch = 1;
+  g.alpha = 1.f;
+  g.res_alpha = 1.f;
+  shai::FoldNormArgs n{};
+  auto row = [&](const optional<Tensor>& t, const char* name) -> const shai::bf16_t* {
+    if (!t) return nullptr;
+    check_bf16(*t, name);
+    SHAI_CHECK(t->numel() == g.N && t->is_contiguous(), "gemm_norm: ", name);
+    return cptr(*t);
+  };
+  n.bias = g.bias = row(bias, "bias");
+  n.gamma = row(gamma, "gamma");
+  n.beta = row(beta, "beta");
+  if (residual) {
+    check_bf16(*residual, "residual");
+    SHAI_CHECK(residual->dim() == 2 && residual->size(0) == g.M && residual->size(1) == g.N && residual->stride(1) == 1, "gemm_norm: residual");
+    n.residual = g.residual = cptr(*residual);
+    n.ldr = g.ldr = residual->stride(0);
+  }
+  n.y = g.C;
+  n.out = mptr(out);
+  n.rows = g.M;
+  n.D = g.N;
+  n.rms = rms;
+  n.res_alpha = 1.f;
+  n.eps = eps;
+  if (g.M == 0) return;
+  OutStats st;
+  st.norm = &n;
+  if (force_cfg >= 0) {
+    const bool tile = force_cfg >= 3000;
+    const Choice c{tile ? (int)(force_cfg - 3000) % 100 : kSkinnyCfg, tile ? (int)(force_cfg - 3000) / 100 : (int)force_cfg - kSkinnyCfg};
+    SHAI_CHECK(c.splits >= 1 && c.splits <= 64 && (tile ? c.cfg < shai::gemm2_num_cfgs() && shai::gemm2_cfg_supported(g, c.cfg)
+                                                        : shai::skinny_supported(g)), "gemm_norm: bad force_cfg");
+    launch_final(g, a, c, &st);
+    return;
+  }
+  run_gemm(g, a, (long)g.M * g.lda * 2, (long)g.N * g.ldw * 2, 0, &st);
+}
+
 void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tensor>& bias,
           const optional<Tensor>& bias2d, int64_t rows_per_bias2d, const optional<Tensor>& residual, double alpha,
           double res_alpha, int64_t act, bool glu, const optional<Tensor>& gate, int64_t rows_per_gate,
@@ -1803,6 +1922,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("col_partials(Tensor x, Tensor(a!) part) -> ()");
   m.def("row_moments(Tensor x, Tensor(a!) mr, float eps) -> ()");
   m.def("gemm(Tensor a, Tensor w, Tensor(a!) c, Tensor? bias, Tensor? bias2d, int rows_per_bias2d, Tensor? residual, float alpha, float res_alpha, int act, bool glu, Tensor? gate=None, int rows_per_gate=1, int force_cfg=-1, float rms_eps=-1.0, Tensor? w_scale=None, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, int w_slice_rows=0) -> ()");
+  m.def("gemm_norm(Tensor a, Tensor w, Tensor(a!) y, Tensor? bias, Tensor? residual, Tensor? gamma, Tensor? beta, Tensor(b!) out, float eps, bool rms, int force_cfg=-1) -> ()");
   m.def("dequant_fp8(Tensor w8, Tensor scale, Tensor(a!) out) -> ()");
   m.def("layernorm_mod(Tensor x, Tensor scale, Tensor shift, Tensor(a!) out, int rows_per_mod, float eps) -> ()");
   m.def("qk_norm_rope(Tensor(a!) x, Tensor? q_w, Tensor? k_w, Tensor? cos, Tensor? sin, int H, int D, int S, float eps) -> ()");
@@ -1848,6 +1968,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("groupnorm_apply", &groupnorm_apply);
   m.impl("groupnorm_one", &groupnorm_one);
   m.impl("gemm", &gemm);
+  m.impl("gemm_norm", &gemm_norm);
   m.impl("dequant_fp8", &dequant_fp8);
   m.impl("gemm_f8", &gemm_f8);
   m.impl("gemm_lnout", &gemm_lnout);

@@ -51,11 +51,18 @@ class FusedSelfAttention(nn.Module):
         v = qkv[..., (H + Hk) * hd:].view(B, T, Hk, hd)
         return q, k, v
 
-    def forward(self, x, residual=None, causal: bool = False, kv_lens=None, bias=None, scale=None):
+    def _attend(self, x, causal=False, kv_lens=None, bias=None, scale=None):
         B, T, _ = x.shape
         q, k, v = self.split(self.qkv(x))
         o = ops.attention(q, k, v, scale=scale, causal=causal, kv_lens=kv_lens, bias=bias)
-        return self.out(o.view(B, T, self.heads * self.head_dim), residual=residual)
+        return o.view(B, T, self.heads * self.head_dim)
+
+    def forward(self, x, residual=None, causal: bool = False, kv_lens=None, bias=None, scale=None):
+        return self.out(self._attend(x, causal, kv_lens, bias, scale), residual=residual)
+
+    def forward_norm(self, x, residual, norm, causal: bool = False):
+        """(y, norm(y)) of y = self(x) + residual."""
+        return self.out.forward_norm(self._attend(x, causal), residual, norm)
 
 
 class CrossAttention(nn.Module):
@@ -75,12 +82,12 @@ class CrossAttention(nn.Module):
     def context_kv(self, ctx: torch.Tensor) -> torch.Tensor:
         return self.kv(ctx)
 
-    def forward(self, x, ctx_kv: torch.Tensor, residual=None, kv_lens=None):
+    def forward_norm(self, x, ctx_kv: torch.Tensor, residual, norm):
+        """(y, norm(y)) of y = attention of x to the context + residual."""
         B, T, _ = x.shape
         S = ctx_kv.shape[1]
         H, hd = self.heads, self.head_dim
         q = self.q(x).view(B, T, H, hd)
         k = ctx_kv[..., : H * hd].view(ctx_kv.shape[0], S, H, hd)
         v = ctx_kv[..., H * hd:].view(ctx_kv.shape[0], S, H, hd)
-        o = ops.attention(q, k, v, kv_lens=kv_lens)
-        return self.out(o.view(B, T, H * hd), residual=residual)
+        return self.out.forward_norm(ops.attention(q, k, v).view(B, T, H * hd), residual, norm)

@@ -44,6 +44,10 @@ class Linear(nn.Module):
         """(y, statistics of y for the next norm) -- see ``ops.linear_stats``."""
         return ops.linear_stats(x, self.weight, self.bias, residual=residual, stats=stats, eps=eps)
 
+    def forward_norm(self, x, residual, norm):
+        """(y, norm(y)) of y = self(x) + residual -- see ``ops.linear_norm``."""
+        return ops.linear_norm(x, self.weight, self.bias, residual, norm)
+
     def folded(self, ln: "LayerNorm"):
         """(w', bias', s) of this projection with LayerNorm ``ln`` folded in (``ops.fold_layernorm``); cached
         until the weights change."""

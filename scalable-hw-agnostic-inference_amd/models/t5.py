@@ -78,16 +78,17 @@ class T5Block(nn.Module):
         self.wo = RowParallelLinear(c.d_ff, c.d_model, bias=False)
         self.h = self.qkv.h_local
 
-    def forward(self, x, bias, lens):
+    def forward(self, x, n, bias, lens, next_norm):
+        """``n``: x normalised by ``ln_attn``.  Returns the block's output and that normalised by ``next_norm``."""
         B, S, _ = x.shape
         h, d = self.h, self.c.d_kv
-        qkv = self.qkv(self.ln_attn(x))
+        qkv = self.qkv(n)
         q = qkv[..., : h * d].view(B, S, h, d)
         k = qkv[..., h * d:2 * h * d].view(B, S, h, d)
         v = qkv[..., 2 * h * d:].view(B, S, h, d)
         a = ops.attention(q, k, v, scale=1.0, kv_lens=lens, bias=bias)
-        x = self.o(a.view(B, S, h * d), residual=x)
-        return self.wo(self.wi(self.ln_ff(x)), residual=x)
+        x, n = self.o.forward_norm(a.view(B, S, h * d), x, self.ln_ff)
+        return self.wo.forward_norm(self.wi(n), x, next_norm)
 
 
 class T5EncoderModel(nn.Module):
@@ -126,9 +127,11 @@ class T5EncoderModel(nn.Module):
                     else torch.full((B,), S, dtype=torch.int32, device=input_ids.device))
         x = self.shared(input_ids)
         bias = self.position_bias(S, input_ids.device)
-        for blk in self.blocks:
-            x = blk(x, bias, lens)
-        return self.final_layer_norm(x)
+        norms = [blk.ln_attn for blk in self.blocks] + [self.final_layer_norm]
+        n = norms[0](x)
+        for blk, following in zip(self.blocks, norms[1:]):
+            x, n = blk(x, n, bias, lens, following)
+        return n
 
     def convert_hf_state_dict(self, sd: dict) -> dict:
         out = {}

@@ -167,9 +167,9 @@ class BasicTransformerBlock(nn.Module):
         self.ff = FeedForward(dim)
 
     def forward(self, x, ctx_kv):
-        x = self.attn1(self.norm1(x), residual=x)
-        x = self.attn2(self.norm2(x), ctx_kv, residual=x)
-        return self.ff(self.norm3(x), residual=x)
+        x, n = self.attn1.forward_norm(self.norm1(x), x, self.norm2)
+        x, n = self.attn2.forward_norm(n, ctx_kv, x, self.norm3)
+        return self.ff(n, residual=x)
 
     def forward_folded(self, x, ctx_kv, mr, next_eps=None, defer_down: bool = False):
         """forward with every LayerNorm folded into the projection that consumes it: ``mr`` = (mean, rstd) [rows, 2]

@@ -75,9 +75,10 @@ class ViTLayer(nn.Module):
         self.output = Linear(c.intermediate_size, c.hidden_size)
         self.act = c.hidden_act
 
-    def forward(self, x):
-        x = self.attention(self.layernorm_before(x), residual=x)
-        return self.output(self.intermediate(self.layernorm_after(x), act=self.act), residual=x)
+    def forward(self, x, n, next_norm):
+        """``n``: x normalised by ``layernorm_before``.  Returns the layer's output and that normalised by ``next_norm``."""
+        x, n = self.attention.forward_norm(n, x, self.layernorm_after)
+        return self.output.forward_norm(self.intermediate(n, act=self.act), x, next_norm)
 
     def forward_folded(self, x, mr, next_eps=None):
         """forward with both LayerNorms folded into the QKV / fc1 GEMMs (``ops.fold_layernorm``): ``mr`` = (mean,
@@ -95,11 +96,11 @@ class ViTLayer(nn.Module):
             return self.output(h, residual=x), None
         return self.output.forward_stats(h, residual=x, stats="ln", eps=next_eps)
 
-    def forward_cls(self, x, mr=None, keep: int = 1, tail: bool = False):
+    def forward_cls(self, x, mr=None, keep: int = 1, tail: bool = False, n=None):
         """The last layer when only some tokens leave the encoder: the first ``keep`` (token 0, CLS: image
         classification) or, with ``tail``, the last ``keep`` (YOLOS's detection tokens).  K / V of every token, the
         rest -- attention queries, out-projection, MLP -- for the kept tokens only (M = B keep instead of B T).
-        ``mr``: x's LayerNorm moments for the folded QKV (None: the plain norm).  Returns [B, keep, d]."""
+        ``mr``: x's LayerNorm moments for the folded QKV, or ``n``: x normalised.  Returns [B, keep, d]."""
         B, T, C = x.shape
         sel = slice(T - keep, T) if tail else slice(0, keep)
         a = self.attention
@@ -107,7 +108,7 @@ class ViTLayer(nn.Module):
             w, b, s = a.qkv.folded(self.layernorm_before)
             qkv = ops.linear(x, w, b, row_affine=(mr, s))
         else:
-            qkv = a.qkv(self.layernorm_before(x))
+            qkv = a.qkv(n)
         q, k, v = a.split(qkv)
         o = ops.attention(q[:, sel], k, v).reshape(B, keep, a.heads * a.head_dim)
         x0 = a.out(o, residual=x[:, sel].contiguous())
@@ -196,11 +197,13 @@ class ViTEncoderModel(nn.Module):
                 nxt = layers[i + 1].layernorm_before.eps if i + 1 < len(layers) else None
                 x, mr = layer.forward_folded(x, mr, nxt)
             return self.layernorm(x)
-        for i, layer in enumerate(self.layers):
-            if (cls_only or det_only) and i + 1 == len(self.layers):
-                return self.layernorm(layer.forward_cls(x, None, *self._kept(cls_only)))
-            x = layer(x)
-        return self.layernorm(x)
+        norms = [layer.layernorm_before for layer in layers] + [self.layernorm]
+        n = norms[0](x)
+        for i, layer in enumerate(layers):
+            if (cls_only or det_only) and i + 1 == len(layers):
+                return self.layernorm(layer.forward_cls(x, None, *self._kept(cls_only), n=n))
+            x, n = layer(x, n, norms[i + 1])
+        return n
 
 
 def preprocess(images_u8: torch.Tensor, size: Tuple[int, int], mean, std, device) -> torch.Tensor:

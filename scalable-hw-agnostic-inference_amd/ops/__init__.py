@@ -294,6 +294,28 @@ def stats_supported(rows: int, cols: int, kind: str, hw: Optional[int] = None) -
     return True
 
 
+# outputs up to which a product and the row norm behind it are one call of the kernels (linear_norm): from there on no K is split
+# (us, product and norm apart -> one call: 512 x 1280 x 5120 25.2 -> 21.3, 128 x 1024 x 1024 9.5 -> 8.4; 512 x 1280 x 1280 and 1232 x 640 x 1024
+# split nothing and take the same time)
+LINEAR_NORM_MAX = 1 << 20
+
+
+def linear_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], residual: torch.Tensor, norm):
+    """(y, norm(y)) with y = x @ w^T + bias + residual, ``norm`` a module with ``weight``, ``bias`` (None: RMS norm) and ``eps``.
+    On the GPU a small product whose K is split leaves its fold to the norm's launch."""
+    M, N = x.numel() // x.shape[-1], w.shape[0]
+    gain, shift, rms = norm.weight, getattr(norm, "bias", None), getattr(norm, "w_offset", None) is not None
+    rows = residual.is_contiguous() and residual.shape[-1] == N
+    if not (_gpu(x) and rows and 0 < M * N <= LINEAR_NORM_MAX and N % 8 == 0 and N <= 2048 and w.dtype == torch.bfloat16
+            and gain is not None and not getattr(norm, "w_offset", 0.0)):
+        y = linear(x, w, bias, residual=residual)
+        return y, norm(y)
+    x2 = x.reshape(M, -1) if (x.dim() == 2 or x.is_contiguous()) else x.contiguous().reshape(M, -1)
+    y, out = (torch.empty(M, N, dtype=x.dtype, device=x.device) for _ in range(2))
+    _K().gemm_norm(x2, w, y, bias, residual.reshape(M, N), gain, shift, out, float(norm.eps), rms)
+    return y.view(*x.shape[:-1], N), out.view(*x.shape[:-1], N)
+
+
 def fold_profitable(rows: int, cols: int) -> bool:
     """A LayerNorm folded into a GEMM pins that GEMM to the v4 kernel (256-row tiles, unsplit): worth it only when
     the problem has about a wave of 256 x 320 tiles for the 256 CUs -- otherwise the standalone norm pass plus the

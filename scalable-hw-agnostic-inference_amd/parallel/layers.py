@@ -120,6 +120,13 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
             y = ops.bias_act(y, self.bias, residual)
         return y
 
+    def forward_norm(self, x, residual, norm):
+        """(y, norm(y)) of y = self(x) + residual -- see ``ops.linear_norm``."""
+        if self.tp_size == 1 and self.w_scale is None:
+            return ops.linear_norm(x, self.weight, self.bias, residual, norm)
+        y = self(x, residual=residual)
+        return y, norm(y)
+
 
 class QKVParallelLinear(_ShardLoadMixin, nn.Module):
     """Fused [q; k; v] projection; rows of the full weight ordered q (H*hd), k (Hk*hd), v (Hk*hd)."""

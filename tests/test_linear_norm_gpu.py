@@ -1,0 +1,80 @@
+"""A product, its residual and the row norm behind it (ops.linear_norm) against the same in fp32, and the split forms' y against the
+separate fold's, bit for bit.
+
+Tolerance: y is rounded to bf16 once (2.3e-3 rms); its norm is taken of the rounded values and rounded again: 2^0.5 of that, 5e-3 with
+the statistics' share."""
+import pytest
+import torch
+
+from shai_amd import ops
+from shai_amd.models.layers import LayerNorm, RMSNorm
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    a, b = a.float().cpu(), b.float().cpu()
+    return ((a - b).norm() / b.norm()).item()
+
+
+def _norm(kind, n, dev):
+    m = (LayerNorm if kind == "layer" else RMSNorm)(n, 1e-6).to(dev)
+    m.weight.data.normal_(1.0, 0.2)
+    if kind == "layer":
+        m.bias.data.normal_(0.0, 0.2)
+    return m
+
+
+def _problem(M, N, K, dev):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    make = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    return make(M, K).bfloat16(), (make(N, K) / K ** 0.5).bfloat16(), make(N).bfloat16(), make(M, N).bfloat16()
+
+
+def _want(y, norm):
+    y = y.float().cpu()
+    if isinstance(norm, RMSNorm):
+        return y * torch.rsqrt((y * y).mean(-1, keepdim=True) + norm.eps) * norm.weight.float().cpu()
+    return torch.nn.functional.layer_norm(y, y.shape[-1:], norm.weight.float().cpu(), norm.bias.float().cpu(), norm.eps)
+
+
+# one row, spare lanes in the last chunk, every number of chunks, more parts than are in flight, more than there are K-tiles
+@pytest.mark.parametrize("M,N,K", [(1, 8, 512), (3, 264, 512), (32, 1024, 2816), (33, 520, 520), (50, 1280, 640), (197, 768, 3072), (20, 2048, 512)])
+@pytest.mark.parametrize("kind", ["layer", "rms"])
+@pytest.mark.parametrize("force", [1001, 1003, 1008, 3116, 3216, 3516, 3319])
+def test_split_forms(cuda, M, N, K, kind, force):
+    if force < 3000 and M > 64:
+        pytest.skip("the skinny kernel takes up to 64 rows")
+    norm = _norm(kind, N, cuda)
+    a, w, b, r = _problem(M, N, K, cuda)
+    y, h = (torch.full((M + 1, N), 7.0, device=cuda, dtype=torch.bfloat16) for _ in range(2))
+    ops._K().gemm_norm(a, w, y[:M], b, r, norm.weight, getattr(norm, "bias", None), h[:M], norm.eps, kind == "rms", force)
+    assert _rel(y[:M], a.float() @ w.float().t() + b.float() + r.float()) < 4e-3
+    assert _rel(h[:M], _want(y[:M], norm)) < 5e-3
+    assert bool((y[M] == 7).all()) and bool((h[M] == 7).all())
+    if force >= 3000:
+        apart = torch.empty_like(r)
+        ops.gemm_into(a, w, apart, b, residual=r, force_cfg=force)
+        assert torch.equal(apart, y[:M])
+
+
+# the rule: both sides of the largest output, a residual in place of the output's memory, widths and strides that go the separate way
+@pytest.mark.parametrize("shape,N,K", [((2, 77), 1024, 1024), ((1, 1024), 1024, 256), ((1, 1025), 1024, 256), ((5,), 2056, 256)])
+@pytest.mark.parametrize("kind", ["layer", "rms"])
+def test_rule(cuda, shape, N, K, kind):
+    norm = _norm(kind, N, cuda)
+    a, w, b, r = _problem(torch.Size(shape).numel(), N, K, cuda)
+    y, h = ops.linear_norm(a.view(*shape, K), w, None, r.view(*shape, N), norm)
+    assert y.shape == h.shape == (*shape, N)
+    want = (a.float() @ w.float().t() + r.float()).view(*shape, N)
+    assert _rel(y, want) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
+
+
+def test_refusals(cuda):
+    a, w, b, r = _problem(16, 64, 64, cuda)
+    y, h = torch.empty_like(r), torch.empty_like(r)
+    for bad in (dict(w=w[:60]), dict(residual=r[:8]), dict(gamma=b[:8]), dict(y=torch.empty(16, 128, device=cuda, dtype=torch.bfloat16)[:, :64]),
+                dict(rms=True), dict(force=1065)):
+        args = dict(w=w, y=y, residual=r, gamma=b, rms=False, force=-1, **{}) | bad
+        with pytest.raises(RuntimeError, match="gemm_norm"):
+            ops._K().gemm_norm(a, args["w"], args["y"], b, args["residual"], args["gamma"], b, h, 1e-5, args["rms"], args["force"])
