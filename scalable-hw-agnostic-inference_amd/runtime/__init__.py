@@ -42,6 +42,8 @@ def lib():
         L.shai_build_decode.argtypes = [_I, _IP, _IP, _IP, _I, _IP, _IP, _IP, _IP]
         L.shai_build_prefill.argtypes = [_I, _I, _IP, _IP, _IP, _IP, _I, _IP, _IP, _IP, _IP, _IP, _IP]
         L.shai_build_prefill_packed.argtypes = [_I, _IP, _IP, _IP, _IP, _I, _IP, _IP, _IP, _IP, _IP, _IP, _IP]
+        L.shai_hash_rows.argtypes = [ctypes.c_char_p, _I64P, _I, _I, _I, _I, _I, _I, _I, _I64P, _I64P]
+        L.shai_hash_rows.restype = _I
         _lib = L
     return _lib
 
@@ -123,6 +125,21 @@ class SlotPool:
 
     def release(self, slot: int) -> None:
         self._free.append(slot)
+
+
+def hash_rows(texts: Sequence[str], first: int, span: int, bos: int, eos: int, pad: int, width: int, trim: bool):
+    """(ids, mask) int64 [rows, width] of ASCII texts (``shai_hash_rows``); ``trim``: only as wide as the longest row.  None where a
+    text has other characters."""
+    raw = "".join(texts)
+    if not raw.isascii():
+        return None
+    ends = np.cumsum(np.fromiter(map(len, texts), np.int64, len(texts)))
+    if trim:
+        width = min(width, max(map(len, texts)) + 2)
+    ids, mask = np.empty((len(texts), width), np.int64), np.empty((len(texts), width), np.int64)
+    at = lambda a: a.ctypes.data_as(_I64P)  # noqa: E731
+    n = lib().shai_hash_rows(raw.encode(), at(ends), len(texts), first, span, bos, eos, pad, width, at(ids), at(mask))
+    return (np.ascontiguousarray(ids[:, :n]), np.ascontiguousarray(mask[:, :n])) if trim else (ids, mask)
 
 
 def sched_admit(prompt_tokens: Sequence[int], free_blocks: int, running: int, max_seqs: int, token_budget: int,

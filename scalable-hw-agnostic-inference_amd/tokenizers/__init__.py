@@ -16,6 +16,8 @@ from typing import List, Optional, Sequence
 
 import torch
 
+from .. import native
+
 _WORDS = ("the a of and to in is it that on for with as was at by an be this from or are his her they we you "
           "image photo light warrior chief astronaut horse mars city river cat dog portrait detailed sky night "
           "blue red green gold old young sunset forest mountain ocean robot castle dragon flower garden").split()
@@ -61,11 +63,23 @@ class HashTokenizer:
                 ids = ids + [self.eos_token_id]
         return ids
 
+    def _native(self, texts: Sequence[str], width: int, trim: bool):
+        """(ids, mask) of the native runtime for what it takes; None: the words are found here."""
+        if not native.runtime_available() or not all(isinstance(t, str) for t in texts):
+            return None
+        from ..runtime import hash_rows
+        bos, eos = (-1 if i is None else i for i in (self.bos_token_id, self.eos_token_id))
+        return hash_rows(texts, self.n_special, max(1, self._hi - self.n_special), bos, eos, self.pad_token_id, width, trim)
+
     def __call__(self, texts: Sequence[str] | str, max_length: Optional[int] = None, padding: str = "max_length",
                  truncation: bool = True, return_tensors: str = "pt"):
         if isinstance(texts, str):
             texts = [texts]
         L = max_length or self.model_max_length
+        if truncation and L > 0 and len(texts) and self._special_re is None:
+            out = self._native(texts, L, padding != "max_length")
+            if out is not None:
+                return {"input_ids": torch.from_numpy(out[0]), "attention_mask": torch.from_numpy(out[1])}
         rows = []
         for t in texts:
             ids = self.encode(t)
