@@ -335,6 +335,10 @@ bool gemm2_cfg_supported(const GemmArgs& a, int cfg) {
     if (cfg >= kV4Cfg && cfg < kV4Cfg + 4) return gemm4_supported(a);
     if (a.conv || a.in_scale != nullptr) return false;
   }
+  // 192 x 128 and 128 x 128 with two groups of waves along K: up to 8192 rows.  They fill one round of the chip where other tiles
+  // need more or a split (4096 x 1280 x 5120: 57.8 us, two workgroups of 192 x 128 to a CU 74.4); with more rows rounds are full anyway
+  // (16384 x 640 x 2560 66.0 and 64.0, x 640 29.7 and 25.6), and the sums of long prompts stay in one order whatever their rows.
+  if ((cfg == kDeepCfg + 3 || cfg == kDeepCfg + 4) && a.M > 8192) return false;
   if (cfg >= kDeepCfg) return cfg < kDeepCfg + kDeepCfgs && gemm_deep_supported(a);
   if (cfg == kWsCfg) return gemm_ws_supported(a);
   if (cfg == kW4Cfg) return gemm_w4_supported(a);

@@ -1,5 +1,6 @@
 // Token ids of texts without a checkpoint's tokenizer (host C++, C ABI): a word's or mark's id is its CRC-32's place among the
-// ordinary ids.  A batch of 32 captions of 130 words took the interpreter 0.95 ms, in front of 4.2 ms of an encoder's kernels; here 0.1.
+// ordinary ids.  32 captions of up to 132 words, ids and mask, took the interpreter 2.4 ms in a container of 8 CPUs, in front of
+// 4.1 ms of an encoder's kernels; here 0.06.  One text of 32: 37 us and 19.
 #include <algorithm>
 #include <array>
 #include <cstdint>

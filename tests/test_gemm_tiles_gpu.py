@@ -80,6 +80,16 @@ def test_rows_of_images(cuda, cfg):
     assert _close(out, ACTS["silu"](y) + 2.0 * r.float())
 
 
+@pytest.mark.parametrize("cfg", [19, 20])
+def test_wave_groups_up_to_8192_rows(cuda, cfg):
+    a, w, b, r = _problem(8193, 64, 64, cuda)
+    out = torch.empty_like(r)
+    with pytest.raises(RuntimeError, match="bad force_cfg"):
+        ops.gemm_into(a, w, out, b, force_cfg=cfg)
+    ops.gemm_into(a[:8192], w, out[:8192], b, force_cfg=cfg)
+    assert _close(out[:8192], a[:8192].float() @ w.float().t() + b.float())
+
+
 @pytest.mark.parametrize("splits", [2, 5])
 @pytest.mark.parametrize("cfg", GROUPS)
 def test_split_k(cuda, splits, cfg):
