@@ -73,8 +73,7 @@ class HashTokenizer:
 
     def __call__(self, texts: Sequence[str] | str, max_length: Optional[int] = None, padding: str = "max_length",
                  truncation: bool = True, return_tensors: str = "pt"):
-        if isinstance(texts, str):
-            texts = [texts]
+        texts = [texts] if isinstance(texts, str) else list(texts)
         L = max_length or self.model_max_length
         if truncation and L > 0 and len(texts) and self._special_re is None:
             out = self._native(texts, L, padding != "max_length")

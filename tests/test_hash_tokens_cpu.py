@@ -31,6 +31,13 @@ def test_rows(bos, eos, length, padding, monkeypatch):
             assert g[name].dtype == want[name].dtype and g[name].shape == want[name].shape and bool((g[name] == want[name]).all()), (b, name)
 
 
+# whatever is iterated over once, as before
+def test_any_iterable():
+    tok = HashTokenizer(1000, None, 1, 0, 16)
+    want = tok(["a b", "c"])["input_ids"]
+    assert bool((tok(t for t in ("a b", "c"))["input_ids"] == want).all()) and bool((tok(("a b", "c"))["input_ids"] == want).all())
+
+
 # a word whose id is the first token's stays the row's beginning; special strings and rows that may not be cut go the Python way
 def test_first_token_and_specials():
     probe = HashTokenizer(1000, None, None, 0, 16)
