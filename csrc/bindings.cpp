@@ -1722,7 +1722,8 @@ int64_t gemm_tuning_import(const std::vector<std::string>& entries) {
   return n;
 }
 
-void patches_u8(const Tensor& x, const Tensor& out, int64_t P, at::ArrayRef<double> mean, at::ArrayRef<double> inv_std) {
+void patches_u8(const Tensor& x, const Tensor& out, int64_t P, at::ArrayRef<double> mean, at::ArrayRef<double> inv_std,
+                const optional<Tensor>& w, const optional<Tensor>& w_out) {
   SHAI_CHECK(x.is_cuda() && x.scalar_type() == at::kByte && x.is_contiguous() && x.dim() == 4 && x.size(3) == 3, "patches_u8: uint8 [B, H, W, 3]");
   check_bf16(out, "out");
   SHAI_CHECK(P > 0 && P % 8 == 0 && x.size(1) % P == 0 && x.size(2) % P == 0 && mean.size() == 3 && inv_std.size() == 3,
@@ -1737,6 +1738,16 @@ void patches_u8(const Tensor& x, const Tensor& out, int64_t P, at::ArrayRef<doub
   a.W = x.size(2);
   a.P = P;
   for (int c = 0; c < 3; ++c) a.mean[c] = mean[c], a.inv_std[c] = inv_std[c];
+  if (w) {
+    SHAI_CHECK(w_out.has_value(), "patches_u8: w needs w_out");
+    check_bf16(*w, "w");
+    check_bf16(*w_out, "w_out");
+    SHAI_CHECK(w->is_contiguous() && w_out->is_contiguous() && w->numel() % (8 * P * P) == 0 && w_out->numel() == w->numel() / 8 * 3,
+               "patches_u8: w [D, P P 8], w_out [D, P P 3]");
+    a.w = cptr(*w);
+    a.w_out = mptr(*w_out);
+    a.w_pixels = w->numel() / 8;
+  }
   shai::launch_patches_u8(a, stream());
 }
 
@@ -1941,7 +1952,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("sched_step(Tensor model_out, Tensor(a!) latents, bool cfg, float guidance, int pred_type, float a_t, float a_prev, float dt) -> ()");
   m.def("sched_step_rows(Tensor model_out, Tensor(a!) latents, bool cfg, float guidance, int pred_type, Tensor rows_params) -> ()");
   m.def("softmax_(Tensor(a!) x, float scale) -> ()");
-  m.def("patches_u8(Tensor x, Tensor(a!) out, int P, float[] mean, float[] inv_std) -> ()");
+  m.def("patches_u8(Tensor x, Tensor(a!) out, int P, float[] mean, float[] inv_std, Tensor? w=None, Tensor(b!)? w_out=None) -> ()");
   m.def("tokens(Tensor patches, Tensor cls, Tensor? det, Tensor pos, Tensor(a!) out, Tensor(b!)? mr, float eps) -> ()");
   m.def("mean_tokens(Tensor x, Tensor(a!) out) -> ()");
   m.def("embedding(Tensor ids, Tensor table, Tensor(a!) out) -> ()");

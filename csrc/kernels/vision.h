@@ -7,12 +7,17 @@ namespace shai {
 typedef uint16_t bf16_t;
 
 // out [B (H / P) (W / P), P P 3] bf16: the pixels of every patch in the order (row, column, channel), normalised
-// (u8 / 255 - mean) inv_std.  x [B, H, W, 3]; P % 8 == 0, H and W multiples of P, x 8-byte aligned.
+// (u8 / 255 - mean) inv_std.  x [B, H, W, 3]; P % 8 == 0, H and W multiples of P, x 8-byte aligned.  With w, the weight of the
+// convolution that they stand for, [w_pixels, 8] with channels of which three count, its [w_pixels, 3] goes to w_out: the product of
+// the two needs no padded channels.  w_pixels % 4 == 0, both 16-byte aligned.
 struct PatchArgs {
   const uint8_t* x;
   bf16_t* out;
   int B, H, W, P;
   float mean[3], inv_std[3];
+  const bf16_t* w;
+  bf16_t* w_out;
+  long w_pixels;
 };
 void launch_patches_u8(const PatchArgs& a, hipStream_t s);
 

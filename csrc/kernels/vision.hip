@@ -8,8 +8,21 @@
 
 namespace shai {
 
-// A thread takes 8 adjacent bytes of a patch's row: 16 bytes out.
-__global__ void __launch_bounds__(256) patches_u8_kernel(const PatchArgs a, long total) {
+// A thread takes 8 adjacent bytes of a patch's row: 16 bytes out.  Workgroups from image_blocks on take the weight, 4 pixels a thread: on
+// every call, so that the product reads the parameter as it is then, also in a replay of a graph.
+__global__ void __launch_bounds__(256) patches_u8_kernel(const PatchArgs a, long total, unsigned image_blocks) {
+  if (blockIdx.x >= image_blocks) {
+    const long j = (blockIdx.x - image_blocks) * 256L + threadIdx.x;
+    if (j * 4 >= a.w_pixels) return;
+    uint2_ v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = *reinterpret_cast<const uint2_*>(a.w + (j * 4 + e) * 8);
+    uint2_* out = reinterpret_cast<uint2_*>(a.w_out + j * 12);
+    out[0] = uint2_{v[0][0], (v[0][1] & 0xffffu) | v[1][0] << 16};
+    out[1] = uint2_{v[1][0] >> 16 | v[1][1] << 16, v[2][0]};
+    out[2] = uint2_{(v[2][1] & 0xffffu) | v[3][0] << 16, v[3][0] >> 16 | v[3][1] << 16};
+    return;
+  }
   const long i = blockIdx.x * 256L + threadIdx.x;
   if (i >= total) return;
   const int per_row = a.P * 3 / 8;                     // 8-byte pieces of a patch's row
@@ -36,7 +49,8 @@ __global__ void __launch_bounds__(256) patches_u8_kernel(const PatchArgs a, long
 
 void launch_patches_u8(const PatchArgs& a, hipStream_t s) {
   const long total = (long)a.B * a.H * a.W * 3 / 8;
-  if (total > 0) patches_u8_kernel<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(a, total);
+  const unsigned images = (unsigned)((total + 255) / 256), weight = a.w ? (unsigned)((a.w_pixels / 4 + 255) / 256) : 0;
+  if (images + weight > 0) patches_u8_kernel<<<images + weight, 256, 0, s>>>(a, total, images);
 }
 
 // One wave a row, held in registers; mean and variance in two passes over them.

@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .attention import FusedSelfAttention, merge_linear_keys
-from .layers import Conv2d, LayerNorm, Linear, _wkey
+from .layers import Conv2d, LayerNorm, Linear
 
 
 # LayerNorms folded into the GEMMs that consume them, moments handed over by the producing GEMM (unet2d.py);
@@ -150,30 +150,14 @@ class ViTEncoderModel(nn.Module):
         patch = patch.flatten(2).transpose(1, 2).to(pe.dtype)
         return torch.cat([cls_pe, patch, det_pe], dim=1)
 
-    def _patch_weight(self):
-        """The patch convolution's weight without the channels that pad 3 to 8, [d, P P 3]; rebuilt when the weight changes.  None
-        when first needed inside a graph capture."""
-        key = _wkey(self.patch.weight)
-        cached = getattr(self, "_w_patch", None)
-        if cached is None or cached[0] != key:
-            if torch.cuda.is_current_stream_capturing():
-                return None
-            w = self.patch.weight.data
-            cached = (key, w.view(w.shape[0], -1, self.patch.cin_p)[..., :3].reshape(w.shape[0], -1).contiguous())
-            self._w_patch = cached
-        return cached[1]
-
     def forward_u8(self, images: torch.Tensor, mean, std, cls_only: bool = False):
         """``forward`` of uint8 images [B, H, W, 3] at the model's resolution, normalised with the channels' ``mean`` and ``std``
         on the way into the patches; None where their sizes or address do not fit that kernel."""
         P = self.cfg.patch_size
         if not ops.patches_u8_ok(images, P):
             return None
-        w = self._patch_weight()
-        if w is None:
-            return None
         B, H, W, _ = images.shape
-        x = ops.linear(ops.patches_u8(images, P, mean, std), w, self.patch.bias)
+        x = ops.linear(*ops.patches_u8(images, P, mean, std, self.patch.weight), self.patch.bias)
         return self._encode(x.view(B, H // P, W // P, -1), cls_only, False)
 
     def forward(self, pixels: torch.Tensor, cls_only: bool = False, det_only: bool = False) -> torch.Tensor:

@@ -828,17 +828,20 @@ def patches_u8_ok(images: torch.Tensor, patch: int) -> bool:
             and patch % 8 == 0 and images.shape[1] % patch == 0 and images.shape[2] % patch == 0 and images.data_ptr() % 8 == 0)
 
 
-def patches_u8(images: torch.Tensor, patch: int, mean, std) -> torch.Tensor:
+def patches_u8(images: torch.Tensor, patch: int, mean, std, weight: Optional[torch.Tensor] = None):
     """uint8 images [B, H, W, 3] -> [B (H / patch) (W / patch), patch patch 3] bf16: the patches' pixels in the order (row, column,
-    channel), normalised (u8 / 255 - mean) / std."""
+    channel), normalised (u8 / 255 - mean) / std.  With ``weight`` [D, patch patch 8], a patch convolution's packed one for channels
+    padded from 3 to 8: (patches, the weight without the padding [D, patch patch 3]), whose product is the convolution."""
     B, H, W, _ = images.shape
     if not _gpu(images):
         m, r = torch.tensor(mean, dtype=torch.float32), 1.0 / torch.tensor(std, dtype=torch.float32)
         x = ((images.float() * (1.0 / 255.0) - m) * r).to(torch.bfloat16)
-        return x.view(B, H // patch, patch, W // patch, patch, 3).transpose(2, 3).reshape(-1, patch * patch * 3)
+        x = x.view(B, H // patch, patch, W // patch, patch, 3).transpose(2, 3).reshape(-1, patch * patch * 3)
+        return x if weight is None else (x, weight.view(weight.shape[0], -1, 8)[..., :3].reshape(weight.shape[0], -1))
     out = torch.empty(B * (H // patch) * (W // patch), patch * patch * 3, dtype=torch.bfloat16, device=images.device)
-    _K().patches_u8(images, out, int(patch), [float(m) for m in mean], [1.0 / float(v) for v in std])
-    return out
+    w = torch.empty(weight.shape[0], patch * patch * 3, dtype=weight.dtype, device=images.device) if weight is not None else None
+    _K().patches_u8(images, out, int(patch), [float(m) for m in mean], [1.0 / float(v) for v in std], weight, w)
+    return out if weight is None else (out, w)
 
 
 def tokens(patches: torch.Tensor, cls: torch.Tensor, det: Optional[torch.Tensor], pos: torch.Tensor, eps: Optional[float] = None):

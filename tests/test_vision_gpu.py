@@ -21,6 +21,41 @@ def test_patches(cuda, B, H, W, P):
     assert (y != ops.patches_u8(x.cpu(), P, mean, std).cuda()).double().mean().item() < 1e-4   # the same steps in 32 bits
 
 
+# the weight without its padding, beside the images: workgroups that it ends in and whole ones
+@pytest.mark.parametrize("D,P", [(1, 8), (192, 16), (768, 16), (3, 24)])
+def test_patch_weight(cuda, D, P):
+    torch.manual_seed(D)
+    x = torch.randint(0, 256, (2, 2 * P, P, 3), device="cuda", dtype=torch.uint8)
+    w = torch.randn(D, P * P * 8, device="cuda").bfloat16()
+    y, w3 = ops.patches_u8(x, P, (0.5, 0.4, 0.3), (0.2, 0.3, 0.4), w)
+    assert torch.equal(y, ops.patches_u8(x, P, (0.5, 0.4, 0.3), (0.2, 0.3, 0.4)))
+    assert torch.equal(w3, w.view(D, P * P, 8)[..., :3].reshape(D, -1))
+    for bad in (w[:, :-8].contiguous(), w.float()):
+        with pytest.raises(RuntimeError):
+            ops.patches_u8(x, P, (0.5, 0.4, 0.3), (0.2, 0.3, 0.4), bad)
+
+
+# graphs follow weights that are loaded in place, in whatever way: those of batches captured before, and later ones
+@pytest.mark.parametrize("load", ["load_into", "data"])
+def test_classifier_follows_its_weights(cuda, load):
+    from shai_amd.engines.encoders import ImageClassifierEngine
+    from shai_amd.models.vit import ViTConfig
+    from shai_amd.weights import load_into
+    eng, new = (ImageClassifierEngine(ViTConfig.tiny(), device="cuda:0", seed=s, use_graphs=s == 1) for s in (1, 2))
+    g = torch.Generator().manual_seed(3)
+    x = {b: torch.randint(0, 256, (b, 64, 64, 3), generator=g, dtype=torch.uint8).cuda() for b in (1, 2, 3)}
+    old = {b: eng.logits_u8(x[b]).clone() for b in (1, 2)}
+    if load == "data":
+        for p, q in zip(eng.model.parameters(), new.model.parameters()):
+            p.data.copy_(q)
+    else:
+        load_into(eng.model, new.model.state_dict())
+    for b in (1, 3, 2, 1):
+        got = eng.logits_u8(x[b]).clone()
+        assert torch.equal(got, new.logits_u8(x[b]))
+        assert b not in old or not torch.equal(got, old[b])
+
+
 def test_patches_left_alone(cuda):
     x = torch.zeros(2, 32, 32, 3, device="cuda", dtype=torch.uint8)
     flat = torch.zeros(2 * 32 * 32 * 3 + 4, device="cuda", dtype=torch.uint8)[4:].view(2, 32, 32, 3)
