@@ -17,6 +17,7 @@ import numpy as np
 import torch
 
 from . import capture, new_graph
+from ..models.layers import FoldedWeights
 from ..tokenizers import load_tokenizer
 from ..weights import materialize
 
@@ -117,9 +118,10 @@ class ImageClassifierEngine:
             graph = new_graph(self.device)
             with capture(graph):
                 out = self._forward_u8(static)
-            g = self._graphs[B] = (graph, static, out)
-        graph, static, out = g
+            g = self._graphs[B] = (graph, static, out, FoldedWeights(self.model))
+        graph, static, out, folded = g
         static.copy_(x_u8)
+        folded.refresh()
         graph.replay()
         return out
 

@@ -203,3 +203,30 @@ def test_up2_phase_weights_match_upsample_conv():
     # bf16 packing: the fp32 sums round once
     wb = ref.pack_conv_weight(torch.randn(8, 8, 3, 3)).to(torch.bfloat16)
     assert ops.pack_up2_phase_weight(wb, 8).dtype == torch.bfloat16
+
+
+def test_folded_weights_are_remade_in_place():
+    """A graph that was captured with folded weights holds their addresses: after a load they are remade there, by the next eager call
+    or by ``FoldedWeights.refresh``, also where they were made in inference mode; a norm without a gain, whose fold is the weight
+    itself, is not written through."""
+    from shai_amd.models.layers import FoldedWeights, LayerNorm, Linear
+    torch.manual_seed(1)
+    lin, ln, bare = Linear(32, 16), LayerNorm(32), LayerNorm(32, affine=False)
+    lin.weight.data.normal_()
+    with torch.inference_mode():
+        kept = lin.folded(ln)
+    where, graph = [t.data_ptr() for t in kept], FoldedWeights(lin)
+    assert len(graph.pairs) == 1 and len(FoldedWeights(ln).pairs) == 0
+    for change in (lambda: lin.load_state_dict({"weight": torch.randn(16, 32), "bias": torch.randn(16)}),
+                   lambda: ln.load_state_dict({"weight": torch.randn(32), "bias": torch.randn(32)})):
+        for refresh in (graph.refresh, lambda: lin.folded(ln)):
+            change()
+            refresh()
+            want = ops.fold_layernorm(lin.weight, lin.bias, ln.weight, ln.bias)
+            assert [t.data_ptr() for t in lin.folded(ln)] == where
+            assert all(torch.equal(a, b) for a, b in zip(kept, want))
+    other = Linear(32, 16)
+    other.weight.data.normal_()
+    first = other.folded(bare)[0]
+    before, other.weight = first.clone(), torch.nn.Parameter(torch.randn(16, 32).bfloat16(), requires_grad=False)
+    assert torch.equal(other.folded(bare)[0], other.weight) and torch.equal(first, before)

@@ -35,12 +35,15 @@ def test_patch_weight(cuda, D, P):
             ops.patches_u8(x, P, (0.5, 0.4, 0.3), (0.2, 0.3, 0.4), bad)
 
 
-# graphs follow weights that are loaded in place, in whatever way: those of batches captured before, and later ones
-@pytest.mark.parametrize("load", ["load_into", "data"])
-def test_classifier_follows_its_weights(cuda, load):
+# graphs follow weights that are loaded in place, in whatever way where nothing is folded: those of batches captured before, and later
+# ones
+@pytest.mark.parametrize("load", ["load_into", "data", "folded"])
+def test_classifier_follows_its_weights(cuda, load, monkeypatch):
     from shai_amd.engines.encoders import ImageClassifierEngine
     from shai_amd.models.vit import ViTConfig
     from shai_amd.weights import load_into
+    if load == "folded":
+        monkeypatch.setattr(ops, "FOLD_MIN_TILES", 0)
     eng, new = (ImageClassifierEngine(ViTConfig.tiny(), device="cuda:0", seed=s, use_graphs=s == 1) for s in (1, 2))
     g = torch.Generator().manual_seed(3)
     x = {b: torch.randint(0, 256, (b, 64, 64, 3), generator=g, dtype=torch.uint8).cuda() for b in (1, 2, 3)}
