@@ -912,8 +912,8 @@ void attach_norm_io(shai::GemmArgs& g, const optional<Tensor>& ln_mr, const opti
 // 1000 + parts for the skinny kernel.
 void gemm_norm(const Tensor& a, const Tensor& w, const Tensor& y, const optional<Tensor>& bias, const optional<Tensor>& residual,
                const optional<Tensor>& gamma, const optional<Tensor>& beta, const Tensor& out, double eps, bool rms, int64_t force_cfg) {
-  check_bf16(a, "a");
-  check_bf16(w, "w");
+  check_rows(a, "a");   // the tiles read 16 bytes at a time
+  check_rows(w, "w");
   check_bf16(y, "y");
   check_bf16(out, "out");
   SHAI_CHECK(a.dim() == 2 && w.dim() == 2 && y.dim() == 2 && a.stride(1) == 1 && w.stride(1) == 1, "gemm_norm: rows");

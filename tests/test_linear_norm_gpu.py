@@ -78,3 +78,18 @@ def test_refusals(cuda):
         args = dict(w=w, y=y, residual=r, gamma=b, rms=False, force=-1, **{}) | bad
         with pytest.raises(RuntimeError, match="gemm_norm"):
             ops._K().gemm_norm(a, args["w"], args["y"], b, args["residual"], args["gamma"], b, h, 1e-5, args["rms"], args["force"])
+
+
+# what ops.linear refuses (rows that do not begin at 16 bytes) is refused here too, by the op and by the function; what it takes is taken
+def test_strides(cuda):
+    norm, (a, w, b, r) = _norm("layer", 64, cuda), _problem(16, 64, 512, cuda)
+    wide = lambda t, ld: torch.cat([t, t[:, :ld - t.shape[1]]], 1)[:, :t.shape[1]]  # noqa: E731
+    y, h = ops.linear_norm(a, w, b, r, norm)
+    for x, v in ((wide(a, 520), w), (a, wide(w, 520))):
+        y2, h2 = ops.linear_norm(x, v, b, r, norm)
+        assert torch.equal(y, y2) and torch.equal(h, h2)
+    for x, v in ((wide(a, 514), w), (a, wide(w, 514))):
+        for call in (lambda: ops.linear(x, v, b, residual=r), lambda: ops.linear_norm(x, v, b, r, norm),
+                     lambda: ops._K().gemm_norm(x, v, y, b, r, norm.weight, norm.bias, h, 1e-6, False, 3216)):
+            with pytest.raises(RuntimeError, match="stride not 16B aligned"):
+                call()
