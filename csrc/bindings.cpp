@@ -555,20 +555,21 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
   const char* suffix = norm ? "|norm" : "";
   const std::string key = gemm_key(g) + suffix;
   Choice c{-1, 1};
-  if (!lookup_choice(g, key, &c, suffix)) c = Choice{-1, 1};
-  if (c.cfg < 0) {
+  // One that has none yet takes the plain product's: a split's fold and the norm are one launch there too, and a request of new rows
+  // waits for no tuning (4.7 to 9 ms, the first of a process 30).
+  bool found = lookup_choice(g, key, &c, suffix);
+  if (!found && norm) found = lookup_choice(g, gemm_key(g), &c);
+  if (!found || c.cfg < 0) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hipStreamIsCapturing(stream(), &cs);
     if (cs == hipStreamCaptureStatusNone && autotune_enabled()) {
       c = tune(g, like, false, norm);
       store_choice(g, key, c, suffix);
-    } else if (norm == nullptr || !lookup_choice(g, gemm_key(g), &c)) {
-      if (shai::skinny_supported(g)) {
-        c = Choice{kSkinnyCfg, shai::skinny_kgroups(g)};
-      } else {
-        shai::gemm2_plan(g, &c.cfg, &c.splits);
-        if (!shai::gemm2_cfg_supported(g, c.cfg)) c = fallback_choice(g);
-      }
+    } else if (shai::skinny_supported(g)) {
+      c = Choice{kSkinnyCfg, shai::skinny_kgroups(g)};
+    } else {
+      shai::gemm2_plan(g, &c.cfg, &c.splits);
+      if (!shai::gemm2_cfg_supported(g, c.cfg)) c = fallback_choice(g);
     }
   }
   if (g.row_mr != nullptr) c.splits = 1;  // before the statistics' rule looks at the choice; launch_choice does the same

@@ -93,3 +93,17 @@ def test_strides(cuda):
                      lambda: ops._K().gemm_norm(x, v, y, b, r, norm.weight, norm.bias, h, 1e-6, False, 3216)):
             with pytest.raises(RuntimeError, match="stride not 16B aligned"):
                 call()
+
+
+# rows for which only the plain product's choice is known, by its bucket or exactly: that one, without a tuning; else one of its own
+@pytest.mark.parametrize("M,key,cfg", [(90, 96, "|mbucket=17,2"), (91, 96, "|mbucket=3,1"), (40, 40, "=1000,3"), (92, None, None)])
+def test_choice_of_the_plain_product(cuda, M, key, cfg):
+    N, K = (328, 520) if key else (336, 520)
+    name = lambda m: f"0:{m},{N},{K},b1,g0|0,0,0,0,0,0,0,0,0"  # noqa: E731
+    if key:
+        ops._K().gemm_tuning_import([name(key) + cfg])
+    norm, (a, w, b, r) = _norm("rms", N, cuda), _problem(M, N, K, cuda)
+    y, h = ops.linear_norm(a, w, b, r, norm)
+    assert _rel(y, a.float() @ w.float().t() + b.float() + r.float()) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
+    own = [e for e in ops._K().gemm_tuning_export() if e.startswith(name(M)) and "|norm" in e]
+    assert len(own) == (0 if key else 1)
