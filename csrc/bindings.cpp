@@ -28,6 +28,9 @@ namespace {
 
 hipStream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// A launch that was refused leaves its output as it was allocated: an error, not a result.
+void check_launch(hipError_t e, const char* kernel) { SHAI_CHECK(e == hipSuccess, kernel, " was not launched: ", hipGetErrorString(e)); }
+
 // Halo-tiled conv routing (conv_halo.hip): 0 off (default), 1 GroupNorm-fused convs, 2 also plain 3x3 convs;
 // SHAI_HALO_CONV sets it, the set_halo_conv op changes it at run time (A/B in one process).  g_halo_waves: 0 = the
 // kernel's default wave layout (SHAI_HALO_WAVES), 4 / 8 pin one.  Off by default: at the SD2.1 batch-32 shapes the
@@ -335,7 +338,7 @@ void launch_then_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, sha
   }
   n.parts = ws.data_ptr<float>();
   n.splits = splits;
-  shai::launch_fold_norm(n, stream());
+  check_launch(shai::launch_fold_norm(n, stream()), "fold_norm");
 }
 
 // Candidates are timed into a scratch output so that in-place epilogues (C aliasing
@@ -459,7 +462,7 @@ void launch_with_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, con
   if (!fold) {
     launch_choice(g, like, c);
     n.x = g.C;
-    shai::launch_gn_one(n, stream());
+    check_launch(shai::launch_gn_one(n, stream()), "gn_one");
     return;
   }
   Tensor ws = at::empty({(long)c.splits * g.M * g.N}, like.options().dtype(at::kFloat));
@@ -473,7 +476,7 @@ void launch_with_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, con
   n.residual = g.residual;
   n.res_alpha = g.res_alpha;
   n.raw = st.keep ? g.C : nullptr;
-  shai::launch_gn_one(n, stream());
+  check_launch(shai::launch_gn_one(n, stream()), "gn_one");
 }
 
 void launch_final(shai::GemmArgs g, const Tensor& like, const Choice& c, const OutStats* st) {
@@ -532,7 +535,7 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
     if (st && st->one) {
       shai::GnOneArgs n = *st->one;
       n.x = g.C;
-      shai::launch_gn_one(n, stream());
+      check_launch(shai::launch_gn_one(n, stream()), "gn_one");
     }
     if (st && st->norm) launch_norm(g, *st->norm);
     if (st && st->any()) {  // v1 writes no statistics
@@ -875,7 +878,7 @@ void groupnorm_one(const Tensor& x, const optional<Tensor>& x2, const optional<T
   n.x = cptr(x);
   n.x2 = src.x2;
   n.C1 = src.C1;
-  shai::launch_gn_one(n, stream());
+  check_launch(shai::launch_gn_one(n, stream()), "gn_one");
 }
 
 // ---------------------------------------------------------------- GEMM
@@ -1749,7 +1752,7 @@ void patches_u8(const Tensor& x, const Tensor& out, int64_t P, at::ArrayRef<doub
     a.w_out = mptr(*w_out);
     a.w_pixels = w->numel() / 8;
   }
-  shai::launch_patches_u8(a, stream());
+  check_launch(shai::launch_patches_u8(a, stream()), "patches_u8");
 }
 
 void tokens(const Tensor& patches, const Tensor& cls, const optional<Tensor>& det, const Tensor& pos, const Tensor& out,
@@ -1781,7 +1784,7 @@ void tokens(const Tensor& patches, const Tensor& cls, const optional<Tensor>& de
   a.pos = cptr(pos);
   a.out = mptr(out);
   a.eps = eps;
-  shai::launch_tokens(a, stream());
+  check_launch(shai::launch_tokens(a, stream()), "tokens");
 }
 
 void mean_tokens(const Tensor& x, const Tensor& out) {

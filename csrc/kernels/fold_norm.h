@@ -21,5 +21,5 @@ struct FoldNormArgs {
 };
 // D a multiple of 4 up to 2048, every address and ldr of 8 bytes
 bool fold_norm_supported(const FoldNormArgs& a);
-void launch_fold_norm(const FoldNormArgs& a, hipStream_t s);
+[[nodiscard]] hipError_t launch_fold_norm(const FoldNormArgs& a, hipStream_t s);
 }  // namespace shai

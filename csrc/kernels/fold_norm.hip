@@ -7,6 +7,7 @@
 // 21.3; where K was not split before, splitting it pays now: 197 x 768 x 768 8.6 -> 7.9, 32 x 768 x 768 10.0 -> 6.9.
 #include "fold_norm.h"
 #include "common.h"
+#include "launch.h"
 
 namespace shai {
 
@@ -102,18 +103,17 @@ bool fold_norm_supported(const FoldNormArgs& a) {
   return a.D % 4 == 0 && a.D <= 2048 && (at & 7) == 0 && (a.residual == nullptr || a.ldr % 4 == 0);
 }
 
-void launch_fold_norm(const FoldNormArgs& a, hipStream_t s) {
-  if (a.rows == 0) return;
-#define SHAI_FN(NC) fold_norm_kernel<NC><<<a.rows, 64, 0, s>>>(a)
+hipError_t launch_fold_norm(const FoldNormArgs& a, hipStream_t s) {
+  if (a.rows == 0) return hipSuccess;
+  if (!fold_norm_supported(a)) return hipErrorInvalidValue;
   const int chunks = (a.D + 255) / 256;
-  if (chunks <= 1) SHAI_FN(1);
-  else if (chunks <= 2) SHAI_FN(2);
-  else if (chunks <= 3) SHAI_FN(3);
-  else if (chunks <= 4) SHAI_FN(4);
-  else if (chunks <= 5) SHAI_FN(5);
-  else SHAI_FN(8);
-#undef SHAI_FN
-  SHAI_CHECK_LAUNCH();
+  return launch(chunks <= 1   ? fold_norm_kernel<1>
+                : chunks <= 2 ? fold_norm_kernel<2>
+                : chunks <= 3 ? fold_norm_kernel<3>
+                : chunks <= 4 ? fold_norm_kernel<4>
+                : chunks <= 5 ? fold_norm_kernel<5>
+                              : fold_norm_kernel<8>,
+                a.rows, 64, s, a);
 }
 
 }  // namespace shai

@@ -6,6 +6,7 @@
 // and the fold of a split convolution is another launch less.  A workgroup owns one image's channels of one group (of two where a
 // group's width is no multiple of 4), holds them in registers as bf16, and takes mean and variance in two passes over the registers.
 #include "common.h"
+#include "launch.h"
 #include "launchers.h"
 
 namespace shai {
@@ -202,25 +203,24 @@ bool gn_one_supported(int HW, int C, int G, bool fold) {
   return HW > 0 && geometry(HW, C, G, fold ? kMaxVecFold : kMaxVec, &q);
 }
 
-void launch_gn_one(const GnOneArgs& a, hipStream_t s) {
+hipError_t launch_gn_one(const GnOneArgs& a, hipStream_t s) {
   GnOneGeom q;
   const bool fold = a.parts != nullptr;
-  if (a.N <= 0 || !geometry(a.HW, a.C, a.G, fold ? kMaxVecFold : kMaxVec, &q)) return;   // the bindings refuse such a call
+  if (a.N <= 0) return hipSuccess;
+  if (a.HW <= 0 || !geometry(a.HW, a.C, a.G, fold ? kMaxVecFold : kMaxVec, &q)) return hipErrorInvalidValue;
   const int units = a.G / q.u, threads = (q.active + 63) / 64 * 64;
-  auto go = [&](auto kernel) { kernel<<<a.N * units, threads, 0, s>>>(a, units, q.vp, q.active); };
-#define SHAI_GN1(NV)                                                                    \
-  case NV:                                                                              \
-    if (q.u == 2) fold ? go(gn_one_kernel<NV, true, true>) : go(gn_one_kernel<NV, true, false>);  \
-    else fold ? go(gn_one_kernel<NV, false, true>) : go(gn_one_kernel<NV, false, false>);         \
-    break;
+  auto go = [&](auto kernel) { return launch(kernel, a.N * units, threads, s, a, units, q.vp, q.active); };
+#define SHAI_GN1(NV)                                                                                     \
+  case NV:                                                                                               \
+    return q.u == 2 ? go(fold ? gn_one_kernel<NV, true, true> : gn_one_kernel<NV, true, false>)          \
+                    : go(fold ? gn_one_kernel<NV, false, true> : gn_one_kernel<NV, false, false>);
   switch (q.nv) {
     SHAI_GN1(1)
     SHAI_GN1(2)
     SHAI_GN1(4)
     SHAI_GN1(8)
-    case 16:  // of one group, never behind a fold
-      go(gn_one_kernel<16, false, false>);
-      break;
+    default:  // 16, of one group, never behind a fold
+      return go(gn_one_kernel<16, false, false>);
   }
 #undef SHAI_GN1
 }

@@ -66,7 +66,8 @@ struct GnOneArgs {
   int silu;
 };
 bool gn_one_supported(int HW, int C, int G, bool fold);
-void launch_gn_one(const GnOneArgs& a, hipStream_t s);
+// hipErrorInvalidValue where gn_one_supported says no
+[[nodiscard]] hipError_t launch_gn_one(const GnOneArgs& a, hipStream_t s);
 // Norm statistics produced by a GEMM epilogue (GemmArgs::col_part / row_part) and their fallback passes:
 //   col partials [M / 128, N, 2] (sum, sum of squares per 128-row block and column) of x [M, N] (row stride ldx)
 void launch_col_partials(const bf16_t* x, long M, int N, long ldx, float* part, hipStream_t s);

@@ -19,7 +19,7 @@ struct PatchArgs {
   bf16_t* w_out;
   long w_pixels;
 };
-void launch_patches_u8(const PatchArgs& a, hipStream_t s);
+[[nodiscard]] hipError_t launch_patches_u8(const PatchArgs& a, hipStream_t s);
 
 // x [B, T, D] = (class token | patches | detection tokens) + position embedding, T = 1 + n + nd, and, where mr is given, mean and
 // 1 / standard deviation [B T, 2] of its rows.  D % 8 == 0, D <= 2048.
@@ -33,5 +33,5 @@ struct TokenArgs {
   int B, n, nd, D;
   float eps;
 };
-void launch_tokens(const TokenArgs& a, hipStream_t s);
+[[nodiscard]] hipError_t launch_tokens(const TokenArgs& a, hipStream_t s);
 }  // namespace shai

@@ -4,6 +4,7 @@
 // a cast, two affine passes, a cast, the channels' padding from 3 to 8 (which also made the patch product 2048 deep instead of 768),
 // a concatenation, a copy, an addition and the row moments were launches of their own.
 #include "common.h"
+#include "launch.h"
 #include "vision.h"
 
 namespace shai {
@@ -47,10 +48,10 @@ __global__ void __launch_bounds__(256) patches_u8_kernel(const PatchArgs a, long
   *reinterpret_cast<uint4_*>(a.out + i * 8) = pack8(f);
 }
 
-void launch_patches_u8(const PatchArgs& a, hipStream_t s) {
+hipError_t launch_patches_u8(const PatchArgs& a, hipStream_t s) {
   const long total = (long)a.B * a.H * a.W * 3 / 8;
   const unsigned images = (unsigned)((total + 255) / 256), weight = a.w ? (unsigned)((a.w_pixels / 4 + 255) / 256) : 0;
-  if (images + weight > 0) patches_u8_kernel<<<images + weight, 256, 0, s>>>(a, total, images);
+  return images + weight > 0 ? launch(patches_u8_kernel, images + weight, 256, s, a, total, images) : hipSuccess;
 }
 
 // One wave a row, held in registers; mean and variance in two passes over them.
@@ -97,13 +98,11 @@ __global__ void __launch_bounds__(256) tokens_kernel(const TokenArgs a) {
   if (lane == 0) *reinterpret_cast<float2*>(a.mr + 2 * row) = make_float2(mean, rsqrtf(var + a.eps));
 }
 
-void launch_tokens(const TokenArgs& a, hipStream_t s) {
+hipError_t launch_tokens(const TokenArgs& a, hipStream_t s) {
   const long rows = (long)a.B * (1 + a.n + a.nd);
-  if (rows <= 0) return;
+  if (rows <= 0) return hipSuccess;
   const unsigned grid = (unsigned)((rows + 3) / 4);
-  if (a.D <= 512) tokens_kernel<1><<<grid, 256, 0, s>>>(a);
-  else if (a.D <= 1024) tokens_kernel<2><<<grid, 256, 0, s>>>(a);
-  else tokens_kernel<4><<<grid, 256, 0, s>>>(a);
+  return launch(a.D <= 512 ? tokens_kernel<1> : a.D <= 1024 ? tokens_kernel<2> : tokens_kernel<4>, grid, 256, s, a);
 }
 
 }  // namespace shai
