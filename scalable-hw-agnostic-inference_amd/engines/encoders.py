@@ -94,7 +94,8 @@ class ImageClassifierEngine:
         self._graphs = {}
 
     def _forward_u8(self, x_u8: torch.Tensor) -> torch.Tensor:
-        out = self.model.forward_u8(x_u8, self.cfg.image_mean, self.cfg.image_std)
+        fused = getattr(self.model, "forward_u8", None)      # not every model that may be put in place has one
+        out = fused(x_u8, self.cfg.image_mean, self.cfg.image_std) if fused is not None else None
         if out is not None:
             return out
         px = ((x_u8.float() * (1.0 / 255.0) - self._mean) * self._inv_std).to(torch.bfloat16)

@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from .layers import Linear
+from .layers import Linear, then_norm
 
 
 def merge_linear_keys(sd: dict, prefix: str, parts, merged: str, bias: bool = True) -> None:
@@ -32,6 +32,7 @@ def merge_linear_keys(sd: dict, prefix: str, parts, merged: str, bias: bool = Tr
 
 class FusedSelfAttention(nn.Module):
     """Multi-head (optionally grouped-query) self-attention with a fused QKV GEMM."""
+    FUSED = True
 
     def __init__(self, dim: int, heads: int, head_dim: Optional[int] = None, kv_heads: Optional[int] = None,
                  qkv_bias: bool = True, out_bias: bool = True, out_dim: Optional[int] = None):
@@ -61,13 +62,14 @@ class FusedSelfAttention(nn.Module):
         return self.out(self._attend(x, causal, kv_lens, bias, scale), residual=residual)
 
     def forward_norm(self, x, residual, norm, causal: bool = False):
-        """(y, norm(y)) of y = self(x) + residual."""
-        return self.out.forward_norm(self._attend(x, causal), residual, norm)
+        """(y, norm(y)) of y = self(x, residual, causal)."""
+        return then_norm(self.out, norm, self._attend(x, causal), residual=residual)
 
 
 class CrossAttention(nn.Module):
     """Q from x, fused K/V GEMM from the (static) context.  K/V can be precomputed
     once per request and reused for every denoising step."""
+    FUSED = True
 
     def __init__(self, dim: int, ctx_dim: int, heads: int, head_dim: Optional[int] = None, qkv_bias: bool = False,
                  out_bias: bool = True):
@@ -82,12 +84,18 @@ class CrossAttention(nn.Module):
     def context_kv(self, ctx: torch.Tensor) -> torch.Tensor:
         return self.kv(ctx)
 
-    def forward_norm(self, x, ctx_kv: torch.Tensor, residual, norm):
-        """(y, norm(y)) of y = attention of x to the context + residual."""
+    def _attend(self, x, ctx_kv, kv_lens=None):
         B, T, _ = x.shape
         S = ctx_kv.shape[1]
         H, hd = self.heads, self.head_dim
         q = self.q(x).view(B, T, H, hd)
         k = ctx_kv[..., : H * hd].view(ctx_kv.shape[0], S, H, hd)
         v = ctx_kv[..., H * hd:].view(ctx_kv.shape[0], S, H, hd)
-        return self.out.forward_norm(ops.attention(q, k, v).view(B, T, H * hd), residual, norm)
+        return ops.attention(q, k, v, kv_lens=kv_lens).view(B, T, H * hd)
+
+    def forward(self, x, ctx_kv: torch.Tensor, residual=None, kv_lens=None):
+        return self.out(self._attend(x, ctx_kv, kv_lens), residual=residual)
+
+    def forward_norm(self, x, ctx_kv: torch.Tensor, residual, norm):
+        """(y, norm(y)) of y = self(x, ctx_kv, residual)."""
+        return then_norm(self.out, norm, self._attend(x, ctx_kv), residual=residual)

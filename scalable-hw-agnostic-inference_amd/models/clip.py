@@ -18,7 +18,7 @@ import torch.nn as nn
 
 from .. import ops
 from .attention import FusedSelfAttention, merge_linear_keys
-from .layers import Embedding, LayerNorm, Linear
+from .layers import Embedding, LayerNorm, Linear, chain, then_norm
 
 
 @dataclass
@@ -51,17 +51,24 @@ class CLIPTextConfig:
 
 
 class CLIPMLP(nn.Module):
+    FUSED = True
+
     def __init__(self, cfg: CLIPTextConfig):
         super().__init__()
         self.act = cfg.hidden_act
         self.fc1 = Linear(cfg.hidden_size, cfg.intermediate_size)
         self.fc2 = Linear(cfg.intermediate_size, cfg.hidden_size)
 
+    def forward(self, x, residual):
+        return self.fc2(self.fc1(x, act=self.act), residual=residual)
+
     def forward_norm(self, x, residual, norm):
-        return self.fc2.forward_norm(self.fc1(x, act=self.act), residual, norm)
+        return then_norm(self.fc2, norm, self.fc1(x, act=self.act), residual=residual)
 
 
 class CLIPEncoderLayer(nn.Module):
+    FUSED = True
+
     def __init__(self, cfg: CLIPTextConfig):
         super().__init__()
         self.layer_norm1 = LayerNorm(cfg.hidden_size, cfg.layer_norm_eps)
@@ -69,10 +76,14 @@ class CLIPEncoderLayer(nn.Module):
         self.layer_norm2 = LayerNorm(cfg.hidden_size, cfg.layer_norm_eps)
         self.mlp = CLIPMLP(cfg)
 
-    def forward(self, x, n, next_norm):
-        """``n``: x normalised by ``layer_norm1``.  Returns the layer's output and that normalised by ``next_norm``."""
-        x, n = self.self_attn.forward_norm(n, x, self.layer_norm2, causal=True)
-        return self.mlp.forward_norm(n, x, next_norm)
+    def forward(self, x, kv_lens=None):
+        x = self.self_attn(self.layer_norm1(x), residual=x, causal=True, kv_lens=kv_lens)
+        return self.mlp(self.layer_norm2(x), residual=x)
+
+    def forward_next(self, x, n, next_norm):
+        """(y, next_norm(y)) of y = self(x); ``n``: x normalised by ``layer_norm1``."""
+        x, n = then_norm(self.self_attn, self.layer_norm2, n, residual=x, causal=True)
+        return then_norm(self.mlp, next_norm, n, residual=x)
 
 
 class CLIPTextModel(nn.Module):
@@ -92,11 +103,7 @@ class CLIPTextModel(nn.Module):
         x = self.token_embedding(input_ids)
         x = ops.bias_act(x, None, self.position_embedding[:T].expand(B, T, -1).contiguous()) if x.is_cuda \
             else x + self.position_embedding[:T]
-        norms = [layer.layer_norm1 for layer in self.layers] + [self.final_layer_norm]
-        n = norms[0](x)
-        for layer, following in zip(self.layers, norms[1:]):
-            x, n = layer(x, n, following)
-        x = n
+        x = chain(self.layers, [layer.layer_norm1 for layer in self.layers] + [self.final_layer_norm], x)[1]
         if not output_pooled:
             return x
         if self.cfg.eos_token_id == 2:

@@ -20,6 +20,7 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook as _any_global_hook
 
 from .. import ops
 
@@ -30,7 +31,42 @@ def _round8(c: int) -> int:
     return (c + 7) // 8 * 8
 
 
+def as_called(*modules) -> bool:
+    """Whether a call of each of these modules is its class's ``forward`` and nothing else, so that a fused form may stand for the call: a
+    class that says ``FUSED`` of itself (one derived from it may have another ``forward``), no hooks, no ``forward`` of the object's."""
+    if _any_global_hook():
+        return False
+    for m in modules:
+        d = m.__dict__
+        if ("FUSED" not in type(m).__dict__ or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                or d["_backward_pre_hooks"]):
+            return False
+    return True
+
+
+def then_norm(m: nn.Module, norm: nn.Module, x, *args, residual, **kw):
+    """(y, norm(y)) of y = m(x, *args, residual=residual, **kw): in one call where nothing hooks into either."""
+    if as_called(m, norm):
+        return m.forward_norm(x, *args, residual=residual, norm=norm, **kw)
+    y = m(x, *args, residual=residual, **kw)
+    return y, norm(y)
+
+
+def chain(layers, norms, x, *args):
+    """(y, norm(y)) of y = x through ``layers``; ``norms``: the one that each layer begins with, and the one behind them all.  A layer's
+    last product makes the next layer's norm as well (``forward_next``), unless something hooks into the layer's call."""
+    n = None
+    for layer, own, following in zip(layers, norms, norms[1:]):
+        if as_called(layer):
+            x, n = layer.forward_next(x, own(x) if n is None else n, *args, next_norm=following)
+        else:
+            x, n = layer(x, *args), None
+    return x, norms[-1](x) if n is None else n
+
+
 class Linear(nn.Module):
+    FUSED = True
+
     def __init__(self, in_features: int, out_features: int, bias: bool = True, dtype=BF16):
         super().__init__()
         self.in_features, self.out_features = in_features, out_features
@@ -45,7 +81,7 @@ class Linear(nn.Module):
         return ops.linear_stats(x, self.weight, self.bias, residual=residual, stats=stats, eps=eps)
 
     def forward_norm(self, x, residual, norm):
-        """(y, norm(y)) of y = self(x) + residual -- see ``ops.linear_norm``."""
+        """(y, norm(y)) of y = self(x, residual=residual) -- see ``ops.linear_norm``; called by :func:`then_norm`."""
         return ops.linear_norm(x, self.weight, self.bias, residual, norm)
 
     def folded(self, ln: "LayerNorm"):
@@ -135,6 +171,7 @@ class GLULinear(nn.Module):
 
 class Conv2d(nn.Module):
     """NHWC conv on the implicit-GEMM kernel. Input channels padded to a multiple of 8."""
+    FUSED = True
 
     def __init__(self, cin: int, cout: int, kernel: int, stride: int = 1, padding: int = 0, bias: bool = True,
                  dtype=BF16):
@@ -189,6 +226,8 @@ class Conv2d(nn.Module):
 
 
 class GroupNorm(nn.Module):
+    FUSED = True
+
     def __init__(self, groups: int, channels: int, eps: float = 1e-5, dtype=BF16):
         super().__init__()
         self.groups, self.channels, self.eps = groups, channels, eps
@@ -213,7 +252,8 @@ class GroupNorm(nn.Module):
         return self.weight, self.bias, self.groups, self.eps, silu
 
     def one_ok(self, x, hw: int, channels: int) -> bool:
-        return ops.groupnorm_one_ok(x, hw, channels, self.groups)
+        """Whether this norm of [N, hw, channels], N and the device those of ``x``, runs as one launch, behind a convolution too."""
+        return ops.groupnorm_one_ok(x, hw, channels, self.groups) and as_called(self)
 
     def forward(self, x, silu: bool = False, x2=None, part=None, part2=None):
         """GroupNorm of x, or of cat([x, x2], -1) without materialising the concat.  ``part`` / ``part2``:
@@ -227,6 +267,8 @@ class GroupNorm(nn.Module):
 
 
 class LayerNorm(nn.Module):
+    FUSED = True
+
     def __init__(self, dim: int, eps: float = 1e-5, affine: bool = True, bias: bool = True, dtype=BF16):
         super().__init__()
         self.eps = eps
@@ -239,6 +281,8 @@ class LayerNorm(nn.Module):
 
 
 class RMSNorm(nn.Module):
+    FUSED = True
+
     def __init__(self, dim: int, eps: float = 1e-6, dtype=BF16, w_offset: float = 0.0):
         super().__init__()
         self.eps, self.w_offset = eps, w_offset

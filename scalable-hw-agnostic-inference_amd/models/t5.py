@@ -21,7 +21,7 @@ import torch.nn as nn
 from .. import ops
 from ..parallel.layers import GLUParallelLinear, QKVParallelLinear, RowParallelLinear
 from ..parallel.state import tp
-from .layers import Embedding, GLULinear, RMSNorm
+from .layers import Embedding, GLULinear, RMSNorm, chain, then_norm
 
 
 @dataclass
@@ -66,6 +66,8 @@ def relative_position_bucket(rel: torch.Tensor, num_buckets: int, max_distance: 
 
 
 class T5Block(nn.Module):
+    FUSED = True
+
     def __init__(self, c: T5Config):
         super().__init__()
         self.c = c
@@ -78,17 +80,23 @@ class T5Block(nn.Module):
         self.wo = RowParallelLinear(c.d_ff, c.d_model, bias=False)
         self.h = self.qkv.h_local
 
-    def forward(self, x, n, bias, lens, next_norm):
-        """``n``: x normalised by ``ln_attn``.  Returns the block's output and that normalised by ``next_norm``."""
-        B, S, _ = x.shape
+    def _attend(self, n, bias, lens):
+        B, S, _ = n.shape
         h, d = self.h, self.c.d_kv
         qkv = self.qkv(n)
         q = qkv[..., : h * d].view(B, S, h, d)
         k = qkv[..., h * d:2 * h * d].view(B, S, h, d)
         v = qkv[..., 2 * h * d:].view(B, S, h, d)
-        a = ops.attention(q, k, v, scale=1.0, kv_lens=lens, bias=bias)
-        x, n = self.o.forward_norm(a.view(B, S, h * d), x, self.ln_ff)
-        return self.wo.forward_norm(self.wi(n), x, next_norm)
+        return ops.attention(q, k, v, scale=1.0, kv_lens=lens, bias=bias).view(B, S, h * d)
+
+    def forward(self, x, bias, lens):
+        x = self.o(self._attend(self.ln_attn(x), bias, lens), residual=x)
+        return self.wo(self.wi(self.ln_ff(x)), residual=x)
+
+    def forward_next(self, x, n, bias, lens, next_norm):
+        """(y, next_norm(y)) of y = self(x, bias, lens); ``n``: x normalised by ``ln_attn``."""
+        x, n = then_norm(self.o, self.ln_ff, self._attend(n, bias, lens), residual=x)
+        return then_norm(self.wo, next_norm, self.wi(n), residual=x)
 
 
 class T5EncoderModel(nn.Module):
@@ -127,11 +135,7 @@ class T5EncoderModel(nn.Module):
                     else torch.full((B,), S, dtype=torch.int32, device=input_ids.device))
         x = self.shared(input_ids)
         bias = self.position_bias(S, input_ids.device)
-        norms = [blk.ln_attn for blk in self.blocks] + [self.final_layer_norm]
-        n = norms[0](x)
-        for blk, following in zip(self.blocks, norms[1:]):
-            x, n = blk(x, n, bias, lens, following)
-        return n
+        return chain(self.blocks, [blk.ln_attn for blk in self.blocks] + [self.final_layer_norm], x, bias, lens)[1]
 
     def convert_hf_state_dict(self, sd: dict) -> dict:
         out = {}

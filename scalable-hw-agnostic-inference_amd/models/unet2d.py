@@ -28,7 +28,7 @@ import torch.nn as nn
 
 from .. import ops
 from .attention import CrossAttention, FusedSelfAttention, merge_linear_keys
-from .layers import Conv2d, GLULinear, GroupNorm, LayerNorm, Linear, _wkey, timestep_embedding
+from .layers import Conv2d, GLULinear, GroupNorm, LayerNorm, Linear, _wkey, then_norm, timestep_embedding
 
 # the last transformer block's FF down projection merged into proj_out (Transformer2DModel._merged_out)
 MERGE_PROJ_OUT = os.environ.get("SHAI_MERGE_PROJ_OUT", "1") != "0"
@@ -134,7 +134,7 @@ class ResnetBlock2D(nn.Module):
     def _finish(self, n2, x, x2, follow):
         """conv2 of a small image, and the norm that follows."""
         skip = self._skip(x, x2)
-        if follow is None:
+        if follow is None or not follow[0].one_ok(x, x.shape[1] * x.shape[2], self.cout):
             return self.conv2(n2, residual=skip), None
         out, y = self.conv2(n2, residual=skip, gn=follow[0].spec(follow[1]))
         return out, Normed(y)
@@ -167,8 +167,8 @@ class BasicTransformerBlock(nn.Module):
         self.ff = FeedForward(dim)
 
     def forward(self, x, ctx_kv):
-        x, n = self.attn1.forward_norm(self.norm1(x), x, self.norm2)
-        x, n = self.attn2.forward_norm(n, ctx_kv, x, self.norm3)
+        x, n = then_norm(self.attn1, self.norm2, self.norm1(x), residual=x)
+        x, n = then_norm(self.attn2, self.norm3, n, ctx_kv, residual=x)
         return self.ff(n, residual=x)
 
     def forward_folded(self, x, ctx_kv, mr, next_eps=None, defer_down: bool = False):

@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .attention import FusedSelfAttention, merge_linear_keys
-from .layers import Conv2d, LayerNorm, Linear
+from .layers import Conv2d, LayerNorm, Linear, as_called, chain, then_norm
 
 
 # LayerNorms folded into the GEMMs that consume them, moments handed over by the producing GEMM (unet2d.py);
@@ -66,6 +66,8 @@ class ViTConfig:
 
 
 class ViTLayer(nn.Module):
+    FUSED = True
+
     def __init__(self, c: ViTConfig):
         super().__init__()
         self.layernorm_before = LayerNorm(c.hidden_size, c.layer_norm_eps)
@@ -75,10 +77,14 @@ class ViTLayer(nn.Module):
         self.output = Linear(c.intermediate_size, c.hidden_size)
         self.act = c.hidden_act
 
-    def forward(self, x, n, next_norm):
-        """``n``: x normalised by ``layernorm_before``.  Returns the layer's output and that normalised by ``next_norm``."""
-        x, n = self.attention.forward_norm(n, x, self.layernorm_after)
-        return self.output.forward_norm(self.intermediate(n, act=self.act), x, next_norm)
+    def forward(self, x):
+        x = self.attention(self.layernorm_before(x), residual=x)
+        return self.output(self.intermediate(self.layernorm_after(x), act=self.act), residual=x)
+
+    def forward_next(self, x, n, next_norm):
+        """(y, next_norm(y)) of y = self(x); ``n``: x normalised by ``layernorm_before``."""
+        x, n = then_norm(self.attention, self.layernorm_after, n, residual=x)
+        return then_norm(self.output, next_norm, self.intermediate(n, act=self.act), residual=x)
 
     def forward_folded(self, x, mr, next_eps=None):
         """forward with both LayerNorms folded into the QKV / fc1 GEMMs (``ops.fold_layernorm``): ``mr`` = (mean,
@@ -100,7 +106,7 @@ class ViTLayer(nn.Module):
         """The last layer when only some tokens leave the encoder: the first ``keep`` (token 0, CLS: image
         classification) or, with ``tail``, the last ``keep`` (YOLOS's detection tokens).  K / V of every token, the
         rest -- attention queries, out-projection, MLP -- for the kept tokens only (M = B keep instead of B T).
-        ``mr``: x's LayerNorm moments for the folded QKV, or ``n``: x normalised.  Returns [B, keep, d]."""
+        ``mr``: x's LayerNorm moments for the folded QKV, or ``n``: x normalised (neither: the plain norm).  Returns [B, keep, d]."""
         B, T, C = x.shape
         sel = slice(T - keep, T) if tail else slice(0, keep)
         a = self.attention
@@ -108,7 +114,7 @@ class ViTLayer(nn.Module):
             w, b, s = a.qkv.folded(self.layernorm_before)
             qkv = ops.linear(x, w, b, row_affine=(mr, s))
         else:
-            qkv = a.qkv(n)
+            qkv = a.qkv(self.layernorm_before(x) if n is None else n)
         q, k, v = a.split(qkv)
         o = ops.attention(q[:, sel], k, v).reshape(B, keep, a.heads * a.head_dim)
         x0 = a.out(o, residual=x[:, sel].contiguous())
@@ -116,6 +122,8 @@ class ViTLayer(nn.Module):
 
 
 class ViTEncoderModel(nn.Module):
+    FUSED = True
+
     def __init__(self, c: ViTConfig):
         super().__init__()
         self.cfg = c
@@ -152,9 +160,9 @@ class ViTEncoderModel(nn.Module):
 
     def forward_u8(self, images: torch.Tensor, mean, std, cls_only: bool = False):
         """``forward`` of uint8 images [B, H, W, 3] at the model's resolution, normalised with the channels' ``mean`` and ``std``
-        on the way into the patches; None where their sizes or address do not fit that kernel."""
+        on the way into the patches; None where their sizes or address do not fit that kernel, or something hooks into the calls."""
         P = self.cfg.patch_size
-        if not ops.patches_u8_ok(images, P):
+        if not ops.patches_u8_ok(images, P) or not as_called(self, self.patch):
             return None
         B, H, W, _ = images.shape
         x = ops.linear(*ops.patches_u8(images, P, mean, std, self.patch.weight), self.patch.bias)
@@ -182,12 +190,10 @@ class ViTEncoderModel(nn.Module):
                 x, mr = layer.forward_folded(x, mr, nxt)
             return self.layernorm(x)
         norms = [layer.layernorm_before for layer in layers] + [self.layernorm]
-        n = norms[0](x)
-        for i, layer in enumerate(layers):
-            if (cls_only or det_only) and i + 1 == len(layers):
-                return self.layernorm(layer.forward_cls(x, None, *self._kept(cls_only), n=n))
-            x, n = layer(x, n, norms[i + 1])
-        return n
+        if (cls_only or det_only) and layers:
+            x, n = chain(layers[:-1], norms[:-1], x)
+            return self.layernorm(layers[-1].forward_cls(x, None, *self._kept(cls_only), n=n))
+        return chain(layers, norms, x)[1]
 
 
 def preprocess(images_u8: torch.Tensor, size: Tuple[int, int], mean, std, device) -> torch.Tensor:
@@ -225,6 +231,8 @@ def _convert_vit_keys(sd: dict, prefix: str, n_layers: int) -> dict:
 
 
 class ViTForImageClassification(nn.Module):
+    FUSED = True
+
     def __init__(self, cfg: ViTConfig = None):
         super().__init__()
         self.cfg = cfg or ViTConfig()
@@ -237,7 +245,7 @@ class ViTForImageClassification(nn.Module):
 
     def forward_u8(self, images, mean, std):
         """``forward`` of uint8 images, or None (``ViTEncoderModel.forward_u8``)."""
-        h = self.vit.forward_u8(images, mean, std, cls_only=True)
+        h = self.vit.forward_u8(images, mean, std, cls_only=True) if as_called(self) else None
         return None if h is None else self.classifier(h[:, 0].contiguous())
 
     def convert_hf_state_dict(self, sd: dict) -> dict:

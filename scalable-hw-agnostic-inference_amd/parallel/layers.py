@@ -83,6 +83,8 @@ class ColumnParallelLinear(_ShardLoadMixin, nn.Module):
 
 
 class RowParallelLinear(_ShardLoadMixin, nn.Module):
+    FUSED = True
+
     def __init__(self, in_features: int, out_features: int, bias: bool = True, input_is_parallel: bool = True,
                  dtype=torch.bfloat16):
         super().__init__()
@@ -121,7 +123,7 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
         return y
 
     def forward_norm(self, x, residual, norm):
-        """(y, norm(y)) of y = self(x) + residual -- see ``ops.linear_norm``."""
+        """(y, norm(y)) of y = self(x, residual=residual) -- see ``ops.linear_norm``."""
         if self.tp_size == 1 and self.w_scale is None:
             return ops.linear_norm(x, self.weight, self.bias, residual, norm)
         y = self(x, residual=residual)
