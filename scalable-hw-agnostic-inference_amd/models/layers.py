@@ -253,7 +253,8 @@ class GroupNorm(nn.Module):
 
     def one_ok(self, x, hw: int, channels: int) -> bool:
         """Whether this norm of [N, hw, channels], N and the device those of ``x``, runs as one launch, behind a convolution too."""
-        return ops.groupnorm_one_ok(x, hw, channels, self.groups) and as_called(self)
+        return (ops.groupnorm_one_ok(x, hw, channels, self.groups) and as_called(self) and ops.row_ok(self.weight, channels, 8)
+                and ops.row_ok(self.bias, channels, 8))
 
     def forward(self, x, silu: bool = False, x2=None, part=None, part2=None):
         """GroupNorm of x, or of cat([x, x2], -1) without materialising the concat.  ``part`` / ``part2``:

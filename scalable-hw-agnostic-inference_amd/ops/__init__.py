@@ -300,6 +300,11 @@ def stats_supported(rows: int, cols: int, kind: str, hw: Optional[int] = None) -
 LINEAR_NORM_MAX = 1 << 20
 
 
+def row_ok(t: Optional[torch.Tensor], n: int, align: int = 16) -> bool:
+    """Whether the one-launch norms read ``t`` [n] as it lies: bf16 at multiples of ``align`` bytes.  The other kernels do not ask."""
+    return t is None or (t.dtype == torch.bfloat16 and t.numel() == n and t.is_contiguous() and t.data_ptr() % align == 0)
+
+
 def linear_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], residual: torch.Tensor, norm):
     """(y, norm(y)) with y = x @ w^T + bias + residual, ``norm`` a module with ``weight``, ``bias`` (None: RMS norm) and ``eps``.
     On the GPU a small product whose K is split leaves its fold to the norm's launch."""
@@ -307,7 +312,7 @@ def linear_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     gain, shift, rms = norm.weight, getattr(norm, "bias", None), getattr(norm, "w_offset", None) is not None
     rows = residual.is_contiguous() and residual.shape[-1] == N
     if not (_gpu(x) and rows and 0 < M * N <= LINEAR_NORM_MAX and N % 8 == 0 and N <= 2048 and w.dtype == torch.bfloat16
-            and gain is not None and not getattr(norm, "w_offset", 0.0)):
+            and gain is not None and not getattr(norm, "w_offset", 0.0) and row_ok(gain, N) and row_ok(shift, N)):
         y = linear(x, w, bias, residual=residual)
         return y, norm(y)
     x2 = x.reshape(M, -1) if (x.dim() == 2 or x.is_contiguous()) else x.contiguous().reshape(M, -1)
@@ -848,15 +853,15 @@ def tokens(patches: torch.Tensor, cls: torch.Tensor, det: Optional[torch.Tensor]
     """(x, row moments of x or None): x [B, T, D] = cat(class token, patches, detection tokens) + position embeddings [1, T, D], and
     with ``eps`` the (mean, rstd) [B T, 2] that the first layer's folded LayerNorm consumes."""
     B, n, D = patches.shape
-    if not _gpu(patches) or D % 8 or D > 2048:
+    nd = det.shape[1] if det is not None else 0
+    at = [cls.reshape(-1).contiguous(), det.reshape(nd, D).contiguous() if nd else None, pos.contiguous()]
+    if not _gpu(patches) or D % 8 or D > 2048 or not all(row_ok(t, n) for t, n in zip(at, (D, nd * D, (1 + n + nd) * D))):
         x = torch.cat([cls.expand(B, -1, -1), patches] + ([det.expand(B, -1, -1)] if det is not None else []), 1)
         x = bias_act(x.contiguous(), None, pos.expand(B, -1, -1).contiguous())
         return x, (row_moments(x, eps) if eps is not None else None)
-    nd = det.shape[1] if det is not None else 0
     x = torch.empty(B, 1 + n + nd, D, dtype=patches.dtype, device=patches.device)
     mr = torch.empty(B * (1 + n + nd), 2, dtype=torch.float32, device=x.device) if eps is not None else None
-    _K().tokens(patches.contiguous(), cls.reshape(-1).contiguous(), det.reshape(nd, D).contiguous() if nd else None, pos.contiguous(), x, mr,
-                float(eps) if eps is not None else 0.0)
+    _K().tokens(patches.contiguous(), *at, x, mr, float(eps) if eps is not None else 0.0)
     return x, mr
 
 

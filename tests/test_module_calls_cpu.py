@@ -3,6 +3,7 @@ although fused forms stand for most of them."""
 import pytest
 import torch
 
+from shai_amd import ops
 from shai_amd.models import clip, t5, unet2d, vit
 from shai_amd.models.attention import CrossAttention
 from shai_amd.models.layers import LayerNorm, Linear, as_called, init_random_, then_norm
@@ -122,3 +123,13 @@ def test_what_is_not_a_plain_call():
     finally:
         handle.remove()
     assert as_called(lin)
+
+
+def test_rows_that_the_one_launch_norms_read():
+    room = torch.zeros(64, dtype=torch.bfloat16)
+    at = room.data_ptr() % 16 // 2                     # elements behind an aligned address
+    row = room[(8 - at) % 8:]
+    assert ops.row_ok(None, 8) and ops.row_ok(row[:16], 16) and ops.row_ok(row[4:20], 16, 8)
+    for bad in (row[4:20], row[1:17], row[:8], row[:32:2], row[:16].float()):
+        assert not ops.row_ok(bad, 16)
+    assert not ops.row_ok(row[2:18], 16, 8)

@@ -2,8 +2,9 @@
 import pytest
 import torch
 
+from shai_amd import ops
 from shai_amd.models import t5, unet2d, vit
-from shai_amd.models.layers import GroupNorm, init_random_
+from shai_amd.models.layers import GroupNorm, LayerNorm, init_random_
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,29 @@ def test_small_images(cuda):
         got = m(x, t, kv).float()
         h.remove()
         assert ran and ran[-1] == n and ((got - want).norm() / want.norm()).item() < 2e-2
+
+
+def _at(t, elements):
+    """``t`` at an address so many elements behind an aligned one."""
+    room = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+    v = room[elements:elements + t.numel()].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+def test_parameters_at_other_addresses(cuda):
+    """Norms and tokens take parameters at any address of 4 bytes, as views of one large buffer are: by the kernels that ask for none."""
+    torch.manual_seed(0)
+    rnd = lambda *s: torch.randn(*s, device=cuda).bfloat16()      # noqa: E731
+    a, w, r, ln = rnd(40, 256), rnd(64, 256) / 16, rnd(40, 64), LayerNorm(64).to(cuda)
+    gn, img = GroupNorm(8, 64).to(cuda), rnd(2, 9, 9, 64)
+    args = (rnd(2, 6, 64), rnd(1, 1, 64), rnd(1, 3, 64), rnd(1, 10, 64))
+    for m in (ln, gn):
+        m.weight.data, m.bias.data = rnd(64), rnd(64)
+    assert gn.one_ok(img, 81, 64)
+    want = *ops.linear_norm(a, w, None, r, ln), gn(img, silu=True), ops.tokens(*args)[0]
+    ln.weight.data, gn.bias.data = _at(ln.weight.data, 4), _at(gn.bias.data, 2)
+    assert not gn.one_ok(img, 81, 64) and not ops.row_ok(ln.weight, 64)
+    got = *ops.linear_norm(a, w, None, r, ln), gn(img, silu=True), ops.tokens(args[0], _at(args[1], 2), *args[2:])[0]
+    for x, y in zip(got, want):      # other kernels: the sums of another order, rounded to bf16
+        assert ((x.float() - y.float()).norm() / y.float().norm()).item() < 5e-3
