@@ -48,3 +48,15 @@ def test_first_token_and_specials():
     assert special(["a <|image|>"])["input_ids"][0, :2].tolist() == [probe.encode("a")[0], 999]
     with pytest.raises(RuntimeError):
         probe(["a " * 20], max_length=4, truncation=False)
+
+
+# ids that are made another way, by a derived class or on the object, are those of the batch too
+@pytest.mark.parametrize("name", ["encode", "_words", "_tok"])
+def test_other_ids(name):
+    class Other(HashTokenizer):
+        pass
+    other = {"encode": lambda self, text, add_special_tokens=True: [7, 7], "_words": lambda self, text: [7, 7], "_tok": lambda self, w: 7}[name]
+    setattr(Other, name, other)
+    tok, own = Other(1000, None, None, 0, 4), HashTokenizer(1000, None, None, 0, 4)
+    setattr(own, name, other.__get__(own))
+    assert tok(["a b"])["input_ids"].tolist() == own(["a b"])["input_ids"].tolist() == [[7, 7, 0, 0]]
