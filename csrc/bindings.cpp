@@ -90,7 +90,7 @@ std::string gemm_key(const shai::GemmArgs& g) {
   // not be reused by a same-shape problem with a fused epilogue (and vice versa): separate key class
   // a folded-LayerNorm GEMM (row_mr) runs only unsplit: it tunes and caches apart from the plain problem
   return std::string(buf) + (g.rms ? "|rms" : "") + (g.w_scale ? "|fp8w" : "") + (g.row_mr ? "|ln" : "") +
-         (g.w_slice_rows ? "|wslice" + std::to_string(g.w_slice_rows) : "") +
+         (g.w_slice_rows ? "|wslice" + std::to_string(g.w_slice_rows) : "") + (shai::keeps_order(g) ? "|order" : "") +
          (lib_supported(g) && !g.residual ? "|lib" : "");
 }
 
@@ -172,7 +172,7 @@ bool lib_enabled() {  // off by default: every GEMM runs on the hand-written ker
 
 int max_splits_for(const shai::GemmArgs& g) {
   const int batch = g.batch > 0 ? g.batch : 1;
-  if (batch != 1 || g.row_mr != nullptr) return 1;  // folded LayerNorm: applied by unsplit epilogues only
+  if (batch != 1 || g.row_mr != nullptr || shai::keeps_order(g)) return 1;  // folded LayerNorm: applied by unsplit epilogues only
   const long kt = (g.K + 63) / 64;
   int s = 1;
   while (s < 16 && kt / (s * 2) >= 4) s *= 2;
@@ -274,7 +274,7 @@ void launch_choice(const shai::GemmArgs& g, const Tensor& like, Choice c) {
   }
   // a choice reused from another row count of the same bucket must still fit this problem
   if (!shai::gemm2_cfg_supported(g, c.cfg)) c = fallback_choice(g);
-  if (g.row_mr != nullptr) c.splits = 1;  // the planner's or a cached choice; K parts and their fold know no LayerNorm
+  if (g.row_mr != nullptr || shai::keeps_order(g)) c.splits = 1;  // the planner's or a cached choice; K parts and their fold know no LayerNorm
   Tensor ws;
   float* wsp = nullptr;
   if (c.splits > 1) {
@@ -375,7 +375,7 @@ Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only =
     }
   // residual epilogues are in place (C aliases the residual): timing them into the scratch output is not
   // equivalent, so only bias-or-nothing problems race the library
-  if (!skinny_only && lib_enabled() && lib_supported(g_real) && !g_real.residual) cands.push_back({kLibCfg, 1});
+  if (!skinny_only && lib_enabled() && lib_supported(g_real) && !g_real.residual && !shai::keeps_order(g)) cands.push_back({kLibCfg, 1});
   auto launch = [&](const Choice& c) {
     if (norm) launch_then_norm(g, like, c, *norm);
     else launch_choice(g, like, c);
@@ -562,6 +562,11 @@ void run_gemm(const shai::GemmArgs& g, const Tensor& like, long a_bytes, long w_
   // waits for no tuning (4.7 to 9 ms, the first of a process 30).
   bool found = lookup_choice(g, key, &c, suffix);
   if (!found && norm) found = lookup_choice(g, gemm_key(g), &c);
+  if (!found && shai::keeps_order(g)) {  // the choice for any order, where it keeps this one
+    shai::GemmArgs any = g;
+    any.one_order = 0;
+    found = lookup_choice(any, gemm_key(any), &c) && c.splits == 1 && shai::gemm2_cfg_supported(g, c.cfg);
+  }
   if (!found || c.cfg < 0) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hipStreamIsCapturing(stream(), &cs);
@@ -979,7 +984,7 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
           double res_alpha, int64_t act, bool glu, const optional<Tensor>& gate, int64_t rows_per_gate,
           int64_t force_cfg, double rms_eps, const optional<Tensor>& w_scale, const optional<Tensor>& ln_mr,
           const optional<Tensor>& ln_s, const optional<Tensor>& gn_part, const optional<Tensor>& ln_stats,
-          double ln_eps, int64_t w_slice_rows) {
+          double ln_eps, int64_t w_slice_rows, bool one_order) {
   check_rows(a, "a");
   if (w_scale.has_value()) {  // fp8 (e4m3) weights + fp32 per-row scale: skinny (decode-shaped) kernel only
     SHAI_CHECK(w.is_cuda() && w.scalar_type() == at::kFloat8_e4m3fn && w.dim() == 2 && w.stride(1) == 1 &&
@@ -996,6 +1001,7 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
   SHAI_CHECK(a.dim() == w.dim() || w.dim() == 2, "gemm rank mismatch");
   const bool batched = a.dim() == 3;
   shai::GemmArgs g{};
+  g.one_order = one_order;
   g.A = cptr(a);
   g.W = cptr(w);
   g.C = mptr(c);
@@ -1936,7 +1942,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("groupnorm_from_partials(Tensor part1, Tensor? part2, int C1, int C2, int Nimg, int HW, Tensor? gamma, Tensor? beta, Tensor(a!) scale, Tensor(b!) shift, int G, float eps) -> ()");
   m.def("col_partials(Tensor x, Tensor(a!) part) -> ()");
   m.def("row_moments(Tensor x, Tensor(a!) mr, float eps) -> ()");
-  m.def("gemm(Tensor a, Tensor w, Tensor(a!) c, Tensor? bias, Tensor? bias2d, int rows_per_bias2d, Tensor? residual, float alpha, float res_alpha, int act, bool glu, Tensor? gate=None, int rows_per_gate=1, int force_cfg=-1, float rms_eps=-1.0, Tensor? w_scale=None, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, int w_slice_rows=0) -> ()");
+  m.def("gemm(Tensor a, Tensor w, Tensor(a!) c, Tensor? bias, Tensor? bias2d, int rows_per_bias2d, Tensor? residual, float alpha, float res_alpha, int act, bool glu, Tensor? gate=None, int rows_per_gate=1, int force_cfg=-1, float rms_eps=-1.0, Tensor? w_scale=None, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, int w_slice_rows=0, bool one_order=False) -> ()");
   m.def("gemm_norm(Tensor a, Tensor w, Tensor(a!) y, Tensor? bias, Tensor? residual, Tensor? gamma, Tensor? beta, Tensor(b!) out, float eps, bool rms, int force_cfg=-1) -> ()");
   m.def("dequant_fp8(Tensor w8, Tensor scale, Tensor(a!) out) -> ()");
   m.def("layernorm_mod(Tensor x, Tensor scale, Tensor shift, Tensor(a!) out, int rows_per_mod, float eps) -> ()");

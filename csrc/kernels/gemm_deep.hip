@@ -116,6 +116,8 @@ bool gemm_deep_supported(const GemmArgs& a) {
   return !a.conv || (a.Cin % 64 == 0 && (a.A2 == nullptr || a.Cin1 % 64 == 0));
 }
 
+int gemm_deep_wave_groups(int which) { return kDeep[which].wk; }
+
 void gemm_deep_tile(int which, int* bm, int* bn) {
   *bm = kDeep[which].bm;
   *bn = kDeep[which].bn;

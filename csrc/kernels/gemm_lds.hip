@@ -336,10 +336,12 @@ bool gemm2_cfg_supported(const GemmArgs& a, int cfg) {
     if (a.conv || a.in_scale != nullptr) return false;
   }
   // 192 x 128 and 128 x 128 with two groups of waves along K: up to 8192 rows.  They fill one round of the chip where other tiles
-  // need more or a split (4096 x 1280 x 5120: 57.8 us, two workgroups of 192 x 128 to a CU 74.4); with more rows rounds are full anyway
-  // (16384 x 640 x 2560 66.0 and 64.0, x 640 29.7 and 25.6), and the sums of long prompts stay in one order whatever their rows.
+  // need more or a split (4096 x 1280 x 5120: 57.8 us, two workgroups of 192 x 128 to a CU 74.4).  With more rows the better of the two
+  // is ahead of the best other tile by 5 % at most (9364 x 512 x 1024 19.6 and 20.6 us, 8274 x 1280 x 5120 115.7 and 116.2) and
+  // mostly behind it (9364 x 768 x 768 23.2 and 19.9, 12288 x 1280 x 5120 172 and 132, 16384 x 1024 x 2816 108 and 80).
   if ((cfg == kDeepCfg + 3 || cfg == kDeepCfg + 4) && a.M > 8192) return false;
-  if (cfg >= kDeepCfg) return cfg < kDeepCfg + kDeepCfgs && gemm_deep_supported(a);
+  if (cfg >= kDeepCfg)
+    return cfg < kDeepCfg + kDeepCfgs && gemm_deep_supported(a) && !(keeps_order(a) && gemm_deep_wave_groups(cfg - kDeepCfg) > 1);
   if (cfg == kWsCfg) return gemm_ws_supported(a);
   if (cfg == kW4Cfg) return gemm_w4_supported(a);
   if (cfg == kW4Cfg + 1) return false;  // 192 x 320 four-wave tile: lab only (gemm_w4.hip launch_gemm_w4)

@@ -173,7 +173,14 @@ struct GemmArgs {
   // kernel only, w_slice_rows % 256 == 0): a per-image weight, e.g. a GroupNorm's per-image scale folded into W
   int w_slice_rows;
   int no_fold;              // split-K: leave the partial sums to the caller's consumer, launch no fold
+  int one_order;            // the same sums whatever the row count is, from kOneOrderRows rows on (keeps_order)
 };
+// Products of packed prompts (GemmArgs::one_order) of this many rows and more take no split of K, over workgroups or over groups of
+// waves: all other tiles add K in the same order, so that a prompt's rows have the same bits whatever is packed or padded beside them.
+// From here on the rows alone fill the chip at a decoder's widths (4096 x 4096: 256 tiles of 256 x 256); narrower ones lose at most
+// what the wave groups gain (4096 x 1280 x 5120 57.8 us, without 74.4; 6304 x 1280 x 5120 90.8 and 87.7).
+constexpr int kOneOrderRows = 4096;
+inline bool keeps_order(const GemmArgs& a) { return a.one_order != 0 && a.M >= kOneOrderRows; }
 // (conv, GLU, activation) epilogue variants the tile kernels (v2 / v4 / four-wave / W-stationary / halo conv)
 // instantiate: convolutions NONE / SILU, GLU SILU / GELU / GELU_TANH, plain GEMMs every activation.  Any other
 // combination is rejected by every tile config (gemm2_cfg_supported), never run as a neighbouring variant.
@@ -209,6 +216,7 @@ void launch_gemm_w4(const GemmArgs& a, int bn, hipStream_t s);
 constexpr int kDeepCfgs = 6;
 bool gemm_deep_supported(const GemmArgs& a);
 void gemm_deep_tile(int which, int* bm, int* bn);
+int gemm_deep_wave_groups(int which);  // along K
 void launch_gemm_deep(const GemmArgs& a, int which, float* ws, int splits, hipStream_t s);
 // v6: W-stationary low-K GEMM (gemm_ws.hip): K = 320, N % 320 == 0, persistent over M, weights in VGPRs
 bool gemm_ws_supported(const GemmArgs& a);

@@ -175,8 +175,8 @@ class LlamaAttention(nn.Module):
         st = tp()
         self.cfg = cfg
         self.qkv_proj = QKVParallelLinear(cfg.hidden_size, cfg.num_attention_heads, cfg.num_key_value_heads,
-                                          cfg.head_dim)
-        self.o_proj = RowParallelLinear(cfg.num_attention_heads * cfg.head_dim, cfg.hidden_size, bias=False)
+                                          cfg.head_dim, one_order=True)
+        self.o_proj = RowParallelLinear(cfg.num_attention_heads * cfg.head_dim, cfg.hidden_size, bias=False, one_order=True)
         self.h = self.qkv_proj.h_local
         self.hk = self.qkv_proj.kv_local
         self.hd = cfg.head_dim
@@ -215,8 +215,8 @@ class LlamaAttention(nn.Module):
 class LlamaMLP(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
-        self.gate_up_proj = GLUParallelLinear(cfg.hidden_size, cfg.intermediate_size, act="silu")
-        self.down_proj = RowParallelLinear(cfg.intermediate_size, cfg.hidden_size, bias=False)
+        self.gate_up_proj = GLUParallelLinear(cfg.hidden_size, cfg.intermediate_size, act="silu", one_order=True)
+        self.down_proj = RowParallelLinear(cfg.intermediate_size, cfg.hidden_size, bias=False, one_order=True)
 
     def forward(self, x, residual=None, rms_eps=None):
         return self.down_proj(self.gate_up_proj(x, rms_eps=rms_eps), residual=residual)

@@ -336,9 +336,9 @@ class CrossAttention(nn.Module):
 
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
-        self.q_proj = ColumnParallelLinear(cfg.hidden_size, cfg.num_attention_heads * cfg.head_dim, bias=False)
+        self.q_proj = ColumnParallelLinear(cfg.hidden_size, cfg.num_attention_heads * cfg.head_dim, bias=False, one_order=True)
         self.kv_proj = QKVParallelLinear(cfg.hidden_size, 0, cfg.num_key_value_heads, cfg.head_dim)
-        self.o_proj = RowParallelLinear(cfg.num_attention_heads * cfg.head_dim, cfg.hidden_size, bias=False)
+        self.o_proj = RowParallelLinear(cfg.num_attention_heads * cfg.head_dim, cfg.hidden_size, bias=False, one_order=True)
         self.q_norm = RMSNorm(cfg.head_dim, cfg.rms_norm_eps)
         self.k_norm = RMSNorm(cfg.head_dim, cfg.rms_norm_eps)
         self.h = self.q_proj.out_local // cfg.head_dim

@@ -219,7 +219,7 @@ def gemm_f8(a8: torch.Tensor, w8: torch.Tensor, a_scale: torch.Tensor, w_scale: 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act=None,
            residual: Optional[torch.Tensor] = None, glu: bool = False, alpha: float = 1.0,
            res_alpha: float = 1.0, rms_eps: Optional[float] = None,
-           w_scale: Optional[torch.Tensor] = None, row_affine=None, force_cfg: int = -1) -> torch.Tensor:
+           w_scale: Optional[torch.Tensor] = None, row_affine=None, force_cfg: int = -1, one_order: bool = False) -> torch.Tensor:
     """y = act(alpha * x @ w^T + bias) (+ res_alpha * residual).
 
     glu=True: ``w`` rows are interleaved (value_i, gate_i) pairs and the output
@@ -233,6 +233,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     problems (<= 64 rows) stream the fp8 bytes through the skinny kernel (half the weight
     traffic); larger ones run W8A8 on the fp8 MFMA (``FP8_PREFILL``: the activation is quantised per row, with
     the folded RMSNorm in its row scale) or dequantize to bf16 first and run the bf16 GEMMs.
+    one_order: from 4096 rows on a row's bits do not depend on how many rows there are (prompts that are packed into one product: the
+    kernels that cut K into parts are left out).
     """
     if w_scale is not None:
         M = x.numel() // x.shape[-1]
@@ -265,7 +267,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     y = torch.empty(x2.shape[0], Nout, dtype=x.dtype, device=x.device)
     r2 = residual.reshape(-1, Nout) if residual is not None else None
     _K().gemm(x2, w, y, bias, None, 1, r2, float(alpha), float(res_alpha), act_id(act), bool(glu), None, 1, -1,
-              float(rms_eps) if rms_eps is not None else -1.0, w_scale)
+              float(rms_eps) if rms_eps is not None else -1.0, w_scale, one_order=bool(one_order))
     return y.view(*lead, Nout)
 
 

@@ -14,6 +14,8 @@ Semantics match NxD's layers the reference uses for Flux / T5 TP8
   GEMM epilogue on each shard.
 * ``VocabParallelEmbedding`` / ``ParallelLMHead``: vocab-sharded.
 
+``one_order``: the layer of a decoder whose prompts are packed into one product, see ``ops.linear``.
+
 Every layer's ``_load_from_state_dict`` accepts the FULL (unsharded) tensor and
 slices this rank's shard, so one HF checkpoint serves every TP degree.
 """
@@ -61,8 +63,9 @@ class _ShardLoadMixin:
 
 class ColumnParallelLinear(_ShardLoadMixin, nn.Module):
     def __init__(self, in_features: int, out_features: int, bias: bool = True, gather_output: bool = False,
-                 dtype=torch.bfloat16):
+                 dtype=torch.bfloat16, one_order: bool = False):
         super().__init__()
+        self.one_order = one_order
         st = tp()
         self.tp_rank, self.tp_size = st.rank, st.size
         self.in_features, self.out_features = in_features, out_features
@@ -78,7 +81,7 @@ class ColumnParallelLinear(_ShardLoadMixin, nn.Module):
         return (self.out_features, self.in_features) if name == "weight" else (self.out_features,)
 
     def forward(self, x, act=None, rms_eps=None):
-        y = ops.linear(x, self.weight, self.bias, act=act, rms_eps=rms_eps, w_scale=self.w_scale)
+        y = ops.linear(x, self.weight, self.bias, act=act, rms_eps=rms_eps, w_scale=self.w_scale, one_order=self.one_order)
         return comm.all_gather_last(y) if self.gather_output else y
 
 
@@ -86,8 +89,9 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
     FUSED = True
 
     def __init__(self, in_features: int, out_features: int, bias: bool = True, input_is_parallel: bool = True,
-                 dtype=torch.bfloat16):
+                 dtype=torch.bfloat16, one_order: bool = False):
         super().__init__()
+        self.one_order = one_order
         st = tp()
         self.tp_rank, self.tp_size = st.rank, st.size
         self.in_features, self.out_features = in_features, out_features
@@ -108,7 +112,7 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
         if not self.input_is_parallel and self.tp_size > 1:
             x = x.narrow(-1, self.tp_rank * self.in_local, self.in_local).contiguous()
         if self.tp_size == 1:
-            return ops.linear(x, self.weight, self.bias, residual=residual, w_scale=self.w_scale)
+            return ops.linear(x, self.weight, self.bias, residual=residual, w_scale=self.w_scale, one_order=self.one_order)
         rows = x.numel() // x.shape[-1]
         # fused (GEMM into the IPC staging slot, one kernel reduces + adds bias / residual) and, at >= 1024 rows,
         # overlapped (row slab i's reduce runs beside slab i + 1's GEMM); CPU (gloo): the same slab schedule
@@ -116,7 +120,7 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
                                      chunks=comm.overlap_chunks(rows, self.out_features))
         if y is not None:
             return y.view(*x.shape[:-1], self.out_features)
-        y = ops.linear(x, self.weight, None, w_scale=self.w_scale)
+        y = ops.linear(x, self.weight, None, w_scale=self.w_scale, one_order=self.one_order)
         comm.all_reduce(y)
         if self.bias is not None or residual is not None:
             y = ops.bias_act(y, self.bias, residual)
@@ -124,7 +128,7 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
 
     def forward_norm(self, x, residual, norm):
         """(y, norm(y)) of y = self(x, residual=residual) -- see ``ops.linear_norm``."""
-        if self.tp_size == 1 and self.w_scale is None:
+        if self.tp_size == 1 and self.w_scale is None and not self.one_order:
             return ops.linear_norm(x, self.weight, self.bias, residual, norm)
         y = self(x, residual=residual)
         return y, norm(y)
@@ -134,8 +138,9 @@ class QKVParallelLinear(_ShardLoadMixin, nn.Module):
     """Fused [q; k; v] projection; rows of the full weight ordered q (H*hd), k (Hk*hd), v (Hk*hd)."""
 
     def __init__(self, hidden: int, heads: int, kv_heads: int, head_dim: int, bias: bool = False,
-                 dtype=torch.bfloat16):
+                 dtype=torch.bfloat16, one_order: bool = False):
         super().__init__()
+        self.one_order = one_order
         st = tp()
         self.tp_rank, self.tp_size = st.rank, st.size
         self.heads, self.kv_heads, self.head_dim = heads, kv_heads, head_dim
@@ -162,15 +167,16 @@ class QKVParallelLinear(_ShardLoadMixin, nn.Module):
         return (n, self.weight.shape[1]) if name == "weight" else (n,)
 
     def forward(self, x, rms_eps=None):
-        return ops.linear(x, self.weight, self.bias, rms_eps=rms_eps, w_scale=self.w_scale)
+        return ops.linear(x, self.weight, self.bias, rms_eps=rms_eps, w_scale=self.w_scale, one_order=self.one_order)
 
 
 class GLUParallelLinear(_ShardLoadMixin, nn.Module):
     """Fused value/gate projection, rows interleaved (value_i, gate_i); output value*act(gate)."""
 
     def __init__(self, hidden: int, intermediate: int, act: str = "silu", bias: bool = False,
-                 dtype=torch.bfloat16):
+                 dtype=torch.bfloat16, one_order: bool = False):
         super().__init__()
+        self.one_order = one_order
         st = tp()
         self.tp_rank, self.tp_size = st.rank, st.size
         self.act = act
@@ -186,7 +192,8 @@ class GLUParallelLinear(_ShardLoadMixin, nn.Module):
         return (n, self.weight.shape[1]) if name == "weight" else (n,)
 
     def forward(self, x, rms_eps=None):
-        return ops.linear(x, self.weight, self.bias, act=self.act, glu=True, rms_eps=rms_eps, w_scale=self.w_scale)
+        return ops.linear(x, self.weight, self.bias, act=self.act, glu=True, rms_eps=rms_eps, w_scale=self.w_scale,
+                          one_order=self.one_order)
 
 
 class VocabParallelEmbedding(_ShardLoadMixin, nn.Module):

@@ -107,3 +107,42 @@ def test_convolution(cuda, cfg, splits):
     r = subprocess.run([sys.executable, "-c", CONV_SCRIPT.format(root=root, tol=TOL)], env=env, capture_output=True, text=True,
                        timeout=100)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-3000:]
+
+
+# products that keep one order of sums (packed prompts): every tile that they may take gives the same bits, the others are refused
+@pytest.mark.parametrize("N,K,glu", [(512, 1024, False), (320, 320, False), (1536, 776, False), (1024, 512, True)])
+def test_one_order(cuda, N, K, glu):
+    M = 4100
+    a, w, _, _ = _problem(M, N, K, cuda)
+    r = torch.randn(M, N // 2 if glu else N, device=cuda).bfloat16()
+    run = lambda rows, cfg: ops._K().gemm(a[:rows], w, y[:rows], None, None, 1, r[:rows], 1.0, 1.0, ops.act_id("silu" if glu else None), glu,  # noqa: E731
+                                          force_cfg=cfg, one_order=True)
+    y, seen = torch.empty_like(r), {}
+    for cfg in range(22):
+        try:
+            run(M, cfg)
+        except RuntimeError as e:
+            assert "bad force_cfg" in str(e)
+            continue
+        seen[cfg] = y.clone()
+    assert {0, 3, 9, 12, 18, 21} <= set(seen) and not {16, 17, 19, 20} & set(seen)
+    for cfg, out in seen.items():
+        assert torch.equal(out, seen[3]), cfg
+    for cfg in (16, 19):                  # fewer rows: any tile
+        run(4095, cfg)
+    for cfg in (3203, 3410):              # and no split where the rows keep the order
+        run(M, cfg)
+        assert torch.equal(y, seen[3])
+
+
+@pytest.mark.parametrize("N,K,glu,rms", [(512, 1024, False, None), (768, 512, False, 1e-5), (2048, 512, True, 1e-5)])
+def test_rows_do_not_depend_on_how_many(cuda, N, K, glu, rms):
+    """Rows of a packed prompt beside few others and many, on both sides of the sizes where tiles change; also where the shipped or an
+    earlier choice for the rows cuts K."""
+    a, w, _, _ = _problem(16000, N, K, cuda)
+    call = lambda rows: ops.linear(a[:rows], w, act="silu" if glu else None, glu=glu, rms_eps=rms, one_order=True)  # noqa: E731
+    for rows, choice in ((4096, "19,1"), (4864, "10,4"), (9364, "3,2"), (16000, "17,1")):
+        ops._K().gemm_tuning_import([f"0:{rows},{N},{K},b1,g{int(glu)}|0,0,0,0,0,0,0,0,0{t}={choice}" for t in ("", "|lib")])
+    want = call(16000)
+    for rows in (4096, 4864, 9364):
+        assert torch.equal(call(rows), want[:rows])

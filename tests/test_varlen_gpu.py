@@ -138,3 +138,29 @@ def test_engine_packed_prefill_matches_padded(cuda):
     rel = ((l_packed - l_pad).norm() / l_pad.norm()).item()
     assert rel < 2e-2, rel
     assert got == want
+
+
+def test_engine_packed_prefill_matches_padded_below_8192_rows(cuda):
+    """4864 packed rows and 14000 padded ones: tiles that add in another order are open to image and text encoders on one side only
+    (gemm2_cfg_supported), to neither here."""
+    from shai_amd.engines.llm import LLMEngine, SamplingParams
+    from shai_amd.models.llama import LlamaConfig
+    c = LlamaConfig(vocab_size=2048, hidden_size=512, intermediate_size=1024, num_hidden_layers=2,
+                    num_attention_heads=8, num_key_value_heads=2, head_dim=64, max_position_embeddings=16384)
+    prompts = [[(7 * i) % 2000 + 3 for i in range(n)] for n in (64, 1000, 3500, 300)]
+    p = SamplingParams(max_tokens=6, temperature=0.0, ignore_eos=True)
+
+    def run(packed):
+        e = LLMEngine(c, device="cuda:0", max_num_seqs=4, max_model_len=4096, enable_prefix_caching=False,
+                      packed_prefill=packed, mixed_steps=False, prefill_token_budget=16384, seed=3)
+        rec = []
+        fwd = e.model.forward
+        e.model.forward = lambda *a, **k: (lambda y: (rec.append(y.float().clone()), y)[1])(fwd(*a, **k))
+        with torch.inference_mode():
+            out = [s.output for s in e.generate(prompts, p)]
+        return out, rec[0]
+    want, l_pad = run(False)
+    got, l_packed = run(True)
+    rel = ((l_packed - l_pad).norm() / l_pad.norm()).item()
+    assert rel < 2e-2, rel
+    assert got == want
