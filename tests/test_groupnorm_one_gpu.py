@@ -79,3 +79,8 @@ def test_after_convolution(cuda, cfg, splits, side, cin, cout):
             assert off(y, norm64(out, gamma, beta, 32, 1e-5, True)) < 2 ** -8
             plain = ops.conv2d(x, w, b, 3, 3, 1, 1, temb=temb, residual=res)
             assert torch.equal(out, plain)      # the fold's sums in its order
+    # which launch folds: without keep the convolution itself is written only where its K is not split
+    raw = torch.full((N, side, side, cout), 7.0, device="cuda", dtype=torch.bfloat16)
+    native.ops().conv2d(x, None, w, raw, b, temb, None, None, None, 0, 3, 3, 1, 1, False, 0, 1.0, gn_gamma=gamma, gn_beta=beta,
+                        gn_out=torch.empty_like(raw), gn_groups=32, gn_silu=True, keep_out=False)
+    assert bool((raw == 7).all()) == (splits > 1)

@@ -58,7 +58,7 @@ def test_split_forms(cuda, M, N, K, kind, force):
         assert torch.equal(apart, y[:M])
 
 
-# the rule: both sides of the largest output, a residual in place of the output's memory, widths and strides that go the separate way
+# the rule: both sides of the largest output, and a width that goes the separate way
 @pytest.mark.parametrize("shape,N,K", [((2, 77), 1024, 1024), ((1, 1024), 1024, 256), ((1, 1025), 1024, 256), ((5,), 2056, 256)])
 @pytest.mark.parametrize("kind", ["layer", "rms"])
 def test_rule(cuda, shape, N, K, kind):
@@ -68,6 +68,27 @@ def test_rule(cuda, shape, N, K, kind):
     assert y.shape == h.shape == (*shape, N)
     want = (a.float() @ w.float().t() + r.float()).view(*shape, N)
     assert _rel(y, want) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
+
+
+# a residual whose rows lie apart (the function goes the separate way, the op folds it as it lies), and one in place of the output
+@pytest.mark.parametrize("force", [3216, 1003, 3116])
+def test_residuals(cuda, force):
+    norm, (a, w, b, r) = _norm("rms", 264, cuda), _problem(33, 264, 512, cuda)
+    y, h = torch.empty_like(r), torch.empty_like(r)
+    op = lambda y, res: ops._K().gemm_norm(a, w, y, b, res, norm.weight, None, h, norm.eps, True, force)  # noqa: E731
+    op(y, r)
+    want = y.clone(), h.clone()
+    assert _rel(y, a.float() @ w.float().t() + b.float() + r.float()) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
+    wide = torch.full((33, 272), 9.0, device=cuda, dtype=torch.bfloat16)
+    wide[:, :264] = r
+    for out, res in ((torch.empty_like(r), wide[:, :264]), (r.clone(), None)):
+        op(out, out if res is None else res)
+        assert torch.equal(out, want[0]) and torch.equal(h, want[1])
+    y2, h2 = ops.linear_norm(a, w, b, wide[:, :264], norm)
+    assert _rel(y2, want[0]) < 4e-3 and _rel(h2, _want(y2, norm)) < 5e-3
+    three = a.view(3, 11, 512).transpose(0, 1)          # an input that is copied first
+    y3, h3 = ops.linear_norm(three, w, b, r.view(3, 11, 264).transpose(0, 1).contiguous(), norm)
+    assert _rel(y3, want[0].view(3, 11, 264).transpose(0, 1)) < 4e-3 and _rel(h3, _want(y3, norm)) < 5e-3
 
 
 def test_refusals(cuda):
