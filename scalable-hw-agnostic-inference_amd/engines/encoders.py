@@ -122,8 +122,9 @@ class ImageClassifierEngine:
             g = self._graphs[B] = (graph, static, out, FoldedWeights(self.model))
         graph, static, out, folded = g
         static.copy_(x_u8)
-        folded.refresh()
         graph.replay()
+        if folded.refresh():       # looked at beside the replay, which is made again where parameters were written since the last
+            graph.replay()
         return out
 
     @torch.inference_mode()

@@ -14,7 +14,8 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from .layers import Linear, then_norm
+from ..utils.calls import fused, then_norm
+from .layers import Linear
 
 
 def merge_linear_keys(sd: dict, prefix: str, parts, merged: str, bias: bool = True) -> None:
@@ -30,10 +31,9 @@ def merge_linear_keys(sd: dict, prefix: str, parts, merged: str, bias: bool = Tr
                 sd.pop(k, None)
 
 
+@fused
 class FusedSelfAttention(nn.Module):
     """Multi-head (optionally grouped-query) self-attention with a fused QKV GEMM."""
-    FUSED = True
-
     def __init__(self, dim: int, heads: int, head_dim: Optional[int] = None, kv_heads: Optional[int] = None,
                  qkv_bias: bool = True, out_bias: bool = True, out_dim: Optional[int] = None):
         super().__init__()
@@ -66,11 +66,10 @@ class FusedSelfAttention(nn.Module):
         return then_norm(self.out, norm, self._attend(x, causal), residual=residual)
 
 
+@fused
 class CrossAttention(nn.Module):
     """Q from x, fused K/V GEMM from the (static) context.  K/V can be precomputed
     once per request and reused for every denoising step."""
-    FUSED = True
-
     def __init__(self, dim: int, ctx_dim: int, heads: int, head_dim: Optional[int] = None, qkv_bias: bool = False,
                  out_bias: bool = True):
         super().__init__()

@@ -17,8 +17,9 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..utils.calls import chain, fused, then_norm
 from .attention import FusedSelfAttention, merge_linear_keys
-from .layers import Embedding, LayerNorm, Linear, chain, then_norm
+from .layers import Embedding, LayerNorm, Linear
 
 
 @dataclass
@@ -50,9 +51,8 @@ class CLIPTextConfig:
                               num_attention_heads=2, bos_token_id=998, eos_token_id=999)
 
 
+@fused
 class CLIPMLP(nn.Module):
-    FUSED = True
-
     def __init__(self, cfg: CLIPTextConfig):
         super().__init__()
         self.act = cfg.hidden_act
@@ -66,9 +66,8 @@ class CLIPMLP(nn.Module):
         return then_norm(self.fc2, norm, self.fc1(x, act=self.act), residual=residual)
 
 
+@fused
 class CLIPEncoderLayer(nn.Module):
-    FUSED = True
-
     def __init__(self, cfg: CLIPTextConfig):
         super().__init__()
         self.layer_norm1 = LayerNorm(cfg.hidden_size, cfg.layer_norm_eps)

@@ -20,9 +20,9 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-from torch.nn.modules.module import _has_any_global_hook as _any_global_hook
 
 from .. import ops
+from ..utils.calls import as_called, fused
 
 BF16 = torch.bfloat16
 
@@ -31,42 +31,8 @@ def _round8(c: int) -> int:
     return (c + 7) // 8 * 8
 
 
-def as_called(*modules) -> bool:
-    """Whether a call of each of these modules is its class's ``forward`` and nothing else, so that a fused form may stand for the call: a
-    class that says ``FUSED`` of itself (one derived from it may have another ``forward``), no hooks, no ``forward`` of the object's."""
-    if _any_global_hook():
-        return False
-    for m in modules:
-        d = m.__dict__
-        if ("FUSED" not in type(m).__dict__ or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                or d["_backward_pre_hooks"]):
-            return False
-    return True
-
-
-def then_norm(m: nn.Module, norm: nn.Module, x, *args, residual, **kw):
-    """(y, norm(y)) of y = m(x, *args, residual=residual, **kw): in one call where nothing hooks into either."""
-    if as_called(m, norm):
-        return m.forward_norm(x, *args, residual=residual, norm=norm, **kw)
-    y = m(x, *args, residual=residual, **kw)
-    return y, norm(y)
-
-
-def chain(layers, norms, x, *args):
-    """(y, norm(y)) of y = x through ``layers``; ``norms``: the one that each layer begins with, and the one behind them all.  A layer's
-    last product makes the next layer's norm as well (``forward_next``), unless something hooks into the layer's call."""
-    n = None
-    for layer, own, following in zip(layers, norms, norms[1:]):
-        if as_called(layer):
-            x, n = layer.forward_next(x, own(x) if n is None else n, *args, next_norm=following)
-        else:
-            x, n = layer(x, *args), None
-    return x, norms[-1](x) if n is None else n
-
-
+@fused
 class Linear(nn.Module):
-    FUSED = True
-
     def __init__(self, in_features: int, out_features: int, bias: bool = True, dtype=BF16):
         super().__init__()
         self.in_features, self.out_features = in_features, out_features
@@ -81,7 +47,7 @@ class Linear(nn.Module):
         return ops.linear_stats(x, self.weight, self.bias, residual=residual, stats=stats, eps=eps)
 
     def forward_norm(self, x, residual, norm):
-        """(y, norm(y)) of y = self(x, residual=residual) -- see ``ops.linear_norm``; called by :func:`then_norm`."""
+        """(y, norm(y)) of y = self(x, residual=residual) -- see ``ops.linear_norm``; called by ``then_norm``."""
         return ops.linear_norm(x, self.weight, self.bias, residual, norm)
 
     def folded(self, ln: "LayerNorm"):
@@ -118,20 +84,22 @@ def _folded(lin, ln):
 
 
 class FoldedWeights:
-    """The weights with a LayerNorm folded in that ``module`` has by now, for a graph that reads them: :meth:`refresh`, before a replay,
-    remakes them where parameters were written since (24 projections: 6 us where none was)."""
+    """The weights with a LayerNorm folded in that ``module`` has by now, for a graph that reads them: :meth:`refresh` remakes them
+    where parameters were written since the last time, and says so (24 projections: 8 us where none was)."""
 
     def __init__(self, module: nn.Module):
         self.pairs = [(m, m._ln_fold[2]) for m in module.modules() if getattr(m, "_ln_fold", None) is not None]
         self.params = [t for m, ln in self.pairs for t in (m.weight, m.bias, ln.weight, ln.bias) if t is not None and not t.is_inference()]
         self.seen = [t._version for t in self.params]
 
-    def refresh(self):
+    def refresh(self) -> bool:
         now = [t._version for t in self.params]
-        if now != self.seen:
-            for m, ln in self.pairs:
-                m.folded(ln)
-            self.seen = now
+        if now == self.seen:
+            return False
+        for m, ln in self.pairs:
+            m.folded(ln)
+        self.seen = now
+        return True
 
 
 class GLULinear(nn.Module):
@@ -169,10 +137,9 @@ class GLULinear(nn.Module):
         return _folded(self, ln)
 
 
+@fused
 class Conv2d(nn.Module):
     """NHWC conv on the implicit-GEMM kernel. Input channels padded to a multiple of 8."""
-    FUSED = True
-
     def __init__(self, cin: int, cout: int, kernel: int, stride: int = 1, padding: int = 0, bias: bool = True,
                  dtype=BF16):
         super().__init__()
@@ -225,9 +192,8 @@ class Conv2d(nn.Module):
                           x2=x2, norm=norm, temb=temb, residual=residual, act=act, **extra)
 
 
+@fused
 class GroupNorm(nn.Module):
-    FUSED = True
-
     def __init__(self, groups: int, channels: int, eps: float = 1e-5, dtype=BF16):
         super().__init__()
         self.groups, self.channels, self.eps = groups, channels, eps
@@ -252,9 +218,10 @@ class GroupNorm(nn.Module):
         return self.weight, self.bias, self.groups, self.eps, silu
 
     def one_ok(self, x, hw: int, channels: int) -> bool:
-        """Whether this norm of [N, hw, channels], N and the device those of ``x``, runs as one launch, behind a convolution too."""
-        return (ops.groupnorm_one_ok(x, hw, channels, self.groups) and as_called(self) and ops.row_ok(self.weight, channels, 8)
-                and ops.row_ok(self.bias, channels, 8))
+        """Whether this norm of [N, hw, channels], N and the device those of ``x``, runs as one launch, behind a convolution too: that
+        one reads its parameters 8 bytes at a time."""
+        return (ops.groupnorm_one_ok(x, hw, channels, self.groups) and as_called(self)
+                and not (self.weight.data_ptr() | self.bias.data_ptr()) & 7)
 
     def forward(self, x, silu: bool = False, x2=None, part=None, part2=None):
         """GroupNorm of x, or of cat([x, x2], -1) without materialising the concat.  ``part`` / ``part2``:
@@ -267,9 +234,8 @@ class GroupNorm(nn.Module):
         return ops.groupnorm_apply(x, sc, sh, silu, x2=x2)
 
 
+@fused
 class LayerNorm(nn.Module):
-    FUSED = True
-
     def __init__(self, dim: int, eps: float = 1e-5, affine: bool = True, bias: bool = True, dtype=BF16):
         super().__init__()
         self.eps = eps
@@ -281,9 +247,8 @@ class LayerNorm(nn.Module):
         return (y, r) if residual is not None else y
 
 
+@fused
 class RMSNorm(nn.Module):
-    FUSED = True
-
     def __init__(self, dim: int, eps: float = 1e-6, dtype=BF16, w_offset: float = 0.0):
         super().__init__()
         self.eps, self.w_offset = eps, w_offset

@@ -27,8 +27,9 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..utils.calls import then_norm
 from .attention import CrossAttention, FusedSelfAttention, merge_linear_keys
-from .layers import Conv2d, GLULinear, GroupNorm, LayerNorm, Linear, _wkey, then_norm, timestep_embedding
+from .layers import Conv2d, GLULinear, GroupNorm, LayerNorm, Linear, _wkey, timestep_embedding
 
 # the last transformer block's FF down projection merged into proj_out (Transformer2DModel._merged_out)
 MERGE_PROJ_OUT = os.environ.get("SHAI_MERGE_PROJ_OUT", "1") != "0"

@@ -24,8 +24,9 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..utils.calls import as_called, chain, fused, then_norm
 from .attention import FusedSelfAttention, merge_linear_keys
-from .layers import Conv2d, LayerNorm, Linear, as_called, chain, then_norm
+from .layers import Conv2d, LayerNorm, Linear
 
 
 # LayerNorms folded into the GEMMs that consume them, moments handed over by the producing GEMM (unet2d.py);
@@ -65,9 +66,8 @@ class ViTConfig:
                          intermediate_size=128, num_labels=10, num_detection_tokens=5 if detection else 0)
 
 
+@fused
 class ViTLayer(nn.Module):
-    FUSED = True
-
     def __init__(self, c: ViTConfig):
         super().__init__()
         self.layernorm_before = LayerNorm(c.hidden_size, c.layer_norm_eps)
@@ -121,9 +121,8 @@ class ViTLayer(nn.Module):
         return self.output(self.intermediate(self.layernorm_after(x0), act=self.act), residual=x0)
 
 
+@fused
 class ViTEncoderModel(nn.Module):
-    FUSED = True
-
     def __init__(self, c: ViTConfig):
         super().__init__()
         self.cfg = c
@@ -165,7 +164,9 @@ class ViTEncoderModel(nn.Module):
         if not ops.patches_u8_ok(images, P) or not as_called(self, self.patch):
             return None
         B, H, W, _ = images.shape
-        x = ops.linear(*ops.patches_u8(images, P, mean, std, self.patch.weight), self.patch.bias)
+        cols, w = ops.patches_u8(images, P, mean, std, self.patch.weight)
+        x = ops.linear(cols, w, self.patch.bias)
+        del cols
         return self._encode(x.view(B, H // P, W // P, -1), cls_only, False)
 
     def forward(self, pixels: torch.Tensor, cls_only: bool = False, det_only: bool = False) -> torch.Tensor:
@@ -230,9 +231,8 @@ def _convert_vit_keys(sd: dict, prefix: str, n_layers: int) -> dict:
     return out
 
 
+@fused
 class ViTForImageClassification(nn.Module):
-    FUSED = True
-
     def __init__(self, cfg: ViTConfig = None):
         super().__init__()
         self.cfg = cfg or ViTConfig()

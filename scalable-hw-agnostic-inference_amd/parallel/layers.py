@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..utils.calls import fused
 from . import comm
 from .state import tp
 
@@ -85,9 +86,8 @@ class ColumnParallelLinear(_ShardLoadMixin, nn.Module):
         return comm.all_gather_last(y) if self.gather_output else y
 
 
+@fused
 class RowParallelLinear(_ShardLoadMixin, nn.Module):
-    FUSED = True
-
     def __init__(self, in_features: int, out_features: int, bias: bool = True, input_is_parallel: bool = True,
                  dtype=torch.bfloat16, one_order: bool = False):
         super().__init__()

@@ -3,10 +3,11 @@ although fused forms stand for most of them."""
 import pytest
 import torch
 
-from shai_amd import ops
 from shai_amd.models import clip, t5, unet2d, vit
 from shai_amd.models.attention import CrossAttention
-from shai_amd.models.layers import LayerNorm, Linear, as_called, init_random_, then_norm
+from shai_amd.models.layers import LayerNorm, Linear, init_random_
+from shai_amd.utils import calls as module_calls
+from shai_amd.utils.calls import as_called, then_norm
 
 
 def _rand(*shape, seed=0):
@@ -55,8 +56,7 @@ def test_hooks_run_and_change_nothing_else(name, monkeypatch):
         return [m.register_forward_hook(lambda mod, a, y, n=n: into.setdefault(n, []).append((a[0].clone(), y.clone())))
                 for n, m in model.named_modules() if isinstance(m, kinds)]
     with monkeypatch.context() as mp:      # nothing fused: the calls that there are
-        import shai_amd.models.layers as layers
-        mp.setattr(layers, "as_called", lambda *a: False)
+        mp.setattr(module_calls, "as_called", lambda *a: False)
         mp.setattr(vit, "as_called", lambda *a: False)
         handles = record(calls)
         assert torch.equal(run(), want)
@@ -123,13 +123,3 @@ def test_what_is_not_a_plain_call():
     finally:
         handle.remove()
     assert as_called(lin)
-
-
-def test_rows_that_the_one_launch_norms_read():
-    room = torch.zeros(64, dtype=torch.bfloat16)
-    at = room.data_ptr() % 16 // 2                     # elements behind an aligned address
-    row = room[(8 - at) % 8:]
-    assert ops.row_ok(None, 8) and ops.row_ok(row[:16], 16) and ops.row_ok(row[4:20], 16, 8)
-    for bad in (row[4:20], row[1:17], row[:8], row[:32:2], row[:16].float()):
-        assert not ops.row_ok(bad, 16)
-    assert not ops.row_ok(row[2:18], 16, 8)
