@@ -130,6 +130,18 @@ bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out,
   }
   std::string bk = gemm_bucket_key(g);
   if (bk.empty()) return false;
+  if (*suffix) {
+    // Shipped choices of products with a row norm are by the number of 64-row tiles: these products are one round of the chip, and
+    // how often K may be cut for one round changes inside a bucket (cold weights, 768 x 3072: 320 rows in four parts 12.3 us and two 14.1, 576 rows 15.5 and 14.4).
+    shai::GemmArgs t = g;
+    t.M = (g.M + 63) / 64 * 64;
+    it = g_tuned.find(gemm_key(t) + "|m64" + suffix);
+    if (it != g_tuned.end() && usable(it->second)) {
+      *out = it->second;
+      g_tuned[key] = it->second;
+      return true;
+    }
+  }
   bk += suffix;
   it = g_tuned.find(bk);
   if (it == g_tuned.end() || !usable(it->second)) return false;
@@ -917,7 +929,8 @@ void attach_norm_io(shai::GemmArgs& g, const optional<Tensor>& ln_mr, const opti
 }
 
 // a: [M, K] or [B, M, K]; w: [N, K] or [B, N, K]; c: [M, N'] or [B, M, N'] (N' = N or N/2 for glu)
-// y = a w^T + bias + residual and out = RMS norm or LayerNorm of y's rows.  force_cfg, for tests: 3000 + 100 * parts + tile config,
+// y = a w^T + bias + residual and out = RMS norm or LayerNorm of y's rows; a and residual [..., K] and [..., N], contiguous, or rows
+// that lie apart.  force_cfg, for tests: 3000 + 100 * parts + tile config,
 // 1000 + parts for the skinny kernel.
 void gemm_norm(const Tensor& a, const Tensor& w, const Tensor& y, const optional<Tensor>& bias, const optional<Tensor>& residual,
                const optional<Tensor>& gamma, const optional<Tensor>& beta, const Tensor& out, double eps, bool rms, int64_t force_cfg) {
@@ -925,38 +938,41 @@ void gemm_norm(const Tensor& a, const Tensor& w, const Tensor& y, const optional
   check_rows(w, "w");
   check_bf16(y, "y");
   check_bf16(out, "out");
-  SHAI_CHECK(a.dim() == 2 && w.dim() == 2 && y.dim() == 2 && a.stride(1) == 1 && w.stride(1) == 1, "gemm_norm: rows");
+  SHAI_CHECK((a.dim() == 2 || a.is_contiguous()) && w.dim() == 2, "gemm_norm: rows");
   shai::GemmArgs g{};
   g.A = cptr(a);
   g.W = cptr(w);
   g.C = mptr(y);
-  g.M = a.size(0);
-  g.K = a.size(1);
+  g.K = a.size(-1);
   g.N = w.size(0);
-  SHAI_CHECK(w.size(1) == g.K && g.K % 8 == 0 && g.N % 8 == 0 && g.N <= 8192, "gemm_norm: K and N are multiples of 8, N at most 8192");
-  SHAI_CHECK(y.size(0) == g.M && y.size(1) == g.N && y.is_contiguous() && out.sizes() == y.sizes() && out.is_contiguous(), "gemm_norm: outputs");
+  SHAI_CHECK(w.size(1) == g.K && g.K > 0 && g.K % 8 == 0 && g.N % 8 == 0 && g.N <= 8192, "gemm_norm: K and N are multiples of 8, N at most 8192");
+  g.M = a.numel() / g.K;
+  SHAI_CHECK(y.size(-1) == g.N && y.numel() == (long)g.M * g.N && y.is_contiguous() && out.sizes() == y.sizes() && out.is_contiguous(),
+             "gemm_norm: outputs");
   SHAI_CHECK(!rms || !beta, "gemm_norm: an RMS norm has no shift");
-  g.lda = a.stride(0);
+  g.lda = a.dim() == 2 ? a.stride(0) : g.K;
   g.ldw = w.stride(0);
   g.ldc = g.N;
   g.batch = 1;
   g.alpha = 1.f;
   g.res_alpha = 1.f;
   shai::FoldNormArgs n{};
+  // the norm's parameters at any address, as rmsnorm and layernorm take them: launch_then_norm asks where they lie
   auto row = [&](const optional<Tensor>& t, const char* name) -> const shai::bf16_t* {
     if (!t) return nullptr;
-    check_bf16(*t, name);
-    SHAI_CHECK(t->numel() == g.N && t->is_contiguous(), "gemm_norm: ", name);
+    SHAI_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->numel() == g.N && t->is_contiguous(), "gemm_norm: ", name);
     return cptr(*t);
   };
+  if (bias) check_bf16(*bias, "bias");
   n.bias = g.bias = row(bias, "bias");
   n.gamma = row(gamma, "gamma");
   n.beta = row(beta, "beta");
   if (residual) {
     check_bf16(*residual, "residual");
-    SHAI_CHECK(residual->dim() == 2 && residual->size(0) == g.M && residual->size(1) == g.N && residual->stride(1) == 1, "gemm_norm: residual");
+    SHAI_CHECK((residual->dim() == 2 || residual->is_contiguous()) && residual->size(-1) == g.N && residual->numel() == (long)g.M * g.N,
+               "gemm_norm: residual");
     n.residual = g.residual = cptr(*residual);
-    n.ldr = g.ldr = residual->stride(0);
+    n.ldr = g.ldr = residual->dim() == 2 ? residual->stride(0) : g.N;
   }
   n.y = g.C;
   n.out = mptr(out);

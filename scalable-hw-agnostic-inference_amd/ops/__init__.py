@@ -302,11 +302,6 @@ def stats_supported(rows: int, cols: int, kind: str, hw: Optional[int] = None) -
 LINEAR_NORM_MAX = 1 << 20
 
 
-def row_ok(t: Optional[torch.Tensor], n: int, align: int = 16) -> bool:
-    """Whether the one-launch norms read ``t`` [n] as it lies: bf16 at multiples of ``align`` bytes.  The other kernels do not ask."""
-    return t is None or (t.dtype == torch.bfloat16 and t.numel() == n and t.is_contiguous() and t.data_ptr() % align == 0)
-
-
 def linear_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], residual: torch.Tensor, norm):
     """(y, norm(y)) with y = x @ w^T + bias + residual, ``norm`` a module with ``weight``, ``bias`` (None: RMS norm) and ``eps``.
     On the GPU a small product whose K is split leaves its fold to the norm's launch."""
@@ -314,13 +309,13 @@ def linear_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     gain, shift, rms = norm.weight, getattr(norm, "bias", None), getattr(norm, "w_offset", None) is not None
     rows = residual.is_contiguous() and residual.shape[-1] == N
     if not (_gpu(x) and rows and 0 < M * N <= LINEAR_NORM_MAX and N % 8 == 0 and N <= 2048 and w.dtype == torch.bfloat16
-            and gain is not None and not getattr(norm, "w_offset", 0.0) and row_ok(gain, N) and row_ok(shift, N)):
+            and gain is not None and not getattr(norm, "w_offset", 0.0)):
         y = linear(x, w, bias, residual=residual)
         return y, norm(y)
-    x2 = x.reshape(M, -1) if (x.dim() == 2 or x.is_contiguous()) else x.contiguous().reshape(M, -1)
-    y, out = (torch.empty(M, N, dtype=x.dtype, device=x.device) for _ in range(2))
-    _K().gemm_norm(x2, w, y, bias, residual.reshape(M, N), gain, shift, out, float(norm.eps), rms)
-    return y.view(*x.shape[:-1], N), out.view(*x.shape[:-1], N)
+    y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    out = torch.empty_like(y)
+    _K().gemm_norm(x if x.dim() == 2 else x.contiguous(), w, y, bias, residual, gain, shift, out, float(norm.eps), rms)
+    return y, out
 
 
 def fold_profitable(rows: int, cols: int) -> bool:
@@ -857,7 +852,7 @@ def tokens(patches: torch.Tensor, cls: torch.Tensor, det: Optional[torch.Tensor]
     B, n, D = patches.shape
     nd = det.shape[1] if det is not None else 0
     at = [cls.reshape(-1).contiguous(), det.reshape(nd, D).contiguous() if nd else None, pos.contiguous()]
-    if not _gpu(patches) or D % 8 or D > 2048 or not all(row_ok(t, n) for t, n in zip(at, (D, nd * D, (1 + n + nd) * D))):
+    if not _gpu(patches) or D % 8 or D > 2048 or any(t is not None and t.data_ptr() % 16 for t in at):
         x = torch.cat([cls.expand(B, -1, -1), patches] + ([det.expand(B, -1, -1)] if det is not None else []), 1)
         x = bias_act(x.contiguous(), None, pos.expand(B, -1, -1).contiguous())
         return x, (row_moments(x, eps) if eps is not None else None)

@@ -116,8 +116,10 @@ def test_strides(cuda):
                 call()
 
 
-# rows for which only the plain product's choice is known, by its bucket or exactly: that one, without a tuning; else one of its own
-@pytest.mark.parametrize("M,key,cfg", [(90, 96, "|mbucket=17,2"), (91, 96, "|mbucket=3,1"), (40, 40, "=1000,3"), (92, None, None)])
+# rows for which a choice is known by their number of 64-row tiles, or only the plain product's, by its bucket or exactly: that one,
+# without a tuning; else one of its own
+@pytest.mark.parametrize("M,key,cfg", [(90, 96, "|mbucket=17,2"), (91, 96, "|mbucket=3,1"), (40, 40, "=1000,3"), (150, 192, "|m64|norm=18,2"),
+                                       (92, None, None)])
 def test_choice_of_the_plain_product(cuda, M, key, cfg):
     N, K = (328, 520) if key else (336, 520)
     name = lambda m: f"0:{m},{N},{K},b1,g0|0,0,0,0,0,0,0,0,0"  # noqa: E731
@@ -126,5 +128,5 @@ def test_choice_of_the_plain_product(cuda, M, key, cfg):
     norm, (a, w, b, r) = _norm("rms", N, cuda), _problem(M, N, K, cuda)
     y, h = ops.linear_norm(a, w, b, r, norm)
     assert _rel(y, a.float() @ w.float().t() + b.float() + r.float()) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
-    own = [e for e in ops._K().gemm_tuning_export() if e.startswith(name(M)) and "|norm" in e]
-    assert len(own) == (0 if key else 1)
+    own = [e.split("=")[1] for e in ops._K().gemm_tuning_export() if e.startswith(name(M)) and "|norm" in e]
+    assert len(own) == 1 if key is None else own == (["18,2"] if "m64" in cfg else [])
