@@ -93,3 +93,21 @@ def test_yolos_matches_transformers():
         logits, boxes = m(px.permute(0, 2, 3, 1).to(torch.bfloat16))
     assert _rel(logits, ref.logits) < 0.05
     assert _rel(boxes, ref.pred_boxes) < 0.05
+
+
+def test_shipped_choice_of_the_patch_product():
+    """ViT-base's patches of 1 to 64 images, as uint8 images come: a row bucket's or the rows' own choice, so that no call tunes it and the
+    bits of its sums do not change from one process to the next."""
+    import json
+    import os
+
+    from shai_amd.models.vit import ViTConfig
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "config", "gemm_tuning_mi355x.json")
+    with open(path) as f:
+        shipped = {e.split("=")[0] for e in json.load(f)}
+    c = ViTConfig.vit_base()
+    key = lambda m: f"0:{m},{c.hidden_size},{c.patch_size ** 2 * 3},b1,g0|0,0,0,0,0,0,0,0,0|lib"  # noqa: E731
+    buckets = sorted(b for p in range(6, 20) for b in (1 << p, 3 << (p - 1)))
+    for images in range(1, 65):
+        m = images * (c.image_size[0] // c.patch_size) * (c.image_size[1] // c.patch_size)
+        assert key(m) in shipped or key(min(b for b in buckets if b >= m)) + "|mbucket" in shipped, images
