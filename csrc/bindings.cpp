@@ -132,7 +132,8 @@ bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out,
   if (bk.empty()) return false;
   if (*suffix) {
     // Shipped choices of products with a row norm are by the number of 64-row tiles: these products are one round of the chip, and
-    // how often K may be cut for one round changes inside a bucket (cold weights, 768 x 3072: 320 rows in four parts 12.3 us and two 14.1, 576 rows 15.5 and 14.4).
+    // how often K may be cut for one round changes inside a bucket (768 x 3072, cold weights: 320 rows in four parts 12.3 us and in
+    // two 14.1, 576 rows 15.5 and 14.4).
     shai::GemmArgs t = g;
     t.M = (g.M + 63) / 64 * 64;
     it = g_tuned.find(gemm_key(t) + "|m64" + suffix);
@@ -930,8 +931,7 @@ void attach_norm_io(shai::GemmArgs& g, const optional<Tensor>& ln_mr, const opti
 
 // a: [M, K] or [B, M, K]; w: [N, K] or [B, N, K]; c: [M, N'] or [B, M, N'] (N' = N or N/2 for glu)
 // y = a w^T + bias + residual and out = RMS norm or LayerNorm of y's rows; a and residual [..., K] and [..., N], contiguous, or rows
-// that lie apart.  force_cfg, for tests: 3000 + 100 * parts + tile config,
-// 1000 + parts for the skinny kernel.
+// that lie apart.  force_cfg, for tests: 3000 + 100 * parts + tile config, 1000 + parts for the skinny kernel.
 void gemm_norm(const Tensor& a, const Tensor& w, const Tensor& y, const optional<Tensor>& bias, const optional<Tensor>& residual,
                const optional<Tensor>& gamma, const optional<Tensor>& beta, const Tensor& out, double eps, bool rms, int64_t force_cfg) {
   check_rows(a, "a");   // the tiles read 16 bytes at a time
