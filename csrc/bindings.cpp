@@ -201,8 +201,10 @@ constexpr int kSkinnyFixCfg = 1100;
 constexpr int kSkinny2Cfg = 1200;
 // the same kernel with a 6-stage ring (one workgroup per CU, deeper prefetch)
 constexpr int kSkinny2DeepCfg = 1250;
+// Choice.cfg of the skinny kernel without a split over workgroups (csrc/kernels/gemv3.hip); Choice.splits = 1
+constexpr int kSkinny3Cfg = 1300;
 inline bool is_skinny2(int cfg) { return cfg == kSkinny2Cfg || cfg == kSkinny2DeepCfg; }
-inline bool is_skinny(int cfg) { return cfg == kSkinnyCfg || cfg == kSkinnyFixCfg || is_skinny2(cfg); }
+inline bool is_skinny(int cfg) { return cfg == kSkinnyCfg || cfg == kSkinnyFixCfg || cfg == kSkinny3Cfg || is_skinny2(cfg); }
 
 // Last resort when neither the tuner nor the planner produced a usable config: an explicit, directly tested
 // config, never "whichever kernel happens to be numbered highest".  The v2 128x64 tile (cfg 4) runs every
@@ -273,6 +275,10 @@ void launch_choice(const shai::GemmArgs& g, const Tensor& like, Choice c) {
     // falls back to the planner's tile config
     shai::gemm2_plan(g, &c.cfg, &c.splits);
     if (!shai::gemm2_cfg_supported(g, c.cfg)) c = fallback_choice(g);
+  }
+  if (c.cfg == kSkinny3Cfg && shai::skinny3_supported(g)) {
+    shai::launch_skinny3(g, stream());
+    return;
   }
   if (is_skinny2(c.cfg) && shai::skinny2_supported(g)) {
     launch_skinny2_choice(g, like, c.splits, c.cfg == kSkinny2DeepCfg);
@@ -386,6 +392,7 @@ Choice tune(const shai::GemmArgs& g_real, const Tensor& like, bool skinny_only =
       cands.push_back({kSkinny2Cfg, kg});
       cands.push_back({kSkinny2DeepCfg, kg});
     }
+  if (shai::skinny3_supported(g)) cands.push_back({kSkinny3Cfg, 1});
   // residual epilogues are in place (C aliases the residual): timing them into the scratch output is not
   // equivalent, so only bias-or-nothing problems race the library
   if (!skinny_only && lib_enabled() && lib_supported(g_real) && !g_real.residual && !shai::keeps_order(g)) cands.push_back({kLibCfg, 1});
@@ -1094,16 +1101,19 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
   // tests / tools bypass the tuner: force_cfg = gemm2 config, 1000 = skinny kernel (heuristic K groups),
   // 1000 + kg = skinny kernel with kg K groups (separate fold), 1100 + kg = the same with the in-kernel fixup
   // 1200 + kg = the wide skinny kernel (gemv2.hip) with kg K groups (in-kernel fixup), 1250 + kg its 6-stage form
-  const bool force_s2d = force_cfg > kSkinny2DeepCfg && force_cfg < kLibCfg;
-  const bool force_s2 = force_cfg > kSkinny2Cfg && force_cfg < kLibCfg;
+  // 1300 = the skinny kernel without a split over workgroups (gemv3.hip)
+  const bool force_s3 = force_cfg == kSkinny3Cfg;
+  const bool force_s2d = force_cfg > kSkinny2DeepCfg && force_cfg < kSkinny3Cfg;
+  const bool force_s2 = force_cfg > kSkinny2Cfg && force_cfg < kSkinny3Cfg;
   const bool force_skinny = force_cfg >= kSkinnyCfg && force_cfg != kLibCfg;
-  const bool force_fix = force_cfg > kSkinnyFixCfg && force_cfg != kLibCfg && !force_s2;
-  const int force_kg = force_s2d  ? (int)(force_cfg - kSkinny2DeepCfg)
+  const bool force_fix = force_cfg > kSkinnyFixCfg && force_cfg != kLibCfg && !force_s2 && !force_s3;
+  const int force_kg = force_s3    ? 1
+                       : force_s2d ? (int)(force_cfg - kSkinny2DeepCfg)
                        : force_s2 ? (int)(force_cfg - kSkinny2Cfg)
                        : force_fix ? (int)(force_cfg - kSkinnyFixCfg)
                        : force_cfg > kSkinnyCfg ? (int)(force_cfg - kSkinnyCfg)
                                                 : shai::skinny_kgroups(g);
-  const int force_skcfg = force_s2d ? kSkinny2DeepCfg : force_s2 ? kSkinny2Cfg : force_fix ? kSkinnyFixCfg : kSkinnyCfg;
+  const int force_skcfg = force_s3 ? kSkinny3Cfg : force_s2d ? kSkinny2DeepCfg : force_s2 ? kSkinny2Cfg : force_fix ? kSkinnyFixCfg : kSkinnyCfg;
   if (rms_eps >= 0) {
     // RMSNorm(a) folded in (norm gain pre-multiplied into w): fused into the skinny kernel for
     // decode-shaped problems, otherwise an explicit unweighted RMSNorm pass feeds the GEMM.
@@ -1166,7 +1176,7 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
   }
   if (force_cfg >= 0) {
     if (force_skinny) {
-      SHAI_CHECK((force_s2 ? shai::skinny2_supported(g) : shai::skinny_supported(g)) && force_kg >= 1 &&
+      SHAI_CHECK((force_s3 ? shai::skinny3_supported(g) : force_s2 ? shai::skinny2_supported(g) : shai::skinny_supported(g)) && force_kg >= 1 &&
                      force_kg <= 64,
                  "skinny kernel does not support this problem");
       launch_choice(g, a, Choice{force_skcfg, force_kg});

@@ -255,6 +255,9 @@ unsigned* skinny_ticket_slice(hipStream_t s, int ntiles);
 // skinny2 (gemv2.hip): 128-row W tiles, whole K-step per wave, M <= 64, bf16 weights; split-K always fixed up
 // in the launch (ws of skinny2_workspace_bytes)
 bool skinny2_supported(const GemmArgs& a);
+// skinny3 (gemv3.hip): M <= 16, 16 weight rows a workgroup with all of K
+bool skinny3_supported(const GemmArgs& a);
+void launch_skinny3(const GemmArgs& a, hipStream_t s);
 int skinny2_max_kgroups(const GemmArgs& a);
 size_t skinny2_workspace_bytes(const GemmArgs& a, int kg);
 void launch_skinny2(const GemmArgs& a, float* ws, int kg, bool deep, hipStream_t s);

@@ -424,3 +424,22 @@ def test_skinny2_glu_residual_and_graph(cuda, cfg):
         g.replay()
         torch.cuda.synchronize()
         assert _rel(o2, x.float() @ w.float().t()) < 1e-2
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4, 8), (1, 16, 64), (2, 20, 72), (15, 100, 520), (16, 1000, 1016), (16, 768, 3072), (3, 4096, 4096)])
+@pytest.mark.parametrize("act,extra", [(None, False), ("silu", True), ("quick_gelu", False)])
+def test_skinny_whole_k(cuda, M, N, K, act, extra):
+    """The kernel without a split over workgroups (force_cfg 1300): one row and all 16, K that ends inside a unit of 64, in fewer units than
+    there are waves and in more than the ring holds, columns that end inside a workgroup; rows that lie apart.  The result is the fp32 one
+    but for one rounding to bf16 (2^-9) and the order of its sums."""
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device=cuda).bfloat16()[:, :K]
+    w = (torch.randn(N, K, device=cuda) / K ** 0.5).bfloat16()
+    b, r = (torch.randn(*s, device=cuda).bfloat16() if extra else None for s in ((N,), (M, N)))
+    out = torch.full((M, N + 4), 7.0, device=cuda, dtype=torch.bfloat16)
+    ops.gemm_into(x, w, out[:, :N], b, act=act, residual=r, force_cfg=1300)
+    y = x.double() @ w.double().t() + (b.double() if extra else 0)
+    y = {None: lambda t: t, "silu": torch.nn.functional.silu, "quick_gelu": lambda t: t * torch.sigmoid(1.702 * t)}[act](y)
+    y = y + (r.double() if extra else 0)
+    assert (out[:, :N].double() - y).abs().max() <= 2 ** -8 * max(1.0, float(y.abs().max()))
+    assert _rel(out[:, :N], y) < 2 ** -8 and (out[:, N:] == 7.0).all()
