@@ -1,0 +1,56 @@
+// A decode step of a layer's two mixers in one launch: attention over a paged cache (attn_decode.h) and the delta rule (rule_rows.h),
+// which read different columns of the layer's rows and write different columns of its outputs.
+//
+// One after the other, an attention of a few workgroups waits for its chain of loads (block table, keys, values: 11.6 us for 132 keys and
+// one sequence, 15.2 for 64 sequences, 0.25 to 1.3 TB/s), and then the recurrence begins.  Here the attention's workgroups are the first of
+// the grid, so that their chains start at once, and the recurrence's, bound by the state's traffic, take the rest of the chip.
+#include "attn_decode.h"
+#include "rule_rows.h"
+
+namespace shai_lm {
+
+template <int D, int RH, int MODE, int SD>
+__global__ void __launch_bounds__(256, 3) attn_rule_kernel(const AttnArgs a, const RuleArgs r, int per_group, int heads, int n_attn) {
+  const int i = blockIdx.x;
+  if (i < n_attn) {
+    const int j = i / heads;
+    attn_decode<D, D, RH, true>(a, per_group, 1, i - j * heads, j % a.B, j / a.B);
+  } else {
+    const int b = (i - n_attn) / r.H;
+    rule_rows<bf16_t, MODE, SD, SD, 256, true>(r, i - n_attn - b * r.H, b);
+  }
+}
+
+template <int D, int RH, int MODE, int SD>
+static void attn_rule(const AttnArgs& a, const RuleArgs& r, hipStream_t s) {
+  const int n_attn = a.G * a.B * a.splits;
+  attn_rule_kernel<D, RH, MODE, SD><<<n_attn + r.H * r.B, 256, 0, s>>>(a, r, a.H / a.G, a.G, n_attn);
+}
+
+template <int D, int RH>
+static void attn_rule(const AttnArgs& a, const RuleArgs& r, hipStream_t s) {
+  if (r.mode == kHead) r.dk == 64 ? attn_rule<D, RH, kHead, 64>(a, r, s) : attn_rule<D, RH, kHead, 128>(a, r, s);
+  else r.dk == 64 ? attn_rule<D, RH, kChannel, 64>(a, r, s) : attn_rule<D, RH, kChannel, 128>(a, r, s);
+}
+
+// The head sizes and groups whose registers fit the recurrence's three workgroups a CU; others run one after the other.
+static bool fits(const AttnArgs& a, const RuleArgs& r) {
+  const long grid = (long)a.G * a.B * a.splits + (long)r.H * r.B;
+  return a.own_kv && a.rope && a.H / a.G <= 8 && a.dk == a.dv && a.dk <= 128 && r.mode != kRetention && r.dk == r.dv && r.dk <= 128 &&
+         r.q_lens == nullptr && grid <= 0x7fffffffL;
+}
+
+void launch_attn_beside_rule(const AttnArgs& a, const RuleArgs& r, bool f32, hipStream_t s) {
+  if (f32 || !fits(a, r)) {
+    launch_attn_decode(a, f32, s);
+    launch_rule_rows(r, f32, s);
+    return;
+  }
+  const bool few = a.H / a.G <= 4;
+  if (a.dk == 64) few ? attn_rule<64, 4>(a, r, s) : attn_rule<64, 8>(a, r, s);
+  else few ? attn_rule<128, 4>(a, r, s) : attn_rule<128, 8>(a, r, s);
+  if (a.splits > 1) launch_attn_decode_fold(a, s);
+  SHAI_CHECK_LAUNCH();
+}
+
+}  // namespace shai_lm

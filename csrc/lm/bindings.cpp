@@ -1115,12 +1115,12 @@ void gated_attn_prefill(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, 
   shai_lm::launch_attn_prefill(a, is_f32(qkvg), stream());
 }
 
-void gated_attn_decode(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, const Tensor& o, const Tensor& bt,
-                       const Tensor& ctx, const Tensor& slots, const Tensor& ws, int64_t heads, int64_t splits,
-                       int64_t chunk, double scale, bool window, bool per_element, bool own_kv,
-                       const optional<Tensor>& rope, int64_t dim, double eps, const optional<Tensor>& q_gain,
-                       const optional<Tensor>& k_gain, const optional<Tensor>& temp, const optional<Tensor>& sink,
-                       double out_scale) {
+shai_lm::AttnArgs decode_args(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, const Tensor& o, const Tensor& bt,
+                              const Tensor& ctx, const Tensor& slots, const Tensor& ws, int64_t heads, int64_t splits,
+                              int64_t chunk, double scale, bool window, bool per_element, bool own_kv,
+                              const optional<Tensor>& rope, int64_t dim, double eps, const optional<Tensor>& q_gain,
+                              const optional<Tensor>& k_gain, const optional<Tensor>& temp, const optional<Tensor>& sink,
+                              double out_scale) {
   shai_lm::AttnArgs a = attn_args(qkvg, kc, vc, &o, heads, per_element, own_kv, sink.has_value());
   set_turn(a, rope, dim, eps, q_gain, k_gain);
   set_ungated(a, temp, sink, out_scale);
@@ -1141,7 +1141,34 @@ void gated_attn_decode(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, c
   a.chunk = std::min<int64_t>(chunk, 1 << 30);
   a.window = window;
   a.scale = scale;
+  return a;
+}
+
+void gated_attn_decode(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, const Tensor& o, const Tensor& bt,
+                       const Tensor& ctx, const Tensor& slots, const Tensor& ws, int64_t heads, int64_t splits,
+                       int64_t chunk, double scale, bool window, bool per_element, bool own_kv,
+                       const optional<Tensor>& rope, int64_t dim, double eps, const optional<Tensor>& q_gain,
+                       const optional<Tensor>& k_gain, const optional<Tensor>& temp, const optional<Tensor>& sink,
+                       double out_scale) {
+  const shai_lm::AttnArgs a = decode_args(qkvg, kc, vc, o, bt, ctx, slots, ws, heads, splits, chunk, scale, window, per_element,
+                                          own_kv, rope, dim, eps, q_gain, k_gain, temp, sink, out_scale);
   shai_lm::launch_attn_decode(a, is_f32(qkvg), stream());
+}
+
+// Attention without gates and the delta rule of one decode step: the arguments of gated_attn_decode, then those of rule_rows.
+void attn_beside_rule(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, const Tensor& o, const Tensor& bt, const Tensor& ctx,
+                      const Tensor& slots, const Tensor& ws, int64_t heads, int64_t splits, int64_t chunk, double scale,
+                      const Tensor& rope, int64_t dim, double eps, const optional<Tensor>& q_gain, const optional<Tensor>& k_gain,
+                      const Tensor& temp, const Tensor& sink, double out_scale, const Tensor& x, const Tensor& gate,
+                      const Tensor& state, const Tensor& out, const Tensor& pos, const Tensor& state_slots, int64_t kv_heads,
+                      int64_t rule_dim, int64_t vdim, int64_t gate_kind, double rule_eps, const Tensor& rate, const Tensor& decay,
+                      const Tensor& beta, const Tensor& conv, const Tensor& bias, const Tensor& gain, const Tensor& ring) {
+  const shai_lm::AttnArgs a = decode_args(qkvg, kc, vc, o, bt, ctx, slots, ws, heads, splits, chunk, scale, true, false, true, rope,
+                                          dim, eps, q_gain, k_gain, temp, sink, out_scale);
+  const shai_lm::RuleArgs r = rule_args(x, gate, state, out, pos, state_slots, kv_heads, rule_dim, vdim, gate_kind, rule_eps, rate,
+                                        decay, beta, conv, bias, gain, ring, c10::nullopt, c10::nullopt, c10::nullopt);
+  SHAI_CHECK(a.T == r.T && qkvg.scalar_type() == x.scalar_type(), "attention and delta rule: rows of one step");
+  if (a.T > 0) shai_lm::launch_attn_beside_rule(a, r, is_f32(qkvg), stream());
 }
 
 void sample(const Tensor& logits, const Tensor& temps, const Tensor& top_k, const Tensor& top_p,
@@ -1201,6 +1228,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("ring_commit(Tensor x, Tensor(a!) ring, Tensor pos, Tensor q_start, Tensor q_lens, Tensor slots) -> ()");
   m.def("gated_attn_prefill(Tensor qkvg, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor ctx_lens, Tensor q_lens, Tensor q_start, int max_q, int heads, int chunk, float scale, bool window=False, bool per_element=False, bool own_kv=True, Tensor? temp=None, Tensor? sink=None, float out_scale=1.) -> ()");
   m.def("gated_attn_decode(Tensor qkvg, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, Tensor ctx_lens, Tensor slots, Tensor(d!) ws, int heads, int splits, int chunk, float scale, bool window=False, bool per_element=False, bool own_kv=True, Tensor? rope=None, int dim=0, float eps=0., Tensor? q_gain=None, Tensor? k_gain=None, Tensor? temp=None, Tensor? sink=None, float out_scale=1.) -> ()");
+  m.def("attn_beside_rule(Tensor qkvg, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, Tensor ctx_lens, Tensor slots, Tensor(d!) ws, int heads, int splits, int chunk, float scale, Tensor rope, int dim, float eps, Tensor? q_gain, Tensor? k_gain, Tensor temp, Tensor sink, float out_scale, Tensor x, Tensor gate, Tensor(e!) state, Tensor(f!) out, Tensor pos, Tensor state_slots, int kv_heads, int rule_dim, int vdim, int gate_kind, float rule_eps, Tensor rate, Tensor decay, Tensor beta, Tensor conv, Tensor bias, Tensor gain, Tensor(g!) ring) -> ()");
   m.def("sample(Tensor logits, Tensor temps, Tensor top_k, Tensor top_p, Tensor uniforms, Tensor(a!) out) -> ()");
   m.def("token_feedback(Tensor(a!) ids, Tensor rowmap, Tensor prev) -> ()");
 }
@@ -1230,6 +1258,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("ring_commit", &ring_commit);
   m.impl("gated_attn_prefill", &gated_attn_prefill);
   m.impl("gated_attn_decode", &gated_attn_decode);
+  m.impl("attn_beside_rule", &attn_beside_rule);
   m.impl("sample", &sample);
   m.impl("token_feedback", &token_feedback);
 }

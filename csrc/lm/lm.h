@@ -202,6 +202,7 @@ void launch_kv_store(const AttnArgs& a, bool f32, hipStream_t s);
 void launch_head_prep(const AttnArgs& a, bool f32, hipStream_t s);     // q in place, k (turned, normed) and v to the cache
 void launch_attn_prefill(const AttnArgs& a, bool f32, hipStream_t s);
 void launch_attn_decode(const AttnArgs& a, bool f32, hipStream_t s);
+void launch_attn_decode_fold(const AttnArgs& a, hipStream_t s);        // joins the splits of a bf16 decode step
 void launch_latent_prefill(const AttnArgs& a, hipStream_t s);          // bf16
 
 struct LatentPrepArgs {
@@ -308,6 +309,7 @@ struct RuleArgs {          // delta rule (mode 1: a decay per head, 2: per key c
 };
 void launch_rule_rows(const RuleArgs& a, bool f32, hipStream_t s);     // row by row
 void launch_rule_chunks(const RuleArgs& a, hipStream_t s);             // bf16, 32 rows at a time; heads head0 .. of a prefill step
+void launch_attn_beside_rule(const AttnArgs& a, const RuleArgs& r, bool f32, hipStream_t s);   // a decode step of both (beside.hip)
 // workspace of one chunk of `heads` heads and `keys` heads of queries and keys (those of every head with a decay per channel)
 long rule_chunk_bytes(int dk, int dv, int heads, int keys, bool channel);
 // workspace of a segment of `heads` heads

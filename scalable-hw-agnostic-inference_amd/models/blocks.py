@@ -14,6 +14,7 @@ import torch
 import torch.nn as nn
 
 from ..ops import lm
+from ..utils.calls import as_called, fused
 
 
 def _param(*shape, dtype):
@@ -747,11 +748,17 @@ class JointLayer(nn.Module):
         n = self.out_cols + self.fp
         rows = torch.empty(h.shape[0], n + self.in_rows, dtype=h.dtype, device=h.device)
         side = lm.matmul_joint(h, self.w_in, rows[:, self.out_cols:], self.fp, self.side_rows)
+        mixers, args = list(self.mixers.values()), []
         i, s, o = n, 0, 0
-        for m in self.mixers.values():
-            m(rows[:, i:i + m.in_rows], side[:, s:s + m.side_rows] if m.side_rows else None, rows[:, o:o + m.out_cols], batch,
-              cache if m.cached else state, step)
+        for m in mixers:
+            args.append((rows[:, i:i + m.in_rows], side[:, s:s + m.side_rows] if m.side_rows else None, rows[:, o:o + m.out_cols]))
             i, s, o = i + m.in_rows, s + m.side_rows, o + m.out_cols
+        if not batch.is_prefill and [type(m) for m in mixers] == [TiedAttention, DeltaRule] and as_called(*mixers):
+            (x, _, out), rule = args[0], mixers[1].step_of(*args[1], state)
+            mixers[0].beside(x, out, batch, cache, step, rule)
+        else:
+            for m, a in zip(mixers, args):
+                m(*a, batch, cache if m.cached else state, step)
         return lm.matmul_parts(rows[:, :n], self.w_out)
 
     def cache_shapes(self, blocks: int, block: int):
@@ -781,6 +788,7 @@ class TiedAttentionConfig:
             raise ValueError(f"bad attention sizes: {self}")
 
 
+@fused
 class TiedAttention(nn.Module):
     """Causal attention whose values are the projected keys: queries and keys rms-normed per head with a gain and then rotated
     (half against half), a factor per head on the scores, a learned sink per head in the denominator."""
@@ -816,11 +824,17 @@ class TiedAttention(nn.Module):
     def pack_out(self, get):
         return _head_columns(get("o"), self.c.heads, self.c.dim, self.dk, lm.pad64(self.width))
 
-    def forward(self, x, side, out, batch, cache, step):
+    def _forms(self, out, step):
         c = self.c
-        lm.gated_attention(x, *cache, batch, c.heads, lm.WHOLE, c.scale, window=True,
-                           turn=lm.HeadTurn(step.rope(self), c.dim, self.eps, self.q_gain, self.k_gain),
-                           plain=lm.Ungated(self.temp, self.sink, out, c.out_scale))
+        return dict(turn=lm.HeadTurn(step.rope(self), c.dim, self.eps, self.q_gain, self.k_gain),
+                    plain=lm.Ungated(self.temp, self.sink, out, c.out_scale))
+
+    def forward(self, x, side, out, batch, cache, step):
+        lm.gated_attention(x, *cache, batch, self.c.heads, lm.WHOLE, self.c.scale, window=True, **self._forms(out, step))
+
+    def beside(self, x, out, batch, cache, step, rule: lm.RuleStep):
+        """``forward`` and a delta rule of the same decode step."""
+        lm.attention_beside_rule(x, *cache, batch, self.c.heads, lm.WHOLE, self.c.scale, rule=rule, **self._forms(out, step))
 
     def cache_shapes(self, blocks: int, block: int):
         return ((blocks, self.c.kv_heads, block, self.dk),) * 2
@@ -848,6 +862,7 @@ class DeltaRuleConfig:
             raise ValueError(f"short convolutions of 1 to {lm.MAX_TAPS} taps are supported, got {self.taps}")
 
 
+@fused
 class DeltaRule(nn.Module):
     """Linear attention whose matrix state per head is decayed (per head, or per key channel) and written by the delta rule;
     queries, keys and values pass a short convolution and silu, queries and keys are unit vectors, every head's output is
@@ -917,13 +932,17 @@ class DeltaRule(nn.Module):
     def pack_out(self, get):
         return _head_columns(get("o"), self.c.heads, self.c.vdim, self.dv, lm.pad64(self.width))
 
-    def forward(self, x, side, out, batch, state, step):
+    def step_of(self, x, side, out, state) -> lm.RuleStep:
         H, n = self.c.heads, self.channels
         gate, decay = x[:, n:], side[:, H:]
         if self.low:
             gate, decay = lm.matmul_with_side(gate, self.up, H * self.dk)
-        lm.delta_rule(x[:, :n], gate, decay, side[:, :H], self.conv, self.rate, self.bias, self.gain, *state, batch, out,
-                      self.shape, self.eps)
+        return lm.RuleStep(x[:, :n], gate, decay, side[:, :H], self.conv, self.rate, self.bias, self.gain, *state, out, self.shape,
+                           self.eps)
+
+    def forward(self, x, side, out, batch, state, step):
+        r = self.step_of(x, side, out, state)
+        lm.delta_rule(r.x, r.gate, r.decay, r.beta, r.conv, r.rate, r.bias, r.gain, r.state, r.ring, batch, r.out, r.shape, r.eps)
 
     def state_shapes(self):
         return [((self.c.heads, self.dk, self.dv), True), ((self.c.taps, self.channels), False)]

@@ -276,6 +276,10 @@ class Ungated:
     out_scale: float = 1.0
 
 
+def _decode_splits(batch, size: int) -> int:
+    return max(1, min(int(batch.num_splits or 1), (size + 63) // 64, 64))
+
+
 def gated_attention(qkvg, k_cache, v_cache, batch, heads: int, size: int, scale: float, window: bool = False,
                     per_element: bool = False, own_kv: bool = True, turn: Optional[HeadTurn] = None,
                     plain: Optional[Ungated] = None):
@@ -308,12 +312,48 @@ def gated_attention(qkvg, k_cache, v_cache, batch, heads: int, size: int, scale:
                                 batch.q_start, int(batch.S), int(heads), int(size), float(scale), window, per_element, own_kv,
                                 **more)
         return o
-    ns = max(1, min(int(batch.num_splits or 1), (size + 63) // 64, 64))
+    ns = _decode_splits(batch, size)
     ws = torch.empty(T * heads * ns * (dv + 2) if ns > 1 else 0, dtype=torch.float32, device=qkvg.device)
     _K().gated_attn_decode(qkvg, k_cache, v_cache, o, batch.block_table, batch.ctx_lens, batch.slots, ws, int(heads),
                            ns, int(size), float(scale), window, per_element, own_kv,
                            *(turn and (turn.rope, int(turn.dim), float(turn.eps)) or ()), **gains, **more)
     return o
+
+
+@dataclass
+class RuleStep:
+    """The arguments of :func:`delta_rule` but the step's batch."""
+    x: torch.Tensor
+    gate: torch.Tensor
+    decay: torch.Tensor
+    beta: torch.Tensor
+    conv: torch.Tensor
+    rate: torch.Tensor
+    bias: torch.Tensor
+    gain: torch.Tensor
+    state: torch.Tensor
+    ring: torch.Tensor
+    out: torch.Tensor
+    shape: "RuleShape"
+    eps: float
+
+
+def attention_beside_rule(qk, k_cache, v_cache, batch, heads: int, size: int, scale: float, turn: HeadTurn, plain: Ungated,
+                          rule: RuleStep) -> None:
+    """:func:`gated_attention` in a window without gates and :func:`delta_rule` of one decode step: neither reads what the other
+    writes, and on the GPU they are one launch."""
+    if not qk.is_cuda or batch.is_prefill:
+        gated_attention(qk, k_cache, v_cache, batch, heads, size, scale, window=True, turn=turn, plain=plain)
+        delta_rule(rule.x, rule.gate, rule.decay, rule.beta, rule.conv, rule.rate, rule.bias, rule.gain, rule.state, rule.ring, batch,
+                   rule.out, rule.shape, rule.eps)
+        return
+    ns = _decode_splits(batch, size)
+    ws = torch.empty(qk.shape[0] * heads * ns * (v_cache.shape[3] + 2) if ns > 1 else 0, dtype=torch.float32, device=qk.device)
+    _K().attn_beside_rule(qk, k_cache, v_cache, plain.out, batch.block_table, batch.ctx_lens, batch.slots, ws, int(heads), ns, int(size),
+                          float(scale), turn.rope, int(turn.dim), float(turn.eps), turn.q_gain, turn.k_gain, plain.temp, plain.sink,
+                          float(plain.out_scale), rule.x, rule.gate, rule.state, rule.out, batch.positions, batch.state_slots,
+                          int(rule.shape.kv_heads), int(rule.shape.dim), int(rule.shape.vdim), int(rule.shape.gate), float(rule.eps),
+                          rule.rate, rule.decay, rule.beta, rule.conv, rule.bias, rule.gain, rule.ring)
 
 
 def chunk_attention(qkvg, k_cache, v_cache, batch, heads: int, chunk: int, scale: float):

@@ -85,3 +85,51 @@ def test_prompts_in_segments(cuda, monkeypatch, rows):
     monkeypatch.setattr(C.lm, "rule_segment", lambda *_: rows)
     for check in (C.check_delta, C.check_delta_memory, C.check_retention, C.check_mixers):
         check(cuda, torch.bfloat16)
+
+
+@pytest.mark.parametrize("B,H,G,d,rule,channels,splits", [
+    (1, 4, 1, 128, (4, 2, 128), True, 1), (3, 8, 1, 64, (2, 1, 64), False, 2), (5, 2, 2, 64, (3, 3, 128), True, 1),
+    (2, 12, 1, 64, (2, 2, 64), True, 1), (64, 16, 4, 128, (16, 16, 128), True, 1), (1, 4, 4, 128, (2, 2, 256), False, 1)])
+def test_mixers_of_a_step_in_one_launch(cuda, B, H, G, d, rule, channels, splits):
+    """Attention and delta rule together against one after the other: caches, states and both outputs.  Groups and head sizes that the one
+    launch takes and that it does not (12 heads to a group, heads of 256); contexts of one key, of whole blocks and past them; sequences
+    without a slot.  The sums are the same in the same order, compiled twice: a last bit of the bf16 outputs, 2^-16 of the fp32 states."""
+    from types import SimpleNamespace
+    lm, (R, K, s) = C.lm, rule
+    g = torch.Generator(device=cuda).manual_seed(B * H + s)
+    rand = lambda *shape, dtype=torch.bfloat16: torch.randn(*shape, generator=g, device=cuda).to(dtype)
+    i32 = lambda t: torch.tensor(t, dtype=torch.int32, device=cuda)
+    lens = [(1, 64, 65, 200, 7)[i % 5] for i in range(B)]
+    blocks, ch = 4, 2 * K * s + R * s
+    batch = SimpleNamespace(is_prefill=False, num_splits=splits, ctx_lens=i32(lens), positions=i32([n - 1 for n in lens]),
+                            block_table=i32([[b * blocks + j for j in range(blocks)] for b in range(B)]),
+                            slots=i32([-1 if b == 4 else b * blocks * 64 + n - 1 for b, n in enumerate(lens)]),
+                            state_slots=i32([-1 if b == 4 else B - 1 - b for b in range(B)]))
+    rows = rand(B, (H + G) * d + ch + R * s)
+    caches = [rand(B * blocks, G, 64, d) for _ in range(2)]
+    state, ring = rand(B, R, s, s, dtype=torch.float32), rand(B, 4, ch)
+    turn = lm.HeadTurn(lm.rope_rows(batch.positions, lm.rope_freq(1e4, d // 2).to(cuda)), d, 1e-6, rand(d, dtype=torch.float32),
+                       rand(d, dtype=torch.float32))
+    f32 = dict(dtype=torch.float32)
+    decay, beta = rand(B, R * (s if channels else 1), **f32), rand(B, R, **f32)
+    conv, rate, bias, gain = rand(4, ch, **f32), rand(R, **f32).exp(), rand(decay.shape[1], **f32), rand(s, **f32)
+    temp, sink = rand(H, **f32), rand(H, **f32)
+
+    def run(together):
+        out = torch.zeros(B, H * d + R * s, dtype=torch.bfloat16, device=cuda)
+        kc, vc, st, rg = caches[0].clone(), caches[1].clone(), state.clone(), ring.clone()
+        r = lm.RuleStep(rows[:, (H + G) * d:(H + G) * d + ch], rows[:, (H + G) * d + ch:], decay, beta, conv, rate, bias, gain, st, rg,
+                        out[:, H * d:], lm.RuleShape(K, s, s), 1e-6)
+        a = (rows[:, :(H + G) * d], kc, vc, batch, H, lm.WHOLE, d ** -0.5)
+        plain = lm.Ungated(temp, sink, out[:, :H * d], 0.7)
+        if together:
+            lm.attention_beside_rule(*a, turn=turn, plain=plain, rule=r)
+        else:
+            lm.gated_attention(*a, window=True, turn=turn, plain=plain)
+            lm.delta_rule(r.x, r.gate, r.decay, r.beta, r.conv, r.rate, r.bias, r.gain, r.state, r.ring, batch, r.out, r.shape, r.eps)
+        return out, kc, vc, st, rg
+    one, two = run(True), run(False)
+    for i, (a, b) in enumerate(zip(one, two)):
+        assert torch.isfinite(b.float()).all()
+        assert (a.float() - b.float()).norm() <= (2 ** -16 if a.dtype == torch.float32 else 2 ** -9) * b.float().norm(), i
+    assert torch.equal(one[2], two[2]) and torch.equal(one[4], two[4])
