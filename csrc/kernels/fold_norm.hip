@@ -1,10 +1,11 @@
 // Fold of split-K partial sums, residual and the next row norm in one launch.
 //
 // A layer of a small batch is a chain of launches that cost 3.5 to 4.5 us each whatever they do: a product whose K is split over
-// workgroups, its fold, the norm of the result, the next product.  The fold and the norm read some hundred KB; here a wave takes
-// a row, all its loads issued before the first addition, and the row never leaves its registers between the two.
-// 154 x 1024 x 4096: product, fold and norm 13.9 us -> 10.9, 197 x 768 x 3072 13.5 -> 10.2, 32 x 768 x 3072 11.6 -> 8.6, 512 x 1280 x 5120 25.2 ->
-// 21.3; where K was not split before, splitting it pays now: 197 x 768 x 768 8.6 -> 7.9, 32 x 768 x 768 10.0 -> 6.9.
+// workgroups, its fold, the norm of the result, the next product.  The fold and the norm read some hundred KB: all loads of a row are
+// issued before the first addition, by a wave for every 256 columns, and the row never leaves the registers between the two.
+// us apart -> one launch: 154 x 1024 x 4096 13.9 -> 10.5, 197 x 768 x 3072 13.5 -> 9.9, 512 x 1280 x 5120 25.2 -> 21.3; where K was not split
+// before, splitting it pays now: 197 x 768 x 768 8.6 -> 7.6.  A row a wave, its parts four at a time, took 0.3 to 1.2 us longer: 32 x 1024 x
+// 2816 in 8 parts 9.0 -> 7.8, 128 x 1280 x 1280 in 2 9.7 -> 9.1, 197 x 768 x 3072 in 4 10.1 -> 9.8.
 #include "fold_norm.h"
 #include "common.h"
 #include "launch.h"
@@ -17,83 +18,79 @@ __device__ __forceinline__ float at4(const uint2_& t, int e) { return bf2f(e & 1
 
 __device__ __forceinline__ uint2_ pack4(const float (&f)[4]) { return uint2_{pack2(f[0], f[1]), pack2(f[2], f[3])}; }
 
-// NC: 256-column chunks of a row, 4 columns a lane each.  The parts are added in the order, and the bias and the residual with the
-// operations, of gemm_splitk_reduce: y has the bits that it writes.
-template <int NC>
-__global__ void __launch_bounds__(64) fold_norm_kernel(const FoldNormArgs p) {
-  constexpr int ROUND = NC <= 4 ? 4 : 2;   // parts in flight
-  const int lane = threadIdx.x;
+// W: waves, each 256 columns of the row, 4 a lane.  The parts are added in the order, and the bias and the residual with the operations, of
+// gemm_splitk_reduce: y has the bits that it writes.
+template <int W>
+__global__ void __launch_bounds__(64 * W) fold_norm_kernel(const FoldNormArgs p) {
+  constexpr int ROUND = 16;   // parts in flight
+  __shared__ float red[2][W];
+  const int tid = threadIdx.x;
   const long row = blockIdx.x, slab = (long)p.rows * p.D;
-  const float* src = p.parts + row * p.D;
-  float v[NC][4];
-  uint2_ r[NC], bias[NC], gain[NC], shift[NC];
-  bool in[NC];
-  int col[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    in[c] = (c * 64 + lane) * 4 < p.D;
-    col[c] = in[c] ? (c * 64 + lane) * 4 : 0;   // spare lanes read column 0
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[c][e] = 0.f;
-    auto load = [&](const bf16_t* at) { return *reinterpret_cast<const uint2_*>(at + col[c]); };
-    const uint2_ one = {0x3f803f80u, 0x3f803f80u}, zero = {0u, 0u};
-    r[c] = p.residual ? load(p.residual + row * p.ldr) : zero;
-    bias[c] = p.bias ? load(p.bias) : zero;
-    gain[c] = p.gamma ? load(p.gamma) : one;
-    shift[c] = p.beta ? load(p.beta) : zero;
-  }
+  const bool in = tid * 4 < p.D;
+  const int col = in ? tid * 4 : 0;   // spare lanes read column 0
+  const float* src = p.parts + row * p.D + col;
+  auto load = [&](const bf16_t* at) { return *reinterpret_cast<const uint2_*>(at + col); };
+  const uint2_ one = {0x3f803f80u, 0x3f803f80u}, zero = {0u, 0u};
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  uint2_ r, bias, gain, shift;
   for (int s0 = 0; s0 < p.splits; s0 += ROUND) {
-    float4_ x[ROUND][NC];
+    float4_ x[ROUND];
 #pragma unroll
     for (int u = 0; u < ROUND; ++u)
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-        x[u][c] = s0 + u < p.splits ? *reinterpret_cast<const float4_*>(src + (s0 + u) * slab + col[c]) : float4_{0.f, 0.f, 0.f, 0.f};
+      if (s0 + u < p.splits) x[u] = *reinterpret_cast<const float4_*>(src + (s0 + u) * slab);
+    if (s0 == 0) {
+      r = p.residual ? load(p.residual + row * p.ldr) : zero;
+      bias = p.bias ? load(p.bias) : zero;
+      gain = p.gamma ? load(p.gamma) : one;
+      shift = p.beta ? load(p.beta) : zero;
+    }
 #pragma unroll
     for (int u = 0; u < ROUND; ++u)
+      if (s0 + u < p.splits) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[c][e] += x[u][c][e];
+        for (int e = 0; e < 4; ++e) v[e] += x[u][e];
+      }
   }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (p.bias) v[e] += at4(bias, e);
+    if (p.residual) v[e] += at4(r, e) * p.res_alpha;
+  }
+  const uint2_ w = pack4(v);
+  if (in) *reinterpret_cast<uint2_*>(p.y + row * p.D + col) = w;
   float sum = 0.f, sq = 0.f;
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (p.bias) v[c][e] += at4(bias[c], e);
-      if (p.residual) v[c][e] += at4(r[c], e) * p.res_alpha;
-    }
-    const uint2_ w = pack4(v[c]);
-    if (in[c]) *reinterpret_cast<uint2_*>(p.y + row * p.D + col[c]) = w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[c][e] = in[c] ? at4(w, e) : 0.f;   // as the next layer reads it
-      sum += v[c][e];
-      sq += v[c][e] * v[c][e];
-    }
+  for (int e = 0; e < 4; ++e) {
+    v[e] = in ? at4(w, e) : 0.f;   // as the next layer reads it
+    sum += v[e];
+    sq += v[e] * v[e];
   }
+  auto total = [&](float t, float* at) {   // over the row
+    t = wave_sum(t);
+    if constexpr (W == 1) return t;
+    if ((tid & 63) == 0) at[tid >> 6] = t;
+    __syncthreads();
+    t = at[0];
+#pragma unroll
+    for (int u = 1; u < W; ++u) t += at[u];
+    return t;
+  };
   float mean = 0.f, rstd;
   if (p.rms) {
-    rstd = rsqrtf(wave_sum(sq) / p.D + p.eps);
+    rstd = rsqrtf(total(sq, red[0]) / p.D + p.eps);
   } else {
-    mean = wave_sum(sum) / p.D;
+    mean = total(sum, red[0]) / p.D;
     float var = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float d = in[c] ? v[c][e] - mean : 0.f;
-        var += d * d;
-      }
-    rstd = rsqrtf(wave_sum(var) / p.D + p.eps);
+    for (int e = 0; e < 4; ++e) {
+      const float d = in ? v[e] - mean : 0.f;
+      var += d * d;
+    }
+    rstd = rsqrtf(total(var, red[1]) / p.D + p.eps);
   }
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[c][e] = (v[c][e] - mean) * rstd * at4(gain[c], e) + at4(shift[c], e);
-    if (in[c]) *reinterpret_cast<uint2_*>(p.out + row * p.D + col[c]) = pack4(v[c]);
-  }
+  for (int e = 0; e < 4; ++e) v[e] = (v[e] - mean) * rstd * at4(gain, e) + at4(shift, e);
+  if (in) *reinterpret_cast<uint2_*>(p.out + row * p.D + col) = pack4(v);
 }
 
 }  // namespace
@@ -106,14 +103,10 @@ bool fold_norm_supported(const FoldNormArgs& a) {
 hipError_t launch_fold_norm(const FoldNormArgs& a, hipStream_t s) {
   if (a.rows == 0) return hipSuccess;
   if (!fold_norm_supported(a)) return hipErrorInvalidValue;
-  const int chunks = (a.D + 255) / 256;
-  return launch(chunks <= 1   ? fold_norm_kernel<1>
-                : chunks <= 2 ? fold_norm_kernel<2>
-                : chunks <= 3 ? fold_norm_kernel<3>
-                : chunks <= 4 ? fold_norm_kernel<4>
-                : chunks <= 5 ? fold_norm_kernel<5>
-                              : fold_norm_kernel<8>,
-                a.rows, 64, s, a);
+  const int waves = (a.D + 255) / 256;
+  auto go = [&](auto kernel, int w) { return launch(kernel, a.rows, 64 * w, s, a); };
+  return waves <= 1 ? go(fold_norm_kernel<1>, 1) : waves <= 2 ? go(fold_norm_kernel<2>, 2) : waves <= 3 ? go(fold_norm_kernel<3>, 3)
+         : waves <= 4 ? go(fold_norm_kernel<4>, 4) : waves <= 5 ? go(fold_norm_kernel<5>, 5) : go(fold_norm_kernel<8>, 8);
 }
 
 }  // namespace shai
