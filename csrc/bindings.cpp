@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "kernels/attn_proj.h"
 #include "kernels/fold_norm.h"
 #include "kernels/launchers.h"
 #include "kernels/vision.h"
@@ -1189,6 +1190,76 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
   run_gemm(g, a, a_bytes, (long)g.N * g.ldw * 2, 0);
 }
 
+// y = attention(q, k, v) w^T + bias + residual and out = RMS norm or LayerNorm of y, in two launches: every head's attention with its
+// part of the product, then the sum of the parts with the norm.
+void attn_proj_norm(const Tensor& q, const Tensor& k, const Tensor& v, const optional<Tensor>& kv_lens, const optional<Tensor>& attn_bias,
+                    double scale, bool causal, const Tensor& w, const optional<Tensor>& bias, const Tensor& residual, const Tensor& gamma,
+                    const optional<Tensor>& beta, const Tensor& y, const Tensor& out, double eps, bool rms) {
+  for (auto* t : {&q, &k, &v}) {
+    check_bf16(*t, "q, k, v");
+    SHAI_CHECK(t->dim() == 4 && t->size(3) == 64 && t->stride(2) == 64 && t->size(0) == q.size(0) && t->size(2) == q.size(2),
+               "attn_proj_norm: q, k, v must be [B, S, H, 64], heads packed");
+  }
+  check_rows(w, "w");
+  check_bf16(y, "y");
+  check_bf16(out, "out");
+  shai::AttnProjArgs a{};
+  a.q = cptr(q);
+  a.k = cptr(k);
+  a.v = cptr(v);
+  a.q_bs = q.stride(0), a.q_ts = q.stride(1);
+  a.k_bs = k.stride(0), a.k_ts = k.stride(1);
+  a.v_bs = v.stride(0), a.v_ts = v.stride(1);
+  a.B = q.size(0);
+  a.Sq = q.size(1);
+  a.H = q.size(2);
+  a.Skv = k.size(1);
+  a.N = w.size(0);
+  a.W = cptr(w);
+  a.ldw = w.stride(0);
+  a.scale = scale;
+  a.causal = causal;
+  const long rows = (long)a.B * a.Sq;
+  SHAI_CHECK(v.size(1) == a.Skv && w.dim() == 2 && w.size(1) == (long)a.H * 64, "attn_proj_norm: keys, values and weight columns");
+  for (auto* t : {&y, &out, &residual})
+    SHAI_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->is_contiguous() && t->numel() == rows * a.N && t->size(-1) == a.N,
+               "attn_proj_norm: residual and outputs must be contiguous [B, S, N]");
+  auto row = [&](const Tensor& t, const char* name) {
+    SHAI_CHECK(t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.numel() == a.N && t.is_contiguous(), "attn_proj_norm: ", name);
+    return cptr(t);
+  };
+  shai::FoldNormArgs n{};
+  if (bias) n.bias = row(*bias, "bias");
+  n.gamma = row(gamma, "gamma");
+  if (beta) n.beta = row(*beta, "beta");
+  SHAI_CHECK(!rms || !beta, "attn_proj_norm: an RMS norm has no shift");
+  if (kv_lens) {
+    SHAI_CHECK(kv_lens->is_cuda() && kv_lens->scalar_type() == at::kInt && kv_lens->is_contiguous() && kv_lens->numel() == a.B, "attn_proj_norm: kv_lens");
+    a.kv_lens = kv_lens->data_ptr<int>();
+  }
+  if (attn_bias) {
+    SHAI_CHECK(attn_bias->is_cuda() && attn_bias->scalar_type() == at::kBFloat16 && attn_bias->is_contiguous() && attn_bias->dim() == 3 &&
+                   attn_bias->size(0) == a.H && attn_bias->size(1) == a.Sq && attn_bias->size(2) == a.Skv,
+               "attn_proj_norm: the bias must be [H, Sq, Skv]");
+    a.bias = cptr(*attn_bias);
+  }
+  if (rows == 0) return;
+  Tensor ws = at::empty({(long)a.H * rows * a.N}, q.options().dtype(at::kFloat));
+  n.parts = a.parts = ws.data_ptr<float>();
+  n.splits = a.H;
+  n.residual = cptr(residual);
+  n.ldr = n.D = a.N;
+  n.rows = rows;
+  n.rms = rms;
+  n.res_alpha = 1.f;
+  n.eps = eps;
+  n.y = mptr(y);
+  n.out = mptr(out);
+  SHAI_CHECK(shai::attn_proj_supported(a) && shai::fold_norm_supported(n), "attn_proj_norm: up to 256 keys, N a multiple of 16 up to 2048, aligned operands");
+  check_launch(shai::launch_attn_proj(a, stream()), "attn_proj");
+  check_launch(shai::launch_fold_norm(n, stream()), "fold_norm");
+}
+
 // x: [N, H, W, C1] NHWC; x2 optional [N, H, W, C2]; w: [Cout, KH*KW*Cin]; out: [N, OH, OW, Cout]
 void conv2d(const Tensor& x, const optional<Tensor>& x2, const Tensor& w, const Tensor& out,
             const optional<Tensor>& bias, const optional<Tensor>& bias2d, const optional<Tensor>& residual,
@@ -1976,6 +2047,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("conv2d(Tensor x, Tensor? x2, Tensor w, Tensor(a!) out, Tensor? bias, Tensor? bias2d, Tensor? residual, Tensor? in_scale, Tensor? in_shift, int in_act, int kh, int kw, int stride, int pad, bool upsample, int act, float res_alpha, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, bool up_phases=False, Tensor? gn_gamma=None, Tensor? gn_beta=None, Tensor(d!)? gn_out=None, int gn_groups=0, float gn_eps=1e-5, bool gn_silu=False, bool keep_out=True) -> ()");
   m.def("groupnorm_one(Tensor x, Tensor? x2, Tensor? gamma, Tensor? beta, Tensor(a!) out, int G, float eps, bool silu) -> ()");
   m.def("groupnorm_one_supported(int HW, int C, int G, bool fold) -> bool", &groupnorm_one_supported);
+  m.def("attn_proj_norm(Tensor q, Tensor k, Tensor v, Tensor? kv_lens, Tensor? attn_bias, float scale, bool causal, Tensor w, Tensor? bias, Tensor residual, Tensor gamma, Tensor? beta, Tensor(a!) y, Tensor(b!) out, float eps, bool rms) -> ()");
   m.def("flash_attn(Tensor q, Tensor k, Tensor v, Tensor(a!) o, float scale, bool causal, int causal_offset, Tensor? kv_lens, Tensor? q_lens, Tensor? bias, Tensor? block_table) -> ()");
   m.def("paged_attn_varlen(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor kv_lens, Tensor q_lens, Tensor q_start, int max_q, float scale, bool causal) -> ()");
   m.def("decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor ctx_lens, Tensor(b!) ws, int num_splits, float scale) -> ()");
@@ -2016,6 +2088,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("groupnorm_one", &groupnorm_one);
   m.impl("gemm", &gemm);
   m.impl("gemm_norm", &gemm_norm);
+  m.impl("attn_proj_norm", &attn_proj_norm);
   m.impl("dequant_fp8", &dequant_fp8);
   m.impl("gemm_f8", &gemm_f8);
   m.impl("gemm_lnout", &gemm_lnout);

@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from ..utils.calls import fused, then_norm
+from ..utils.calls import as_called, fused, then_norm
 from .layers import Linear
 
 
@@ -63,6 +63,8 @@ class FusedSelfAttention(nn.Module):
 
     def forward_norm(self, x, residual, norm, causal: bool = False):
         """(y, norm(y)) of y = self(x, residual, causal)."""
+        if as_called(self.out, norm) and self.kv_heads == self.heads:
+            return ops.attention_linear_norm(*self.split(self.qkv(x)), self.out.weight, self.out.bias, residual, norm, causal=causal)
         return then_norm(self.out, norm, self._attend(x, causal), residual=residual)
 
 

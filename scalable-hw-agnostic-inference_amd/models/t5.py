@@ -21,7 +21,7 @@ import torch.nn as nn
 from .. import ops
 from ..parallel.layers import GLUParallelLinear, QKVParallelLinear, RowParallelLinear
 from ..parallel.state import tp
-from ..utils.calls import chain, fused, then_norm
+from ..utils.calls import as_called, chain, fused, then_norm
 from .layers import Embedding, GLULinear, RMSNorm
 
 
@@ -80,13 +80,13 @@ class T5Block(nn.Module):
         self.wo = RowParallelLinear(c.d_ff, c.d_model, bias=False)
         self.h = self.qkv.h_local
 
-    def _attend(self, qkv, bias, lens):
+    def _heads(self, qkv):
         B, S, _ = qkv.shape
         h, d = self.h, self.c.d_kv
-        q = qkv[..., : h * d].view(B, S, h, d)
-        k = qkv[..., h * d:2 * h * d].view(B, S, h, d)
-        v = qkv[..., 2 * h * d:].view(B, S, h, d)
-        return ops.attention(q, k, v, scale=1.0, kv_lens=lens, bias=bias).view(B, S, h * d)
+        return [t.view(B, S, h, d) for t in (qkv[..., : h * d], qkv[..., h * d:2 * h * d], qkv[..., 2 * h * d:])]
+
+    def _attend(self, qkv, bias, lens):
+        return ops.attention(*self._heads(qkv), scale=1.0, kv_lens=lens, bias=bias).view(*qkv.shape[:2], self.h * self.c.d_kv)
 
     def forward(self, x, bias, lens):
         x = self.o(self._attend(self.qkv(self.ln_attn(x)), bias, lens), residual=x)
@@ -95,8 +95,11 @@ class T5Block(nn.Module):
     def forward_next(self, x, n, bias, lens, next_norm):
         """(y, next_norm(y)) of y = self(x, bias, lens); ``n``: x normalised by ``ln_attn``."""
         qkv = self.qkv(n)      # kept beside the block: products that wrote where these heads lay made a graph's replay 3 % slower
-        a = self._attend(qkv, bias, lens)
-        x, n = then_norm(self.o, self.ln_ff, a, residual=x)
+        if as_called(self.o, self.ln_ff) and self.o.whole:
+            x, n = ops.attention_linear_norm(*self._heads(qkv), self.o.weight, self.o.bias, x, self.ln_ff, scale=1.0, kv_lens=lens,
+                                             attn_bias=bias)
+        else:
+            x, n = then_norm(self.o, self.ln_ff, self._attend(qkv, bias, lens), residual=x)
         return then_norm(self.wo, next_norm, self.wi(n), residual=x)
 
 

@@ -302,14 +302,20 @@ def stats_supported(rows: int, cols: int, kind: str, hw: Optional[int] = None) -
 LINEAR_NORM_MAX = 1 << 20
 
 
+def _norm_fuses(M: int, w, residual, norm) -> bool:
+    """Whether the fold of partial sums, the residual and this norm can be one launch."""
+    N = w.shape[0]
+    rows = residual.is_contiguous() and residual.shape[-1] == N
+    return (rows and 0 < M * N <= LINEAR_NORM_MAX and N % 8 == 0 and N <= 2048 and w.dtype == torch.bfloat16
+            and norm.weight is not None and not getattr(norm, "w_offset", 0.0))
+
+
 def linear_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], residual: torch.Tensor, norm):
     """(y, norm(y)) with y = x @ w^T + bias + residual, ``norm`` a module with ``weight``, ``bias`` (None: RMS norm) and ``eps``.
     On the GPU a small product whose K is split leaves its fold to the norm's launch."""
     M, N = x.numel() // x.shape[-1], w.shape[0]
     gain, shift, rms = norm.weight, getattr(norm, "bias", None), getattr(norm, "w_offset", None) is not None
-    rows = residual.is_contiguous() and residual.shape[-1] == N
-    if not (_gpu(x) and rows and 0 < M * N <= LINEAR_NORM_MAX and N % 8 == 0 and N <= 2048 and w.dtype == torch.bfloat16
-            and gain is not None and not getattr(norm, "w_offset", 0.0)):
+    if not (_gpu(x) and _norm_fuses(M, w, residual, norm)):
         y = linear(x, w, bias, residual=residual)
         return y, norm(y)
     y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
@@ -603,6 +609,38 @@ def attention(q, k, v, scale: Optional[float] = None, causal: bool = False, caus
     _K().flash_attn(q, k, v, o, float(scale), bool(causal), int(causal_offset), _i32(kv_lens), _i32(q_lens), bias,
                     None)
     return o
+
+
+# partial sums (rows x columns x heads) below which attention and its projection are one launch: beyond, writing and reading them costs
+# more than the launch (us apart -> one: 16 heads to 1024 columns, 154 rows 14.9 -> 14.1, 160 rows 13.6 -> 13.5, 200 rows 15.6 -> 16.4)
+ATTENTION_LINEAR_PARTS = 5 << 19
+
+
+def attention_linear_norm(q, k, v, w, bias, residual, norm, scale: Optional[float] = None, causal: bool = False, kv_lens=None,
+                          attn_bias=None):
+    """(y, norm(y)) with y = attention(q, k, v) @ w^T + bias + residual, ``norm`` as in :func:`linear_norm`.  q [B, Sq, H, D], k / v
+    [B, Skv, H, D]; ``kv_lens``, ``attn_bias`` [H, Sq, Skv]: see :func:`attention`.  On the GPU a few rows of a few keys take two launches:
+    the heads' attention and projection, then the sum over heads with the norm."""
+    B, S, H, D = q.shape
+    if not (_gpu(q) and _attention_linear_fits(q, k, v, w, bias, residual, norm, attn_bias)):
+        o = attention(q, k, v, scale=scale, causal=causal, kv_lens=kv_lens, bias=attn_bias)
+        return linear_norm(o.reshape(B, S, H * D), w, bias, residual, norm)
+    y = torch.empty(B, S, w.shape[0], dtype=q.dtype, device=q.device)
+    out = torch.empty_like(y)
+    _K().attn_proj_norm(q, k, v, _i32(kv_lens), attn_bias, float(scale if scale is not None else D ** -0.5), bool(causal), w, bias, residual,
+                        norm.weight, getattr(norm, "bias", None), y, out, float(norm.eps), getattr(norm, "w_offset", None) is not None)
+    return y, out
+
+
+def _attention_linear_fits(q, k, v, w, bias, residual, norm, attn_bias) -> bool:
+    B, S, H, D = q.shape
+    heads = lambda t: t.stride(3) == 1 and t.stride(2) == D and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0
+    params = [t for t in (bias, residual, norm.weight, getattr(norm, "bias", None)) if t is not None]
+    return (D == 64 and B * S * H * w.shape[0] < ATTENTION_LINEAR_PARTS and k.shape[1] <= 256 and k.shape == v.shape and k.shape[0] == B and k.shape[2] == H
+            and _norm_fuses(B * S, w, residual, norm) and w.shape[0] % 16 == 0 and w.shape[1] == H * D and w.stride(1) == 1
+            and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0 and all(heads(t) for t in (q, k, v))
+            and all(t.dtype == torch.bfloat16 for t in (q, k, v, *params)) and all(t.data_ptr() % 8 == 0 for t in params)
+            and (attn_bias is None or (attn_bias.is_contiguous() and attn_bias.dtype == torch.bfloat16)))
 
 
 def paged_attention(q, k_cache, v_cache, block_table, kv_lens, q_lens, scale=None, causal=True):

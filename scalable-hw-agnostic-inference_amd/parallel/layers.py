@@ -126,9 +126,14 @@ class RowParallelLinear(_ShardLoadMixin, nn.Module):
             y = ops.bias_act(y, self.bias, residual)
         return y
 
+    @property
+    def whole(self) -> bool:
+        """Whether a call is one product with the weight as it is, its sums in any order."""
+        return self.tp_size == 1 and self.w_scale is None and not self.one_order
+
     def forward_norm(self, x, residual, norm):
         """(y, norm(y)) of y = self(x, residual=residual) -- see ``ops.linear_norm``."""
-        if self.tp_size == 1 and self.w_scale is None and not self.one_order:
+        if self.whole:
             return ops.linear_norm(x, self.weight, self.bias, residual, norm)
         y = self(x, residual=residual)
         return y, norm(y)
