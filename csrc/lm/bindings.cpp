@@ -8,6 +8,7 @@
 
 #include "kernels/launchers.h"
 #include "lm/lm.h"
+#include "lm/normed_gemm.h"
 
 using at::Tensor;
 using c10::optional;
@@ -308,6 +309,75 @@ void lm_gemm_parts(const Tensor& A, const Tensor& W, const Tensor& C) {
   const bool tile = !f32 && g.M > 64 && (long)g.M * g.lda * 2 < lim && (long)g.N * g.K * 2 < lim;
   if (tile) shai_lm::launch_gemm_tile(g, stream());
   else shai_lm::launch_gemm(g, f32, stream());
+}
+
+// C = epi(h W^T) with h the norm of x + sum of delta's parts (residual_norm without a norm on delta, lm_gemm), for a few bf16 rows
+void normed_gemm(const optional<Tensor>& x, const optional<Tensor>& ids, const optional<Tensor>& table, double scale,
+                 const optional<Tensor>& delta, const Tensor& w, double eps, int64_t width, const optional<Tensor>& x_out,
+                 const Tensor& W, const Tensor& C, const optional<Tensor>& side, int64_t act) {
+  shai_lm::NormedGemmArgs a{};
+  shai_lm::GemmArgs& g = a.g;
+  check(W, at::kBFloat16, "W");
+  SHAI_CHECK(W.dim() == 2 && C.dim() == 2 && (C.scalar_type() == at::kFloat || C.scalar_type() == at::kBFloat16), "normed_gemm: W [N, K], C bf16 or fp32");
+  check_rows(C, C.scalar_type(), "C");
+  g.M = g.a_rows = C.size(0);
+  g.N = W.size(0);
+  g.K = W.size(1);
+  g.batch = 1;
+  g.out_f32 = C.scalar_type() == at::kFloat;
+  SHAI_CHECK(shai_lm::normed_gemm_fits(g.M, g.K) && g.N >= 1, "normed_gemm: ", g.M, " rows of ", g.K, ": one or two of up to 4096");
+  check_width(g.K, width);
+  SHAI_CHECK(x.has_value() != ids.has_value(), "normed_gemm: a residual or token ids");
+  auto matrix = [&](const Tensor& t, const char* name) {
+    check(t, at::kFloat, name);
+    SHAI_CHECK(t.dim() == 2 && t.size(0) == g.M && t.size(1) == g.K, name, " must be [rows, K]");
+    return t.data_ptr<float>();
+  };
+  if (x) {
+    a.x = matrix(*x, "x");
+  } else {
+    check_i32(*ids, "ids");
+    SHAI_CHECK(table.has_value() && ids->numel() == g.M, "token ids, one a row, need a table");
+    check(*table, at::kBFloat16, "table");
+    SHAI_CHECK(table->dim() == 2 && table->size(1) == g.K && table->size(0) >= 1, "table must be [V, K]");
+    a.ids = ids->data_ptr<int>();
+    a.table = table->data_ptr();
+    a.V = table->size(0);
+    a.scale = scale;
+  }
+  if (delta) {
+    check(*delta, at::kFloat, "delta");
+    SHAI_CHECK(delta->dim() == 3 && delta->size(0) >= 1 && delta->size(0) <= 8 && delta->size(1) == g.M && delta->size(2) == g.K,
+               "delta must be [1 to 8 parts, rows, K]");
+    a.delta = delta->data_ptr<float>();
+    a.parts = delta->size(0);
+    a.part_stride = (long)g.M * g.K;
+  }
+  if (x_out) {
+    a.x_out = matrix(*x_out, "x_out");
+    SHAI_CHECK(a.x_out != a.x, "x_out must lie apart from x");
+  }
+  check(w, at::kFloat, "w");
+  SHAI_CHECK(w.numel() == g.K, "w must be [K]");
+  a.w = w.data_ptr<float>();
+  a.eps = eps;
+  a.width = width;
+  g.n_main = g.N;
+  if (side) {
+    check(*side, at::kFloat, "side");
+    SHAI_CHECK(side->dim() == 2 && side->size(0) == g.M && side->size(1) >= 1 && side->size(1) < g.N, "side output: [M, last rows of W]");
+    g.n_main = g.N - side->size(1);
+    SHAI_CHECK(g.n_main % 4 == 0, "side output: the other rows of W must be a multiple of 4");
+    g.side = side->data_ptr<float>();
+  }
+  SHAI_CHECK(reinterpret_cast<uintptr_t>(C.data_ptr()) % 16 == 0 && C.size(1) == g.n_main, "C: 16-byte aligned, the columns of the product");
+  SHAI_CHECK(act >= 0 && act % 4 == 0 && act <= g.n_main, "act: leading columns, a multiple of 4");
+  g.epi = act > 0 ? shai_lm::EPI_RELU2 : shai_lm::EPI_NONE;
+  g.n_act = act > 0 ? act : g.n_main;
+  g.ldc = g.M > 1 ? C.stride(0) : std::max<int64_t>(C.stride(0), C.size(1));
+  g.W = W.data_ptr();
+  g.C = C.data_ptr();
+  shai_lm::launch_normed_gemm(a, stream());
 }
 
 // Which kernel a plain bf16 product runs on (for tests and tools); n_tiles > 0: grouped, in that many tiles of up to 256 rows
@@ -1207,6 +1277,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("lm_gemm_heads(Tensor a, Tensor w, Tensor(a!) c) -> ()");
   m.def("lm_gemm_parts(Tensor a, Tensor w, Tensor(a!) c) -> ()");
   m.def("residual_norm(Tensor? x, Tensor? ids, Tensor? table, float scale, Tensor? delta, Tensor? wb, float mult, Tensor? step, Tensor(a!)? x_out, Tensor? rows, Tensor? w, float eps, int width, Tensor(b!)? h, Tensor? cw=None, Tensor(c!)? state=None, Tensor(d!)? tail=None, Tensor? row_seq=None, Tensor? q_start=None, Tensor? q_lens=None, Tensor? pos=None, Tensor? slots=None, Tensor? bb=None, Tensor? b=None, Tensor? ye=None, Tensor? slot_of=None, Tensor? wts=None) -> ()");
+  m.def("normed_gemm(Tensor? x, Tensor? ids, Tensor? table, float scale, Tensor? delta, Tensor w, float eps, int width, Tensor(a!)? x_out, Tensor W, Tensor(b!) C, Tensor(c!)? side=None, int act=0) -> ()");
   m.def("conv_commit(Tensor(a!) state, Tensor tail, Tensor q_lens, Tensor slots) -> ()");
   m.def("rope_rows(Tensor pos, Tensor freq, Tensor(a!) out) -> ()");
   m.def("latent_prep(Tensor d, Tensor wq, Tensor wkv, Tensor rope, Tensor slots, Tensor(a!) cache, Tensor(b!) cq, float eps, int q_rank, int kv_rank) -> ()");
@@ -1240,6 +1311,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("lm_gemm_heads", &lm_gemm_heads);
   m.impl("lm_gemm_parts", &lm_gemm_parts);
   m.impl("residual_norm", &residual_norm);
+  m.impl("normed_gemm", &normed_gemm);
   m.impl("conv_commit", &conv_commit);
   m.impl("rope_rows", &rope_rows);
   m.impl("latent_prep", &latent_prep);

@@ -239,6 +239,7 @@ class MoE(nn.Module):
         _init_packed(self, self.pack, self.shapes(), gen)
 
 
+@fused
 class SoftcapHead(nn.Module):
     """fp32 logits = cap * tanh(h W^T / cap); no cap: h W^T."""
 
@@ -249,6 +250,12 @@ class SoftcapHead(nn.Module):
 
     def forward(self, h):
         return lm.matmul(h, self.weight, torch.float32, lm.EPI_SOFTCAP if self.cap else lm.EPI_NONE, self.cap or 0.0)
+
+    def forward_normed(self, n: lm.Normed, rows: int):
+        """``forward`` of a norm (no cap): the norm made by the product."""
+        out = torch.empty(rows, self.weight.shape[0], dtype=torch.float32, device=self.weight.device)
+        lm.normed_matmul(n, self.weight, out, keep=False)
+        return out
 
     def init_random_(self, gen):
         self.weight[:, :self.width].normal_(0, self.width ** -0.5, generator=gen)
@@ -697,6 +704,7 @@ class TokenSide(nn.Module):
 
 
 # ---------------------------------------------------------------------------------------------- joint layers
+@fused
 class JointLayer(nn.Module):
     """Sublayers that read one norm's output and whose sum is added to the residual: one or more mixers and an ungated
     squared-ReLU feed-forward (``ff`` 0: none).  One product gives every mixer's inputs and the activated feed-forward, one
@@ -745,9 +753,18 @@ class JointLayer(nn.Module):
 
     def forward(self, h, batch, cache, state, step):
         """``cache`` / ``state``: what the mixers that have a key-value cache / a recurrent state keep of this layer run."""
-        n = self.out_cols + self.fp
-        rows = torch.empty(h.shape[0], n + self.in_rows, dtype=h.dtype, device=h.device)
+        rows = torch.empty(h.shape[0], self.out_cols + self.fp + self.in_rows, dtype=h.dtype, device=h.device)
         side = lm.matmul_joint(h, self.w_in, rows[:, self.out_cols:], self.fp, self.side_rows)
+        return self._rest(rows, side, batch, cache, state, step)
+
+    def forward_normed(self, n: lm.Normed, batch, cache, state, step):
+        """(x, ``forward`` of x's norm): the norm made by the product that reads it."""
+        rows = torch.empty(batch.B, self.out_cols + self.fp + self.in_rows, dtype=self.w_in.dtype, device=self.w_in.device)
+        x, side = lm.normed_matmul(n, self.w_in, rows[:, self.out_cols:], self.fp, self.side_rows)
+        return x, self._rest(rows, side, batch, cache, state, step)
+
+    def _rest(self, rows, side, batch, cache, state, step):
+        n = self.out_cols + self.fp
         mixers, args = list(self.mixers.values()), []
         i, s, o = n, 0, 0
         for m in mixers:

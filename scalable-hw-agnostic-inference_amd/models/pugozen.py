@@ -22,6 +22,7 @@ from .blocks import (DeltaRule, DeltaRuleConfig, GainNorm, JointLayer, Retention
 from .llama import KV_BLOCK, Batch
 from ..ops import lm
 from ..parallel.state import tp
+from ..utils.calls import as_called
 
 
 @dataclass
@@ -204,11 +205,20 @@ class PugozenForCausalLM(nn.Module):
         norm = lambda source, delta, w, **kw: lm.residual_norm(source, delta, lm.PLAIN, 1.0, None, w, cfg.eps, cfg.width,
                                                                self.dtype, batch=batch, **kw)
         x, delta = lm.Embedding(batch.input_ids, self.embed, cfg.embed_scale), None
+        ahead = lambda w: lm.Normed(x, delta, w, cfg.eps, cfg.width)   # a norm that the product behind it makes
+        alone = not batch.is_prefill and trail is None
         for r, layer in enumerate(self.runs()):
+            n = ahead(layer.norm1.weight)
+            if alone and lm.normed_fits(n, layer.joint.w_in) and as_called(layer.joint):
+                x, delta = layer.joint.forward_normed(n, batch, kv_caches[r], batch.states[r], step)
+                continue
             x, h = norm(x, delta, layer.norm1.weight)
             delta = layer.joint(h, batch, kv_caches[r], batch.states[r], step)
             if trail is not None:
                 trail.append(norm(x.clone(), delta, None)[0][:, :cfg.width])
+        n = ahead(self.final_norm.weight)
+        if alone and self.head.cap is None and lm.normed_fits(n, self.head.weight) and as_called(self.head):
+            return self.head.forward_normed(n, batch.B)
         rows = batch.last_index.int() if batch.is_prefill else None
         return self.head(norm(x, delta, self.final_norm.weight, rows=rows, keep=False)[1])
 

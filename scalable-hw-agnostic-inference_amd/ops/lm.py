@@ -17,7 +17,7 @@ GPU tensors run the native kernels (raising if the library is missing); CPU tens
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import List, NamedTuple, Optional
+from typing import List, NamedTuple, Optional, Union
 
 import numpy as np
 import torch
@@ -429,6 +429,40 @@ def residual_norm(source, delta, wb, mult: float, step, w, eps: float, width: in
         _K().residual_norm(*args, conv.weight, conv.state, conv.tail, batch.row_seq, batch.q_start, batch.q_lens,
                            batch.positions, batch.state_slots, **ye)
     return x, h
+
+
+@dataclass
+class Normed:
+    """A product's input that is yet to be made: the norm with gain ``w`` of x = source + the sum of ``delta``'s parts, as
+    ``residual_norm(source, delta, PLAIN, 1.0, None, w, ...)`` has it."""
+    source: Union[torch.Tensor, Embedding]
+    delta: Optional[torch.Tensor]
+    w: torch.Tensor
+    eps: float
+    width: int
+
+
+NORMED_ROWS = 2
+
+
+def normed_fits(n: Normed, weight: torch.Tensor) -> bool:
+    """Whether :func:`normed_matmul` takes this norm: bf16 weights, one or two rows of up to 4096, parts in fp32."""
+    emb = isinstance(n.source, Embedding)
+    rows, K = (n.source.ids.shape[0], n.source.table.shape[1]) if emb else n.source.shape
+    d = n.delta
+    return (weight.is_cuda and weight.dtype == torch.bfloat16 and 1 <= rows <= NORMED_ROWS and K <= 4096
+            and not isinstance(n.w, Affine) and (d is None or (isinstance(d, torch.Tensor) and d.dim() == 3 and d.shape[0] <= 8)))
+
+
+def normed_matmul(n: Normed, weight, out, act: int = 0, side: int = 0, keep: bool = True):
+    """(x, side product) of :func:`matmul_joint` of the norm's output, and the norm's x (``keep`` False: None)."""
+    emb = isinstance(n.source, Embedding)
+    ids, table, scale = n.source if emb else (None, None, 1.0)
+    K, dev = weight.shape[1], weight.device
+    x = torch.empty(out.shape[0], K, dtype=torch.float32, device=dev) if keep else None
+    s = torch.empty(out.shape[0], side, dtype=torch.float32, device=dev) if side else None
+    _K().normed_gemm(None if emb else n.source, ids, table, float(scale), n.delta, n.w, float(n.eps), int(n.width), x, weight, out, s, int(act))
+    return x, s
 
 
 def conv_commit(state, tail, batch) -> None:

@@ -133,3 +133,46 @@ def test_mixers_of_a_step_in_one_launch(cuda, B, H, G, d, rule, channels, splits
         assert torch.isfinite(b.float()).all()
         assert (a.float() - b.float()).norm() <= (2 ** -16 if a.dtype == torch.float32 else 2 ** -9) * b.float().norm(), i
     assert torch.equal(one[2], two[2]) and torch.equal(one[4], two[4])
+
+
+@pytest.mark.parametrize("M,K,width,N,act,side,parts,source,out", [
+    (1, 64, 40, 16, 0, 0, 0, "table", torch.bfloat16), (1, 64, 64, 20, 8, 4, 1, "rows", torch.bfloat16),
+    (2, 192, 180, 9000, 0, 0, 4, "rows", torch.float32), (1, 2048, 2048, 17424, 8448, 16, 4, "rows", torch.bfloat16),
+    (2, 2048, 2000, 999, 64, 3, 8, "table", torch.bfloat16), (1, 2112, 2112, 8200, 0, 0, 5, "rows", torch.float32),
+    (2, 4096, 4096, 333, 0, 0, 3, "rows", torch.float32)])
+def test_norm_made_by_its_product(cuda, M, K, width, N, act, side, parts, source, out):
+    """A product that makes its input's norm against the two launches: rows of one step of the ring and of many, a K that the waves do not
+    share evenly, fewer tiles than workgroups and more, columns that end in a tile.  The residual has the same bits; the norm's mean square
+    is summed in another order (2^-20), which may turn a bf16 rounding of h (2^-9 of one of K terms)."""
+    lm = C.lm
+    g = torch.Generator(device=cuda).manual_seed(K + N)
+    rand = lambda *s: torch.randn(*s, generator=g, device=cuda)
+    pad = (torch.arange(K, device=cuda) < width).float()
+    w, W = (rand(K).abs() + 0.5) * pad, (rand(N, K) / K ** 0.5).bfloat16()
+    x, table = rand(M, K) * pad, (rand(50, K) * pad).bfloat16()
+    src = x if source == "rows" else lm.Embedding(torch.tensor([49, 7][:M], dtype=torch.int32, device=cuda), table, 3.0)
+    delta = rand(parts, M, K) * pad if parts else None
+    n = lm.Normed(src, delta, w, 1e-5, width)
+    assert lm.normed_fits(n, W)
+    got = torch.full((M, N - side), 5.0, dtype=out, device=cuda)
+    gx, gs = lm.normed_matmul(n, W, got, act, side)
+    wx, h = lm.residual_norm(x.clone() if source == "rows" else src, delta, lm.PLAIN, 1.0, None, w, 1e-5, width, torch.bfloat16)
+    c = h.double() @ W.double().T
+    c[:, :act] = torch.relu(c[:, :act]) ** 2
+    assert torch.equal(gx, wx)
+    tol = 2 ** -8 if out == torch.bfloat16 else 2 ** -9
+    assert (got.double() - c[:, :N - side]).norm() <= tol * c.norm()
+    if side:
+        assert (gs.double() - c[:, N - side:]).norm() <= 2 ** -9 * c.norm()
+
+
+def test_norms_that_stay_apart(cuda):
+    """More rows, a wider residual, fp32 weights, sums in bf16 or in more parts, a norm with a bias."""
+    lm = C.lm
+    W, w = torch.zeros(16, 128, dtype=torch.bfloat16, device=cuda), torch.zeros(128, device=cuda)
+    x, d = torch.zeros(2, 128, device=cuda), torch.zeros(4, 2, 128, device=cuda)
+    fits = lambda x, d, w, W: lm.normed_fits(lm.Normed(x, d, w, 1e-5, 128), W)
+    assert fits(x, d, w, W) and fits(x, None, w, W)
+    assert not fits(torch.zeros(3, 128, device=cuda), None, w, W) and not fits(torch.zeros(1, 4160, device=cuda), None, w, W)
+    assert not fits(x, d, w, W.float()) and not fits(x, d[0].bfloat16(), w, W) and not fits(x, torch.zeros(9, 2, 128, device=cuda), w, W)
+    assert not fits(x, d, lm.Affine(w, w), W)
