@@ -32,12 +32,27 @@ __global__ void __launch_bounds__(256) row_norm_kernel(
   }
   const bf16_t* xr = x + (long)row * x_stride;
   uint4_ v[MAXC];
+  // Gain and shift are asked for with the row, where registers allow: behind the sums they were a second latency (us, 512 x
+  // 1280 5.2 -> 4.8, 128 x 1280 4.2 -> 3.8; by rows of 320 below 8192 5.5 -> 4.4, 65536 19.5 -> 16.8).
+  constexpr bool EARLY = MAXC <= 4;
+  uint4_ wv[EARLY ? MAXC : 1], bv[EARLY ? MAXC : 1];
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+      const int col = (c * 64 + lane) * 8;
+      if (col < D) {
+        v[c] = *reinterpret_cast<const uint4_*>(xr + col);
+        if (w) wv[c] = *reinterpret_cast<const uint4_*>(w + col);
+        if (LAYERNORM && b) bv[c] = *reinterpret_cast<const uint4_*>(b + col);
+      }
+    }
+  }
   float sum = 0.f, sumsq = 0.f;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
     const int col = (c * 64 + lane) * 8;
     if (col < D) {
-      v[c] = *reinterpret_cast<const uint4_*>(xr + col);
+      if constexpr (!EARLY) v[c] = *reinterpret_cast<const uint4_*>(xr + col);
       if (residual) {
         const uint4_ r = *reinterpret_cast<const uint4_*>(residual + (long)row * D + col);
         float f[8], g[8];
@@ -85,11 +100,11 @@ __global__ void __launch_bounds__(256) row_norm_kernel(
     if (col < D) {
       float f[8], wf[8], bf[8];
       unpack8(v[c], f);
-      if (w) unpack8(*reinterpret_cast<const uint4_*>(w + col), wf);
+      if (w) unpack8(EARLY ? wv[c % (EARLY ? MAXC : 1)] : *reinterpret_cast<const uint4_*>(w + col), wf);
       else
 #pragma unroll
         for (int i = 0; i < 8; ++i) wf[i] = 1.f;
-      if (LAYERNORM && b) unpack8(*reinterpret_cast<const uint4_*>(b + col), bf);
+      if (LAYERNORM && b) unpack8(EARLY ? bv[c % (EARLY ? MAXC : 1)] : *reinterpret_cast<const uint4_*>(b + col), bf);
       else
 #pragma unroll
         for (int i = 0; i < 8; ++i) bf[i] = 0.f;
@@ -119,9 +134,13 @@ __global__ void __launch_bounds__(256) row_norm8_kernel(
     if (b) b += wo;
   }
   const bf16_t* xr = x + (long)r * x_stride;
-  uint4_ v[NV];
+  uint4_ v[NV], wv[NV], bv[NV];
 #pragma unroll
-  for (int c = 0; c < NV; ++c) v[c] = *reinterpret_cast<const uint4_*>(xr + (c * 8 + sub) * 8);
+  for (int c = 0; c < NV; ++c) {
+    v[c] = *reinterpret_cast<const uint4_*>(xr + (c * 8 + sub) * 8);
+    if (w) wv[c] = *reinterpret_cast<const uint4_*>(w + (c * 8 + sub) * 8);
+    if (LAYERNORM && b) bv[c] = *reinterpret_cast<const uint4_*>(b + (c * 8 + sub) * 8);
+  }
   if (residual) {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
@@ -176,11 +195,11 @@ __global__ void __launch_bounds__(256) row_norm8_kernel(
     const int col = (c * 8 + sub) * 8;
     float f[8], wf[8], bf[8];
     unpack8(v[c], f);
-    if (w) unpack8(*reinterpret_cast<const uint4_*>(w + col), wf);
+    if (w) unpack8(wv[c], wf);
     else
 #pragma unroll
       for (int i = 0; i < 8; ++i) wf[i] = 1.f;
-    if (LAYERNORM && b) unpack8(*reinterpret_cast<const uint4_*>(b + col), bf);
+    if (LAYERNORM && b) unpack8(bv[c], bf);
     else
 #pragma unroll
       for (int i = 0; i < 8; ++i) bf[i] = 0.f;
@@ -579,36 +598,34 @@ void launch_groupnorm_apply(const GroupNormArgs& a, hipStream_t s) {
 // Norm statistics handed from a GEMM epilogue to the next norm (GemmArgs::col_part / row_part, gemm_8ph.hip), and
 // the passes that produce the same statistics when the producing kernel could not (fallbacks).
 
-// col partials [M / 128, N, 2] of x [M, N]: block = 128 rows x 64 channel vectors (512 channels); 256 threads =
-// 64 vectors x 4 row lanes, each lane 32 rows with 8 independent 16-B loads in flight (batch-1 steps give only a
-// few 128-row blocks, so the per-thread loop must not be latency-bound)
-__global__ void __launch_bounds__(256) col_partials_kernel(const bf16_t* __restrict__ x, long M, int N, long ldx,
-                                                           float* __restrict__ part) {
-  __shared__ float4_ red[4][64][4];  // [row lane][vector][sum 0-3, sum 4-7, sq 0-3, sq 4-7]
+// col partials [M / 128, N, 2] of x [M, N]: block = 128 rows x 64 channel vectors (512 channels); 1024 threads = 64 vectors x 16 row
+// lanes, whose 8 rows are all on their way at once (a batch-1 step has a few dozen blocks, each a latency and a few sums long; four lanes
+// of 32 rows were four latencies: 8192 x 320 4.8 us, now 4.0)
+__global__ void __launch_bounds__(1024) col_partials_kernel(const bf16_t* __restrict__ x, long M, int N, long ldx,
+                                                            float* __restrict__ part) {
+  constexpr int L = 16;
+  __shared__ float4_ red[L][64][4];  // [row lane][vector][sum 0-3, sum 4-7, sq 0-3, sq 4-7]
   const int C8 = N >> 3, t = threadIdx.x;
   const int v = t & 63, rl = t >> 6;
   const int cv = blockIdx.y * 64 + v;
-  const long r0 = (long)blockIdx.x * 128 + rl * 32;
+  const long r0 = (long)blockIdx.x * 128 + rl * 8;
   float s[8], q[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) s[e] = q[e] = 0.f;
   if (cv < C8) {
     const bf16_t* src = x + r0 * ldx + cv * 8;
+    uint4_ u[8];
 #pragma unroll
-    for (int r8 = 0; r8 < 32; r8 += 8) {
-      uint4_ u[8];
+    for (int k = 0; k < 8; ++k)
+      u[k] = r0 + k < M ? *reinterpret_cast<const uint4_*>(src + (long)k * ldx) : uint4_{0, 0, 0, 0};
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        u[k] = r0 + r8 + k < M ? *reinterpret_cast<const uint4_*>(src + (long)(r8 + k) * ldx) : uint4_{0, 0, 0, 0};
+    for (int k = 0; k < 8; ++k) {
+      float f[8];
+      unpack8(u[k], f);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        float f[8];
-        unpack8(u[k], f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          s[e] += f[e];
-          q[e] = fmaf(f[e], f[e], q[e]);
-        }
+      for (int e = 0; e < 8; ++e) {
+        s[e] += f[e];
+        q[e] = fmaf(f[e], f[e], q[e]);
       }
     }
   }
@@ -617,27 +634,22 @@ __global__ void __launch_bounds__(256) col_partials_kernel(const bf16_t* __restr
   red[rl][v][2] = float4_{q[0], q[1], q[2], q[3]};
   red[rl][v][3] = float4_{q[4], q[5], q[6], q[7]};
   __syncthreads();
-  if (rl == 0 && cv < C8) {
-    float4_ a0 = red[0][v][0], a1 = red[0][v][1], b0 = red[0][v][2], b1 = red[0][v][3];
+  const int part_of = t & 3, vec = t >> 2;   // four threads finish a vector: sums of its channels 0-3, 4-7, their squares
+  const int cw = blockIdx.y * 64 + vec;
+  if (vec < 64 && cw < C8) {
+    float4_ a = red[0][vec][part_of];
 #pragma unroll
-    for (int l = 1; l < 4; ++l) {
-      a0 += red[l][v][0];
-      a1 += red[l][v][1];
-      b0 += red[l][v][2];
-      b1 += red[l][v][3];
-    }
-    float4_* dst = reinterpret_cast<float4_*>(part + ((long)blockIdx.x * N + cv * 8) * 2);
-    dst[0] = float4_{a0[0], b0[0], a0[1], b0[1]};
-    dst[1] = float4_{a0[2], b0[2], a0[3], b0[3]};
-    dst[2] = float4_{a1[0], b1[0], a1[1], b1[1]};
-    dst[3] = float4_{a1[2], b1[2], a1[3], b1[3]};
+    for (int l = 1; l < L; ++l) a += red[l][vec][part_of];
+    float* dst = part + ((long)blockIdx.x * N + cw * 8 + 4 * (part_of & 1)) * 2 + (part_of >> 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[2 * e] = a[e];
   }
 }
 
 void launch_col_partials(const bf16_t* x, long M, int N, long ldx, float* part, hipStream_t s) {
   if (M <= 0) return;
   const int C8 = N >> 3;
-  col_partials_kernel<<<dim3((unsigned)((M + 127) / 128), (C8 + 63) / 64), 256, 0, s>>>(x, M, N, ldx, part);
+  col_partials_kernel<<<dim3((unsigned)((M + 127) / 128), (C8 + 63) / 64), 1024, 0, s>>>(x, M, N, ldx, part);
 }
 
 // GroupNorm (scale, shift) from the col partials of x (channels [0, C1)) and x2 ([C1, C1 + C2)): one wave per
