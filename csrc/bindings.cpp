@@ -17,6 +17,7 @@
 
 #include "kernels/attn_proj.h"
 #include "kernels/fold_norm.h"
+#include "kernels/groupnorm_two.h"
 #include "kernels/launchers.h"
 #include "kernels/vision.h"
 
@@ -497,6 +498,11 @@ void launch_with_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, con
   n.residual = g.residual;
   n.res_alpha = g.res_alpha;
   n.raw = st.keep ? g.C : nullptr;
+  if (shai::gn_two_wanted(n)) {
+    Tensor stats = at::empty({shai::gn_two_floats(n)}, like.options().dtype(at::kFloat));
+    check_launch(shai::launch_gn_two(n, g.C, stats.data_ptr<float>(), stream()), "gn_two");
+    return;
+  }
   check_launch(shai::launch_gn_one(n, stream()), "gn_one");
 }
 

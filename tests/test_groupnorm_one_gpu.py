@@ -84,3 +84,30 @@ def test_after_convolution(cuda, cfg, splits, side, cin, cout):
     native.ops().conv2d(x, None, w, raw, b, temb, None, None, None, 0, 3, 3, 1, 1, False, 0, 1.0, gn_gamma=gamma, gn_beta=beta,
                         gn_out=torch.empty_like(raw), gn_groups=32, gn_silu=True, keep_out=False)
     assert bool((raw == 7).all()) == (splits > 1)
+
+
+# 81920 values of a group's parts and more: the fold and the norm are two launches.  Groups of 4 n channels and two groups to a workgroup,
+# images of whole segments and of uneven ones (25 x 25: 157, 157, 157, 154 pixels), an image that has 16 segments, and the border below
+@pytest.mark.parametrize("N,side,cout,splits", [(2, 32, 640, 4), (1, 32, 640, 8), (2, 16, 1280, 8), (2, 32, 320, 8), (1, 16, 960, 16), (2, 25, 640, 8),
+                                                (1, 28, 1280, 3), (2, 16, 1280, 7)])
+def test_large_fold(cuda, N, side, cout, splits):
+    """Against the unfused convolution's own output, a last bit of y (its mean square is combined from segments, 2^-20); the same with an
+    offset of 50 standard deviations, where E[x^2] - mean^2 in fp32 would lose 2500 x 2^-24."""
+    torch.manual_seed(side + splits)
+    cin = 1024 * splits // 16
+    x, b, res = rnd(N, side, side, cin), rnd(cout), rnd(N, side, side, cout)
+    w = (torch.randn(cout, 9 * cin, device="cuda") * (9 * cin) ** -0.5).bfloat16()
+    gamma, beta, M, K = rnd(cout), rnd(cout), N * side * side, 9 * cin
+    native.ops().gemm_tuning_import([f"1:{M},{cout},{K},b1,g0|{N},{side},{side},{cin},{cin},3,1,0,0=18,{splits}"])
+    for far in (0, 50):
+        r = (res + far).bfloat16()
+        plain = ops.conv2d(x, w, b, 3, 3, 1, 1, residual=r)
+        for silu in (True, False):
+            out, y = ops.conv2d(x, w, b, 3, 3, 1, 1, residual=r, gn=(gamma, beta, 32, 1e-5, silu))
+            assert torch.equal(out, plain)
+            assert off(y, norm64(out, gamma, beta, 32, 1e-5, silu)) < 2 ** -8
+    raw = torch.full((N, side, side, cout), 7.0, device="cuda", dtype=torch.bfloat16)
+    native.ops().conv2d(x, None, w, raw, b, None, None, None, None, 0, 3, 3, 1, 1, False, 0, 1.0, gn_gamma=gamma, gn_beta=beta,
+                        gn_out=torch.empty_like(raw), gn_groups=32, keep_out=False)
+    two = side * side * cout // 32 * splits >= 81920
+    assert bool((raw == 7).any()) != two
