@@ -130,6 +130,20 @@ bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out,
     *out = it->second;
     return true;
   }
+  auto take = [&](const std::string& k) {
+    it = g_tuned.find(k);
+    if (it == g_tuned.end() || !usable(it->second)) return false;
+    *out = it->second;
+    g_tuned[key] = it->second;
+    return true;
+  };
+  if (!g.conv && g.M <= 64) {
+    // Shipped choices of prompts of a few tokens are by 16 rows: products of 4 to 9 us, of which the tuner's events tell neighbours apart
+    // by chance (5632 x 1024 GLU, 32 rows: 7.7 and 8.3 us, either taken).
+    shai::GemmArgs t = g;
+    t.M = (g.M + 15) / 16 * 16;
+    return take(gemm_key(t) + "|m16" + suffix);
+  }
   std::string bk = gemm_bucket_key(g);
   if (bk.empty()) return false;
   if (*suffix) {
@@ -138,19 +152,9 @@ bool lookup_choice(const shai::GemmArgs& g, const std::string& key, Choice* out,
     // two 14.1, 576 rows 15.5 and 14.4).
     shai::GemmArgs t = g;
     t.M = (g.M + 63) / 64 * 64;
-    it = g_tuned.find(gemm_key(t) + "|m64" + suffix);
-    if (it != g_tuned.end() && usable(it->second)) {
-      *out = it->second;
-      g_tuned[key] = it->second;
-      return true;
-    }
+    if (take(gemm_key(t) + "|m64" + suffix)) return true;
   }
-  bk += suffix;
-  it = g_tuned.find(bk);
-  if (it == g_tuned.end() || !usable(it->second)) return false;
-  *out = it->second;
-  g_tuned[key] = it->second;
-  return true;
+  return take(bk + suffix);
 }
 
 void store_choice(const shai::GemmArgs& g, const std::string& key, const Choice& c, const char* suffix = "") {

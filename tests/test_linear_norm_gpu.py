@@ -130,3 +130,18 @@ def test_choice_of_the_plain_product(cuda, M, key, cfg):
     assert _rel(y, a.float() @ w.float().t() + b.float() + r.float()) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
     own = [e.split("=")[1] for e in ops._K().gemm_tuning_export() if e.startswith(name(M)) and "|norm" in e]
     assert len(own) == 1 if key is None else own == (["18,2"] if "m64" in cfg else [])
+
+
+# up to 64 rows a choice known by their number of 16-row tiles is taken, with the norm and without, and is filed under the rows
+@pytest.mark.parametrize("M,tile", [(1, 16), (16, 16), (17, 32), (49, 64), (64, 64)])
+def test_choice_by_sixteen_rows(cuda, M, tile):
+    N, K = 344, 520
+    name = lambda m: f"0:{m},{N},{K},b1,g0|0,0,0,0,0,0,0,0,0"  # noqa: E731
+    ops._K().gemm_tuning_import([name(tile) + "|m16=1000,2", name(tile) + "|m16|norm=1000,4"])
+    norm, (a, w, b, r) = _norm("rms", N, cuda), _problem(M, N, K, cuda)
+    y, h = ops.linear_norm(a, w, b, r, norm)
+    want = a.float() @ w.float().t() + b.float() + r.float()
+    assert _rel(y, want) < 4e-3 and _rel(h, _want(y, norm)) < 5e-3
+    assert _rel(ops.linear(a, w, b, residual=r), want) < 4e-3
+    have = ops._K().gemm_tuning_export()
+    assert name(M) + "|norm=1000,4" in have and name(M) + "=1000,2" in have
