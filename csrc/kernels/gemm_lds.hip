@@ -126,8 +126,8 @@ constexpr int kNumCfgs = 5;
 // (cached choices run on v4); kNumCfgs + 4 / + 5 the 8-phase ping-pong v4 kernel (gemm_8ph.hip) with 256 / 320 wide tiles,
 // kNumCfgs + 6 / + 7 the same in its persistent form (next tile's operands prefetched under the epilogue).
 constexpr int kV4Cfg = kNumCfgs + 4;
-// kV4Cfg + 4 / + 5: the four-wave kernel (gemm_w4.hip) with 256 x 256 / 192 x 320 tiles (128 x 128 / 96 x 160
-// wave tiles; plain GEMM, GLU, conv; no split-K).
+// kV4Cfg + 4 / + 5: the four-wave kernel (gemm_w4.hip) with 256 x 256 / 256 x 192 tiles (128 x 128 / 128 x 96
+// wave tiles; plain GEMM, GLU, folded LayerNorm; conv with the former; no split-K).
 constexpr int kW4Cfg = kV4Cfg + 4;
 // kW4Cfg + 2: the W-stationary low-K kernel (gemm_ws.hip): K = 320, N a multiple of 320, weights resident in VGPRs,
 // persistent over M (plain / bias / act / GLU / residual / folded LayerNorm; no split-K).
@@ -268,7 +268,7 @@ void launch_gemm2_cfg(const GemmArgs& a, float* ws, int cfg, int splits, hipStre
     return;
   }
   if (cfg == kW4Cfg || cfg == kW4Cfg + 1) {  // whole K per tile: a split-K choice is run unsplit
-    launch_gemm_w4(a, cfg == kW4Cfg ? 256 : 320, s);
+    launch_gemm_w4(a, cfg == kW4Cfg ? 256 : 192, s);
     return;
   }
   if (cfg >= kV4Cfg) {
@@ -315,9 +315,8 @@ void launch_splitk_epilogue(const GemmArgs& a, const float* ws, int splits, hipS
 int gemm2_num_cfgs() { return kDeepCfg + kDeepCfgs; }
 
 // Configs the autotuner races: not the retired v3 indices (kNumCfgs .. + 3; the pipelined kernel held 2 cached
-// shapes when it was removed in round 5 -- every index stays valid for old caches) nor the lab-only 192 x 320
-// four-wave tile.
-bool gemm2_cfg_candidate(int cfg) { return !(cfg >= kNumCfgs && cfg < kV4Cfg) && cfg != kW4Cfg + 1; }
+// shapes when it was removed -- every index stays valid for old caches).
+bool gemm2_cfg_candidate(int cfg) { return !(cfg >= kNumCfgs && cfg < kV4Cfg); }
 
 bool gemm2_cfg_splittable(int cfg) { return cfg != kW4Cfg && cfg != kW4Cfg + 1 && cfg != kWsCfg; }
 
@@ -327,11 +326,11 @@ bool gemm2_cfg_supported(const GemmArgs& a, int cfg) {
   // phase-decomposed upsample conv (upsample == 2) / weight slices: only the v4 kernel maps rows to output pixels
   // and tiles to weight slices
   if (a.upsample == 2 || a.w_slice_rows != 0) return cfg >= kV4Cfg && cfg < kV4Cfg + 4 && gemm4_supported(a);
-  // folded LayerNorm (row_mr): applied by the unsplit epilogues of this file's tiles (plain GEMMs) and of the v4 and the
-  // W-stationary kernel, batch 1.  The small tiles: 6304 x 2304 x 768 37.6 us (256 x 256) instead of v4's 44.9.
+  // folded LayerNorm (row_mr): applied by the unsplit epilogues of this file's tiles (plain GEMMs) and of the v4, the 192-wide four-wave
+  // and the W-stationary kernel, batch 1.  The small tiles: 6304 x 2304 x 768 37.6 us (256 x 256) instead of v4's 44.9.
   if (a.row_mr != nullptr) {
     if (cfg == kWsCfg) return gemm_ws_supported(a);
-    if (a.batch > 1 || (cfg >= kNumCfgs && cfg < kV4Cfg) || cfg == kW4Cfg || cfg == kW4Cfg + 1) return false;
+    if (a.batch > 1 || (cfg >= kNumCfgs && cfg < kV4Cfg) || cfg == kW4Cfg) return false;
     if (cfg >= kV4Cfg && cfg < kV4Cfg + 4) return gemm4_supported(a);
     if (a.conv || a.in_scale != nullptr) return false;
   }
@@ -344,7 +343,7 @@ bool gemm2_cfg_supported(const GemmArgs& a, int cfg) {
     return cfg < kDeepCfg + kDeepCfgs && gemm_deep_supported(a) && !(keeps_order(a) && gemm_deep_wave_groups(cfg - kDeepCfg) > 1);
   if (cfg == kWsCfg) return gemm_ws_supported(a);
   if (cfg == kW4Cfg) return gemm_w4_supported(a);
-  if (cfg == kW4Cfg + 1) return false;  // 192 x 320 four-wave tile: lab only (gemm_w4.hip launch_gemm_w4)
+  if (cfg == kW4Cfg + 1) return !a.conv && gemm_w4_supported(a);
   if (cfg >= kV4Cfg) return cfg < kV4Cfg + 4 && gemm4_supported(a);
   if (cfg >= kNumCfgs) return gemm4_supported(a);  // retired v3 -> v4
   if (a.in_scale != nullptr) return false;
@@ -362,9 +361,9 @@ void gemm2_cfg_info(int cfg, int* bm, int* bn) {
     *bn = -320;
     return;
   }
-  if (cfg == kW4Cfg || cfg == kW4Cfg + 1) {  // four-wave kernel: reported as "4x-256" / "4x-320"
+  if (cfg == kW4Cfg || cfg == kW4Cfg + 1) {  // four-wave kernel: reported as "4x-256" / "4x-192"
     *bm = 4;
-    *bn = cfg == kW4Cfg ? -256 : -320;
+    *bn = cfg == kW4Cfg ? -256 : -192;
     return;
   }
   if (cfg >= kV4Cfg) {  // 8-phase v4 kernel: reported as "8x-<BN>" ("9x-<BN>" persistent)

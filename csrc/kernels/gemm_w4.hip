@@ -3,8 +3,11 @@
 //
 //   C[b, m, n] = gate * act(alpha * sum_k A[b, m, k] * W[b, n, k] + bias[n] + bias2d[m / rpb, n]) + res_alpha * R
 //
-// Configs: 256 x 256 tiles (8 x 8 blocks per wave: LLM / Flux / ViT widths, every multiple of 256); a 192 x 320
-// lab config (6 x 10 blocks per wave) for the SD2.1 channel widths lost to v4 (see launch_gemm_w4).
+// Configs: 256 x 256 tiles (8 x 8 blocks per wave: LLM / Flux / ViT widths, every multiple of 256) and 256 x 192 ones (8 x 6,
+// products only) where they fit the 256 CUs better: 4096 x 3072 x 1024 is 192 tiles of the one (42.2 us with a residual, 34.8
+// without) and 256 of the other (34.9 and 30.1), 5122 x 2304 x 768 with a folded LayerNorm 32.3 and 25.5. 192 x 320 tiles (6 x 10)
+// for the SD2.1 channel widths lost to v4 on every shape (unet64_320 conv 949 and 1135 TF/s), and 256 x 320 ones (8 x 10 blocks, 320
+// accumulators) spill 32 to 85 VGPRs.
 //
 // Why: the v4 kernel (gemm_8ph.hip) pairs two waves per SIMD that each own a 128 x 64 (or 128 x 80) slice;
 // per 64-deep K-tile a CU then reads 8 x (128 + 80) x 128 B = 213 KB of fragments out of LDS and re-syncs
@@ -49,13 +52,13 @@ template <int BMB, int BNB>
 struct W4T {
   static constexpr int BM = 32 * BMB, BN = 32 * BNB;   // 2 x 2 waves of 16 BMB x 16 BNB
   static constexpr int WM = BM / 2, WN = BN / 2;         // rows / columns per wave
-  static constexpr int STAGE = (BM + BN) * W4_BK;        // elements per LDS stage (64 KB for both configs)
+  static constexpr int STAGE = (BM + BN) * W4_BK;        // elements per LDS stage (64 KB, 56 KB)
   static constexpr int AJ = BM / 32, WJ = BN / 32;       // DMA instructions (8 rows) per wave per K-tile
-  static constexpr int GT = AJ + WJ;                     // 16
-  static constexpr int NF = BMB + BNB;                   // fragments per k-step (16)
+  static constexpr int GT = AJ + WJ;                     // 16, 14
+  static constexpr int NF = BMB + BNB;                   // fragments per k-step (16, 14)
   static constexpr int RPG = (NF + BMB / 2 - 1) / (BMB / 2);  // fragment reads per MFMA group (first half)
   static constexpr int DPG = (GT + BMB - 1) / BMB;             // DMA instructions per MFMA group
-  static_assert(GT == 16 && NF == 16 && BNB % 2 == 0, "geometry");
+  static_assert(GT <= 16 && NF <= 16 && BMB % 2 == 0 && BNB % 2 == 0, "geometry");
 };
 
 // sched_group_barrier needs literal counts: the per-group counts of the interleave are template arguments
@@ -236,7 +239,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
   for (int g = 0; g < T::GT; ++g) dma(0, 0, g);
 #pragma unroll
   for (int g = 0; g < T::GT; ++g) dma(1, 1, g);   // nk == 1: zero fill past K, never read
-  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(T::GT) : "memory");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -304,30 +307,61 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
   bf16_t* C = p.C + (long)b * p.batch_c;
   const bf16_t* R = p.residual ? p.residual + (long)b * p.batch_r : nullptr;
   const uintptr_t ptrs = (uintptr_t)C | (uintptr_t)R | (uintptr_t)p.bias | (uintptr_t)p.bias2d | (uintptr_t)p.gate;
-  const bool full = n0 + BN <= p.N && ((p.ldc | (R ? p.ldr : 0)) & 7) == 0 && (ptrs & 15) == 0 &&
+  const bool full = (p.N & 7) == 0 && ((p.ldc | (R ? p.ldr : 0)) & 7) == 0 && (ptrs & 15) == 0 &&
                     (p.bias2d == nullptr || (p.bias2d_ld & 7) == 0) && (p.gate == nullptr || (p.gate_stride & 7) == 0);
   constexpr int NQ = BNB / 2;
+  if constexpr (BNB == 6) {  // with 256 accumulators the factors spill, and the tile was the best one for no folded product
+    if (p.row_mr != nullptr) {  // LayerNorm of A folded in (host: batch 1): acc <- rstd[m] * (acc - mean[m] * s[n]), W carries the gain
+      float2 mr[BMB];
+#pragma unroll
+      for (int i = 0; i < BMB; ++i) mr[i] = *reinterpret_cast<const float2*>(p.row_mr + 2 * (long)min(m0 + wr * WM + 16 * i + fr, p.M - 1));
+#pragma unroll
+      for (int jb = 0; jb < BNB; ++jb) {
+        const int n = n0 + wc * WN + (jb >> 1) * 32 + 8 * fq + 4 * (jb & 1);
+        float sc[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[e] = n + e < p.N ? p.col_s[n + e] : 0.f;
+#pragma unroll
+        for (int i = 0; i < BMB; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][jb][e] = mr[i].y * fmaf(-mr[i].x, sc[e], acc[i][jb][e]);
+      }
+    }
+  }
   if (full) {
-    // Rows may end inside the tile: it reads clamped rows and guards its stores.  Taken through the element-wise form below, such a
+    // Rows and columns may end inside the tile: it reads clamped ones and guards its stores.  Taken through the element-wise form below, such a
     // tile took several times the others' time: 8000 x 4096 x 4096 275 -> 224 us, 8000 x 28672 x 4096 gated 1575 -> 1429, 1600 x
     // 4096 x 14336 339 -> 307; whole tiles as before (8192 x 28672 x 4096 1440 and 1435; a second copy of the epilogue for them: 3 %
-    // slower on gated products).
+    // slower on gated products). Columns likewise: 16384 x 640 x 640 115 -> 34, 256 x 192 tiles 62 -> 27.
     float bq[NQ][8];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      if (p.bias) unpack8(*reinterpret_cast<const uint4_*>(p.bias + n0 + wc * WN + q * 32 + 8 * fq), bq[q]);
+      if (p.bias) unpack8(*reinterpret_cast<const uint4_*>(p.bias + min(n0 + wc * WN + q * 32 + 8 * fq, p.N - 8)), bq[q]);
       else
 #pragma unroll
         for (int e = 0; e < 8; ++e) bq[q][e] = 0.f;
     }
+    // the residual of IG rows in the registers that the fragments have left: asked for block by block, each was waited for by itself
+    // (us, 8192 x 4096 x 4096 241 -> 228 and without a residual 214, 8192 x 4096 x 14336 740 -> 720, 4096 x 1024 x 1024 39.8 -> 33.6)
+    constexpr int IG = BNB == 6 ? 8 : 4;
+    using res_t = std::conditional_t<GLU, uint2_, uint4_>;
+    res_t rr[IG][NQ];
 #pragma unroll
     for (int i = 0; i < BMB; ++i) {
+      if (i % IG == 0 && R) {
+#pragma unroll
+        for (int u = 0; u < IG; ++u)
+#pragma unroll
+          for (int q = 0; q < NQ; ++q)
+            rr[u][q] = *reinterpret_cast<const res_t*>(R + (long)min(m0 + wr * WM + 16 * (i + u) + fr, p.M - 1) * p.ldr +
+                                                       (min(n0 + wc * WN + q * 32 + 8 * fq, p.N - 8) >> (GLU ? 1 : 0)));
+      }
       const int row = m0 + wr * WM + 16 * i + fr, m = min(row, p.M - 1);
       const bf16_t* b2 = p.bias2d ? p.bias2d + (long)(m / p.rows_per_bias2d) * p.bias2d_ld : nullptr;
       const bf16_t* gr = p.gate ? p.gate + ((long)b * p.M + m) / p.rows_per_gate * p.gate_stride : nullptr;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
-        const int n = n0 + wc * WN + q * 32 + 8 * fq;
+        const int col = n0 + wc * WN + q * 32 + 8 * fq, n = min(col, p.N - 8);
         float v[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -350,14 +384,14 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
             o[2] *= bf2f(g2[1] & 0xffff); o[3] *= bf2f(g2[1] >> 16);
           }
           if (R) {
-            const uint2_ r2 = *reinterpret_cast<const uint2_*>(R + (long)m * p.ldr + (n >> 1));
+            const uint2_ r2 = rr[i % IG][q];
             o[0] += bf2f(r2[0] & 0xffff) * p.res_alpha; o[1] += bf2f(r2[0] >> 16) * p.res_alpha;
             o[2] += bf2f(r2[1] & 0xffff) * p.res_alpha; o[3] += bf2f(r2[1] >> 16) * p.res_alpha;
           }
           uint2_ w;
           w[0] = pack2(o[0], o[1]);
           w[1] = pack2(o[2], o[3]);
-          if (row < p.M) *reinterpret_cast<uint2_*>(C + (long)m * p.ldc + (n >> 1)) = w;
+          if (row < p.M && col < p.N) *reinterpret_cast<uint2_*>(C + (long)m * p.ldc + (n >> 1)) = w;
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = apply_act<ACT>(v[e]);
@@ -369,17 +403,17 @@ __global__ void __launch_bounds__(256, 1) gemm_w4_kernel(const GemmArgs p) {
           }
           if (R) {
             float r8[8];
-            unpack8(*reinterpret_cast<const uint4_*>(R + (long)m * p.ldr + n), r8);
+            unpack8(rr[i % IG][q], r8);
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] += r8[e] * p.res_alpha;
           }
           const uint4_ w = pack8(v);
-          if (row < p.M) *reinterpret_cast<uint4_*>(C + (long)m * p.ldc + n) = w;
+          if (row < p.M && col < p.N) *reinterpret_cast<uint4_*>(C + (long)m * p.ldc + n) = w;
         }
       }
     }
   } else {
-    // columns that end inside the tile, odd strides and bases: element-wise, guarded (no array indexed at run time: every index is
+    // odd widths, strides and bases: element-wise, guarded (no array indexed at run time: every index is
     // unrolled, no early loop exits -- a run-time-bounded loop over the accumulators sends all of them to scratch)
 #pragma unroll
     for (int i = 0; i < BMB; ++i) {
@@ -432,17 +466,7 @@ static void w4_go(const GemmArgs& a, hipStream_t s) {
 }
 
 template <int BMB, int BNB>
-static void w4_dispatch(const GemmArgs& a, hipStream_t s) {
-  if (a.conv) {
-    if (a.upsample) {
-      if (a.act == ACT_SILU) w4_go<BMB, BNB, 2, false, ACT_SILU>(a, s);
-      else w4_go<BMB, BNB, 2, false, ACT_NONE>(a, s);
-    } else {
-      if (a.act == ACT_SILU) w4_go<BMB, BNB, 1, false, ACT_SILU>(a, s);
-      else w4_go<BMB, BNB, 1, false, ACT_NONE>(a, s);
-    }
-    return;
-  }
+static void w4_product(const GemmArgs& a, hipStream_t s) {
   if (a.glu) {
     if (a.act == ACT_SILU) w4_go<BMB, BNB, 0, true, ACT_SILU>(a, s);
     else if (a.act == ACT_GELU_TANH) w4_go<BMB, BNB, 0, true, ACT_GELU_TANH>(a, s);
@@ -459,19 +483,20 @@ static void w4_dispatch(const GemmArgs& a, hipStream_t s) {
   }
 }
 
-// bn = 256: 256 x 256 tiles; bn = 320 (lab builds only): 192 x 320 tiles.  The 192 x 320 config lost to v4's
-// persistent 256 x 320 kernel on every SD2.1 shape in the round-4 lab (unet64_320 conv 949 vs 1135 TF/s: 5.3
-// tile rounds per CU instead of 4, and ~10 % slower per tile), and a 256 x 320 four-wave tile (8 x 10 blocks,
-// 320 accumulators) spills 32-85 VGPRs, so production keeps v4 for the 320-wide problems.
+// bn: columns of a tile, 256 or 192 (products only)
 void launch_gemm_w4(const GemmArgs& a, int bn, hipStream_t s) {
-#ifdef SHAI_GEMM_LAB
-  if (bn == 320) {
-    w4_dispatch<6, 10>(a, s);
+  if (!a.conv) {
+    if (bn == 192) w4_product<8, 6>(a, s);
+    else w4_product<8, 8>(a, s);
     return;
   }
-#endif
-  (void)bn;
-  w4_dispatch<8, 8>(a, s);
+  if (a.upsample) {
+    if (a.act == ACT_SILU) w4_go<8, 8, 2, false, ACT_SILU>(a, s);
+    else w4_go<8, 8, 2, false, ACT_NONE>(a, s);
+  } else {
+    if (a.act == ACT_SILU) w4_go<8, 8, 1, false, ACT_SILU>(a, s);
+    else w4_go<8, 8, 1, false, ACT_NONE>(a, s);
+  }
 }
 
 }  // namespace shai

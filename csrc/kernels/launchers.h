@@ -209,7 +209,7 @@ void launch_gemm2_cfg(const GemmArgs& a, float* ws, int cfg, int splits, hipStre
 int gemm2_num_cfgs();
 bool gemm2_cfg_supported(const GemmArgs& a, int cfg);
 bool gemm2_cfg_splittable(int cfg);  // false: the config always runs the whole K (split-K choices are moot)
-// v5: four-wave GEMM / implicit-GEMM conv (gemm_w4.hip), bn = 256: 256 x 256 tiles, bn = 320: 192 x 320 tiles
+// v5: four-wave GEMM / implicit-GEMM conv (gemm_w4.hip), 256 x bn tiles, bn = 256 or, products only, 192
 bool gemm_w4_supported(const GemmArgs& a);
 void launch_gemm_w4(const GemmArgs& a, int bn, hipStream_t s);
 // small tiles with a deep ring of K-tiles in flight (gemm_deep.hip)

@@ -146,3 +146,28 @@ def test_rows_do_not_depend_on_how_many(cuda, N, K, glu, rms):
     want = call(16000)
     for rows in (4096, 4864, 9364):
         assert torch.equal(call(rows), want[:rows])
+
+
+# four waves of 128 x 128 and of 128 x 96: columns that end inside the tile (by eights, and not), in a wave's first and second half; the
+# latter's folded LayerNorm, whose factors the products' sums take before bias and activation
+@pytest.mark.parametrize("act,glu", [(None, False), ("gelu", False), ("gelu_tanh", True)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (257, 192, 64), (255, 200, 72), (130, 388, 128), (513, 456, 776)])
+@pytest.mark.parametrize("cfg", [13, 14])
+def test_four_waves(cuda, cfg, M, N, K, act, glu):
+    if glu and N % 8:
+        pytest.skip("gated widths are multiples of 8")
+    a, w, b, r = _problem(M, N, K, cuda)
+    no = N // 2 if glu else N
+    r = r[:, :no].contiguous()
+    f = (lambda y: y[:, 0::2] * ACTS[act](y[:, 1::2])) if glu else ACTS[act]
+    y = a.float() @ w.float().t()
+    out = torch.full((M + 1, no), 7.0, device=cuda, dtype=torch.bfloat16)
+    out[:M] = r
+    ops.gemm_into(a, w, out[:M], b, act=act, residual=out[:M], glu=glu, force_cfg=cfg)
+    assert _close(out[:M], f(y + b.float()) + r.float()) and bool((out[M] == 7).all())
+    if cfg == 13:
+        return
+    g = torch.Generator(device=cuda).manual_seed(N)
+    mr, s = torch.rand(M, 2, generator=g, device=cuda) + 0.5, torch.randn(N, generator=g, device=cuda)
+    ops._K().gemm(a, w, out[:M], b, None, 1, r, 1.0, 1.0, ops.act_id(act), glu, None, 1, cfg, -1.0, None, mr, s)
+    assert _close(out[:M], f(mr[:, 1:] * (y - mr[:, :1] * s) + b.float()) + r.float()) and bool((out[M] == 7).all())
