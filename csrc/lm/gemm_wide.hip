@@ -160,29 +160,182 @@ __device__ __forceinline__ void tile(const GemmArgs& p, bf16_t* smem, int m0, in
   }
 }
 
+struct Place {
+  int m0, n0;
+};
+
+// Tiles one after the other, the next one's first two k-tiles fetched during the last two of the one before: no launch, no first loads to
+// wait for, and the stores go out beside the next products (the first wait counts them, as they are younger than what it waits for).  A
+// register kept over both halves of an epilogue would spill: one path of stores, no branches in it.  Rows and columns take 16-byte stores, K is at least two k-tiles, no rows are
+// gathered.  next(Place&) gives the workgroup's next tile, false: none.
+template <typename Next>
+__device__ __forceinline__ void chain(const GemmArgs& p, bf16_t* smem, Place at, Next next) {
+  constexpr int NB = 8, B = kTile, FR = 2 * NB, STAGE = 2 * B * 64, NQ = NB / 2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wid >> 1, wn = wid & 1;
+  const __amdgpu_buffer_rsrc_t rW = rsrc(p.W, (long)p.N * p.K * 2), rA = rsrc(p.A, ((long)(p.a_rows - 1) * p.lda + p.K) * 2);
+
+  // byte offset of this lane's 16-byte chunk of the NB + NB row groups its wave stages, at k = 0; the bank swizzle is on the source.
+  // W's rows are permuted inside pairs of blocks of 16, so that a lane's results are 8 neighbouring columns.
+  const int lrow = lane >> 3, lpos = lane & 7;
+  uint32_t off[FR];
+  auto place = [&](const Place& t, bool any) {
+    int lr = lrow, lp = lpos;
+    asm volatile("" : "+v"(lr), "+v"(lp));
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int r = wid * (B / 4) + j * 8 + lr, ch = (lp ^ ((r >> 1) & 7)) * 8, m = t.m0 + r;
+      const int wave = r / (B / 2), l = r % (B / 2), n = t.n0 + wave * (B / 2) + (l >> 5) * 32 + ((l & 15) >> 2) * 8 + ((l >> 4) & 1) * 4 + (l & 3);
+      off[j] = any && m < p.M ? (uint32_t)(((long)m * p.lda + ch) * 2) : kOob;
+      off[NB + j] = any && n < p.N ? (uint32_t)(((long)n * p.K + ch) * 2) : kOob;
+    }
+  };
+  const int nk = p.K / 64;
+  int base = 0;                                  // the tile's first k-tile in the sequence of all, which the stages follow
+  // row group g of the place's k-tile k into the stage of the tile's k-tile t
+  auto dma = [&](int t, int k, int g) {
+    bf16_t* dst = smem + ((base + t) & 1) * STAGE + ((g < NB ? 0 : B) + wid * (B / 4) + (g % NB) * 8) * 64;
+    dma16(g < NB ? rA : rW, dst, off[g] + (uint32_t)k * 128u);
+  };
+  // fragment f of k-step s: W's blocks of 16 rows first, the first MFMAs need all of them
+  const int fr = lane & 15, fq = lane >> 4;
+  typedef bf16x8 Set[FR];
+  auto read = [&](int t, int s, int f, Set& x) {
+    const int row = f < NB ? B + wn * (B / 2) + 16 * f : wm * (B / 2) + 16 * (f - NB);
+    x[f] = *reinterpret_cast<const bf16x8*>(smem + ((base + t) & 1) * STAGE + (row + fr) * 64 + (((fq + 4 * s) ^ ((fr >> 1) & 7)) << 3));
+  };
+  // a set is redefined after its inline wait: the compiler's own wait counts do not see that one
+  auto landed = [](Set& x) {
+#pragma unroll
+    for (int f = 0; f < FR; ++f) asm volatile("" : "+v"(x[f]));
+  };
+
+  float4_ acc[NB][NB];
+  Set x0, x1;
+  place(at, true);
+#pragma unroll
+  for (int g = 0; g < 2 * FR; ++g) dma(g / FR, g / FR, g % FR);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FR) : "memory");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int f = 0; f < FR; ++f) read(0, 0, f, x0);
+
+  auto half0 = [&](int t, auto first) {
+#pragma unroll
+    for (int g = 0; g < NB; ++g) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (g < NB / 2) read(t, 1, 4 * g + u, x1);
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x0[j], x0[NB + g], decltype(first)::value ? float4_{} : acc[g][j], 0, 0, 0);
+    }
+    interleave<NB, 0>(std::make_integer_sequence<int, NB>{});
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // k: the place's k-tile that goes into the stage of t + 2; behind: the last tile's stores are younger than the loads waited for
+  auto half1 = [&](int t, int k, bool behind) {
+    if (behind) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NB * NQ) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    landed(x1);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < NB; ++g) {
+      dma(t + 2, k, 2 * g);
+      dma(t + 2, k, 2 * g + 1);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (g < NB / 2) read(t + 1, 0, 4 * g + u, x0);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x1[j], x1[NB + g], acc[g][j], 0, 0, 0);
+    }
+    interleave<NB, 2>(std::make_integer_sequence<int, NB>{});
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    landed(x0);
+  };
+
+  bf16_t* C = static_cast<bf16_t*>(p.C);
+  for (;;) {
+    Place to;
+    const bool more = next(to);
+    half0(0, std::true_type{});
+    for (int t = 0; t + 1 < nk; ++t) {
+      if (t == nk - 2) place(to, more);
+      half1(t, t + 2 < nk ? t + 2 : t + 2 - nk, base > 0 && t == 0);
+      half0(t + 1, std::false_type{});
+    }
+    half1(nk - 1, 1, false);
+
+    const __amdgpu_buffer_rsrc_t rC = rsrc(C + (long)at.m0 * p.ldc, 0x7fffffffL);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int r = wm * (B / 2) + 16 * i + fr, m = at.m0 + r;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int n = at.n0 + wn * (B / 2) + 32 * q + 8 * fq;
+        float4_ u = acc[i][2 * q], v = acc[i][2 * q + 1];
+        const bool su = p.epi == EPI_RELU2 && n < p.n_act, sv = p.epi == EPI_RELU2 && n + 4 < p.n_act;   // epilogue_cols without branches
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = fmaxf(u[e], 0.f), y = fmaxf(v[e], 0.f);
+          u[e] = su ? x * x : u[e];
+          v[e] = sv ? y * y : v[e];
+        }
+        const uint4_ o = {pack2(u[0], u[1]), pack2(u[2], u[3]), pack2(v[0], v[1]), pack2(v[2], v[3])};
+        // always NB * NQ stores: they are counted above
+        __builtin_amdgcn_raw_buffer_store_b128(o, rC, m < p.M && n < p.n_main ? ((uint32_t)r * (uint32_t)p.ldc + (uint32_t)n) * 2u : kOob, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!more) return;
+    at = to;
+    base += nk;
+  }
+}
+
 }  // namespace
 
-// Workgroups 0 .. whole - 1 take one tile each, every four behind them the quarters of one of the remaining tiles.
-__global__ void __launch_bounds__(256, 1) gemm_wide_kernel(const GemmArgs p, int whole) {
+// Workgroups 0 .. step - 1 take tiles step apart of the first `whole`, every four behind them the quarters of one of the remaining tiles.
+// The columns of tiles from `lines` on, with side columns, come last: a chain (step < whole) has none.
+__global__ void __launch_bounds__(256, 1) gemm_wide_kernel(const GemmArgs p, int whole, int step, int lines) {
   extern __shared__ __attribute__((aligned(16))) bf16_t smem[];
   const int tiles_m = p.tiles ? p.n_tiles : (p.M + kTile - 1) / kTile, tiles_n = (p.N + kTile - 1) / kTile;
-  int bid = blockIdx.x, part = 0;
-  const bool quarter = bid >= whole;
-  if (quarter) {
-    part = (bid - whole) & 3;
-    bid = whole + ((bid - whole) >> 2);
-  } else {
-    const int xcd = bid & 7, q = whole >> 3, r = whole & 7;
-    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
-  }
   constexpr int GROUP = 8;
-  const int group = bid / (GROUP * tiles_n), first_m = group * GROUP;
-  const int gsize = min(tiles_m - first_m, GROUP);
-  const int in_group = bid - group * GROUP * tiles_n;
-  const int mt = first_m + in_group % gsize, n0 = (in_group / gsize) * kTile;
-  if (quarter) {
+  auto tile_of = [&](int bid, int& mt, int& n0) {
+    const int first_n = bid < tiles_m * lines ? 0 : lines, cols = first_n ? tiles_n - lines : lines;
+    bid -= tiles_m * first_n;
+    const int group = bid / (GROUP * cols), first_m = group * GROUP;
+    const int gsize = min(tiles_m - first_m, GROUP);
+    const int in_group = bid - group * GROUP * cols;
+    mt = first_m + in_group % gsize;
+    n0 = (first_n + in_group / gsize) * kTile;
+  };
+  int bid = blockIdx.x, mt, n0;
+  if (bid >= step) {
+    const int part = (bid - step) & 3;
+    tile_of(whole + ((bid - step) >> 2), mt, n0);
     const int m = mt * kTile + (part >> 1) * 128, n = n0 + (part & 1) * 128;
     if (m < p.M && n < p.N) tile<4, 4>(p, smem, m, p.M, n, static_cast<const bf16_t*>(p.W));
+    return;
+  }
+  auto take = [&] {
+    const int xcd = bid & 7, q = whole >> 3, r = whole & 7;
+    tile_of((xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3), mt, n0);
+    bid += step;
+  };
+  take();
+  if (step < whole) {
+    chain(p, smem, Place{mt * kTile, n0}, [&](Place& t) {
+      if (bid >= whole) return false;
+      take();
+      t = Place{mt * kTile, n0};
+      return true;
+    });
     return;
   }
   int m0 = mt * kTile, m_end = p.M, expert = 0;
@@ -196,10 +349,16 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(const GemmArgs p, int
 }
 
 void launch_gemm_wide(const GemmArgs& a, hipStream_t s) {
-  const int tiles = (a.tiles ? a.n_tiles : (a.M + kTile - 1) / kTile) * ((a.N + kTile - 1) / kTile), left = tiles % 256;
-  const int whole = !a.tiles && tiles > 256 && left <= 128 ? tiles - left : tiles;
+  const int tiles_m = a.tiles ? a.n_tiles : (a.M + kTile - 1) / kTile, tiles_n = (a.N + kTile - 1) / kTile, tiles = tiles_m * tiles_n;
+  const int left = tiles % 256, whole = !a.tiles && tiles > 256 && left <= 128 ? tiles - left : tiles;
+  // A chain where whole rounds are more than one and have neither side columns nor rows without 16-byte stores.  Those columns are last, so
+  // that they are among the quarters.  us: 7700 x 14848 x 2048 414 -> 396, 7700 x 17424 with 16 side columns 500 -> 481, 7700 x
+  // 16640 465 -> 462, 8192 x 8192 x 8192 837 -> 824, and all of a prompt of 7 x 1100 tokens 9.29 -> 8.89 ms; one round is the slower through the direct stores (7700 x 2048 x 10496: 262 and 269).
+  const int lines = a.n_main == a.N ? tiles_n : a.n_main / kTile;
+  const bool chain = !a.tiles && !a.gather && whole > 256 && a.K >= 128 && a.ldc % 8 == 0 && a.n_main % 8 == 0 && whole <= tiles_m * lines;
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-  gemm_wide_kernel<<<whole + 4 * (tiles - whole), 256, kLds, s>>>(a, whole);
+  const int step = chain ? 256 : whole;
+  gemm_wide_kernel<<<step + 4 * (tiles - whole), 256, kLds, s>>>(a, whole, step, chain ? lines : tiles_n);
   SHAI_CHECK_LAUNCH();
 }
 

@@ -35,6 +35,25 @@ def test_plain(cuda, M, N, K):
     assert bool((out[:, :8] == 3).all()) and bool((out[:, N + 8:] == 3).all())
 
 
+# more than one whole round, tile after tile in a workgroup: two, three and odd counts of k-tiles; a last row and columns that end inside
+# a tile, the last round not whole (391 tiles), cut in quarters (544 and 32 more) or with side columns among the quarters (512 and 64)
+@pytest.mark.parametrize("M,N,side,act", [(4100, 5640, 0, None), (4352, 8192, 0, 4100), (4096, 8976, 272, None), (8191, 4352, 0, None)])
+@pytest.mark.parametrize("K", [128, 192, 1600])
+def test_chain(cuda, M, N, side, act, K):
+    a, w = _problem(M, N, K, cuda, spare=8)
+    want = a.double() @ w.double().T
+    if side:
+        main, extra = lm.matmul_with_side(a, w, side)
+        assert _rel(main, want[:, :-side]) < 2.3e-3 and _rel(extra, want[:, -side:]) < 1e-5
+        return
+    out = torch.full((M + 1, N + 16), 3.0, device=cuda, dtype=torch.bfloat16)
+    lm.matmul_joint(a, w, out[:M, 8:N + 8], act or 0, 0)
+    if act:
+        want[:, :act] = want[:, :act].clamp(min=0) ** 2
+    assert _rel(out[:M, 8:N + 8], want) < 2.3e-3
+    assert bool((out[:, :8] == 3).all()) and bool((out[:, N + 8:] == 3).all()) and bool((out[M] == 3).all())
+
+
 # smaller tiles: fewer k-tiles than the ring holds, one more, many; 64 x 64, one 128 x 128 tile per CU and more than one
 @pytest.mark.parametrize("M,N", [(65, 64), (129, 452), (300, 2052), (1030, 4100), (2100, 4100)])
 @pytest.mark.parametrize("K", [64, 192, 256, 320, 2112])
