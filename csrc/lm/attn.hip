@@ -181,9 +181,11 @@ __global__ void __launch_bounds__(256, DK + DV > (LAT ? 320 : 256) ? 1 : 2) attn
   bf16_t* sV = smem + 2 * KT * DK;
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, fh = lane >> 5;
-  const int b = blockIdx.z, h = blockIdx.y;
+  // the last queries, which have the most keys, first: the others even out the end of the grid (7 x 1100 tokens, 16 heads: about 107 ->
+  // 71 us, of a pass of 8.89 ms 0.14)
+  const int b = blockIdx.y, h = blockIdx.x;
   const int hk = h / (p.H / p.G);
-  const int q_len = p.q_lens[b], q0 = blockIdx.x * 128;
+  const int q_len = p.q_lens[b], q0 = (gridDim.z - 1 - blockIdx.z) * 128;
   if (q0 >= q_len) return;
   const int ctx = p.ctx[b], c_off = ctx - q_len;
   const int qi = q0 + wid * 32 + fr, pos = qi + c_off, lo = LAT ? 0 : first_key(p, pos);
@@ -408,7 +410,7 @@ static void prefill(const AttnArgs& a, hipStream_t s) {
   constexpr int lds = 2 * 64 * (DK + DV) * 2;
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attn_prefill_kernel<DK, DV, LAT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  attn_prefill_kernel<DK, DV, LAT><<<dim3((a.max_q + 127) / 128, a.H, a.B), 256, lds, s>>>(a);
+  attn_prefill_kernel<DK, DV, LAT><<<dim3(a.H, a.B, (a.max_q + 127) / 128), 256, lds, s>>>(a);
 }
 
 void launch_latent_prefill(const AttnArgs& a, hipStream_t s) {
