@@ -531,15 +531,11 @@ __global__ void __launch_bounds__(256) gn_apply_kernel(const bf16_t* __restrict_
     b0 = *reinterpret_cast<const float4_*>(sh);
     b1 = *reinterpret_cast<const float4_*>(sh + 4);
   };
+  uint4_ v = src[pix * srcw];
   load_ss();
-  for (; i < total8; i += stride, pix += pstep) {
-    if (pix >= next) {  // crossed into another image (rare unless HW is small)
-      n = (int)(pix / HW);
-      next = (long)(n + 1) * HW;
-      load_ss();
-    }
+  while (true) {
     float f[8];
-    unpack8(src[pix * srcw], f);
+    unpack8(v, f);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       f[k] = f[k] * a0[k] + b0[k];
@@ -549,6 +545,15 @@ __global__ void __launch_bounds__(256) gn_apply_kernel(const bf16_t* __restrict_
 #pragma unroll
       for (int k = 0; k < 8; ++k) f[k] = silu_f(f[k]);
     reinterpret_cast<uint4_*>(out)[i] = pack8(f);
+    i += stride;
+    pix += pstep;
+    if (i >= total8) return;
+    v = src[pix * srcw];
+    if (pix >= next) {  // crossed into another image (rare unless HW is small)
+      n = (int)(pix / HW);
+      next = (long)(n + 1) * HW;
+      load_ss();
+    }
   }
 }
 
@@ -581,8 +586,13 @@ void launch_groupnorm_stats(const GroupNormArgs& a, hipStream_t s) {
 
 void launch_groupnorm_apply(const GroupNormArgs& a, hipStream_t s) {
   const long total8 = (long)a.N * a.HW * a.C / 8;
-  long blocks = (total8 + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
+  // A thread has one vector, more in very large tensors: with a few each, the workgroups of the last round had the chip to themselves
+  // (us, 4096 workgroups and this: 16 x 4096 x 640 43.5 and 34.5, x 960 71.1 and 49.4, 16 x 1024 x 1280 23.8 and 19.7, 8 x 16384 x 512 69.5
+  // and 51.4, 8 x 262144 x 256 458 and 422). Where 4096 come out even with up to four vectors they save loads of scale and shift (1 x
+  // 65536 x 256 14.7 and 16.0, 1 x 262144 x 128 26.2 and 27.7). Two or four vectors on their way in a thread: slower at every size.
+  constexpr long kEven = 4096 * 256;
+  long blocks = total8 % kEven == 0 && total8 <= 4 * kEven ? 4096 : (total8 + 255) / 256;
+  if (blocks > 65536) blocks = 65536;
   // grid threads a multiple of C / 8 (the kernel keeps one channel vector per thread)
   const int C8 = a.C / 8;
   int g = C8, b = 256;
