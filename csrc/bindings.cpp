@@ -1200,6 +1200,21 @@ void gemm(const Tensor& a, const Tensor& w, const Tensor& c, const optional<Tens
   run_gemm(g, a, a_bytes, (long)g.N * g.ldw * 2, 0);
 }
 
+// Whether attn_proj_norm takes these strides, types and addresses (the sizes that are worth it: the caller's; in Python this took longer
+// than the launches).
+bool attn_proj_fits(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& w, const optional<Tensor>& bias, const Tensor& residual,
+                    const Tensor& gamma, const optional<Tensor>& beta, const optional<Tensor>& attn_bias) {
+  auto at = [](const Tensor& t, int64_t bytes) { return t.scalar_type() == at::kBFloat16 && reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0; };
+  const int64_t H = q.size(2), D = q.size(3);
+  auto heads = [&](const Tensor& t) {
+    return at(t, 16) && t.dim() == 4 && t.stride(3) == 1 && t.stride(2) == D && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0;
+  };
+  return D == 64 && heads(q) && heads(k) && heads(v) && k.size(1) <= 256 && k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(2) == H &&
+         at(w, 16) && w.size(0) % 16 == 0 && w.size(1) == H * D && w.stride(1) == 1 && w.stride(0) % 8 == 0 && (!bias || at(*bias, 8)) &&
+         at(residual, 8) && at(gamma, 8) && (!beta || at(*beta, 8)) &&
+         (!attn_bias || (attn_bias->is_contiguous() && attn_bias->scalar_type() == at::kBFloat16));
+}
+
 // y = attention(q, k, v) w^T + bias + residual and out = RMS norm or LayerNorm of y, in two launches: every head's attention with its
 // part of the product, then the sum of the parts with the norm.
 void attn_proj_norm(const Tensor& q, const Tensor& k, const Tensor& v, const optional<Tensor>& kv_lens, const optional<Tensor>& attn_bias,
@@ -2057,6 +2072,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("conv2d(Tensor x, Tensor? x2, Tensor w, Tensor(a!) out, Tensor? bias, Tensor? bias2d, Tensor? residual, Tensor? in_scale, Tensor? in_shift, int in_act, int kh, int kw, int stride, int pad, bool upsample, int act, float res_alpha, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, bool up_phases=False, Tensor? gn_gamma=None, Tensor? gn_beta=None, Tensor(d!)? gn_out=None, int gn_groups=0, float gn_eps=1e-5, bool gn_silu=False, bool keep_out=True) -> ()");
   m.def("groupnorm_one(Tensor x, Tensor? x2, Tensor? gamma, Tensor? beta, Tensor(a!) out, int G, float eps, bool silu) -> ()");
   m.def("groupnorm_one_supported(int HW, int C, int G, bool fold) -> bool", &groupnorm_one_supported);
+  m.def("attn_proj_fits(Tensor q, Tensor k, Tensor v, Tensor w, Tensor? bias, Tensor residual, Tensor gamma, Tensor? beta, Tensor? attn_bias) -> bool");
   m.def("attn_proj_norm(Tensor q, Tensor k, Tensor v, Tensor? kv_lens, Tensor? attn_bias, float scale, bool causal, Tensor w, Tensor? bias, Tensor residual, Tensor gamma, Tensor? beta, Tensor(a!) y, Tensor(b!) out, float eps, bool rms) -> ()");
   m.def("flash_attn(Tensor q, Tensor k, Tensor v, Tensor(a!) o, float scale, bool causal, int causal_offset, Tensor? kv_lens, Tensor? q_lens, Tensor? bias, Tensor? block_table) -> ()");
   m.def("paged_attn_varlen(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor kv_lens, Tensor q_lens, Tensor q_start, int max_q, float scale, bool causal) -> ()");
@@ -2099,6 +2115,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("gemm", &gemm);
   m.impl("gemm_norm", &gemm_norm);
   m.impl("attn_proj_norm", &attn_proj_norm);
+  m.impl("attn_proj_fits", &attn_proj_fits);
   m.impl("dequant_fp8", &dequant_fp8);
   m.impl("gemm_f8", &gemm_f8);
   m.impl("gemm_lnout", &gemm_lnout);

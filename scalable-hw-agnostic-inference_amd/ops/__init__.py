@@ -634,13 +634,8 @@ def attention_linear_norm(q, k, v, w, bias, residual, norm, scale: Optional[floa
 
 def _attention_linear_fits(q, k, v, w, bias, residual, norm, attn_bias) -> bool:
     B, S, H, D = q.shape
-    heads = lambda t: t.stride(3) == 1 and t.stride(2) == D and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0
-    params = [t for t in (bias, residual, norm.weight, getattr(norm, "bias", None)) if t is not None]
-    return (D == 64 and B * S * H * w.shape[0] < ATTENTION_LINEAR_PARTS and k.shape[1] <= 256 and k.shape == v.shape and k.shape[0] == B and k.shape[2] == H
-            and _norm_fuses(B * S, w, residual, norm) and w.shape[0] % 16 == 0 and w.shape[1] == H * D and w.stride(1) == 1
-            and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0 and all(heads(t) for t in (q, k, v))
-            and all(t.dtype == torch.bfloat16 for t in (q, k, v, *params)) and all(t.data_ptr() % 8 == 0 for t in params)
-            and (attn_bias is None or (attn_bias.is_contiguous() and attn_bias.dtype == torch.bfloat16)))
+    return (B * S * H * w.shape[0] < ATTENTION_LINEAR_PARTS and _norm_fuses(B * S, w, residual, norm)
+            and _K().attn_proj_fits(q, k, v, w, bias, residual, norm.weight, getattr(norm, "bias", None), attn_bias))
 
 
 def paged_attention(q, k_cache, v_cache, block_table, kv_lens, q_lens, scale=None, causal=True):
