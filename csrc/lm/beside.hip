@@ -3,7 +3,8 @@
 //
 // One after the other, an attention of a few workgroups waits for its chain of loads (block table, keys, values: 11.6 us for 132 keys and
 // one sequence, 15.2 for 64 sequences, 0.25 to 1.3 TB/s), and then the recurrence begins.  Here the attention's workgroups are the first of
-// the grid, so that their chains start at once, and the recurrence's, bound by the state's traffic, take the rest of the chip.
+// the grid, so that their chains start at once, and the recurrence's, bound by the state's traffic, take the rest of the chip (kernels of
+// one sequence 25.3 -> 16.5 us with what prepares them, of 64 sequences 1.0 of 33.9 ms a pass).
 #include "attn_decode.h"
 #include "rule_rows.h"
 

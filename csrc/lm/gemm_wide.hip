@@ -355,7 +355,8 @@ void launch_gemm_wide(const GemmArgs& a, hipStream_t s) {
   // that they are among the quarters.  us: 7700 x 14848 x 2048 414 -> 396, 7700 x 17424 with 16 side columns 500 -> 481, 7700 x
   // 16640 465 -> 462, 8192 x 8192 x 8192 837 -> 824, and all of a prompt of 7 x 1100 tokens 9.29 -> 8.89 ms; one round is the slower through the direct stores (7700 x 2048 x 10496: 262 and 269).
   const int lines = a.n_main == a.N ? tiles_n : a.n_main / kTile;
-  const bool chain = !a.tiles && !a.gather && whole > 256 && a.K >= 128 && a.ldc % 8 == 0 && a.n_main % 8 == 0 && whole <= tiles_m * lines;
+  const bool chain = !a.tiles && !a.gather && whole > 256 && a.K >= 128 && a.ldc % 8 == 0 && a.ldc <= 1 << 21 &&
+                     a.n_main % 8 == 0 && whole <= tiles_m * lines;   // a tile's stores are at 32-bit offsets
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   const int step = chain ? 256 : whole;
   gemm_wide_kernel<<<step + 4 * (tiles - whole), 256, kLds, s>>>(a, whole, step, chain ? lines : tiles_n);

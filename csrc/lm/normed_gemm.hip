@@ -5,8 +5,9 @@
 // the XCD's L2 while they travel.  The first workgroup writes the residual (to memory that no workgroup reads).
 //
 // A workgroup takes every gridDim-th tile of 16 rows of W, so that the norm is made once for all of them (one tile a workgroup: 1089 norms,
-// 19.1 us for 1 x 17424 x 2048 where norm and product apart take 19.5).  Eight waves split K in steps of 64, and a wave's steps follow each other
-// across tiles through a ring of D in registers: the end of a tile, where the waves' sums meet in LDS, has the next one's weights beside it.
+// 19.1 us for 1 x 17424 x 2048 where norm and product apart take 19.4; 256 workgroups 20.8, 512 17.7, 1024 18.6).  Eight waves split
+// K in steps of 64, and a wave's steps follow each other across tiles through a ring of D in registers: the end of a tile, where the
+// waves' sums meet in LDS, has the next one's weights beside it.
 #include "lm_device.h"
 #include "normed_gemm.h"
 
@@ -16,7 +17,7 @@ namespace {
 
 constexpr int NW = 8, NT = 512;           // waves, threads
 constexpr int kGrid = 512;                // two workgroups for each CU
-constexpr int kRows = 2;                  // most rows
+constexpr int kRows = 2;                  // most rows; norm and product apart, and this: one 19.4 and 17.7 us, two 19.9 and 19.5, four 20.6 and 22.8
 constexpr int kMaxK = 4096;
 
 template <typename O, int M, int NV, bool MANY>   // NV: groups of 4 columns a thread and row has; MANY: more than four parts
