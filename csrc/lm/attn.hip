@@ -181,8 +181,8 @@ __global__ void __launch_bounds__(256, DK + DV > (LAT ? 320 : 256) ? 1 : 2) attn
   bf16_t* sV = smem + 2 * KT * DK;
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, fh = lane >> 5;
-  // the last queries, which have the most keys, first: the others even out the end of the grid (7 x 1100 tokens, 16 heads: about 107 ->
-  // 71 us, of a pass of 8.89 ms 0.14)
+  // the last queries, which have the most keys, first: the others even out the end of the grid (7 x 1100 tokens, 16 heads: 107 ->
+  // 87 us)
   const int b = blockIdx.y, h = blockIdx.x;
   const int hk = h / (p.H / p.G);
   const int q_len = p.q_lens[b], q0 = (gridDim.z - 1 - blockIdx.z) * 128;
