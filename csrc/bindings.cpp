@@ -895,6 +895,9 @@ shai::GnOneArgs gn_one_args(const optional<Tensor>& gamma, const optional<Tensor
   return n;
 }
 
+// Workgroups of groupnorm_apply's launch (for tests and tools)
+int64_t groupnorm_apply_blocks(int64_t N, int64_t HW, int64_t C) { return shai::gn_apply_blocks(N, HW, C); }
+
 bool groupnorm_one_supported(int64_t HW, int64_t C, int64_t G, bool fold) {
   return HW < (1 << 20) && C <= 8192 && shai::gn_one_supported(HW, C, G, fold);
 }
@@ -2071,6 +2074,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("qk_norm_rope(Tensor(a!) x, Tensor? q_w, Tensor? k_w, Tensor? cos, Tensor? sin, int H, int D, int S, float eps) -> ()");
   m.def("conv2d(Tensor x, Tensor? x2, Tensor w, Tensor(a!) out, Tensor? bias, Tensor? bias2d, Tensor? residual, Tensor? in_scale, Tensor? in_shift, int in_act, int kh, int kw, int stride, int pad, bool upsample, int act, float res_alpha, Tensor? ln_mr=None, Tensor? ln_s=None, Tensor(b!)? gn_part=None, Tensor(c!)? ln_stats=None, float ln_eps=1e-5, bool up_phases=False, Tensor? gn_gamma=None, Tensor? gn_beta=None, Tensor(d!)? gn_out=None, int gn_groups=0, float gn_eps=1e-5, bool gn_silu=False, bool keep_out=True) -> ()");
   m.def("groupnorm_one(Tensor x, Tensor? x2, Tensor? gamma, Tensor? beta, Tensor(a!) out, int G, float eps, bool silu) -> ()");
+  m.def("groupnorm_apply_blocks(int N, int HW, int C) -> int", &groupnorm_apply_blocks);
   m.def("groupnorm_one_supported(int HW, int C, int G, bool fold) -> bool", &groupnorm_one_supported);
   m.def("attn_proj_fits(Tensor q, Tensor k, Tensor v, Tensor w, Tensor? bias, Tensor residual, Tensor gamma, Tensor? beta, Tensor? attn_bias) -> bool");
   m.def("attn_proj_norm(Tensor q, Tensor k, Tensor v, Tensor? kv_lens, Tensor? attn_bias, float scale, bool causal, Tensor w, Tensor? bias, Tensor residual, Tensor gamma, Tensor? beta, Tensor(a!) y, Tensor(b!) out, float eps, bool rms) -> ()");

@@ -43,6 +43,7 @@ struct GroupNormArgs {
 };
 int gn_num_blocks(int N, int HW, int C);
 void launch_groupnorm_stats(const GroupNormArgs& a, hipStream_t s);
+long gn_apply_blocks(int N, int HW, int C);
 void launch_groupnorm_apply(const GroupNormArgs& a, hipStream_t s);
 // GroupNorm (+ SiLU) in one launch (groupnorm.hip), of x (and x2: channels [C1, C)), or of the fp32 partial sums
 // [splits][N HW][C] of a split-K convolution with what its fold adds.

@@ -12,6 +12,8 @@
 #include "common.h"
 #include "launchers.h"
 
+#include <algorithm>
+
 namespace shai {
 
 // ----------------------------------------------------------------------------
@@ -584,23 +586,31 @@ void launch_groupnorm_stats(const GroupNormArgs& a, hipStream_t s) {
     gn_finalize_kernel<<<dim3(a.N, a.G), 64, 0, s>>>(a.partials, a.gamma, a.beta, a.scale, a.shift, a.HW, a.C, a.G, NB, a.eps);
 }
 
-void launch_groupnorm_apply(const GroupNormArgs& a, hipStream_t s) {
-  const long total8 = (long)a.N * a.HW * a.C / 8;
-  // A thread has one vector, more in very large tensors: with a few each, the workgroups of the last round had the chip to themselves
-  // (us, 4096 workgroups and this: 16 x 4096 x 640 43.5 and 34.5, x 960 71.1 and 49.4, 16 x 1024 x 1280 23.8 and 19.7, 8 x 16384 x 512 69.5
-  // and 51.4, 8 x 262144 x 256 458 and 422). Where 4096 come out even with up to four vectors they save loads of scale and shift (1 x
-  // 65536 x 256 14.7 and 16.0, 1 x 262144 x 128 26.2 and 27.7). Two or four vectors on their way in a thread: slower at every size.
-  constexpr long kEven = 4096 * 256;
-  long blocks = total8 % kEven == 0 && total8 <= 4 * kEven ? 4096 : (total8 + 255) / 256;
+// Workgroups of the apply pass.  A thread has one vector, or two or three (as there are 2^18 of them, 1024 workgroups) of one or two large
+// images: they lie a grid apart, mostly in one image, and share its scale and shift.  With more images every vector loads a set of its
+// own, and the workgroups of the last round have the chip to themselves.  us for one, two, three vectors: 1 x 16384 x 512 7.9, 7.2, 7.2, 1 x
+// 64512 x 256 14.2, 12.7, 12.8, 1 x 102400 x 256 20.3, 19.8, 18.5, 1 x 262144 x 128 25.0, 23.5, 22.7, 1 x 262144 x 256 48.0, 43.1, 42.8, 1 x 589824 x
+// 128 52.1, 47.7, 47.0, 2 x 9216 x 640 9.9, 9.5, 9.3, 2 x 65536 x 256 24.5, 23.4, 22.4, 1 x 8192 x 512 5.4, 5.2, 5.4; below 2^19 vectors 1 x 6144 x
+// 512 4.5, 4.6, 4.8, 2 x 4096 x 320 4.1, 4.5, 4.7; more images 4 x 9216 x 640 18.4, 18.7, 20.6, 8 x 16384 x 512 46.5, 47.2, 50.9, 16 x 4096 x 640 30.6,
+// 31.9, 36.8.  4096 workgroups at every size: 8 x 16384 x 512 64.0, 16 x 4096 x 640 40.1.  Two or four vectors on their way in a thread:
+// slower at every size.
+long gn_apply_blocks(int N, int HW, int C) {
+  const long total8 = (long)N * HW * C / 8;
+  const long each = N > 2 ? 1 : std::min(3L, std::max(1L, total8 >> 18));
+  long blocks = (total8 + 256 * each - 1) / (256 * each);
   if (blocks > 65536) blocks = 65536;
   // grid threads a multiple of C / 8 (the kernel keeps one channel vector per thread)
-  const int C8 = a.C / 8;
+  const int C8 = C / 8;
   int g = C8, b = 256;
   while (b) { const int t = g % b; g = b; b = t; }  // gcd(C8, 256)
   const long unit = C8 / g;
-  blocks = (blocks + unit - 1) / unit * unit;
-  gn_apply_kernel<<<(int)blocks, 256, 0, s>>>(a.x, a.x2, a.x2 ? a.C1 : a.C, a.scale, a.shift, a.out, total8, a.HW,
-                                              a.C, a.silu);
+  return (blocks + unit - 1) / unit * unit;
+}
+
+void launch_groupnorm_apply(const GroupNormArgs& a, hipStream_t s) {
+  const long total8 = (long)a.N * a.HW * a.C / 8;
+  gn_apply_kernel<<<(int)gn_apply_blocks(a.N, a.HW, a.C), 256, 0, s>>>(a.x, a.x2, a.x2 ? a.C1 : a.C, a.scale, a.shift, a.out,
+                                                                       total8, a.HW, a.C, a.silu);
 }
 
 

@@ -90,6 +90,18 @@ def test_groupnorm_two_source(cuda, N, HW, C1, C2, fused, monkeypatch):
         assert int(ops._gn_tickets(x, N)[:N].abs().sum()) == 0  # re-armed
 
 
+# one, two and three vectors a thread, with remainders; two images, whose border lies between a thread's vectors; channels that 256 threads
+# do not divide
+@pytest.mark.parametrize("N,HW,C", [(1, 1, 8), (1, 16385, 256), (1, 24577, 264), (2, 12289, 384), (3, 5000, 320)])
+def test_groupnorm_apply_sizes(cuda, N, HW, C):
+    """Against 64 bits: the rounding of the bf16 result, 2^-9 of a value."""
+    torch.manual_seed(HW)
+    x, sc, sh = rnd(N, HW, C), torch.randn(N, C, device=cuda), torch.randn(N, C, device=cuda)
+    y = x.double() * sc.double()[:, None] + sh.double()[:, None]
+    y = y * torch.sigmoid(y)
+    assert (ops.groupnorm_apply(x, sc, sh, True).double() - y).norm() <= 2 ** -9 * y.norm()
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (1000, 320, 1280), (77, 1024, 1024), (8192, 640, 320),
                                    (5, 4096, 4096), (300, 96, 72)])
 @pytest.mark.parametrize("act", ["none", "silu", "gelu"])
