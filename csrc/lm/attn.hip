@@ -440,7 +440,7 @@ void launch_attn_prefill(const AttnArgs& a, bool f32, hipStream_t s) {
 // ------------------------------------------------------------------------------------------------ decode (bf16)
 template <int DK, int DV, int RH, bool PREP>
 __global__ void __launch_bounds__(256) attn_decode_kernel(const AttnArgs p, int per_group, int store) {
-  attn_decode<DK, DV, RH, PREP>(p, per_group, store, blockIdx.x, blockIdx.y, blockIdx.z);
+  attn_decode<DK, DV, RH, PREP, 16>(p, per_group, store, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 __global__ void __launch_bounds__(256) attn_decode_fold_kernel(const AttnArgs p) {

@@ -73,11 +73,11 @@ __device__ __forceinline__ float out_factor(const AttnArgs& p, const bf16_t* row
 }
 
 // One workgroup: kv head g's query heads h0 .. h0 + R - 1 (R <= 16, RH = R rounded up) of sequence b, one split of the
-// visible 64-key blocks.  Wave w takes blocks w, w + 4, ... of the split.
-template <int DK, int DV, int RH, bool PREP>
+// visible 64-key blocks.  Wave w takes blocks w, w + 4, ... of the split.  VMAX: most V loads in flight.
+template <int DK, int DV, int RH, bool PREP, int VMAX>
 __device__ __forceinline__ void attn_decode(const AttnArgs& p, int per_group, int store, int bx, int b, int split) {
   constexpr int LPK = DV / 8, KP = 64 / LPK, IT = 64 / KP;   // V: LPK lanes per key, KP keys at a time
-  constexpr int VB = IT > 16 ? 16 : IT;                      // V loads in flight
+  constexpr int VB = IT > VMAX ? VMAX : IT;                  // V loads in flight
   __shared__ float sp[4][64][RH];
   __shared__ __attribute__((aligned(16))) float so[4][RH][DV];
   __shared__ __attribute__((aligned(16))) bf16_t sq[PREP ? RH : 1][PREP ? DK : 8];

@@ -10,12 +10,19 @@
 
 namespace shai_lm {
 
+// Workgroups a CU that the registers are for: three, and two where eight heads of 128 to a group hold 198 of them.  The recurrence alone has
+// 128, for four.  Given to both, with half as many V loads in flight, nothing spills either, but the attention's chain is the longer and
+// decides (us, 16 heads of 128, 4 a group: one sequence of 132 keys 12.7 at three and 13.9 at four, 64 of 900 keys 59.1 and 68.1).  Eight a group at
+// three spill 51 to 53: 64 sequences of 900 keys 72.9, at two 50.8, one after the other 67.4; of 132 keys 39.5, 36.7 and 45.7.
+constexpr int workgroups(int D, int RH) { return D == 128 && RH == 8 ? 2 : 3; }
+
+// Eight V loads in flight: as fast as the sixteen of the attention alone, which spill 7 registers here (64 sequences of 132 keys 39.4 -> 38.3).
 template <int D, int RH, int MODE, int SD>
-__global__ void __launch_bounds__(256, 3) attn_rule_kernel(const AttnArgs a, const RuleArgs r, int per_group, int heads, int n_attn) {
+__global__ void __launch_bounds__(256, workgroups(D, RH)) attn_rule_kernel(const AttnArgs a, const RuleArgs r, int per_group, int heads, int n_attn) {
   const int i = blockIdx.x;
   if (i < n_attn) {
     const int j = i / heads;
-    attn_decode<D, D, RH, true>(a, per_group, 1, i - j * heads, j % a.B, j / a.B);
+    attn_decode<D, D, RH, true, 8>(a, per_group, 1, i - j * heads, j % a.B, j / a.B);
   } else {
     const int b = (i - n_attn) / r.H;
     rule_rows<bf16_t, MODE, SD, SD, 256, true>(r, i - n_attn - b * r.H, b);
@@ -34,7 +41,7 @@ static void attn_rule(const AttnArgs& a, const RuleArgs& r, hipStream_t s) {
   else r.dk == 64 ? attn_rule<D, RH, kChannel, 64>(a, r, s) : attn_rule<D, RH, kChannel, 128>(a, r, s);
 }
 
-// The head sizes and groups whose registers fit the recurrence's three workgroups a CU; others run one after the other.
+// The head sizes and groups that are compiled; others run one after the other.
 static bool fits(const AttnArgs& a, const RuleArgs& r) {
   const long grid = (long)a.G * a.B * a.splits + (long)r.H * r.B;
   return a.own_kv && a.rope && a.H / a.G <= 8 && a.dk == a.dv && a.dk <= 128 && r.mode != kRetention && r.dk == r.dv && r.dk <= 128 &&

@@ -24,7 +24,8 @@ __device__ __forceinline__ float gate_act(float z, int kind) {
 // convolution's taps one after the other, each waited for, cost 10 us of a step), and the state after it: convolutions, norms and
 // decays are done when it arrives.  64 sequences x 16 heads of 128 x 128 (134 MB of state),
 // us: decay per head 37.6 -> 34.8, per channel 39.8 -> 35.1, retention 28.7 (the rate of a large copy: 27); one sequence 7.1 -> 6.6 and
-// 7.6 -> 6.8.  The one row of a step is compiled apart from prompts': 126 registers instead of 168, four workgroups per CU.
+// 7.6 -> 6.8.  The one row of a step is compiled apart from prompts': 126 registers instead of 168, four workgroups per CU
+// (three beside a step's attention, beside.hip: 64 sequences are then more than are resident at once).
 template <typename T, int MODE, int DK, int DV, int NT, bool STEP>   // STEP: decode of the delta rule
 __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
   constexpr bool DELTA = MODE != kRetention;
