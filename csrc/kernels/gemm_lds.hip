@@ -180,7 +180,7 @@ void gemm2_plan(const GemmArgs& a, int* cfg, int* splits) {
     const long tiles = tm * tn * batch;
     const long lds = 2L * (t.bm + t.bn) * BK2 * 2;
     const long per_cu = std::max(1L, std::min(163840L / lds, 2048L / ((t.bm / 64) * (t.bn / 64) * 64 > 512 ? 512 : 256)));
-    for (int sp = 1; sp <= 16; sp *= 2) {
+    for (int sp = 1; sp <= 16; sp *= 2) {   // (the tuner's counts made this model choose worse: 1.7 % over 204 problems)
       if (sp > 1 && (batch != 1 || kt / sp < 4)) break;
       const long blocks = tiles * sp;
       const long slots = 256 * per_cu;
@@ -319,6 +319,39 @@ int gemm2_num_cfgs() { return kDeepCfg + kDeepCfgs; }
 bool gemm2_cfg_candidate(int cfg) { return !(cfg >= kNumCfgs && cfg < kV4Cfg); }
 
 bool gemm2_cfg_splittable(int cfg) { return cfg != kW4Cfg && cfg != kW4Cfg + 1 && cfg != kWsCfg; }
+
+// One count from each of 2 to 3, 4 to 6, 7 to 12 and 13 to 16: the one with which the tiles' parts leave the fewest slots of the chip's last
+// round empty.  (2, 4, 8 and 16, as many launches to time, were 1.026 times the best of all counts to 16, in the mean of the 175 convolutions of
+// requests of 448 x 576, 640 x 384, 512 x 512 and 768 x 768 pixels and of small batches, up to 1.19, 55 of them over 1.03; these are 1.002, up to
+// 1.07, 5.  Plain products 1.002 either way.)  No part is empty or under 4 k-tiles.
+int gemm2_split_counts(int M, int N, int K, int cfg, int most, int* out) {
+  int bm, bn, per_cu = 1;
+  if (cfg >= kDeepCfg) {
+    gemm_deep_tile(cfg - kDeepCfg, &bm, &bn);
+    per_cu = gemm_deep_per_cu(cfg - kDeepCfg);
+  } else if (cfg >= kNumCfgs) {
+    bm = 256, bn = cfg >= kV4Cfg && ((cfg - kV4Cfg) & 1) ? 320 : 256;
+  } else {
+    bm = kCfgs[cfg].bm, bn = kCfgs[cfg].bn;
+    per_cu = 160 * 1024 / (2 * (bm + bn) * BK2 * (int)sizeof(bf16_t));
+  }
+  const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn), slots = 256 * per_cu;
+  const int kt = (K + BK2 - 1) / BK2;
+  int n = 0;
+  out[n++] = 1;
+  for (int p = 2; p <= most && p <= 16; p *= 2) {
+    int best = 0;
+    long best_left = 0, best_rounds = 1;
+    for (int s = (4 * p + 4) / 5; 5 * s < 8 * p && s <= 16; ++s) {
+      const int per = (kt + s - 1) / s;
+      if (kt / s < 4 || (kt + per - 1) / per != s) continue;
+      const long rounds = (tiles * s + slots - 1) / slots, left = rounds * slots - tiles * s;
+      if (best == 0 || left * best_rounds < best_left * rounds) best = s, best_left = left, best_rounds = rounds;
+    }
+    if (best) out[n++] = best;
+  }
+  return n;
+}
 
 bool gemm2_cfg_supported(const GemmArgs& a, int cfg) {
   // an epilogue activation no tile kernel instantiates is never accepted (it would run as another one)

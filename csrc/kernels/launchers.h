@@ -209,6 +209,8 @@ void gemm2_plan(const GemmArgs& a, int* cfg, int* splits);
 void launch_gemm2_cfg(const GemmArgs& a, float* ws, int cfg, int splits, hipStream_t s);
 int gemm2_num_cfgs();
 bool gemm2_cfg_supported(const GemmArgs& a, int cfg);
+// counts of parts of K, up to `most` (a power of two), that are worth timing with config cfg, 1 first: at most 5, the number of them
+int gemm2_split_counts(int M, int N, int K, int cfg, int most, int* out);
 bool gemm2_cfg_splittable(int cfg);  // false: the config always runs the whole K (split-K choices are moot)
 // v5: four-wave GEMM / implicit-GEMM conv (gemm_w4.hip), 256 x bn tiles, bn = 256 or, products only, 192
 bool gemm_w4_supported(const GemmArgs& a);
@@ -218,6 +220,7 @@ constexpr int kDeepCfgs = 6;
 bool gemm_deep_supported(const GemmArgs& a);
 void gemm_deep_tile(int which, int* bm, int* bn);
 int gemm_deep_wave_groups(int which);  // along K
+int gemm_deep_per_cu(int which);       // workgroups that a CU's LDS holds
 void launch_gemm_deep(const GemmArgs& a, int which, float* ws, int splits, hipStream_t s);
 // v6: W-stationary low-K GEMM (gemm_ws.hip): K = 320, N % 320 == 0, persistent over M, weights in VGPRs
 bool gemm_ws_supported(const GemmArgs& a);

@@ -109,6 +109,19 @@ def test_convolution(cuda, cfg, splits):
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-3000:]
 
 
+# counts of parts that are no powers of two, 45 k-tiles: 15, 9, 7 and 3, and 4 with a last part of one
+@pytest.mark.parametrize("splits", [3, 5, 7, 12, 15])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 9, 10, 11, 12] + GROUPS)
+def test_convolution_in_parts(cuda, cfg, splits):
+    g = torch.Generator(device=cuda).manual_seed(splits)
+    make = lambda *s: torch.randn(*s, generator=g, device=cuda)  # noqa: E731
+    x, w4, b, r = make(2, 9, 11, 320).bfloat16(), (make(328, 320, 3, 3) / 2880 ** 0.5).bfloat16(), make(328).bfloat16(), make(2, 9, 11, 328).bfloat16()
+    ops._K().gemm_tuning_import([f"1:198,328,2880,b1,g0|2,9,11,320,320,3,1,0,0={cfg},{splits}"])
+    y = ops.conv2d(x, ops.pack_conv_weight(w4), b, 3, 3, 1, 1, residual=r)
+    want = torch.nn.functional.conv2d(x.double().permute(0, 3, 1, 2).cpu(), w4.double().cpu(), b.double().cpu(), padding=1).permute(0, 2, 3, 1)
+    assert _close(y, want + r.double().cpu())
+
+
 # products that keep one order of sums (packed prompts): every tile that they may take gives the same bits, the others are refused
 @pytest.mark.parametrize("N,K,glu", [(512, 1024, False), (320, 320, False), (1536, 776, False), (1024, 512, True)])
 def test_one_order(cuda, N, K, glu):
