@@ -395,6 +395,18 @@ std::string lm_gemm_form(int64_t M, int64_t N, int64_t K, int64_t splits, int64_
   return shai_lm::gemm_ring_fits(g) ? "ring" : "stream";
 }
 
+// Tiles of a wide product that follow each other in their workgroups (for tests and tools): N columns, `side` of them side columns
+int64_t lm_gemm_chained(int64_t M, int64_t N, int64_t K, int64_t side) {
+  shai_lm::GemmArgs g{};
+  g.M = g.a_rows = M;
+  g.N = N;
+  g.n_main = g.n_act = N - side;
+  g.K = g.lda = K;
+  g.ldc = (g.n_main + 7) / 8 * 8;
+  g.batch = 1;
+  return shai_lm::gemm_wide_chained(g);
+}
+
 void residual_norm(const optional<Tensor>& x, const optional<Tensor>& ids, const optional<Tensor>& table, double scale,
                    const optional<Tensor>& delta, const optional<Tensor>& wb, double mult, const optional<Tensor>& step,
                    const optional<Tensor>& x_out, const optional<Tensor>& rows, const optional<Tensor>& w, double eps,
@@ -1294,6 +1306,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("rule_rows(Tensor x, Tensor gate, Tensor(a!) state, Tensor(b!) out, Tensor pos, Tensor slots, int kv_heads, int dim, int vdim, int gate_kind, float eps, Tensor rate, Tensor? decay=None, Tensor? beta=None, Tensor? conv=None, Tensor? bias=None, Tensor? gain=None, Tensor(c!)? ring=None, Tensor? rope=None, Tensor? q_start=None, Tensor? q_lens=None) -> ()");
   m.def("rule_chunks(Tensor x, Tensor gate, Tensor(a!) state, Tensor(b!) out, Tensor pos, Tensor slots, int kv_heads, int dim, int vdim, int gate_kind, float eps, Tensor rate, Tensor? decay=None, Tensor? beta=None, Tensor? conv=None, Tensor? bias=None, Tensor? gain=None, Tensor? ring=None, Tensor? rope=None, *, Tensor q_start, Tensor q_lens, Tensor(c!) ws, int max_q, int head0, int heads, int seg=0, Tensor(d!)? seg_ws=None) -> ()");
   m.def("rule_segment_bytes(int dk, int dv, int heads, bool retention) -> int", &rule_segment_bytes);
+  m.def("lm_gemm_chained(int M, int N, int K, int side=0) -> int", &lm_gemm_chained);
   m.def("lm_gemm_form(int M, int N, int K, int splits=1, int n_tiles=0) -> str", &lm_gemm_form);
   m.def("rule_chunk_bytes(int dk, int dv, int heads, int keys, bool channel) -> int", &rule_chunk_bytes);
   m.def("ring_commit(Tensor x, Tensor(a!) ring, Tensor pos, Tensor q_start, Tensor q_lens, Tensor slots) -> ()");

@@ -14,6 +14,7 @@
 #include "lm_device.h"
 #include "lm.h"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -348,18 +349,31 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(const GemmArgs p, int
   tile<8, 2>(p, smem, m0, m_end, n0, static_cast<const bf16_t*>(p.W) + (long)expert * p.N * p.K);
 }
 
+// Tiles of whole rounds; a last round of up to half of the CUs is cut in quarters.
+static int whole_rounds(const GemmArgs& a, int tiles) {
+  const int left = tiles % 256;
+  return !a.tiles && tiles > 256 && left <= 128 ? tiles - left : tiles;
+}
+
+// Tiles that follow each other in their workgroups, 0: every tile has one of its own.  More than a round of tiles without side columns, rows of
+// 16-byte stores at 32-bit offsets.  The tiles with side columns are the last and go to quarters, those past the columns exit at once; more than
+// an eighth of all are not worth it (4096 x 8192 x 2048 with 2048 side columns 127 -> 133 us).  us: 7700 x 14848 x 2048 414 -> 396, 7700 x 16640
+// 465 -> 462, 8192 x 8192 x 8192 837 -> 824; with 32 side columns 7700 x 14624 452 -> 397, 2048 x 14624 122 -> 109, 33000 x 14624 1836 -> 1590; with
+// 16, 8192 x 17424 557 -> 480, 7700 x 17424 500 -> 466; one round is the slower through the direct stores (7700 x 2048 x 10496: 262 and 269).
+int gemm_wide_chained(const GemmArgs& a) {
+  const int tiles_m = (a.M + kTile - 1) / kTile, tiles_n = (a.N + kTile - 1) / kTile;
+  const int rounds = whole_rounds(a, tiles_m * tiles_n), lines = a.n_main == a.N ? tiles_n : a.n_main / kTile;
+  const int n = std::min(rounds, tiles_m * lines);
+  const bool fits = !a.tiles && !a.gather && a.K >= 128 && a.ldc % 8 == 0 && a.ldc <= 1 << 21 && a.n_main % 8 == 0;
+  return fits && n > 256 && 8L * n >= 7L * rounds ? n : 0;
+}
+
 void launch_gemm_wide(const GemmArgs& a, hipStream_t s) {
-  const int tiles_m = a.tiles ? a.n_tiles : (a.M + kTile - 1) / kTile, tiles_n = (a.N + kTile - 1) / kTile, tiles = tiles_m * tiles_n;
-  const int left = tiles % 256, whole = !a.tiles && tiles > 256 && left <= 128 ? tiles - left : tiles;
-  // A chain where whole rounds are more than one and have neither side columns nor rows without 16-byte stores.  Those columns are last, so
-  // that they are among the quarters.  us: 7700 x 14848 x 2048 414 -> 396, 7700 x 17424 with 16 side columns 500 -> 481, 7700 x
-  // 16640 465 -> 462, 8192 x 8192 x 8192 837 -> 824, and all of a prompt of 7 x 1100 tokens 9.29 -> 8.89 ms; one round is the slower through the direct stores (7700 x 2048 x 10496: 262 and 269).
-  const int lines = a.n_main == a.N ? tiles_n : a.n_main / kTile;
-  const bool chain = !a.tiles && !a.gather && whole > 256 && a.K >= 128 && a.ldc % 8 == 0 && a.ldc <= 1 << 21 &&
-                     a.n_main % 8 == 0 && whole <= tiles_m * lines;   // a tile's stores are at 32-bit offsets
+  const int tiles_n = (a.N + kTile - 1) / kTile, tiles = (a.tiles ? a.n_tiles : (a.M + kTile - 1) / kTile) * tiles_n;
+  const int chained = gemm_wide_chained(a), whole = chained ? chained : whole_rounds(a, tiles), step = chained ? 256 : whole;
+  const int lines = chained && a.n_main != a.N ? a.n_main / kTile : tiles_n;
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-  const int step = chain ? 256 : whole;
-  gemm_wide_kernel<<<step + 4 * (tiles - whole), 256, kLds, s>>>(a, whole, step, chain ? lines : tiles_n);
+  gemm_wide_kernel<<<step + 4 * (tiles - whole), 256, kLds, s>>>(a, whole, step, lines);
   SHAI_CHECK_LAUNCH();
 }
 

@@ -142,6 +142,7 @@ void launch_gemm_ring(const GemmArgs& a, hipStream_t s);
 void launch_gemm(const GemmArgs& a, bool f32, hipStream_t s);          // streaming kernel, any M
 void launch_gemm_tile(const GemmArgs& a, hipStream_t s);               // LDS-tiled bf16 kernel (gemm_tile.hip)
 const char* gemm_tile_name(const GemmArgs& a);                         // which of its forms that is
+int gemm_wide_chained(const GemmArgs& a);                             // how many of them follow each other in a workgroup
 void launch_gemm_wide(const GemmArgs& a, hipStream_t s);               // its 256 x 256 tiles without an epilogue (gemm_wide.hip)
 
 struct RouteArgs {

@@ -56,3 +56,13 @@ def test_tiles(M, N, K, splits, want):
 @pytest.mark.parametrize("N,K,want", [(1024, 1600, "wide"), (1024, 4096, "wide"), (1536, 512, "256x256"), (1536, 1536, "256x256")])
 def test_grouped(N, K, want):
     assert form(5000, N, K, 1, 27) == want
+
+
+# tiles one after the other in a workgroup: all whole rounds; with side columns all tiles without them where the whole rounds reach into
+# theirs, as many as an eighth; not a single round, a width or a K that it does not take
+@pytest.mark.parametrize("M,N,K,side,want", [
+    (7700, 14848, 2048, 0, 1792), (8192, 8192, 8192, 0, 1024), (7700, 17424, 2048, 16, 2048), (7700, 14624, 2048, 32, 31 * 57),
+    (8192, 17424, 2048, 16, 32 * 68), (4096, 8192, 2048, 1024, 16 * 28), (4096, 8192, 2048, 1032, 0), (7700, 2048, 4096, 0, 0),
+    (4096, 4104, 2048, 8, 0), (4352, 4104, 2048, 8, 0), (6400, 4104, 2048, 8, 25 * 16), (7700, 14624, 64, 32, 0), (7700, 14624, 128, 32, 31 * 57), (7700, 14628, 2048, 0, 0)])
+def test_chained_tiles(M, N, K, side, want):
+    assert native.lm_ops().lm_gemm_chained(M, N, K, side) == want

@@ -36,8 +36,10 @@ def test_plain(cuda, M, N, K):
 
 
 # more than one whole round, tile after tile in a workgroup: two, three and odd counts of k-tiles; a last row and columns that end inside
-# a tile, the last round not whole (391 tiles), cut in quarters (544 and 32 more) or with side columns among the quarters (512 and 64)
-@pytest.mark.parametrize("M,N,side,act", [(4100, 5640, 0, None), (4352, 8192, 0, 4100), (4096, 8976, 272, None), (8191, 4352, 0, None)])
+# a tile, the last round not whole (391 tiles), cut in quarters (544 and 32 more) or with side columns among the quarters (512 and 64); tiles
+# with side columns that the whole rounds reach into (510 of 527 tiles without, 391 of 408, 400 of 425)
+@pytest.mark.parametrize("M,N,side,act", [(4100, 5640, 0, None), (4352, 8192, 0, 4100), (4096, 8976, 272, None), (8191, 4352, 0, None),
+                                           (4100, 7712, 32, None), (4100, 5904, 16, None), (6400, 4104, 8, None)])
 @pytest.mark.parametrize("K", [128, 192, 1600])
 def test_chain(cuda, M, N, side, act, K):
     a, w = _problem(M, N, K, cuda, spare=8)
