@@ -325,7 +325,8 @@ void normed_gemm(const optional<Tensor>& x, const optional<Tensor>& ids, const o
   g.K = W.size(1);
   g.batch = 1;
   g.out_f32 = C.scalar_type() == at::kFloat;
-  SHAI_CHECK(shai_lm::normed_gemm_fits(g.M, g.K) && g.N >= 1, "normed_gemm: ", g.M, " rows of ", g.K, ": one or two of up to 4096");
+  SHAI_CHECK(shai_lm::normed_gemm_fits(g.M, g.K, delta ? delta->size(0) : 0) && g.N >= 1, "normed_gemm: ", g.M, " rows of ", g.K,
+             ": a form that is made in two launches");
   check_width(g.K, width);
   SHAI_CHECK(x.has_value() != ids.has_value(), "normed_gemm: a residual or token ids");
   auto matrix = [&](const Tensor& t, const char* name) {
@@ -394,6 +395,9 @@ std::string lm_gemm_form(int64_t M, int64_t N, int64_t K, int64_t splits, int64_
   if (n_tiles > 0 || M > 64) return shai_lm::gemm_tile_name(g);
   return shai_lm::gemm_ring_fits(g) ? "ring" : "stream";
 }
+
+// Whether normed_gemm takes so many rows, columns and parts
+bool normed_gemm_fits(int64_t M, int64_t K, int64_t parts) { return shai_lm::normed_gemm_fits(M, K, parts); }
 
 // Tiles of a wide product that follow each other in their workgroups (for tests and tools): N columns, `side` of them side columns
 int64_t lm_gemm_chained(int64_t M, int64_t N, int64_t K, int64_t side) {
@@ -1306,6 +1310,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("rule_rows(Tensor x, Tensor gate, Tensor(a!) state, Tensor(b!) out, Tensor pos, Tensor slots, int kv_heads, int dim, int vdim, int gate_kind, float eps, Tensor rate, Tensor? decay=None, Tensor? beta=None, Tensor? conv=None, Tensor? bias=None, Tensor? gain=None, Tensor(c!)? ring=None, Tensor? rope=None, Tensor? q_start=None, Tensor? q_lens=None) -> ()");
   m.def("rule_chunks(Tensor x, Tensor gate, Tensor(a!) state, Tensor(b!) out, Tensor pos, Tensor slots, int kv_heads, int dim, int vdim, int gate_kind, float eps, Tensor rate, Tensor? decay=None, Tensor? beta=None, Tensor? conv=None, Tensor? bias=None, Tensor? gain=None, Tensor? ring=None, Tensor? rope=None, *, Tensor q_start, Tensor q_lens, Tensor(c!) ws, int max_q, int head0, int heads, int seg=0, Tensor(d!)? seg_ws=None) -> ()");
   m.def("rule_segment_bytes(int dk, int dv, int heads, bool retention) -> int", &rule_segment_bytes);
+  m.def("normed_gemm_fits(int M, int K, int parts) -> bool", &normed_gemm_fits);
   m.def("lm_gemm_chained(int M, int N, int K, int side=0) -> int", &lm_gemm_chained);
   m.def("lm_gemm_form(int M, int N, int K, int splits=1, int n_tiles=0) -> str", &lm_gemm_form);
   m.def("rule_chunk_bytes(int dk, int dv, int heads, int keys, bool channel) -> int", &rule_chunk_bytes);

@@ -19,7 +19,7 @@ struct NormedGemmArgs {
   float* x_out;            // [M, K] x + delta, apart from x; or null
   GemmArgs g;              // A: the norm of x_out in bf16
 };
-bool normed_gemm_fits(int M, int K);
+bool normed_gemm_fits(int M, int K, int parts);
 void launch_normed_gemm(const NormedGemmArgs& a, hipStream_t s);       // plain and squared-ReLU epilogues
 
 }  // namespace shai_lm

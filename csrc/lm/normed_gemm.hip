@@ -1,8 +1,8 @@
 // C = epi(norm(x + sum of a sublayer's parts) W^T) of a decode step's few rows, and x + parts for the next layer.
 //
 // The norm of one row is 2.7 us on one CU, 4.7 with its launch, and the product behind it waits for all of it.  Here every workgroup makes
-// the norm itself: its weights are on their way before the row's values are asked for, and the 8 (1 + parts) KB of a row of 2048 come from
-// the XCD's L2 while they travel.  The first workgroup writes the residual (to memory that no workgroup reads).
+// the norm itself: the row, its parts and the gain are asked for first (8 (2 + parts) KB of a row of 2048, from the XCD's L2), the first weights
+// right behind them, and these travel while the norm is made.  The first workgroup writes the residual (to memory that no workgroup reads).
 //
 // A workgroup takes every gridDim-th tile of 16 rows of W, so that the norm is made once for all of them (one tile a workgroup: 1089 norms,
 // 19.1 us for 1 x 17424 x 2048 where norm and product apart take 19.4; 256 workgroups 20.8, 512 17.7, 1024 18.6).  Eight waves split
@@ -16,9 +16,7 @@ namespace shai_lm {
 namespace {
 
 constexpr int NW = 8, NT = 512;           // waves, threads
-constexpr int kGrid = 512;                // two workgroups for each CU
-constexpr int kRows = 2;                  // most rows; norm and product apart, and this: one 19.4 and 17.7 us, two 19.9 and 19.5, four 20.6 and 22.8
-constexpr int kMaxK = 4096;
+constexpr int kGrid = 512;                // two workgroups for each CU: every form that is compiled has at most 128 registers
 
 template <typename O, int M, int NV, bool MANY>   // NV: groups of 4 columns a thread and row has; MANY: more than four parts
 __global__ void __launch_bounds__(NT, 2) normed_gemm_kernel(const NormedGemmArgs p) {
@@ -143,23 +141,24 @@ __global__ void __launch_bounds__(NT, 2) normed_gemm_kernel(const NormedGemmArgs
   }
 }
 
-template <typename O, int M, int NV>
-void go(const NormedGemmArgs& a, hipStream_t s) {
-  const int tiles = (a.g.N + 15) / 16, grid = tiles < kGrid ? tiles : kGrid;
-  if (a.parts > 4) normed_gemm_kernel<O, M, NV, true><<<grid, NT, 0, s>>>(a);
-  else normed_gemm_kernel<O, M, NV, false><<<grid, NT, 0, s>>>(a);
-}
-
 template <typename O>
 void rows(const NormedGemmArgs& a, hipStream_t s) {
-  const bool wide = a.g.K > NT * 4;
-  if (a.g.M == 1) wide ? go<O, 1, 2>(a, s) : go<O, 1, 1>(a, s);
-  else wide ? go<O, 2, 2>(a, s) : go<O, 2, 1>(a, s);
+  const int tiles = (a.g.N + 15) / 16, grid = tiles < kGrid ? tiles : kGrid;
+  auto go = [&](auto kernel) { kernel<<<grid, NT, 0, s>>>(a); };
+  if (a.g.M == 2) go(normed_gemm_kernel<O, 2, 1, false>);
+  else if (a.g.K > NT * 4) go(normed_gemm_kernel<O, 1, 2, false>);
+  else if (a.parts > 4) go(normed_gemm_kernel<O, 1, 1, true>);
+  else go(normed_gemm_kernel<O, 1, 1, false>);
 }
 
 }  // namespace
 
-bool normed_gemm_fits(int M, int K) { return M >= 1 && M <= kRows && K <= kMaxK && K % 64 == 0; }
+// The forms of which a CU holds two workgroups.  us apart and in one launch, bf16 outputs of 17424 columns: one row of 2048 in four parts 19.3 and
+// 17.7, in eight 19.6 and 18.7, of 4096 in four 31.7 and 29.8; two rows of 2048 in four 19.5 and 19.1.  The others need 147 to 224 registers: one
+// row of 4096 in eight parts 32.2 and 36.7, two of 2048 in eight 19.8 and 22.7, two of 4096 32.2 and 37.3; four rows of 2048 20.6 and 22.8.
+bool normed_gemm_fits(int M, int K, int parts) {
+  return K % 64 == 0 && (M == 1 ? parts <= 4 ? K <= 4096 : parts <= 8 && K <= 2048 : M == 2 && parts <= 4 && K <= 2048);
+}
 
 void launch_normed_gemm(const NormedGemmArgs& a, hipStream_t s) {
   if (a.g.out_f32) rows<float>(a, s);

@@ -394,12 +394,12 @@ class Conv:
 
 
 def residual_norm(source, delta, wb, mult: float, step, w, eps: float, width: int, dtype, conv: Optional[Conv] = None,
-                  batch=None, rows=None, keep: bool = True):
+                  batch=None, rows=None, keep: bool = True, apart: bool = False):
     """x = source (+ mult * norm(delta)) (+ step); h = norm(x), plus its convolution with ``conv``.
 
     source: the fp32 residual [T, D] or an :class:`Embedding`.  delta: [T, D], partial sums [parts, T, D] fp32, or
     :class:`Experts` without a dense part.  wb, w: the norms' gains (RMS norm) or :class:`Affine` (layer norm); wb PLAIN:
-    delta is added as it is; w PLAIN: h = x.  Returns (x, h); the residual may be updated in place.  ``w`` None: no h.  ``rows`` (int32): h of these rows
+    delta is added as it is; w PLAIN: h = x.  Returns (x, h); the residual may be updated in place, unless ``apart``.  ``w`` None: no h.  ``rows`` (int32): h of these rows
     only, and with ``keep`` False x is None."""
     emb = isinstance(source, Embedding)
     if not (source.ids if emb else source).is_cuda:
@@ -415,7 +415,7 @@ def residual_norm(source, delta, wb, mult: float, step, w, eps: float, width: in
         delta = None
     x = None
     if keep:
-        x = torch.empty(T, D, dtype=torch.float32, device=dev) if emb or conv is not None else source
+        x = torch.empty(T, D, dtype=torch.float32, device=dev) if emb or conv is not None or apart else source
     h = torch.empty(T if rows is None else rows.shape[0], D, dtype=dtype, device=dev) if not no_h else None
     ye.update(bb=bb, b=b)
     args = (None if emb else source, ids, table, float(scale), delta, wb, float(mult), step, x, rows, w, float(eps),
@@ -442,12 +442,11 @@ class Normed:
     width: int
 
 
-# us, norm and product apart and one launch, rows x 17424 x 2048: one 19.4 and 17.7, two 19.9 and 19.5, four 20.6 and 22.8
 NORMED_ROWS = 2
 
 
 def normed_fits(n: Normed, weight: torch.Tensor) -> bool:
-    """Whether :func:`normed_matmul` takes this norm: bf16 weights, one or two rows of up to 4096, parts in fp32."""
+    """Whether :func:`normed_matmul` takes this norm: bf16 weights, one or two rows of up to 4096, up to eight parts in fp32."""
     emb = isinstance(n.source, Embedding)
     rows, K = (n.source.ids.shape[0], n.source.table.shape[1]) if emb else n.source.shape
     d = n.delta
@@ -456,10 +455,14 @@ def normed_fits(n: Normed, weight: torch.Tensor) -> bool:
 
 
 def normed_matmul(n: Normed, weight, out, act: int = 0, side: int = 0, keep: bool = True):
-    """(x, side product) of :func:`matmul_joint` of the norm's output, and the norm's x (``keep`` False: None)."""
+    """(x, side product) of :func:`matmul_joint` of the norm's output, and the norm's x (``keep`` False: None): in one launch where that is
+    the faster way, of few rows, columns and parts."""
     emb = isinstance(n.source, Embedding)
     ids, table, scale = n.source if emb else (None, None, 1.0)
     K, dev = weight.shape[1], weight.device
+    if not _K().normed_gemm_fits(out.shape[0], K, 0 if n.delta is None else n.delta.shape[0]):
+        x, h = residual_norm(n.source, n.delta, PLAIN, 1.0, None, n.w, n.eps, n.width, weight.dtype, keep=keep, apart=True)
+        return x, matmul_joint(h, weight, out, act, side)
     x = torch.empty(out.shape[0], K, dtype=torch.float32, device=dev) if keep else None
     s = torch.empty(out.shape[0], side, dtype=torch.float32, device=dev) if side else None
     _K().normed_gemm(None if emb else n.source, ids, table, float(scale), n.delta, n.w, float(n.eps), int(n.width), x, weight, out, s, int(act))

@@ -14,15 +14,15 @@ if READELF is None or not os.path.exists(native.KERNELS_LIB) or not os.path.exis
     pytest.skip("needs the native libraries and llvm-readelf", allow_module_level=True)
 
 
-def spills(lib, tmp_path):
-    """{kernel: registers spilled} over the device objects of a library."""
+def spills(lib, tmp_path, what="vgpr_spill_count"):
+    """{kernel: registers spilled} over the device objects of a library; ``what``: another of the counts."""
     data, out = open(lib, "rb").read(), {}
     at = [m.start() for m in re.finditer(b"\x7fELF", data)][1:]     # behind the library's own header
     for i, (a, b) in enumerate(zip(at, at[1:] + [len(data)])):
         f = tmp_path / f"{i}.o"
         f.write_bytes(data[a:b])
         notes = subprocess.run([READELF, "--notes", str(f)], capture_output=True, text=True).stdout
-        for name, n in re.findall(r"\.name:\s+(_Z\w+).*?\.vgpr_spill_count:\s+(\d+)", notes, re.S):
+        for name, n in re.findall(rf"\.name:\s+(_Z\w+).*?\.{what}:\s+(\d+)", notes, re.S):
             out[name] = int(n)
     return out
 
@@ -51,3 +51,9 @@ def test_joined_and_fused_kernels_do_not_spill(tmp_path):
         found = {k: n for k, n in lib.items() if name in k}
         assert len(found) >= least, name
         assert not {k: n for k, n in found.items() if n}
+
+
+def test_two_workgroups_a_cu(tmp_path):
+    """A norm in its product: the grid is two workgroups of eight waves a CU, which have 128 registers a lane."""
+    found = {k: n for k, n in spills(native.LM_LIB, tmp_path, "vgpr_count").items() if "normed_gemm_kernel" in k}
+    assert len(found) >= 6 and max(found.values()) <= 128
