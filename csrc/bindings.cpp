@@ -510,7 +510,7 @@ void launch_with_norm(shai::GemmArgs g, const Tensor& like, const Choice& c, con
   n.residual = g.residual;
   n.res_alpha = g.res_alpha;
   n.raw = st.keep ? g.C : nullptr;
-  if (shai::gn_two_wanted(n)) {
+  if (((uintptr_t)g.C & 15) == 0 && shai::gn_two_wanted(n)) {
     Tensor stats = at::empty({shai::gn_two_floats(n)}, like.options().dtype(at::kFloat));
     check_launch(shai::launch_gn_two(n, g.C, stats.data_ptr<float>(), stream()), "gn_two");
     return;

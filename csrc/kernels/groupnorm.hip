@@ -18,11 +18,16 @@ namespace {
 // as many workgroups, and with 16 vectors it was the slower way (4 x 32 x 32 x 960: 14.8 us, statistics and apply 12.8; 4 x 48 x 48 x
 // 320: 12.1 and 11.6; with 8, 4 x 16 x 16 x 960: 7.3 and 9.8).
 constexpr int kMaxVec = 16, kMaxVecTwo = 8, kMaxVecFold = 8;
-// A group's values of all parts from which the fold and the norm are two launches, the fold on every CU.  us with the convolution, one launch
-// and two: 2 x 32 x 32 x 640 in 4 parts 49.4 and 42.7, in 16 108.5 and 82.4, 1 x 32 x 32 x 640 in 8 53.0 and 34.5, 2 x 16 x 16 x 1280 in 8 42.4
-// and 41.9 (all from 81920 values); 2 x 12 x 12 x 1280 in 8 34.1 and 36.9, 4 x 16 x 16 x 1280 in 4 52.1 and 55.4, 2 x 8 x 8 x 1280 in 16 22.4
-// and 25.8.
-constexpr long kFoldTwo = 5 << 14;
+// Pixels of all parts, times a group's width and 160, from which the fold and the norm are two launches, the fold on every CU, where the
+// one launch has up to 64 workgroups. What a pixel costs the one launch grows little with the width: it is a row of its own in every part.
+// us with the convolution, one launch and two, above: 2 x 32 x 32 x 640 in 4 parts 54.3 and 48.2, 1 x 32 x 32 x 640 in 8 58.4 and 39.7, 2 x
+// 24 x 24 x 640 in 4 42.8 and 41.6, 2 x 40 x 40 x 320 in 3 44.8 and 29.9, 1 x 16 x 16 x 1280 in 8 35.2 and 34.3, 2 x 16 x 16 x 1280 in 8
+// 52.8 and 53.2, in 12 50.9 and 49.0, 2 x 20 x 20 x 1280 in 6 60.4 and 59.5; below: 2 x 16 x 16 x 640 in 8 26.9 and 27.0, 2 x 24 x 24 x 640
+// in 3 47.7 and 47.5, 2 x 20 x 20 x 1280 in 4 69.5 and 70.3, 2 x 16 x 16 x 1280 in 6 38.2 and 39.8, 1 x 12 x 12 x 2560 in 8 34.6 and 38.5.
+// With 96 and 128 workgroups: 3 x 16 x 16 x 1280 in 8 56.3 and 62.2, 4 x 16 x 16 x 1280 in 8 73.5 and 76.0, 4 x 24 x 24 x 640 in 6 58.0 and
+// 58.3.
+constexpr long kFoldTwo = 2048 * 200;
+constexpr int kFoldTwoUnits = 64;
 
 struct GnOneGeom {
   int u;        // groups per workgroup
@@ -319,7 +324,8 @@ hipError_t launch_gn_one(const GnOneArgs& a, hipStream_t s) {
 
 bool gn_two_wanted(const GnOneArgs& a) {
   GnTwoGeom q;
-  return a.parts != nullptr && a.HW * (long)(a.C / a.G) * a.splits >= kFoldTwo && ((uintptr_t)a.out & 15) == 0 && two_geometry(a, &q);
+  return a.parts != nullptr && (long)a.HW * a.splits * (a.C / a.G + 160) >= kFoldTwo && ((uintptr_t)a.out & 15) == 0 && two_geometry(a, &q) &&
+         a.N * (a.G / q.one.u) <= kFoldTwoUnits;
 }
 
 long gn_two_floats(const GnOneArgs& a) {

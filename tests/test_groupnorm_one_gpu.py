@@ -111,3 +111,20 @@ def test_large_fold(cuda, N, side, cout, splits):
                         gn_out=torch.empty_like(raw), gn_groups=32, keep_out=False)
     two = side * side * cout // 32 * splits >= 81920
     assert bool((raw == 7).any()) != two
+
+
+# which folds take two launches: narrow groups of many pixels, wide ones of few, both sides of the border, and no more than 64 workgroups of the one
+@pytest.mark.parametrize("N,side,cout,splits,two", [(1, 24, 640, 4, True), (2, 40, 320, 3, True), (2, 16, 960, 12, True), (2, 16, 960, 8, False),
+                                                    (1, 12, 2560, 8, False), (2, 20, 1280, 4, False), (3, 16, 1280, 8, False),
+                                                    (4, 16, 1280, 8, False), (4, 24, 640, 8, False)])
+def test_which_folds_take_two(cuda, N, side, cout, splits, two):
+    cin, M = 64, N * side * side
+    x, b, gamma, beta = rnd(N, side, side, cin), rnd(cout), rnd(cout), rnd(cout)
+    w = rnd(cout, 9 * cin, scale=(9 * cin) ** -0.5)
+    native.ops().gemm_tuning_import([f"1:{M},{cout},{9 * cin},b1,g0|{N},{side},{side},{cin},{cin},3,1,0,0=18,{splits}"])
+    raw, y = torch.full((N, side, side, cout), 7.0, device="cuda", dtype=torch.bfloat16), torch.empty(N, side, side, cout, device="cuda", dtype=torch.bfloat16)
+    native.ops().conv2d(x, None, w, raw, b, None, None, None, None, 0, 3, 3, 1, 1, False, 0, 1.0, gn_gamma=gamma, gn_beta=beta, gn_out=y,
+                        gn_groups=32, keep_out=False)
+    assert bool((raw == 7).all()) != two     # the one launch leaves the convolution unwritten
+    plain = ops.conv2d(x, w, b, 3, 3, 1, 1)
+    assert off(y, norm64(plain, gamma, beta, 32, 1e-5, False)) < 2 ** -8
