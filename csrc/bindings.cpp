@@ -1230,10 +1230,11 @@ bool attn_proj_fits(const Tensor& q, const Tensor& k, const Tensor& v, const Ten
   auto heads = [&](const Tensor& t) {
     return at(t, 16) && t.dim() == 4 && t.stride(3) == 1 && t.stride(2) == D && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0;
   };
-  return D == 64 && heads(q) && heads(k) && heads(v) && k.size(1) <= 256 && k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(2) == H &&
+  return D == 64 && heads(q) && heads(k) && heads(v) && k.size(1) >= 1 && k.size(1) <= 256 && k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(2) == H &&
          at(w, 16) && w.size(0) % 16 == 0 && w.size(1) == H * D && w.stride(1) == 1 && w.stride(0) % 8 == 0 && (!bias || at(*bias, 8)) &&
          at(residual, 8) && at(gamma, 8) && (!beta || at(*beta, 8)) &&
-         (!attn_bias || (attn_bias->is_contiguous() && attn_bias->scalar_type() == at::kBFloat16));
+         (!attn_bias || (attn_bias->is_contiguous() && attn_bias->scalar_type() == at::kBFloat16 && attn_bias->dim() == 3 && attn_bias->size(0) == H &&
+                         attn_bias->size(1) == q.size(1) && attn_bias->size(2) == k.size(1)));
 }
 
 // y = attention(q, k, v) w^T + bias + residual and out = RMS norm or LayerNorm of y, in two launches: every head's attention with its

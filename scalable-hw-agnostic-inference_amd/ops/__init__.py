@@ -622,7 +622,8 @@ def attention_linear_norm(q, k, v, w, bias, residual, norm, scale: Optional[floa
     [B, Skv, H, D]; ``kv_lens``, ``attn_bias`` [H, Sq, Skv]: see :func:`attention`.  On the GPU a few rows of a few keys take two launches:
     the heads' attention and projection, then the sum over heads with the norm."""
     B, S, H, D = q.shape
-    if not (_gpu(q) and _attention_linear_fits(q, k, v, w, bias, residual, norm, attn_bias)):
+    lens = kv_lens is None or kv_lens.numel() == B
+    if not (_gpu(q) and lens and _attention_linear_fits(q, k, v, w, bias, residual, norm, attn_bias)):
         o = attention(q, k, v, scale=scale, causal=causal, kv_lens=kv_lens, bias=attn_bias)
         return linear_norm(o.reshape(B, S, H * D), w, bias, residual, norm)
     y = torch.empty(B, S, w.shape[0], dtype=q.dtype, device=q.device)

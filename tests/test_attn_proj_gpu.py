@@ -84,3 +84,15 @@ def test_what_does_not_fit_takes_the_general_path(cuda):
         y, n = ops.attention_linear_norm(*a)
         assert (y.double() - want).norm() <= 2 ** -8 * want.norm()
         assert (n.double() - a[-1](y).double()).norm() <= 2 ** -8 * n.double().norm()
+
+
+def test_what_attention_takes_is_not_refused(cuda):
+    """A bias with a batch dimension of one and lengths of more sequences than there are, which attention takes: the general path."""
+    args, kw = problem(cuda, 2, 33, 33, 4, 256, False, True, [20, 33], True)
+    want = wanted(args, kw)
+    bias, lens = kw["attn_bias"], kw["kv_lens"]
+    assert ops._attention_linear_fits(*args, bias) and not ops._attention_linear_fits(*args, bias[None])
+    for change in (dict(attn_bias=bias[None]), dict(kv_lens=torch.cat([lens, lens]))):
+        y, n = ops.attention_linear_norm(*args, **{**kw, **change})
+        assert (y.double() - want).norm() <= 2 ** -8 * want.norm()
+        assert (n.double() - args[-1](y).double()).norm() <= 2 ** -8 * n.double().norm()
