@@ -244,13 +244,13 @@ int main(int argc, char** argv) {
     const char* name;
     int kind;  // 0: v3 256 4-stage, 1: v3 256 2-stage, 2: v3 320 2-stage, 10+v: v4 schedule variant v
   };
-  const Var vars[] = {{"v4_256w", 30}, {"v4_256pwn", 70}, {"v4_320w", 130}, {"v4_320pwn", 170}, {"w4_256", 5}, {"w4_320", 6},
+  const Var vars[] = {{"v4_256w", 30}, {"v4_256pwn", 70}, {"v4_320w", 130}, {"v4_320pwn", 170}, {"w4_256", 5}, {"w4_192", 6},
                       {"ws_320", 7}, {"ws_nost", 107}, {"ws_nomfma", 207}, {"ws_nodma", 407}, {"ws_dmaonly", 307}};
   constexpr int NV = sizeof(vars) / sizeof(vars[0]);
   auto run = [&](const Var& v, const shai::GemmArgs& g) {
     switch (v.kind) {
       case 5: shai::launch_gemm_w4(g, 256, s); break;
-      case 6: shai::launch_gemm_w4(g, 320, s); break;
+      case 6: shai::launch_gemm_w4(g, 192, s); break;
       case 7: case 107: case 207: case 307: case 407:
         shai::gemm_ws_set_ablation(v.kind / 100);
         shai::launch_gemm_ws(g, s);
