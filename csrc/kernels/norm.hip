@@ -586,17 +586,19 @@ void launch_groupnorm_stats(const GroupNormArgs& a, hipStream_t s) {
     gn_finalize_kernel<<<dim3(a.N, a.G), 64, 0, s>>>(a.partials, a.gamma, a.beta, a.scale, a.shift, a.HW, a.C, a.G, NB, a.eps);
 }
 
-// Workgroups of the apply pass.  A thread has one vector, or two or three (as there are 2^18 of them, 1024 workgroups) of one or two large
-// images: they lie a grid apart, mostly in one image, and share its scale and shift.  With more images every vector loads a set of its
-// own, and the workgroups of the last round have the chip to themselves.  us for one, two, three vectors: 1 x 16384 x 512 7.9, 7.2, 7.2, 1 x
-// 64512 x 256 14.2, 12.7, 12.8, 1 x 102400 x 256 20.3, 19.8, 18.5, 1 x 262144 x 128 25.0, 23.5, 22.7, 1 x 262144 x 256 48.0, 43.1, 42.8, 1 x 589824 x
-// 128 52.1, 47.7, 47.0, 2 x 9216 x 640 9.9, 9.5, 9.3, 2 x 65536 x 256 24.5, 23.4, 22.4, 1 x 8192 x 512 5.4, 5.2, 5.4; below 2^19 vectors 1 x 6144 x
-// 512 4.5, 4.6, 4.8, 2 x 4096 x 320 4.1, 4.5, 4.7; more images 4 x 9216 x 640 18.4, 18.7, 20.6, 8 x 16384 x 512 46.5, 47.2, 50.9, 16 x 4096 x 640 30.6,
-// 31.9, 36.8.  4096 workgroups at every size: 8 x 16384 x 512 64.0, 16 x 4096 x 640 40.1.  Two or four vectors on their way in a thread:
-// slower at every size.
+// Workgroups of the apply pass. A thread has one vector, or two or three of large tensors, as there are 2^18 of them (1024 workgroups): up
+// to three of one or two images, two of three or four. They lie a grid apart, and those in one image share its scale and shift; with more
+// images every vector loads a set of its own, and the workgroups of the last round have the chip to themselves. us for one, two, three
+// vectors: 1 x 16384 x 512 7.9, 7.2, 7.2, 1 x 64512 x 256 14.2, 12.7, 12.8, 1 x 102400 x 256 20.3, 19.8, 18.5, 1 x 262144 x 128 25.0, 23.5,
+// 22.7, 1 x 262144 x 256 48.0, 43.1, 42.8, 1 x 589824 x 128 52.1, 47.7, 47.0, 2 x 9216 x 640 9.9, 9.5, 9.3, 2 x 65536 x 256 24.5, 23.4,
+// 22.4, 1 x 8192 x 512 5.4, 5.2, 5.4; below 2^19 vectors 1 x 6144 x 512 4.5, 4.6, 4.8, 2 x 4096 x 320 4.1, 4.5, 4.7; three and four images
+// 4 x 4096 x 640 9.2, 9.0, 8.8, 3 x 16384 x 512 19.5, 19.2, 20.8, 4 x 9216 x 640 18.4, 18.7, 20.6, 4 x 16384 x 512 24.7, 24.5, 27.2, 3 x
+// 65536 x 256 35.0, 33.8, 34.7, 4 x 65536 x 256 45.8, 44.7, 45.8; more 8 x 16384 x 512 46.5, 47.2, 50.9, 16 x 4096 x 640 30.6, 31.9, 36.8.
+// 4096 workgroups at every size: 8 x 16384 x 512 64.0, 16 x 4096 x 640 40.1. Two or four vectors on their way in a thread: slower at every
+// size.
 long gn_apply_blocks(int N, int HW, int C) {
   const long total8 = (long)N * HW * C / 8;
-  const long each = N > 2 ? 1 : std::min(3L, std::max(1L, total8 >> 18));
+  const long each = std::max(1L, std::min(N <= 2 ? 3L : N <= 4 ? 2L : 1L, total8 >> 18));
   long blocks = (total8 + 256 * each - 1) / (256 * each);
   if (blocks > 65536) blocks = 65536;
   // grid threads a multiple of C / 8 (the kernel keeps one channel vector per thread)

@@ -16,7 +16,7 @@ def each(N, HW, C):
 
 @pytest.mark.parametrize("N,HW,C,want", [
     (1, 4096, 320, 1), (2, 4096, 384, 1), (1, 16383, 256, 1), (1, 16384, 256, 2), (1, 24575, 256, 2), (1, 24576, 256, 3), (2, 147456, 256, 3),
-    (3, 4096, 960, 1), (16, 4096, 640, 1)])
+    (3, 4096, 960, 2), (3, 1024, 1280, 1), (4, 65536, 256, 2), (5, 65536, 256, 1), (16, 4096, 640, 1)])
 def test_by_size_and_images(N, HW, C, want):
     assert each(N, HW, C) == want
 

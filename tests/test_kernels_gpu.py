@@ -92,7 +92,7 @@ def test_groupnorm_two_source(cuda, N, HW, C1, C2, fused, monkeypatch):
 
 # one, two and three vectors a thread, with remainders; two images, whose border lies between a thread's vectors; channels that 256 threads
 # do not divide
-@pytest.mark.parametrize("N,HW,C", [(1, 1, 8), (1, 16385, 256), (1, 24577, 264), (2, 12289, 384), (3, 5000, 320)])
+@pytest.mark.parametrize("N,HW,C", [(1, 1, 8), (1, 16385, 256), (1, 24577, 264), (2, 12289, 384), (3, 5000, 320), (4, 3333, 328)])
 def test_groupnorm_apply_sizes(cuda, N, HW, C):
     """Against 64 bits: the rounding of the bf16 result, 2^-9 of a value."""
     torch.manual_seed(HW)
