@@ -118,11 +118,6 @@ bool gemm_deep_supported(const GemmArgs& a) {
 
 int gemm_deep_wave_groups(int which) { return kDeep[which].wk; }
 
-int gemm_deep_per_cu(int which) {
-  const Deep& d = kDeep[which];
-  return 160 * 1024 / (d.stages * (d.bm + d.bn) * BK2 * (int)sizeof(bf16_t));
-}
-
 void gemm_deep_tile(int which, int* bm, int* bn) {
   *bm = kDeep[which].bm;
   *bn = kDeep[which].bn;

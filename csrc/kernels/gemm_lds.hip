@@ -320,22 +320,24 @@ bool gemm2_cfg_candidate(int cfg) { return !(cfg >= kNumCfgs && cfg < kV4Cfg); }
 
 bool gemm2_cfg_splittable(int cfg) { return cfg != kW4Cfg && cfg != kW4Cfg + 1 && cfg != kWsCfg; }
 
-// One count from each of 2 to 3, 4 to 6, 7 to 12 and 13 to 16: the one with which the tiles' parts leave the fewest slots of the chip's last
-// round empty.  (2, 4, 8 and 16, as many launches to time, were 1.026 times the best of all counts to 16, in the mean of the 175 convolutions of
-// requests of 448 x 576, 640 x 384, 512 x 512 and 768 x 768 pixels and of small batches, up to 1.19, 55 of them over 1.03; these are 1.002, up to
-// 1.07, 5.  Plain products 1.002 either way.)  No part is empty or under 4 k-tiles.
+// One count from each of 2 to 3, 4 to 6, 7 to 12 and 13 to 16: the one with which the tiles' parts leave the fewest of the 256 CUs without one
+// in the last round. Workgroups of small tiles share a CU, but where every CU has as many of them none waits: counted by the places that a CU's
+// LDS has for them, 4096 columns of 110 rows lost the 256 workgroups of 64 x 64 tiles in two parts to 384 in three, of which half the CUs had
+// two (K = 4096, cold weights: 16.9 and 20.9 us with what was taken in their stead).
+// Times of what is picked over the best of all counts to 16, in the mean and at most, for 322 convolutions of requests of 320 x 256 to 768 x 768
+// pixels and of small batches: 2, 4, 8 and 16, as many launches to time, 1.019 and 1.24, 69 of them over 1.03; by places in LDS 1.0017 and 1.09, 7;
+// by CUs 1.0007 and 1.05, 2. For 78 plain products of 70 to 600 rows 1.0025 and 1.09, 1.0020 and 1.04, 1.0007 and 1.03. No part is empty or
+// under 4 k-tiles.
 int gemm2_split_counts(int M, int N, int K, int cfg, int most, int* out) {
-  int bm, bn, per_cu = 1;
+  int bm, bn;
   if (cfg >= kDeepCfg) {
     gemm_deep_tile(cfg - kDeepCfg, &bm, &bn);
-    per_cu = gemm_deep_per_cu(cfg - kDeepCfg);
   } else if (cfg >= kNumCfgs) {
     bm = 256, bn = cfg >= kV4Cfg && ((cfg - kV4Cfg) & 1) ? 320 : 256;
   } else {
     bm = kCfgs[cfg].bm, bn = kCfgs[cfg].bn;
-    per_cu = 160 * 1024 / (2 * (bm + bn) * BK2 * (int)sizeof(bf16_t));
   }
-  const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn), slots = 256 * per_cu;
+  const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   const int kt = (K + BK2 - 1) / BK2;
   int n = 0;
   out[n++] = 1;
@@ -345,7 +347,7 @@ int gemm2_split_counts(int M, int N, int K, int cfg, int most, int* out) {
     for (int s = (4 * p + 4) / 5; 5 * s < 8 * p && s <= 16; ++s) {
       const int per = (kt + s - 1) / s;
       if (kt / s < 4 || (kt + per - 1) / per != s) continue;
-      const long rounds = (tiles * s + slots - 1) / slots, left = rounds * slots - tiles * s;
+      const long rounds = (tiles * s + 255) / 256, left = rounds * 256 - tiles * s;
       if (best == 0 || left * best_rounds < best_left * rounds) best = s, best_left = left, best_rounds = rounds;
     }
     if (best) out[n++] = best;

@@ -220,7 +220,6 @@ constexpr int kDeepCfgs = 6;
 bool gemm_deep_supported(const GemmArgs& a);
 void gemm_deep_tile(int which, int* bm, int* bn);
 int gemm_deep_wave_groups(int which);  // along K
-int gemm_deep_per_cu(int which);       // workgroups that a CU's LDS holds
 void launch_gemm_deep(const GemmArgs& a, int which, float* ws, int splits, hipStream_t s);
 // v6: W-stationary low-K GEMM (gemm_ws.hip): K = 320, N % 320 == 0, persistent over M, weights in VGPRs
 bool gemm_ws_supported(const GemmArgs& a);

@@ -10,8 +10,8 @@ from shai_amd import native
 if not os.path.exists(native.KERNELS_LIB):
     pytest.skip("the native library is not built", allow_module_level=True)
 
-# tile rows, columns and workgroups a CU of some configs
-TILES = {1: (256, 256, 1), 3: (128, 128, 2), 4: (128, 64, 3), 9: (256, 256, 1), 10: (256, 320, 1), 16: (64, 64, 2), 18: (128, 128, 1), 21: (192, 128, 2)}
+# tile rows and columns of some configs
+TILES = {1: (256, 256), 3: (128, 128), 4: (128, 64), 9: (256, 256), 10: (256, 320), 16: (64, 64), 17: (128, 64), 18: (128, 128), 21: (192, 128)}
 
 
 def counts(M, N, K, cfg):
@@ -20,18 +20,23 @@ def counts(M, N, K, cfg):
 
 @pytest.mark.parametrize("cfg", sorted(TILES))
 @pytest.mark.parametrize("M,N,K", [(126, 1280, 11520), (120, 1280, 23040), (2048, 640, 17280), (504, 640, 5760), (8064, 4, 2880), (77, 320, 520),
-                                   (2, 8, 64), (18432, 320, 8640)])
+                                   (2, 8, 64), (18432, 320, 8640), (110, 4096, 4096)])
 def test_counts_fill_rounds(M, N, K, cfg):
     """From each of four ranges the count whose last round is the fullest, no more of them than powers of two, no part empty or short."""
-    bm, bn, per_cu = TILES[cfg]
-    tiles, slots, kt = -(-M // bm) * -(-N // bn), 256 * per_cu, -(-K // 64)
-    fill = lambda s: tiles * s / (-(-tiles * s // slots) * slots)
+    bm, bn = TILES[cfg]
+    tiles, kt = -(-M // bm) * -(-N // bn), -(-K // 64)
+    fill = lambda s: tiles * s / (-(-tiles * s // 256) * 256)
     got, want = counts(M, N, K, cfg), [1]
     for lo, hi, power in ((2, 3, 2), (4, 6, 4), (7, 12, 8), (13, 16, 16)):
         fit = [s for s in range(lo, hi + 1) if kt // s >= 4 and -(-kt // -(-kt // s)) == s]
         if fit and kt // power >= 4:
             want.append(max(fit, key=lambda s: (round(fill(s), 9), -s)))
     assert got == want and len(got) <= 5
+
+
+def test_a_part_for_every_cu():
+    """Workgroups that share a CU do not hide counts that give every CU one."""
+    assert 2 in counts(110, 4096, 4096, 16) and 4 in counts(110, 4096, 4096, 17)
 
 
 def test_unsplit_tiles():
