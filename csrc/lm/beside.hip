@@ -16,23 +16,32 @@ namespace shai_lm {
 // three spill 51 to 53: 64 sequences of 900 keys 72.9, at two 50.8, one after the other 67.4; of 132 keys 39.5, 36.7 and 45.7.
 constexpr int workgroups(int D, int RH) { return D == 128 && RH == 8 ? 2 : 3; }
 
-// Eight V loads in flight: as fast as the sixteen of the attention alone, which spill 7 registers here (64 sequences of 132 keys 39.4 -> 38.3).
-template <int D, int RH, int MODE, int SD>
-__global__ void __launch_bounds__(256, workgroups(D, RH)) attn_rule_kernel(const AttnArgs a, const RuleArgs r, int per_group, int heads, int n_attn) {
+// V: V loads of the attention in flight. Eight where three workgroups share a CU: sixteen spill 7 registers there (64 sequences of 132 keys, 4 heads
+// of 128 a group, 39.4 -> 38.3 us).
+template <int D, int RH, int MODE, int SD, int V>
+__global__ void __launch_bounds__(256, V == 16 ? 2 : workgroups(D, RH)) attn_rule_kernel(const AttnArgs a, const RuleArgs r, int per_group, int heads, int n_attn) {
   const int i = blockIdx.x;
   if (i < n_attn) {
     const int j = i / heads;
-    attn_decode<D, D, RH, true, 8>(a, per_group, 1, i - j * heads, j % a.B, j / a.B);
+    attn_decode<D, D, RH, true, V>(a, per_group, 1, i - j * heads, j % a.B, j / a.B);
   } else {
     const int b = (i - n_attn) / r.H;
     rule_rows<bf16_t, MODE, SD, SD, 256, true>(r, i - n_attn - b * r.H, b);
   }
 }
 
+// Steps of up to so many workgroups have two on a CU at most, whatever their registers: sixteen loads without a spill (one sequence of 132 keys 12.9 ->
+// 12.4 us).
+constexpr int kFew = 512;
+
 template <int D, int RH, int MODE, int SD>
 static void attn_rule(const AttnArgs& a, const RuleArgs& r, hipStream_t s) {
-  const int n_attn = a.G * a.B * a.splits;
-  attn_rule_kernel<D, RH, MODE, SD><<<n_attn + r.H * r.B, 256, 0, s>>>(a, r, a.H / a.G, a.G, n_attn);
+  const int n_attn = a.G * a.B * a.splits, grid = n_attn + r.H * r.B;
+  auto go = [&](auto kernel) { kernel<<<grid, 256, 0, s>>>(a, r, a.H / a.G, a.G, n_attn); };
+  if constexpr (D == 128 && RH == 4) {
+    if (grid <= kFew) return go(attn_rule_kernel<D, RH, MODE, SD, 16>);
+  }
+  go(attn_rule_kernel<D, RH, MODE, SD, 8>);
 }
 
 template <int D, int RH>

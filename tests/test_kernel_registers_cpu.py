@@ -46,7 +46,7 @@ def test_joined_and_fused_kernels_do_not_spill(tmp_path):
     """Kernels that hold the work of two: attention beside a delta rule, a norm in its product, attention with its projection, products whose
     tiles follow each other, the four-wave tile."""
     a, b = spills(native.KERNELS_LIB, tmp_path), spills(native.LM_LIB, tmp_path)
-    for lib, name, least in ((b, "attn_rule_kernel", 16), (b, "normed_gemm_kernel", 6), (a, "attn_proj_kernel", 9), (b, "gemm_wide_kernel", 1),
+    for lib, name, least in ((b, "attn_rule_kernel", 20), (b, "normed_gemm_kernel", 6), (a, "attn_proj_kernel", 9), (b, "gemm_wide_kernel", 1),
                              (a, "gemm_w4_kernel", 10), (a, "fold_norm_kernel", 6), (a, "skinny3_kernel", 1)):
         found = {k: n for k, n in lib.items() if name in k}
         assert len(found) >= least, name

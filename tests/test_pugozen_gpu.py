@@ -90,11 +90,12 @@ def test_prompts_in_segments(cuda, monkeypatch, rows):
 @pytest.mark.parametrize("B,H,G,d,rule,channels,splits", [
     (1, 4, 1, 128, (4, 2, 128), True, 1), (3, 8, 1, 64, (2, 1, 64), False, 2), (5, 2, 2, 64, (3, 3, 128), True, 1),
     (2, 12, 1, 64, (2, 2, 64), True, 1), (3, 8, 1, 128, (2, 2, 128), True, 2),
-    (2, 14, 2, 128, (2, 1, 64), False, 1), (64, 16, 4, 128, (16, 16, 128), True, 1), (1, 4, 4, 128, (2, 2, 256), False, 1)])
+    (2, 14, 2, 128, (2, 1, 64), False, 1), (64, 16, 4, 128, (16, 16, 128), True, 1), (1, 4, 4, 128, (2, 2, 256), False, 1),
+    (25, 16, 4, 128, (16, 8, 128), False, 1), (26, 16, 4, 128, (16, 16, 64), True, 1)])
 def test_mixers_of_a_step_in_one_launch(cuda, B, H, G, d, rule, channels, splits):
     """Attention and delta rule together against one after the other: caches, states and both outputs.  Groups and head sizes that the one
     launch takes and that it does not (12 heads to a group, heads of 256); contexts of one key, of whole blocks and past them; sequences
-    without a slot.  The sums are the same in the same order, compiled twice: a last bit of the bf16 outputs, 2^-16 of the fp32 states."""
+    without a slot; the most workgroups of the form for few of them, and more.  The sums are the same in the same order, compiled twice: a last bit of the bf16 outputs, 2^-16 of the fp32 states."""
     from types import SimpleNamespace
     lm, (R, K, s) = C.lm, rule
     g = torch.Generator(device=cuda).manual_seed(B * H + s)
