@@ -7,6 +7,11 @@
 //
 // 8 waves: wave w takes the 32 k of sub-step w % 4 and the row blocks of half w / 4; the four k-groups' sums meet in LDS and are
 // added in their order.  Rows past M or N and values past K are out of the buffers' range: zeros, no traffic.
+// A workgroup with all of K begins kTurn steps behind the one before it and goes round: begun together, all of them read the same columns of
+// W, rows of 2^n bytes apart, from a part of the memory's channels.  us in order -> turned, cold weights, 16 / 32 / 64 rows: 28672 x 4096 54.1 / 53.3 /
+// 56.1 -> 43.8 / 43.9 / 46.5, 32768 x 2048 35.9 / 34.3 / 36.7 -> 35.7 / 32.7 / 29.3, 17424 x 2048 19.0 / 19.7 / 22.3 -> 16.7 / 17.1 / 20.0, 8192 x 8192
+// 36.3 / 35.4 / 38.0 -> 26.3 / 26.0 / 31.8 (by one step 35.2, by three 29.9, by five 27.1); nothing is slower (5632 x 1024, 4096 x 4096).
+//
 // LDS rows are 256 bytes; chunk c (16 bytes) of row r is at c ^ (r & 15): no bank conflicts, and the DMA stays lane-linear because
 // the source address carries the permutation.
 //
@@ -25,6 +30,7 @@ namespace {
 
 constexpr uint32_t kOob = 0x80000000u;
 constexpr int KS = 128;                       // k of one ring stage
+constexpr unsigned kTurn = 7;                 // steps by which a workgroup begins behind the one before it
 
 constexpr int ring_stages(int MT, int NT) {   // as many as fit in 160 KB, at most 5
   const int n = 160 * 1024 / ((MT + NT) * 16 * KS * 2);
@@ -55,6 +61,7 @@ __global__ void __launch_bounds__(512) gemm_ring_kernel(const GemmArgs p) {
     steps = (int)((blockIdx.y + 1L) * all / p.splits) - first;
     C += (long)blockIdx.y * p.M * p.N;
   }
+  const int turn = p.splits > 1 ? 0 : (int)(blockIdx.x * kTurn % steps);   // the first step
   uint32_t off[HI];
   int col[HI];                                // first k of this lane's chunk within a stage
 #pragma unroll
@@ -65,7 +72,7 @@ __global__ void __launch_bounds__(512) gemm_ring_kernel(const GemmArgs p) {
     else off[j] = row < p.M ? (uint32_t)(((long)row * p.lda + col[j]) * 2) : kOob;
   }
   auto stage = [&](int buf, int s) {          // step s of this workgroup; past its end: zeros
-    const int k = (first + s) * KS;
+    const int k = (first + (s + turn < steps ? s + turn : s + turn - steps)) * KS;
 #pragma unroll
     for (int j = 0; j < HI; ++j) {
       const int piece = wid + 8 * j;
