@@ -32,6 +32,7 @@
 #include "common.h"
 #include "launchers.h"
 #include "gemm_epilogue.h"
+#include "skinny_turn.h"
 
 #include <cstdlib>
 #include <map>
@@ -133,7 +134,7 @@ __device__ __forceinline__ int sk_f8_off(int row, int c8) {
   return row * 64 + (((c8 >> 1) ^ ((row >> 2) & 3)) << 4) + ((c8 & 1) << 3);
 }
 
-template <int MB, bool GLU, int ACT, bool RMS, bool F8>
+template <int MB, bool GLU, int ACT, bool RMS, bool F8, bool TURN>
 __global__ void __launch_bounds__(SK_WAVES * 64) skinny_gemm_kernel(const GemmArgs p, float* __restrict__ ws,
                                                                     int kg_steps, unsigned* __restrict__ cnt) {
   using G = SkGeom<MB, F8>;
@@ -149,6 +150,7 @@ __global__ void __launch_bounds__(SK_WAVES * 64) skinny_gemm_kernel(const GemmAr
   const int ksteps = (p.K + SK_BK - 1) / SK_BK;
   const int t0 = kg * kg_steps;
   const int nk = max(0, min(ksteps, t0 + kg_steps) - t0);
+  const int turn = TURN ? tile * kSkinnyTurn % nk : 0;   // the first step
 
   const __amdgpu_buffer_rsrc_t rW = sk_rsrc(p.W, (uint32_t)min((long)p.N * p.ldw * (F8 ? 1 : 2), 0x7fffffffL));
   const __amdgpu_buffer_rsrc_t rX = sk_rsrc(p.A, (uint32_t)min((long)p.M * p.lda * 2, 0x7fffffffL));
@@ -171,6 +173,7 @@ __global__ void __launch_bounds__(SK_WAVES * 64) skinny_gemm_kernel(const GemmAr
   auto stage = [&](int buf, int step) {
     bf16_t* sw = sk_smem + buf * G::STAGE_ELEMS;
     bf16_t* sx = sw + G::W_ELEMS;
+    if (TURN) step = step + turn < nk ? step + turn : step + turn - nk;
     const int k0 = (t0 + step) * SK_BK;
     if constexpr (F8) {
       const int n = n0 + f8row, k = k0 + f8c * 16;
@@ -553,7 +556,7 @@ static unsigned* sk_tickets(hipStream_t s, int ntiles) {
 
 unsigned* skinny_ticket_slice(hipStream_t s, int ntiles) { return sk_tickets(s, ntiles); }
 
-template <int MB, bool F8>
+template <int MB, bool F8, bool TURN = false>
 static void launch_skinny_mb(const GemmArgs& a, float* ws, int kg, unsigned* cnt, hipStream_t s) {
   const int ksteps = (a.K + SK_BK - 1) / SK_BK;
   const int kg_steps = (ksteps + kg - 1) / kg;
@@ -561,8 +564,8 @@ static void launch_skinny_mb(const GemmArgs& a, float* ws, int kg, unsigned* cnt
   const size_t lds = SkGeom<MB, F8>::LDS;
 #define SK(G, A)                                                                                          \
   do {                                                                                                    \
-    if (a.rms) skinny_gemm_kernel<MB, G, A, true, F8><<<grid, block, lds, s>>>(a, ws, kg_steps, cnt);  \
-    else skinny_gemm_kernel<MB, G, A, false, F8><<<grid, block, lds, s>>>(a, ws, kg_steps, cnt);       \
+    if (a.rms) skinny_gemm_kernel<MB, G, A, true, F8, TURN><<<grid, block, lds, s>>>(a, ws, kg_steps, cnt);  \
+    else skinny_gemm_kernel<MB, G, A, false, F8, TURN><<<grid, block, lds, s>>>(a, ws, kg_steps, cnt);       \
   } while (0)
 #define SK_ACT(G)                                      \
   switch (a.act) {                                     \
@@ -596,7 +599,15 @@ void launch_skinny_kg(const GemmArgs& a_in, float* ws, int kg, hipStream_t s, bo
   // split-K: fixed up inside the launch when asked for and tickets are available, else a separate fold
   unsigned* cnt = nullptr;
   if (kg > 1 && fixup) cnt = sk_tickets(s, (a.N + SK_BN - 1) / SK_BN);
-  if (a.w_scale) {
+  if (skinny_turned(a, kg)) {
+    if (a.w_scale) {
+      if (a.M <= 32) launch_skinny_mb<32, true, true>(a, ws, kg, cnt, s);
+      else launch_skinny_mb<64, true, true>(a, ws, kg, cnt, s);
+    } else {
+      if (a.M <= 32) launch_skinny_mb<32, false, true>(a, ws, kg, cnt, s);
+      else launch_skinny_mb<64, false, true>(a, ws, kg, cnt, s);
+    }
+  } else if (a.w_scale) {
     if (a.M <= 32) launch_skinny_mb<32, true>(a, ws, kg, cnt, s);
     else launch_skinny_mb<64, true>(a, ws, kg, cnt, s);
   } else {

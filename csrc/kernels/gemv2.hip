@@ -21,6 +21,7 @@
 //   order with sc1 loads (the write-through hand-off of gemv.hip) and runs the fused epilogue.
 #include "common.h"
 #include "launchers.h"
+#include "skinny_turn.h"
 
 namespace shai {
 
@@ -111,7 +112,7 @@ __device__ __forceinline__ void s2_epilogue(const GemmArgs& p, int nbase, int fr
   }
 }
 
-template <bool GLU, int ACT, bool RMS, int S2_STAGES>
+template <bool GLU, int ACT, bool RMS, int S2_STAGES, bool TURN>
 __global__ void __launch_bounds__(256) skinny2_kernel(const GemmArgs p, float* __restrict__ ws, int kg_steps,
                                                       unsigned* __restrict__ cnt) {
   extern __shared__ __attribute__((aligned(16))) bf16_t s2_smem[];
@@ -122,6 +123,7 @@ __global__ void __launch_bounds__(256) skinny2_kernel(const GemmArgs p, float* _
   const int ksteps = (p.K + S2_BK - 1) / S2_BK;
   const int t0 = kg * kg_steps;
   const int nk = max(0, min(ksteps, t0 + kg_steps) - t0);
+  const int turn = TURN ? tile * kSkinnyTurn % nk : 0;   // the first step
 
   const __amdgpu_buffer_rsrc_t rW = s2_rsrc(p.W, (uint32_t)min((long)p.N * p.ldw * 2, 0x7fffffffL));
   const __amdgpu_buffer_rsrc_t rX = s2_rsrc(p.A, (uint32_t)min((long)p.M * p.lda * 2, 0x7fffffffL));
@@ -146,6 +148,7 @@ __global__ void __launch_bounds__(256) skinny2_kernel(const GemmArgs p, float* _
   auto stage = [&](int buf, int step) {
     bf16_t* sw = s2_smem + buf * S2_STAGE;
     bf16_t* sx = sw + S2_W_ELEMS;
+    if (TURN) step = step + turn < nk ? step + turn : step + turn - nk;
     const int k0 = (t0 + step) * S2_BK;
     const bool kin = k0 < p.K;  // K tail: whole chunks past K read as zeros (K % 8 == 0)
 #pragma unroll
@@ -330,15 +333,20 @@ void launch_skinny2(const GemmArgs& a_in, float* ws, int kg, bool deep, hipStrea
   const int kg_steps = (ksteps + kg - 1) / kg;
   kg = (ksteps + kg_steps - 1) / kg_steps;  // no empty K groups (their tickets would never arrive)
   dim3 grid(tiles, kg), block(256);
-#define S2R(G, A, ST)                                                                                   \
+#define S2R(G, A, ST, T)                                                                                \
   do {                                                                                                  \
-    if (a.rms) skinny2_kernel<G, A, true, ST><<<grid, block, s2_lds(ST), s>>>(a, ws, kg_steps, cnt);    \
-    else skinny2_kernel<G, A, false, ST><<<grid, block, s2_lds(ST), s>>>(a, ws, kg_steps, cnt);         \
+    if (a.rms) skinny2_kernel<G, A, true, ST, T><<<grid, block, s2_lds(ST), s>>>(a, ws, kg_steps, cnt);    \
+    else skinny2_kernel<G, A, false, ST, T><<<grid, block, s2_lds(ST), s>>>(a, ws, kg_steps, cnt);         \
   } while (0)
-#define S2(G, A)              \
-  do {                        \
-    if (deep) S2R(G, A, 6);   \
-    else S2R(G, A, 3);        \
+#define S2(G, A)                          \
+  do {                                    \
+    if (skinny_turned(a, kg)) {           \
+      if (deep) S2R(G, A, 6, true);       \
+      else S2R(G, A, 3, true);            \
+    } else {                              \
+      if (deep) S2R(G, A, 6, false);      \
+      else S2R(G, A, 3, false);           \
+    }                                     \
   } while (0)
 #define S2_ACT(G)                                      \
   switch (a.act) {                                     \

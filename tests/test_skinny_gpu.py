@@ -443,3 +443,29 @@ def test_skinny_whole_k(cuda, M, N, K, act, extra):
     y = y + (r.double() if extra else 0)
     assert (out[:, :N].double() - y).abs().max() <= 2 ** -8 * max(1.0, float(y.abs().max()))
     assert _rel(out[:, :N], y) < 2 ** -8 and (out[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M", [1, 33, 64])
+@pytest.mark.parametrize("N,K,ld", [(16384, 2048, 2048), (16390, 2056, 4096), (16384, 64, 2048), (16388, 3000, 4096), (18000, 4096, 4096)])
+@pytest.mark.parametrize("cfg,rms", [(SKINNY + 1, True), (SKINNY2 + 1, True), (SKINNY2_DEEP + 1, False)])
+def test_skinny_turned(cuda, M, N, K, ld, cfg, rms):
+    """Workgroups that begin at different steps of K (rows a multiple of 4 KB apart): all steps and half of them, one step in order, K that ends inside a
+    step, columns that end inside a workgroup.  The fp64 result but for one rounding to bf16 (2^-9, as a 2-norm 2^-8 / sqrt(3) = 2.3e-3 at
+    most) and fp32 sums (1e-5)."""
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K, device=cuda).bfloat16()
+    w = (torch.randn(N, ld, device=cuda) / K ** 0.5).bfloat16()[:, :K]
+    out = torch.empty(M, N, device=cuda, dtype=torch.bfloat16)
+    ops.gemm_into(x, w, out, force_cfg=cfg, rms_eps=1e-5 if rms else -1.0)
+    xd = x.double()
+    want = (xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5) if rms else xd) @ w.double().t()
+    assert _rel(out, want) < 2.4e-3
+
+
+def test_skinny_turned_fp8(cuda):
+    M, N, K = 3, 16400, 4096
+    torch.manual_seed(5)
+    x = torch.randn(M, K, device=cuda).bfloat16()
+    w8, scale = ops.quantize_fp8_rows(torch.randn(N, K, device=cuda) / K ** 0.5)
+    want = x.double() @ (w8.double() * scale.double()[:, None]).t()
+    assert _rel(ops.linear(x, w8, w_scale=scale), want) < 2.4e-3
