@@ -699,3 +699,19 @@ def test_mean_tokens(cuda, B, S, D):
     """fp32 sums of at most 1024 bf16 values: 1e-6 of their spread."""
     x = torch.randn(B, S, D, device=cuda).bfloat16()
     assert (ops.mean_tokens(x).double() - x.double().mean(1)).abs().max().item() < 1e-6
+
+
+@pytest.mark.parametrize("act", ["gelu", "gelu_tanh"])
+def test_gelu_of_every_bf16(cuda, act):
+    """All 2^16 inputs.  One rounding to bf16 (half a unit in the last of 8 bits), and 6e-7 for the fp32 steps: 3.4e-7 (gelu) and 5.2e-7
+    (gelu_tanh) at most over -12 .. 12, behind them the results are 0 and x.  NaN for NaN; -inf times 0 is one too."""
+    x = torch.arange(65536, dtype=torch.int32, device=cuda).to(torch.int16).view(torch.bfloat16).view(256, 256)
+    y, xd = ops.bias_act(x, act=act).double(), x.double()
+    if act == "gelu":
+        want = xd * torch.special.ndtr(xd)
+    else:
+        want = xd * torch.sigmoid(2 * (2 / torch.pi) ** 0.5 * (xd + 0.044715 * xd ** 3))
+    num = torch.isfinite(xd) & (xd.abs() < 1e30)
+    assert bool(((y - want).abs() <= want.abs() * 2 ** -8 + 6e-7)[num].all())
+    assert bool(torch.isnan(y[torch.isnan(xd)]).all()) and bool((y[xd == torch.inf] == torch.inf).all())
+    assert bool(torch.isnan(y[xd == -torch.inf]).all())
