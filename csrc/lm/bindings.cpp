@@ -831,7 +831,7 @@ shai_lm::RuleArgs rule_args(const Tensor& x, const Tensor& gate, const Tensor& s
                             const Tensor& rate, const optional<Tensor>& decay, const optional<Tensor>& beta,
                             const optional<Tensor>& conv, const optional<Tensor>& bias, const optional<Tensor>& gain,
                             const optional<Tensor>& ring, const optional<Tensor>& rope, const optional<Tensor>& q_start,
-                            const optional<Tensor>& q_lens) {
+                            const optional<Tensor>& q_lens, bool made = false) {   // made: decays (per key channel) by the kernel
   const auto dt = x.scalar_type();
   is_f32(x);
   check_rows16(x, dt, "x");
@@ -870,27 +870,27 @@ shai_lm::RuleArgs rule_args(const Tensor& x, const Tensor& gate, const Tensor& s
   a.ldo = out.stride(0);
   a.taps = 1;
   if (conv) {
-    SHAI_CHECK(decay.has_value() && beta.has_value() && bias.has_value() && gain.has_value() && ring.has_value(),
+    SHAI_CHECK(decay.has_value() != made && beta.has_value() && bias.has_value() && gain.has_value() && ring.has_value(),
                "delta rule: decay, beta, bias, gain and ring");
     check(*conv, at::kFloat, "conv");
-    check_rows(*decay, at::kFloat, "decay");
+    if (decay) check_rows(*decay, at::kFloat, "decay");
     check_rows(*beta, at::kFloat, "beta");
     check(*bias, at::kFloat, "bias");
     check(*gain, at::kFloat, "gain");
     check(*ring, dt, "ring");
     a.taps = conv->size(0);
-    a.mode = decay->size(1) == a.H && bias->numel() == a.H ? 1 : 2;
+    const long decays = decay ? decay->size(1) : (long)a.H * a.dk;
+    a.mode = decays == a.H && bias->numel() == a.H ? 1 : 2;
     SHAI_CHECK(conv->dim() == 2 && a.taps >= 1 && a.taps <= 16 && conv->size(1) == channels && ring->dim() == 3 &&
                    ring->size(0) == state.size(0) && ring->size(1) == a.taps && ring->size(2) == channels && rate.numel() == a.H &&
-                   gain->numel() == a.dv && beta->size(0) == a.T && beta->size(1) == a.H && decay->size(0) == a.T &&
-                   (a.mode == 1 || decay->size(1) == (long)a.H * a.dk) && bias->numel() == decay->size(1), "delta rule shapes");
+                   gain->numel() == a.dv && beta->size(0) == a.T && beta->size(1) == a.H && (!decay || decay->size(0) == a.T) &&
+                   (a.mode == 1 || decays == (long)a.H * a.dk) && bias->numel() == decays, "delta rule shapes");
     a.conv = conv->data_ptr<float>();
-    a.decay = decay->data_ptr<float>();
     a.beta = beta->data_ptr<float>();
     a.bias = bias->data_ptr<float>();
     a.gain = gain->data_ptr<float>();
     a.ring = ring->data_ptr();
-    a.ldd = decay->stride(0);
+    if (decay) a.decay = decay->data_ptr<float>(), a.ldd = decay->stride(0);
     a.ldb = beta->stride(0);
   } else {
     SHAI_CHECK(rope.has_value(), "retention: rope");
@@ -1257,6 +1257,36 @@ void attn_beside_rule(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, co
   if (a.T > 0) shai_lm::launch_attn_beside_rule(a, r, is_f32(qkvg), stream());
 }
 
+// The same with gate and decay logits from low [T, a + g] and up [H dv + H dk, a + g] ([0 | gate] above [decay | 0]), a = low_a.  False, and
+// nothing done, for sizes and addresses that take the product of their own.
+bool attn_beside_rule_low(const Tensor& qkvg, const Tensor& kc, const Tensor& vc, const Tensor& o, const Tensor& bt, const Tensor& ctx,
+                          const Tensor& slots, const Tensor& ws, int64_t heads, int64_t splits, int64_t chunk, double scale,
+                          const Tensor& rope, int64_t dim, double eps, const optional<Tensor>& q_gain, const optional<Tensor>& k_gain,
+                          const Tensor& temp, const Tensor& sink, double out_scale, const Tensor& x, const Tensor& low,
+                          const Tensor& state, const Tensor& out, const Tensor& pos, const Tensor& state_slots, int64_t kv_heads,
+                          int64_t rule_dim, int64_t vdim, int64_t gate_kind, double rule_eps, const Tensor& rate, const Tensor& up,
+                          int64_t low_a, const Tensor& beta, const Tensor& conv, const Tensor& bias, const Tensor& gain, const Tensor& ring) {
+  const shai_lm::AttnArgs a = decode_args(qkvg, kc, vc, o, bt, ctx, slots, ws, heads, splits, chunk, scale, true, false, true, rope,
+                                          dim, eps, q_gain, k_gain, temp, sink, out_scale);
+  check_rows(low, x.scalar_type(), "low");
+  check(up, x.scalar_type(), "up");
+  SHAI_CHECK(low.size(0) == x.size(0), "low rows");
+  // (the outputs stand for the gates, which have their shape)
+  shai_lm::RuleArgs r = rule_args(x, out, state, out, pos, state_slots, kv_heads, rule_dim, vdim, gate_kind, rule_eps, rate,
+                                  c10::nullopt, beta, conv, bias, gain, ring, c10::nullopt, c10::nullopt, c10::nullopt, true);
+  SHAI_CHECK(a.T == r.T && qkvg.scalar_type() == x.scalar_type(), "attention and delta rule: rows of one step");
+  SHAI_CHECK(low_a >= 0 && low_a <= low.size(1) && up.dim() == 2 && up.size(1) == low.size(1) && up.size(0) == (long)r.H * (r.dv + r.dk),
+             "up must be [H dv + H dk, columns of low]");
+  r.gate = low.data_ptr();
+  r.ldg = low.stride(0);
+  r.up = up.data_ptr();
+  r.low_a = (int)low_a;
+  r.low_g = (int)(low.size(1) - low_a);
+  if (!shai_lm::attn_rule_low_fits(a, r, is_f32(qkvg))) return false;
+  if (a.T > 0) shai_lm::launch_attn_beside_rule(a, r, false, stream());
+  return true;
+}
+
 void sample(const Tensor& logits, const Tensor& temps, const Tensor& top_k, const Tensor& top_p,
             const Tensor& uniforms, const Tensor& out) {
   SHAI_CHECK(logits.is_cuda() && logits.dim() == 2 && logits.stride(1) == 1, "logits must be a 2D GPU tensor");
@@ -1318,6 +1348,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("gated_attn_prefill(Tensor qkvg, Tensor k_cache, Tensor v_cache, Tensor(a!) o, Tensor block_table, Tensor ctx_lens, Tensor q_lens, Tensor q_start, int max_q, int heads, int chunk, float scale, bool window=False, bool per_element=False, bool own_kv=True, Tensor? temp=None, Tensor? sink=None, float out_scale=1.) -> ()");
   m.def("gated_attn_decode(Tensor qkvg, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, Tensor ctx_lens, Tensor slots, Tensor(d!) ws, int heads, int splits, int chunk, float scale, bool window=False, bool per_element=False, bool own_kv=True, Tensor? rope=None, int dim=0, float eps=0., Tensor? q_gain=None, Tensor? k_gain=None, Tensor? temp=None, Tensor? sink=None, float out_scale=1.) -> ()");
   m.def("attn_beside_rule(Tensor qkvg, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, Tensor ctx_lens, Tensor slots, Tensor(d!) ws, int heads, int splits, int chunk, float scale, Tensor rope, int dim, float eps, Tensor? q_gain, Tensor? k_gain, Tensor temp, Tensor sink, float out_scale, Tensor x, Tensor gate, Tensor(e!) state, Tensor(f!) out, Tensor pos, Tensor state_slots, int kv_heads, int rule_dim, int vdim, int gate_kind, float rule_eps, Tensor rate, Tensor decay, Tensor beta, Tensor conv, Tensor bias, Tensor gain, Tensor(g!) ring) -> ()");
+  m.def("attn_beside_rule_low(Tensor qkvg, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor(c!) o, Tensor block_table, Tensor ctx_lens, Tensor slots, Tensor(d!) ws, int heads, int splits, int chunk, float scale, Tensor rope, int dim, float eps, Tensor? q_gain, Tensor? k_gain, Tensor temp, Tensor sink, float out_scale, Tensor x, Tensor low, Tensor(e!) state, Tensor(f!) out, Tensor pos, Tensor state_slots, int kv_heads, int rule_dim, int vdim, int gate_kind, float rule_eps, Tensor rate, Tensor up, int low_a, Tensor beta, Tensor conv, Tensor bias, Tensor gain, Tensor(g!) ring) -> bool");
   m.def("sample(Tensor logits, Tensor temps, Tensor top_k, Tensor top_p, Tensor uniforms, Tensor(a!) out) -> ()");
   m.def("token_feedback(Tensor(a!) ids, Tensor rowmap, Tensor prev) -> ()");
 }
@@ -1349,6 +1380,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("gated_attn_prefill", &gated_attn_prefill);
   m.impl("gated_attn_decode", &gated_attn_decode);
   m.impl("attn_beside_rule", &attn_beside_rule);
+  m.impl("attn_beside_rule_low", &attn_beside_rule_low);
   m.impl("sample", &sample);
   m.impl("token_feedback", &token_feedback);
 }

@@ -307,10 +307,15 @@ struct RuleArgs {          // delta rule (mode 1: a decay per head, 2: per key c
   int seg, cuts;           // rows of a segment (a multiple of 32), segments of the longest sequence
   int T, B, H, G, dk, dv, dim, vdim, taps, rot, gate_kind, max_q, head0, heads;
   float eps;
+  // a decode step beside attention (beside.hip): gate and decay logits are made from `gate`, rows of low_a + low_g values: the H dv rows of `up`
+  // with the last low_g, the H dk behind them with the first low_a; `decay` is not read
+  const void* up;          // [H dv + H dk, low_a + low_g], null: none
+  int low_a, low_g;
 };
 void launch_rule_rows(const RuleArgs& a, bool f32, hipStream_t s);     // row by row
 void launch_rule_chunks(const RuleArgs& a, hipStream_t s);             // bf16, 32 rows at a time; heads head0 .. of a prefill step
 void launch_attn_beside_rule(const AttnArgs& a, const RuleArgs& r, bool f32, hipStream_t s);   // a decode step of both (beside.hip)
+bool attn_rule_low_fits(const AttnArgs& a, const RuleArgs& r, bool f32);                       // whether it makes the logits from r.up too
 // workspace of one chunk of `heads` heads and `keys` heads of queries and keys (those of every head with a decay per channel)
 long rule_chunk_bytes(int dk, int dv, int heads, int keys, bool channel);
 // workspace of a segment of `heads` heads

@@ -26,7 +26,9 @@ __device__ __forceinline__ float gate_act(float z, int kind) {
 // us: decay per head 37.6 -> 34.8, per channel 39.8 -> 35.1, retention 28.7 (the rate of a large copy: 27); one sequence 7.1 -> 6.6 and
 // 7.6 -> 6.8.  The one row of a step is compiled apart from prompts': 126 registers instead of 168, four workgroups per CU
 // (three beside a step's attention, beside.hip: 64 sequences are then more than are resident at once).
-template <typename T, int MODE, int DK, int DV, int NT, bool STEP>   // STEP: decode of the delta rule
+// LOW: gate and decay logits are products of the row's low_a + low_g values with this head's rows of `up`, 16 rows a matrix instruction, the
+// same values in all its columns (as bf16 for the gate, as the product apart leaves them).
+template <typename T, int MODE, int DK, int DV, int NT, bool STEP, bool LOW = false>   // STEP: decode of the delta rule
 __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
   constexpr bool DELTA = MODE != kRetention;
   constexpr int NC = DV / 4, RG = NT / NC, R = DK / RG, NW = NT / 64, KW = DK / 64;
@@ -34,6 +36,8 @@ __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
   __shared__ __attribute__((aligned(16))) float sq[DK], sk[DK], sg[MODE == kChannel ? DK : 4], sv[DV];
   __shared__ __attribute__((aligned(16))) float sa[DELTA ? NW : 1][DV], so[NW][DV];
   __shared__ float red[NW], skq[NW], rout[NW];
+  static_assert(!LOW || (STEP && MODE == kChannel && DK == 128 && DV == 128 && NT == 256), "two waves for decays and two for gates");
+  __shared__ __attribute__((aligned(16))) float slow[LOW ? DK + DV : 4];   // this head's decay logits, then its gates
   const int tid = threadIdx.x;
   const int c = (tid % NC) * 4, r0 = (tid / NC) * R;
   const int n = !STEP && p.q_lens ? p.q_lens[b] : 1;
@@ -103,20 +107,48 @@ __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
       if (tid < DV) s.v = near(t, v_ch);
       s.beta = p.beta[t * p.ldb + h];
       const int d = MODE == kChannel ? h * DK + min(tid, DK - 1) : h;
-      s.decay = p.decay[t * p.ldd + d];
+      if constexpr (!LOW) s.decay = p.decay[t * p.ldd + d];
       s.bias = p.bias[d];
     }
-    if (tid < DV) s.gate = static_cast<const T*>(p.gate)[t * p.ldg + h * DV + tid];
+    if (!LOW && tid < DV) s.gate = static_cast<const T*>(p.gate)[t * p.ldg + h * DV + tid];
     return s;
   };
   Small in{};
   if constexpr (STEP) in = small(t0);
   const float rate = p.rate[h];
   __builtin_amdgcn_sched_barrier(0);
+  [[maybe_unused]] uint4_ lw[LOW ? 4 : 1][4], lx[4];            // 4 blocks of 16 rows of `up`, 32 of up to 128 columns each
+  if constexpr (LOW) {
+    const int w = tid >> 6, r = tid & 15, q = tid >> 4 & 3;
+    const bool decays = w < 2;
+    const int rank = decays ? p.low_a : p.low_g, col = (decays ? 0 : p.low_a) + 8 * q;
+    const long row = (decays ? (long)p.H * DV + h * DK + w * 64 : (long)h * DV + (w - 2) * 64) + r;
+    const bf16_t* up = static_cast<const bf16_t*>(p.up) + row * (p.low_a + p.low_g) + col;
+    const bf16_t* low = static_cast<const bf16_t*>(p.gate) + t0 * p.ldg + col;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = min(32 * s, rank - 32);
+      lx[s] = *reinterpret_cast<const uint4_*>(low + k);
+      if (32 * s >= rank) lx[s] = uint4_{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lw[i][s] = *reinterpret_cast<const uint4_*>(up + (long)(16 * i) * (p.low_a + p.low_g) + k);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   float4_ S[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) S[i] = old ? load4(st + (long)i * DV) : float4_{0.f, 0.f, 0.f, 0.f};
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (LOW) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float4_ y = float4_{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) y = mac(__builtin_bit_cast(bf16x8, lw[i][s]), __builtin_bit_cast(bf16x8, lx[s]), y);
+      if ((tid & 15) == 0) store4(slow + (tid >> 6) * 64 + 16 * i + 4 * (tid >> 4 & 3), y);
+    }
+    __syncthreads();
+  }
   for (long t = t0; t < t0 + n; ++t) {
     const T* row = x + t * p.ldx;
     if constexpr (!STEP) in = small(t);
@@ -144,7 +176,7 @@ __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
     const int v0 = (DELTA ? 2 * p.G * DK : 2 * p.H * DK) + h * DV;
     if (tid < DV) sv[tid] = DELTA ? conv(t, v_ch, in.v) : load1(row + v0 + tid);
     if constexpr (MODE == kChannel) {
-      if (tid < DK) sg[tid] = expf(-rate * softplus_exact(in.decay + in.bias));
+      if (tid < DK) sg[tid] = expf(-rate * softplus_exact((LOW ? slow[tid] : in.decay) + in.bias));
     }
     __syncthreads();
     float rq = 1.f, rk = 1.f, gh = MODE == kRetention ? rate : 1.f, beta = 1.f;
@@ -231,7 +263,7 @@ __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
       float sum = 0.f;
 #pragma unroll
       for (int w = 0; w < DV / 64; ++w) sum += rout[w];
-      const float z = load1(&in.gate);
+      const float z = LOW ? bf2f(f2bf(slow[DK + tid])) : load1(&in.gate);
       const float r = 1.f / sqrtf(sum / (float)p.vdim + p.eps);
       store1(static_cast<T*>(p.out) + t * p.ldo + h * DV + tid, y * r * (DELTA ? p.gain[tid] : 1.f) * gate_act<false>(z, p.gate_kind));
     }

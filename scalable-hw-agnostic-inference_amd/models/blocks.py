@@ -951,14 +951,12 @@ class DeltaRule(nn.Module):
 
     def step_of(self, x, side, out, state) -> lm.RuleStep:
         H, n = self.c.heads, self.channels
-        gate, decay = x[:, n:], side[:, H:]
-        if self.low:
-            gate, decay = lm.matmul_with_side(gate, self.up, H * self.dk)
-        return lm.RuleStep(x[:, :n], gate, decay, side[:, :H], self.conv, self.rate, self.bias, self.gain, *state, out, self.shape,
-                           self.eps)
+        up, low = (self.up, self.low[0]) if self.low else (None, 0)
+        return lm.RuleStep(x[:, :n], x[:, n:], side[:, H:], side[:, :H], self.conv, self.rate, self.bias, self.gain, *state, out, self.shape,
+                           self.eps, up, low)
 
     def forward(self, x, side, out, batch, state, step):
-        r = self.step_of(x, side, out, state)
+        r = self.step_of(x, side, out, state).made()
         lm.delta_rule(r.x, r.gate, r.decay, r.beta, r.conv, r.rate, r.bias, r.gain, r.state, r.ring, batch, r.out, r.shape, r.eps)
 
     def state_shapes(self):

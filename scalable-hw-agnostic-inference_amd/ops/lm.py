@@ -16,7 +16,7 @@ GPU tensors run the native kernels (raising if the library is missing); CPU tens
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import List, NamedTuple, Optional, Union
 
 import numpy as np
@@ -336,24 +336,39 @@ class RuleStep:
     out: torch.Tensor
     shape: "RuleShape"
     eps: float
+    up: Optional[torch.Tensor] = None    # gate and decay are to be made: ``gate`` [T, a + g] times the rows [0 | gate] above [decay | 0]
+    low: int = 0                         # a
+
+    def made(self) -> "RuleStep":
+        """With gate and decay logits as they are, by a product of their own."""
+        if self.up is None:
+            return self
+        gate, decay = matmul_with_side(self.gate, self.up, self.bias.shape[0])
+        return replace(self, gate=gate, decay=decay, up=None)
 
 
 def attention_beside_rule(qk, k_cache, v_cache, batch, heads: int, size: int, scale: float, turn: HeadTurn, plain: Ungated,
                           rule: RuleStep) -> None:
     """:func:`gated_attention` in a window without gates and :func:`delta_rule` of one decode step: neither reads what the other
-    writes, and on the GPU they are one launch."""
+    writes, and on the GPU they are one launch, for few sequences with the products that ``rule`` leaves to it."""
     if not qk.is_cuda or batch.is_prefill:
+        rule = rule.made()
         gated_attention(qk, k_cache, v_cache, batch, heads, size, scale, window=True, turn=turn, plain=plain)
         delta_rule(rule.x, rule.gate, rule.decay, rule.beta, rule.conv, rule.rate, rule.bias, rule.gain, rule.state, rule.ring, batch,
                    rule.out, rule.shape, rule.eps)
         return
     ns = _decode_splits(batch, size)
     ws = torch.empty(qk.shape[0] * heads * ns * (v_cache.shape[3] + 2) if ns > 1 else 0, dtype=torch.float32, device=qk.device)
-    _K().attn_beside_rule(qk, k_cache, v_cache, plain.out, batch.block_table, batch.ctx_lens, batch.slots, ws, int(heads), ns, int(size),
-                          float(scale), turn.rope, int(turn.dim), float(turn.eps), turn.q_gain, turn.k_gain, plain.temp, plain.sink,
-                          float(plain.out_scale), rule.x, rule.gate, rule.state, rule.out, batch.positions, batch.state_slots,
-                          int(rule.shape.kv_heads), int(rule.shape.dim), int(rule.shape.vdim), int(rule.shape.gate), float(rule.eps),
-                          rule.rate, rule.decay, rule.beta, rule.conv, rule.bias, rule.gain, rule.ring)
+    args = (qk, k_cache, v_cache, plain.out, batch.block_table, batch.ctx_lens, batch.slots, ws, int(heads), ns, int(size), float(scale),
+            turn.rope, int(turn.dim), float(turn.eps), turn.q_gain, turn.k_gain, plain.temp, plain.sink, float(plain.out_scale), rule.x)
+    step = (rule.state, rule.out, batch.positions, batch.state_slots, int(rule.shape.kv_heads), int(rule.shape.dim), int(rule.shape.vdim),
+            int(rule.shape.gate), float(rule.eps), rule.rate)
+    rest = (rule.beta, rule.conv, rule.bias, rule.gain, rule.ring)
+    if rule.up is not None:
+        if _K().attn_beside_rule_low(*args, rule.gate, *step, rule.up, int(rule.low), *rest):
+            return
+        rule = rule.made()
+    _K().attn_beside_rule(*args, rule.gate, *step, rule.decay, *rest)
 
 
 def chunk_attention(qkvg, k_cache, v_cache, batch, heads: int, chunk: int, scale: float):

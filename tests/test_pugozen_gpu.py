@@ -137,6 +137,55 @@ def test_mixers_of_a_step_in_one_launch(cuda, B, H, G, d, rule, channels, splits
     assert torch.equal(one[2], two[2]) and torch.equal(one[4], two[4])
 
 
+@pytest.mark.parametrize("B,H,G,R,K,ranks,splits,one", [
+    (1, 16, 4, 16, 16, (128, 128), 1, True), (1, 4, 1, 1, 1, (64, 128), 2, True), (5, 6, 2, 4, 2, (128, 64), 1, True),
+    (25, 16, 4, 16, 8, (64, 64), 1, True), (26, 16, 4, 16, 16, (128, 128), 1, False), (2, 16, 4, 4, 4, (192, 64), 1, False)])
+def test_logits_made_beside_attention(cuda, B, H, G, R, K, ranks, splits, one):
+    """Gate and decay logits made in the launch of a step's two mixers against a product of their own in front of it: both ranks, alike or not,
+    the most workgroups, and what the launch does not take.  The logits are the same products in another order (2^-20 of them), which may
+    turn the rounding of a gate (bf16), and a decay is e^-(rate softplus), rate up to e^2: outputs to a bf16 rounding, states 2^-14."""
+    from types import SimpleNamespace
+    lm, s, d = C.lm, 128, 128
+    g = torch.Generator(device=cuda).manual_seed(B * H + R)
+    rand = lambda *shape, dtype=torch.bfloat16: torch.randn(*shape, generator=g, device=cuda).to(dtype)
+    i32 = lambda t: torch.tensor(t, dtype=torch.int32, device=cuda)
+    lens = [(1, 64, 65, 200, 7)[i % 5] for i in range(B)]
+    blocks, ch, low = 4, 2 * K * s + R * s, sum(ranks)
+    batch = SimpleNamespace(is_prefill=False, num_splits=splits, ctx_lens=i32(lens), positions=i32([n - 1 for n in lens]),
+                            block_table=i32([[b * blocks + j for j in range(blocks)] for b in range(B)]),
+                            slots=i32([-1 if b == 4 else b * blocks * 64 + n - 1 for b, n in enumerate(lens)]),
+                            state_slots=i32([-1 if b == 4 else B - 1 - b for b in range(B)]))
+    rows = rand(B, (H + G) * d + ch + low)
+    caches = [rand(B * blocks, G, 64, d) for _ in range(2)]
+    f32 = dict(dtype=torch.float32)
+    state, ring = rand(B, R, s, s, **f32), rand(B, 4, ch)
+    turn = lm.HeadTurn(lm.rope_rows(batch.positions, lm.rope_freq(1e4, d // 2).to(cuda)), d, 1e-6, rand(d, **f32), rand(d, **f32))
+    up = torch.zeros(R * 2 * s, low, dtype=torch.bfloat16, device=cuda)
+    up[:R * s, ranks[0]:], up[R * s:, :ranks[0]] = rand(R * s, ranks[1]) / 8, rand(R * s, ranks[0]) / 8
+    conv, rate, bias, gain = rand(4, ch, **f32), rand(R, **f32).clamp(max=2).exp(), rand(R * s, **f32), rand(s, **f32)
+    beta, temp, sink = rand(B, R, **f32), rand(H, **f32), rand(H, **f32)
+
+    def run(made):
+        out = torch.zeros(B, H * d + R * s, dtype=torch.bfloat16, device=cuda)
+        kc, vc, st, rg = caches[0].clone(), caches[1].clone(), state.clone(), ring.clone()
+        r = lm.RuleStep(rows[:, (H + G) * d:(H + G) * d + ch], rows[:, (H + G) * d + ch:], None, beta, conv, rate, bias, gain, st, rg,
+                        out[:, H * d:], lm.RuleShape(K, s, s), 1e-6, up, ranks[0])
+        lm.attention_beside_rule(rows[:, :(H + G) * d], kc, vc, batch, H, lm.WHOLE, d ** -0.5, turn=turn,
+                                 plain=lm.Ungated(temp, sink, out[:, :H * d], 0.7), rule=r.made() if made else r)
+        return out, kc, vc, st, rg
+    calls = []
+    real = lm._K()
+    lm_K = SimpleNamespace(**{n: getattr(real, n) for n in ("attn_beside_rule", "lm_gemm")},
+                           attn_beside_rule_low=lambda *a: calls.append(real.attn_beside_rule_low(*a)) or calls[-1])
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(lm, "_K", lambda: lm_K)
+        got = run(False)
+    assert calls == [one]
+    for i, (a, b) in enumerate(zip(got, run(True))):
+        assert torch.isfinite(b.float()).all()
+        assert (a.float() - b.float()).norm() <= (2 ** -14 if a.dtype == torch.float32 else 2 ** -8) * b.float().norm(), i
+
+
 @pytest.mark.parametrize("M,K,width,N,act,side,parts,source,out", [
     (1, 64, 40, 16, 0, 0, 0, "table", torch.bfloat16), (1, 64, 64, 20, 8, 4, 1, "rows", torch.bfloat16),
     (2, 192, 180, 9000, 0, 0, 4, "rows", torch.float32), (1, 2048, 2048, 17424, 8448, 16, 4, "rows", torch.bfloat16),
