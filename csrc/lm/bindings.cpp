@@ -557,16 +557,24 @@ void conv_commit(const Tensor& state, const Tensor& tail, const Tensor& q_lens, 
   if (tail.numel() > 0) shai_lm::launch_conv_commit(a, stream());
 }
 
-void rope_rows(const Tensor& pos, const Tensor& freq, const Tensor& out) {
+void rope_rows_all(const Tensor& pos, at::TensorList freqs, at::TensorList outs) {
   check_i32(pos, "pos");
-  check_f32(freq, "freq");
-  check_f32(out, "out");
-  SHAI_CHECK(freq.dim() == 2 && freq.size(1) == 2 && out.dim() == 2 && out.size(0) <= pos.numel() &&
-                 out.size(1) == 2 * freq.size(0), "rope_rows: freq [n, 2], out [T, 2 n]");
-  shai_lm::RopeRowsArgs a{pos.data_ptr<int>(), freq.data_ptr<float>(), (int)out.size(0), (int)freq.size(0),
-                          out.data_ptr<float>()};
-  if (out.numel() > 0) shai_lm::launch_rope_rows(a, stream());
+  SHAI_CHECK(freqs.size() == outs.size() && freqs.size() >= 1 && freqs.size() <= shai_lm::kRopeTables, "rope_rows: one to four tables");
+  shai_lm::RopeRowsArgs a{};
+  a.pos = pos.data_ptr<int>();
+  a.T = (int)outs[0].size(0);
+  for (size_t i = 0; i < freqs.size(); ++i) {
+    const Tensor &freq = freqs[i], &out = outs[i];
+    check_f32(freq, "freq");
+    check_f32(out, "out");
+    SHAI_CHECK(freq.dim() == 2 && freq.size(1) == 2 && out.dim() == 2 && out.size(0) == a.T && a.T <= pos.numel() &&
+                   out.size(1) == 2 * freq.size(0), "rope_rows: freq [n, 2], out [T, 2 n]");
+    if (out.numel() > 0) a.table[a.tables++] = {freq.data_ptr<float>(), (int)freq.size(0), out.data_ptr<float>()};
+  }
+  if (a.tables > 0) shai_lm::launch_rope_rows(a, stream());
 }
+
+void rope_rows(const Tensor& pos, const Tensor& freq, const Tensor& out) { rope_rows_all(pos, {freq}, {out}); }
 
 void latent_prep(const Tensor& d, const Tensor& wq, const Tensor& wkv, const Tensor& rope, const Tensor& slots,
                  const Tensor& cache, const Tensor& cq, double eps, int64_t q_rank, int64_t kv_rank) {
@@ -1326,6 +1334,7 @@ TORCH_LIBRARY_FRAGMENT(shai, m) {
   m.def("normed_gemm(Tensor? x, Tensor? ids, Tensor? table, float scale, Tensor? delta, Tensor w, float eps, int width, Tensor(a!)? x_out, Tensor W, Tensor(b!) C, Tensor(c!)? side=None, int act=0) -> ()");
   m.def("conv_commit(Tensor(a!) state, Tensor tail, Tensor q_lens, Tensor slots) -> ()");
   m.def("rope_rows(Tensor pos, Tensor freq, Tensor(a!) out) -> ()");
+  m.def("rope_rows_all(Tensor pos, Tensor[] freqs, Tensor(a!)[] outs) -> ()");
   m.def("latent_prep(Tensor d, Tensor wq, Tensor wkv, Tensor rope, Tensor slots, Tensor(a!) cache, Tensor(b!) cq, float eps, int q_rank, int kv_rank) -> ()");
   m.def("latent_gather(Tensor cache, Tensor block_table, Tensor seqs, Tensor ctx, Tensor start, int max_ctx, Tensor(a!) out) -> ()");
   m.def("latent_attn_prefill(Tensor q, Tensor kv, Tensor lat, Tensor(a!) o, Tensor ctx, Tensor q_lens, Tensor q_start, Tensor kv_start, Tensor sink, int max_q, int heads, int np, int rot, int rank, float scale) -> ()");
@@ -1363,6 +1372,7 @@ TORCH_LIBRARY_IMPL(shai, CUDA, m) {
   m.impl("normed_gemm", &normed_gemm);
   m.impl("conv_commit", &conv_commit);
   m.impl("rope_rows", &rope_rows);
+  m.impl("rope_rows_all", &rope_rows_all);
   m.impl("latent_prep", &latent_prep);
   m.impl("latent_gather", &latent_gather);
   m.impl("latent_attn_prefill", &latent_attn_prefill);

@@ -88,11 +88,15 @@ struct ConvCommitArgs {    // the tails of a prefill step into the state of ever
 };
 void launch_conv_commit(const ConvCommitArgs& a, hipStream_t s);
 
-struct RopeRowsArgs {      // cos / sin of pos * freq, every row of a step
+constexpr int kRopeTables = 4;
+struct RopeRowsArgs {      // cos / sin of pos * freq, every row of a step, for several sets of frequencies
   const int* pos;
-  const float* freq;       // [n][2]: frequency as a float and its remainder
-  int T, n;
-  float* out;              // [T, n, 2]
+  int T, tables;
+  struct {
+    const float* freq;     // [n][2]: frequency as a float and its remainder
+    int n;
+    float* out;            // [T, n, 2]
+  } table[kRopeTables];
 };
 void launch_rope_rows(const RopeRowsArgs& a, hipStream_t s);
 

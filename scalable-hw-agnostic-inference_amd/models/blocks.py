@@ -405,16 +405,18 @@ class LatentAttention(nn.Module):
 
 
 class StepShared:
-    """What the layers of one step share: rotation angles per (base, dims) and the attention plan per kind."""
+    """What the layers of one step share: rotation angles per (base, dims) and the attention plan per kind.  ``turning``: mixers that will
+    ask for angles, which are made together."""
 
-    def __init__(self, batch):
-        self.batch, self._ropes, self._plans = batch, {}, {}
+    def __init__(self, batch, turning=()):
+        self.batch, self.turning, self._ropes, self._plans = batch, turning, {}, {}
 
     def rope(self, mix):
         """Angles for a mixer with ``rope_key`` (what its frequencies follow from) and ``freq``."""
         key = mix.rope_key
         if key not in self._ropes:
-            self._ropes[key] = lm.rope_rows(self.batch.positions, mix.freq)
+            todo = {m.rope_key: m.freq for m in (mix, *self.turning) if m.rope_key not in self._ropes}
+            self._ropes.update(zip(todo, lm.rope_rows_all(self.batch.positions, list(todo.values()))))
         return self._ropes[key]
 
     def plan(self, expands: bool):

@@ -165,6 +165,7 @@ class PugozenForCausalLM(nn.Module):
         self.layers = nn.ModuleDict({str(i): PugozenLayer(cfg, cfg.layers[i], dtype) for i in sorted(set(self.order))})
         self.final_norm = GainNorm(cfg.width)
         self.head = SoftcapHead(cfg.vocab_size, cfg.width, None, dtype)
+        self._turning = [m for layer in self.layers.values() for m in layer.joint.mixers.values() if hasattr(m, "rope_key")]
 
     def runs(self) -> List[PugozenLayer]:
         """The weights of every layer run."""
@@ -201,7 +202,7 @@ class PugozenForCausalLM(nn.Module):
     def forward(self, batch: Batch, kv_caches, trail: Optional[list] = None) -> torch.Tensor:
         """fp32 logits [rows, vocab]: every row of a decode step, the rows ``batch.last_index`` of a prefill step.
         ``trail`` (a list) receives the residual stream after every layer."""
-        cfg, step = self.cfg, StepShared(batch)
+        cfg, step = self.cfg, StepShared(batch, self._turning)
         norm = lambda source, delta, w, **kw: lm.residual_norm(source, delta, lm.PLAIN, 1.0, None, w, cfg.eps, cfg.width,
                                                                self.dtype, batch=batch, **kw)
         x, delta = lm.Embedding(batch.input_ids, self.embed, cfg.embed_scale), None

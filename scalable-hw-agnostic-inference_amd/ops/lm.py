@@ -524,6 +524,19 @@ def rope_rows(positions, freq):
     return out
 
 
+ROPE_TABLES = 4
+
+
+def rope_rows_all(positions, freqs):
+    """:func:`rope_rows` of each of ``freqs``, on the GPU up to four in a launch."""
+    if not positions.is_cuda:
+        return [ref.rope_rows(positions, f) for f in freqs]
+    outs = [torch.empty(positions.shape[0], 2 * f.shape[0], dtype=torch.float32, device=positions.device) for f in freqs]
+    for i in range(0, len(freqs), ROPE_TABLES):
+        _K().rope_rows_all(positions, freqs[i:i + ROPE_TABLES], outs[i:i + ROPE_TABLES])
+    return outs
+
+
 # ---------------------------------------------------------------------------------------------- latent attention
 def latent_head_pad(dk: int, dv: int) -> Optional[tuple]:
     """Head sizes of the prefill kernel that hold (dk, dv), or None."""

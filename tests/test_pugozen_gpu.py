@@ -227,3 +227,14 @@ def test_norms_that_stay_apart(cuda):
     assert not fits(torch.zeros(3, 128, device=cuda), None, w, W) and not fits(torch.zeros(1, 4160, device=cuda), None, w, W)
     assert not fits(x, d, w, W.float()) and not fits(x, d[0].bfloat16(), w, W) and not fits(x, torch.zeros(9, 2, 128, device=cuda), w, W)
     assert not fits(x, d, lm.Affine(w, w), W)
+
+
+@pytest.mark.parametrize("T", [1, 3, 300])
+@pytest.mark.parametrize("dims", [(2,), (64, 128), (128, 2, 62, 64, 32)])
+def test_angles_of_several_tables(cuda, T, dims):
+    """Tables of unlike widths in one launch, and more than it takes: the bits of one by one."""
+    lm = C.lm
+    pos = (torch.arange(T, dtype=torch.int32, device=cuda) * 7919) % 100003
+    freqs = [lm.rope_freq(1e4 * (i + 1), d).to(cuda) for i, d in enumerate(dims)]
+    for got, f in zip(lm.rope_rows_all(pos, freqs), freqs):
+        assert torch.equal(got, lm.rope_rows(pos, f))
