@@ -18,7 +18,7 @@ constexpr int workgroups(int D, int RH) { return D == 128 && RH == 8 ? 2 : 3; }
 
 // V: V loads of the attention in flight. Eight where three workgroups share a CU: sixteen spill 7 registers there (64 sequences of 132 keys, 4 heads
 // of 128 a group, 39.4 -> 38.3 us).
-template <int D, int RH, int MODE, int SD, int V, bool LOW = false>
+template <int D, int RH, int MODE, int SD, int V, int LOW = 0>
 __global__ void __launch_bounds__(256, V == 16 ? 2 : workgroups(D, RH)) attn_rule_kernel(const AttnArgs a, const RuleArgs r, int per_group, int heads, int n_attn) {
   const int i = blockIdx.x;
   if (i < n_attn) {
@@ -40,7 +40,7 @@ static void attn_rule(const AttnArgs& a, const RuleArgs& r, hipStream_t s) {
   auto go = [&](auto kernel) { kernel<<<grid, 256, 0, s>>>(a, r, a.H / a.G, a.G, n_attn); };
   if constexpr (D == 128 && RH == 4) {
     if constexpr (MODE == kChannel && SD == 128) {
-      if (r.up) return go(attn_rule_kernel<D, RH, MODE, SD, 16, true>);
+      if (r.up) return grid <= kFew ? go(attn_rule_kernel<D, RH, MODE, SD, 16, 1>) : go(attn_rule_kernel<D, RH, MODE, SD, 8, 2>);
     }
     if (grid <= kFew) return go(attn_rule_kernel<D, RH, MODE, SD, 16>);
   }
@@ -61,13 +61,15 @@ static bool fits(const AttnArgs& a, const RuleArgs& r) {
 }
 
 // The logits of gates and decays in this launch: an attention of few sequences takes longer than the recurrence beside it, so that their product (64 KB
-// of weights a head from the XCD's cache) costs little there and a launch of its own less.  us apart and in one, 16 heads, ranks of 128: one sequence
-// of 132 keys 15.2 and 12.1, 8 16.5 and 13.3, 25 26.2 and 22.2; of one key 13.4 and 10.0, 25 20.2 and 16.6.  Past kFew workgroups three share a CU,
-// which leaves no registers for the weights.
+// of weights a head from the XCD's cache) costs little there and a launch of its own less; where three workgroups share a CU they hide it from each
+// other, with the state asked for behind the weights, in the registers that these had.  us apart and in one, 16 heads, ranks of 128: one sequence of 132
+// keys 15.3 and 11.5, 8 16.4 and 13.1, 25 26.3 and 22.0; 32 30.5 and 28.3, 64 46.2 and 42.8, 96 (1920 workgroups) 60.2 and 59.8; of 900 keys 64 69.1 and
+// 67.4; of one key 64 30.6 and 30.9, 96 41.3 and 43.9: up to two rounds of three to a CU.
+constexpr int kLow = 2 * 3 * 256;
 bool attn_rule_low_fits(const AttnArgs& a, const RuleArgs& r, bool f32) {
   const auto rank = [](int n) { return n == 64 || n == 128; };
   return !f32 && fits(a, r) && a.dk == 128 && a.H / a.G <= 4 && r.mode == kChannel && r.dk == 128 && rank(r.low_a) && rank(r.low_g) &&
-         r.ldg % 8 == 0 && (((uintptr_t)r.gate | (uintptr_t)r.up) & 15) == 0 && (long)a.G * a.B * a.splits + (long)r.H * r.B <= kFew;
+         r.ldg % 8 == 0 && (((uintptr_t)r.gate | (uintptr_t)r.up) & 15) == 0 && (long)a.G * a.B * a.splits + (long)r.H * r.B <= kLow;
 }
 
 void launch_attn_beside_rule(const AttnArgs& a, const RuleArgs& r, bool f32, hipStream_t s) {

@@ -27,8 +27,9 @@ __device__ __forceinline__ float gate_act(float z, int kind) {
 // 7.6 -> 6.8.  The one row of a step is compiled apart from prompts': 126 registers instead of 168, four workgroups per CU
 // (three beside a step's attention, beside.hip: 64 sequences are then more than are resident at once).
 // LOW: gate and decay logits are products of the row's low_a + low_g values with this head's rows of `up`, 16 rows a matrix instruction, the
-// same values in all its columns (as bf16 for the gate, as the product apart leaves them).
-template <typename T, int MODE, int DK, int DV, int NT, bool STEP, bool LOW = false>   // STEP: decode of the delta rule
+// same values in all its columns (as bf16 for the gate, as the product apart leaves them).  1: the state is on its way meanwhile, 2: asked for
+// behind them, in the registers they had.
+template <typename T, int MODE, int DK, int DV, int NT, bool STEP, int LOW = 0>   // STEP: decode of the delta rule
 __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
   constexpr bool DELTA = MODE != kRetention;
   constexpr int NC = DV / 4, RG = NT / NC, R = DK / RG, NW = NT / 64, KW = DK / 64;
@@ -136,9 +137,12 @@ __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
     __builtin_amdgcn_sched_barrier(0);
   }
   float4_ S[R];
+  auto ask = [&] {
 #pragma unroll
-  for (int i = 0; i < R; ++i) S[i] = old ? load4(st + (long)i * DV) : float4_{0.f, 0.f, 0.f, 0.f};
-  __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < R; ++i) S[i] = old ? load4(st + (long)i * DV) : float4_{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (LOW != 2) ask();
   if constexpr (LOW) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -146,6 +150,10 @@ __device__ __forceinline__ void rule_rows(const RuleArgs& p, int h, int b) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) y = mac(__builtin_bit_cast(bf16x8, lw[i][s]), __builtin_bit_cast(bf16x8, lx[s]), y);
       if ((tid & 15) == 0) store4(slow + (tid >> 6) * 64 + 16 * i + 4 * (tid >> 4 & 3), y);
+    }
+    if constexpr (LOW == 2) {
+      __builtin_amdgcn_sched_barrier(0);
+      ask();
     }
     __syncthreads();
   }

@@ -139,10 +139,11 @@ def test_mixers_of_a_step_in_one_launch(cuda, B, H, G, d, rule, channels, splits
 
 @pytest.mark.parametrize("B,H,G,R,K,ranks,splits,one", [
     (1, 16, 4, 16, 16, (128, 128), 1, True), (1, 4, 1, 1, 1, (64, 128), 2, True), (5, 6, 2, 4, 2, (128, 64), 1, True),
-    (25, 16, 4, 16, 8, (64, 64), 1, True), (26, 16, 4, 16, 16, (128, 128), 1, False), (2, 16, 4, 4, 4, (192, 64), 1, False)])
+    (25, 16, 4, 16, 8, (64, 64), 1, True), (26, 16, 4, 16, 16, (128, 64), 1, True), (76, 16, 4, 16, 16, (64, 128), 1, True),
+    (77, 16, 4, 16, 16, (128, 128), 1, False), (2, 16, 4, 4, 4, (192, 64), 1, False)])
 def test_logits_made_beside_attention(cuda, B, H, G, R, K, ranks, splits, one):
     """Gate and decay logits made in the launch of a step's two mixers against a product of their own in front of it: both ranks, alike or not,
-    the most workgroups, and what the launch does not take.  The logits are the same products in another order (2^-20 of them), which may
+    the most workgroups of either form, and what the launch does not take.  The logits are the same products in another order (2^-20 of them), which may
     turn the rounding of a gate (bf16), and a decay is e^-(rate softplus), rate up to e^2: outputs to a bf16 rounding, states 2^-14."""
     from types import SimpleNamespace
     lm, s, d = C.lm, 128, 128
