@@ -661,6 +661,52 @@ def test_decode_attn_wave_per_block_matches_split_kernel(cuda, fused):
         ops.set_decode_wb(prev)
 
 
+@pytest.mark.parametrize("ctx", [[1, 2, 3, 4, 5], [16, 17, 33, 49, 63], [64, 65, 66, 128, 129], [192, 193, 255, 256, 257], [320, 321, 449, 513, 2]])
+def test_decode_attn_wave_per_block_edges(cuda, ctx):
+    """Keys at the edges of tiles, blocks and waves against 64 bits, cache rows behind the context NaN.  P and the output are rounded to bf16 (2^-9
+    each, P in the numerator and the denominator), scores and sums are fp32: 2^-8 + 2^-9 + 2^-11 of the largest value.  From partial sums that add
+    up to the rows without rounding: the rows' result and caches, bit for bit."""
+    torch.manual_seed(sum(ctx))
+    D, Hq, Hkv, B = 128, 32, 8, len(ctx)
+    kc, vc, bt = _paged_setup(B, Hkv, D, ctx, nblocks=sum((c + 63) // 64 for c in ctx) + 8)
+    for b, c in enumerate(ctx):
+        if c % 64:
+            kc[bt[b, (c - 1) // 64], :, c % 64:] = float("nan")
+            vc[bt[b, (c - 1) // 64], :, c % 64:] = float("nan")
+    lens = torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    prev = ops.set_decode_wb(1)
+    try:
+        q = rnd(B, Hq, D)
+        o = ops.decode_attention(q, kc, vc, bt, lens, num_splits=1).cpu().double()
+        top = vc.nan_to_num().abs().max().item()
+        for b, c in enumerate(ctx):
+            k, v = (t[bt[b, :(c + 63) // 64].long()].cpu().double().transpose(1, 2).reshape(-1, Hkv, D)[:c].repeat_interleave(Hq // Hkv, 1)
+                    for t in (kc, vc))
+            w = ((q[b].cpu().double() * k).sum(-1) / math.sqrt(D)).softmax(0)
+            assert (o[b] - (w[..., None] * v).sum(0)).abs().max() <= (2 ** -8 + 2 ** -9 + 2 ** -11) * top
+        n = (Hq + 2 * Hkv) * D
+        ang = torch.rand(max(ctx) + 1, D // 2, device="cuda") * 3
+        cos, sin = ang.cos().contiguous(), ang.sin().contiguous()
+        pos = lens - 1
+        slots = torch.stack([bt[b, (c - 1) // 64] * 64 + (c - 1) % 64 for b, c in enumerate(ctx)]).int()
+        for kg in (2, 3, 4, 5, 9):
+            slabs = torch.randint(-20, 21, (kg, B, n), device="cuda").float() / 32  # sums of up to 180 / 32: exact, in bf16 too
+            qkv = slabs.sum(0).bfloat16()
+            assert torch.equal(qkv.float(), slabs.sum(0))
+            ssq = torch.full((kg, B), 64.0, device="cuda")  # sums to K: a scale of 1
+            part = torch.cat([slabs.flatten(), ssq.flatten()])
+            k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+            rows = ops.decode_attention_rope(qkv, k1, v1, bt, lens, pos, cos, sin, slots, Hq, Hkv, num_splits=1)
+            got = torch.empty_like(rows)
+            ws = torch.empty(B * Hq * (D + 2), device="cuda")
+            ops._K().decode_attn_rope(part, k2, v2, got, bt.int(), lens, pos.int(), cos, sin, slots, ws, Hq, Hkv, 1, 1 / math.sqrt(D), part,
+                                      kg, 64 * kg, 0.0)
+            assert torch.equal(got, rows)
+            assert torch.equal(k1.nan_to_num(9), k2.nan_to_num(9)) and torch.equal(v1.nan_to_num(9), v2.nan_to_num(9))
+    finally:
+        ops.set_decode_wb(prev)
+
+
 def test_upsample2d_layer_takes_phase_conv_and_tracks_weight_updates(cuda):
     """Upsample2D (UNet / VAE) on a shape with >= 256 output tiles runs the phase conv with cached phase weights,
     matches the fp32 upsample + 3x3 conv, and rebuilds the phase weights after an in-place weight update."""
