@@ -958,7 +958,7 @@ __global__ void decode_combine_kernel(const DecodeAttnArgs p) {
 }
 
 // ----------------------------------------------------------------------------
-// Short-context decode attention, "wave per block" (D = 128, GQA group G = 4, one split).
+// Decode attention, "wave per block" (D = 128, GQA group G = 4).
 // The split kernel above walks a (sequence, KV head)'s 64-token blocks one after another with ONE block in flight
 // (two-slot ring), so at decode-batch contexts of a few hundred tokens its launch is mostly prologue and per-block
 // HBM latency (B 64 x ctx 192: 18 us for 50 MB, 2.8 TB/s).  Here the G waves of the
@@ -982,12 +982,16 @@ __global__ void decode_combine_kernel(const DecodeAttnArgs p) {
 // cache's bytes.  Dot products on the VALU, with P through LDS and six exchanges a head for its max and sum, took 8 of
 // the 49 us at 256 x 132; the loads of the prologue behind K and V, whose rows they then had to wait for, another 6.
 // us at sequences x keys, 32 / 8 heads, caches out of memory: 1 x 132 8.0 -> 6.3, 64 x 150 17.2 -> 12.8 (3.0 TB/s), 64 x
-// 250 21.4 -> 16.8, 256 x 132 49.1 -> 34.3 (4.0 TB/s).  SHAI_DECODE_WB=0 / set_decode_wb(0) routes these launches back to the split kernel (A/B).
+// 250 21.4 -> 16.8, 256 x 132 49.1 -> 34.3 (4.0 TB/s).
+// SPLIT: a workgroup has one of a row's da_splits parts of at least four blocks, one for each wave, and leaves (m, l, o)
+// for decode_combine_kernel, as the split kernel does; against that one, both with their combine, us: 1 x 1000 in 16
+// (4 after da_splits) 19.0 -> 11.7, 1 x 6000 in 64 33.7 -> 27.3, 8 x 2000 in 8 29.0 -> 24.5, 32 x 1000 in 2 37.2 -> 31.4.
+// SHAI_DECODE_WB=0 / set_decode_wb(0) routes these launches back to the split kernel (A/B).
 constexpr int kWbG = 4;
 constexpr size_t kWbLds = (size_t)kWbG * 64 * 128 * 2 + (size_t)kWbG * 128 * 2;
 
 enum { kHeadsRoped, kHeadsRows, kHeadsParts };  // q as it is; q, k and v of this step as rows or as partial sums
-template <int SRC>
+template <int SRC, bool SPLIT>
 __global__ void __launch_bounds__(kWbG * 64, 2) decode_attn_wb_kernel(const DecodeAttnArgs p) {
   constexpr int G = kWbG, D = 128, CPR = D / 8;
   extern __shared__ __attribute__((aligned(16))) char dsm[];
@@ -997,20 +1001,29 @@ __global__ void __launch_bounds__(kWbG * 64, 2) decode_attn_wb_kernel(const Deco
   float* sO = sM + G * G * 2;                    // [G waves][G heads][D]
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int b = blockIdx.x / p.Hkv, hk = blockIdx.x - b * p.Hkv;
+  const int bh = SPLIT ? blockIdx.x / p.num_splits : blockIdx.x, split = SPLIT ? blockIdx.x - bh * p.num_splits : 0;
+  const int b = bh / p.Hkv, hk = bh - b * p.Hkv;
   const int hq = hk * G + w;  // this wave's head in the prologue and in the merge
   constexpr bool fused = SRC != kHeadsRoped, part = SRC == kHeadsParts;
   const int ctx = p.ctx_lens[b] - (fused ? 1 : 0);  // tokens read from the cache
-  const int nblk = (ctx + 63) / 64;
-  const int nmine = nblk > w ? (nblk - w + G - 1) / G : 0;  // blocks w, w + G, ... of this wave
+  const int nall = (ctx + 63) / 64;
+  int nsp = 1, blk0 = 0, nblk = nall;
+  if constexpr (SPLIT) {
+    nsp = da_splits(nall, p.num_splits);
+    if (split >= nsp) return;
+    const int per = (nall + nsp - 1) / nsp;
+    blk0 = split * per;
+    nblk = min(per, nall - blk0);  // none, or fewer, where the splits before it took all
+  }
+  const int nmine = nblk > w ? (nblk - w + G - 1) / G : 0;  // blocks blk0 + w, + G, ... of this wave
   // physical ids of this wave's blocks, 64 per lane-distributed chunk (independent of ctx: issued beside its load)
   const int* bt = p.block_table + (long)b * p.max_blocks;
   int chunk0 = 0;
-  int my_phys = (w + G * lane < p.max_blocks) ? bt[w + G * lane] : 0;
+  int my_phys = (blk0 + w + G * lane < p.max_blocks) ? bt[blk0 + w + G * lane] : 0;
   auto phys_of = [&](int it) {
     if (it - chunk0 >= 64) {
       chunk0 += 64;
-      const int e = w + G * (chunk0 + lane);
+      const int e = blk0 + w + G * (chunk0 + lane);
       my_phys = e < p.max_blocks ? bt[e] : 0;
     }
     return __builtin_amdgcn_readlane(my_phys, it - chunk0);
@@ -1055,7 +1068,7 @@ __global__ void __launch_bounds__(kWbG * 64, 2) decode_attn_wb_kernel(const Deco
   // ---- prologue: this wave's q head, roped, into sQb; the new token's k / v in registers.  What it reads is asked for
   // before K and V: loads of a wave return in order.
   const int rpos = fused ? p.positions[b] : 0;
-  const bool new_tok = fused && p.slots[b] >= 0;
+  const bool new_tok = fused && split == nsp - 1 && p.slots[b] >= 0;
   const long pslab = (long)p.B * p.qkv_n;
   const int kcol = (p.Hq + hk) * D, vcol = (p.Hq + p.Hkv + hk) * D;
   const int col[6] = {hq * D + lane, hq * D + lane + D / 2, kcol + lane, kcol + lane + D / 2, vcol + 2 * lane,
@@ -1094,8 +1107,9 @@ __global__ void __launch_bounds__(kWbG * 64, 2) decode_attn_wb_kernel(const Deco
   }
   {  // also without a block (no rows, nothing is read): the number of loads in flight is known below, and waits count them
     const int ph = __builtin_amdgcn_readfirstlane(nmine > 0 ? phys_of(0) : 0);
-    issue_k(w, ph);
-    issue_v(w, ph);
+    const int bi = nmine > 0 ? blk0 + w : nall;
+    issue_k(bi, ph);
+    issue_v(bi, ph);
   }
   // nothing is done with the prologue's values before K and V are asked for
   asm volatile("" : "+v"(vn_pair), "+v"(rc), "+v"(rs));
@@ -1157,7 +1171,7 @@ __global__ void __launch_bounds__(kWbG * 64, 2) decode_attn_wb_kernel(const Deco
   for (int s = 0; s < 4; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(sQb + (lane & 3) * D + 32 * s + 8 * lrow);
   const int krow = (lpos >> 2) + 4 * (lpos & 3);
   for (int it = 0; it < nmine; ++it) {
-    const int bi = w + G * it;
+    const int bi = blk0 + w + G * it;
     // this block's K slot has landed (its V loads, issued behind it, may still be in flight)
     asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     float4_ sc[4];  // sc[t][r]: key lrow + 4 (4 t + r)
@@ -1280,6 +1294,16 @@ __global__ void __launch_bounds__(kWbG * 64, 2) decode_attn_wb_kernel(const Deco
       *reinterpret_cast<uint32_t*>(vc + dst + 2 * lane) = vn_pair;
     }
   }
+  if (SPLIT && nsp > 1) {  // joined by the launch behind: ws[b][hq][split] = {m, l, o[D]}
+    float* dst = p.ws + (((long)b * p.Hq + hq) * p.num_splits + split) * (D + 2);
+    if (lane == 0) {
+      dst[0] = M;
+      dst[1] = L;
+    }
+    dst[2 + 2 * lane] = o0;
+    dst[3 + 2 * lane] = o1;
+    return;
+  }
   const float inv = L > 0.f ? 1.f / L : 0.f;
   *reinterpret_cast<uint32_t*>(p.o + (long)b * p.o_bs + (long)hq * D + 2 * lane) = pack2(o0 * inv, o1 * inv);
 }
@@ -1304,13 +1328,6 @@ size_t decode_attn_workspace(int B, int Hq, int D, int num_splits) {
 
 void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t s) {
   const int G = a.Hq / a.Hkv;
-  if (a.D == 128 && G == kWbG && a.num_splits == 1 && decode_wb_mode()) {  // wave-per-block short-context kernel
-    const dim3 grid((unsigned)(a.B * a.Hkv));
-    if (a.qkv_ws) decode_attn_wb_kernel<kHeadsParts><<<grid, kWbG * 64, kWbLds, s>>>(a);
-    else if (a.knew) decode_attn_wb_kernel<kHeadsRows><<<grid, kWbG * 64, kWbLds, s>>>(a);
-    else decode_attn_wb_kernel<kHeadsRoped><<<grid, kWbG * 64, kWbLds, s>>>(a);
-    return;
-  }
   static const int width = [] {  // two workgroups per CU (70 KB of LDS each)
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -1325,6 +1342,25 @@ void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t s) {
     return e ? (e[0] == '1' ? 1 : 0) : -1;
   }();
   const long items = (long)a.B * a.Hkv * a.num_splits;
+  // Wave-per-block kernel: unsplit, or up to two rounds of workgroups, which is what a split count made to fill the chip
+  // gives (faster at every one measured, 250 to 6,000 keys and 1 to 32 rows).  Beyond stands a count raised for one long
+  // row, and most workgroups have none of a short row's parts: the persistent walk of the split kernel is for those.
+  if (a.D == 128 && G == kWbG && decode_wb_mode() && (a.num_splits == 1 || items <= 2 * width)) {
+    auto go = [&](auto split) {
+      constexpr bool SPLIT = decltype(split)::value;
+      const dim3 grid((unsigned)items);
+      if (a.qkv_ws) decode_attn_wb_kernel<kHeadsParts, SPLIT><<<grid, kWbG * 64, kWbLds, s>>>(a);
+      else if (a.knew) decode_attn_wb_kernel<kHeadsRows, SPLIT><<<grid, kWbG * 64, kWbLds, s>>>(a);
+      else decode_attn_wb_kernel<kHeadsRoped, SPLIT><<<grid, kWbG * 64, kWbLds, s>>>(a);
+    };
+    if (a.num_splits == 1) {
+      go(std::false_type());
+    } else {
+      go(std::true_type());
+      decode_combine_kernel<<<dim3(a.B, a.Hq), 128, 0, s>>>(a);
+    }
+    return;
+  }
   const bool persist = force >= 0 ? force == 1 : a.num_splits > 8;
   dim3 grid((unsigned)(persist ? std::min<long>(items, width) : items));
   const size_t lds = (size_t)4 * 64 * a.D * sizeof(bf16_t) + (size_t)8 * a.D * 4 + 8 * 64 * 4;

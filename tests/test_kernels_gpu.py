@@ -707,6 +707,39 @@ def test_decode_attn_wave_per_block_edges(cuda, ctx):
         ops.set_decode_wb(prev)
 
 
+@pytest.mark.parametrize("splits", [2, 3, 7, 64])
+def test_decode_attn_wave_per_block_splits(cuda, splits):
+    """Splits of whole blocks, uneven and empty ones (33 blocks in 7), rows with fewer blocks than would be split and a padding row, against the unsplit
+    form: o is rounded once on either side (2^-8 of the largest value), the caches are the same bits."""
+    torch.manual_seed(splits)
+    D, Hq, Hkv = 128, 32, 8
+    ctx = [1, 256, 257, 258, 512, 700, 2112, 2113, 300]
+    B = len(ctx)
+    kc, vc, bt = _paged_setup(B, Hkv, D, ctx, nblocks=sum((c + 63) // 64 for c in ctx) + 8)
+    lens = torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    slots = torch.stack([bt[b, (c - 1) // 64] * 64 + (c - 1) % 64 for b, c in enumerate(ctx)]).int()
+    slots[-1] = -1
+    ang = torch.rand(max(ctx) + 1, D // 2, device="cuda") * 3
+    qkv, x = rnd(B, (Hq + 2 * Hkv) * D), rnd(B, 512)
+    w = (rnd((Hq + 2 * Hkv) * D, 512).float() * 512 ** -0.5).bfloat16()
+    args = (bt, lens, lens - 1, ang.cos().contiguous(), ang.sin().contiguous(), slots, Hq, Hkv)
+    prev = ops.set_decode_wb(1)
+    try:
+        def outs(n):
+            k, v = (kc.clone(), kc.clone()), (vc.clone(), vc.clone())
+            o = (ops.decode_attention(rnd_q, kc, vc, bt, lens, num_splits=n).reshape(B, -1),
+                 ops.decode_attention_rope(qkv, k[0], v[0], *args, num_splits=n),
+                 ops.decode_attention_rope_qkv(x, w, 1e-5, k[1], v[1], *args, num_splits=n))
+            return o, k + v
+        rnd_q = rnd(B, Hq, D)
+        (got, gc), (want, wc) = outs(splits), outs(1)
+        for a, b in zip(got, want):
+            assert (a.float() - b.float()).abs().max() <= 2 ** -8 * vc.float().abs().max()
+        assert all(torch.equal(a, b) for a, b in zip(gc, wc))
+    finally:
+        ops.set_decode_wb(prev)
+
+
 def test_upsample2d_layer_takes_phase_conv_and_tracks_weight_updates(cuda):
     """Upsample2D (UNet / VAE) on a shape with >= 256 output tiles runs the phase conv with cached phase weights,
     matches the fp32 upsample + 3x3 conv, and rebuilds the phase weights after an in-place weight update."""
