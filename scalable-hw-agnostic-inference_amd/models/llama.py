@@ -250,10 +250,11 @@ class LlamaForCausalLM(nn.Module):
         """(64-token blocks of a decode split, at least; of a context that is not split) for :func:`ops.decode_splits`.  With 4
         query heads of 128 per KV head an unsplit context's blocks go to the waves of one workgroup at a time
         (decode_attn_wb_kernel), and the launch that joins splits is saved, in an engine whose longest context is that short
-        (``LLMEngine.decode_splits`` goes by ``max_model_len``): Mistral-7B, 8 layers, one step at 254 cached tokens
-        932 -> 893 us (batch 1), 967 -> 910 (16), 989 -> 943 (32); at 504 tokens 965 -> 936; at 724 no longer faster."""
+        (``LLMEngine.decode_splits`` goes by ``max_model_len``): Mistral-7B, 8 layers, one step in parts and whole, at 616 cached
+        tokens 834 and 803 us (batch 1), 884 and 839 (8); at 996 837 and 820, 898 and 875.  Attention alone at 1,600: 13.5 and 15.7
+        us (batch 1), 22.5 and 22.8 (8), 28.7 and 26.7 (16)."""
         a = self.layers[0].self_attn
-        return 1, 8 if a.hd == 128 and a.h == 4 * a.hk else 0
+        return 1, 16 if a.hd == 128 and a.h == 4 * a.hk else 0
 
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
