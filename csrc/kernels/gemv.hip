@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(SK_WAVES * 64) skinny_gemm_kernel(const GemmAr
   // ds_write_b128 / ds_read_b128), each lane's 4 consecutive-n accumulators (registers 4q .. 4q + 3: n = 8q + 4fh
   // + 0..3 of its 32-row half, m = 32j + fr) as ONE float4; a thread then owns output quads (m, 4 consecutive n) and
   // sums the 4 waves' float4s in wave order -- 4x fewer LDS instructions than element-wise, the epilogue / partial
-  // stores 8-16 B per lane (gpurun_out/r6m_decode_lab2.log: the element-wise reduction + 4-B stores cost 2.4-3.9 us
+  // stores 8-16 B per lane (the element-wise reduction + 4-B stores cost 2.4-3.9 us
   // per launch over the streaming loop).
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
