@@ -113,11 +113,15 @@ __device__ __forceinline__ float gelu_erf_f(float x) {
   return fmaf(a, 0.5f - __builtin_amdgcn_exp2f(p), 0.5f * x);
 }
 
-// x/2 (1 + tanh u) = x / (1 + e^{-2u}), u = sqrt(2/pi) (x + 0.044715 x^3): the factors of the exponent in its constants, 7 VALU, 52 clocks a wave, where
-// the tanh took 12 and 72.  Saturates at 0 and x; for x < 0 the result keeps its relative precision, which 1 + tanh u lost.
+// x/2 (1 + tanh u) = max(x, 0) - |x| / (1 + e^{2|u|}), u = sqrt(2/pi) (x + 0.044715 x^3), the factors of the exponent in its constants: the fraction, with
+// the exponential's and the reciprocal's errors, is what is taken off, so that x > 0 loses none of its bits to them and x < 0 keeps its relative
+// precision.  10 VALU, 64 clocks a wave.  Against 64 bits over -12 .. 12 at most 2.4e-7; x/2 (1 + tanh u) as it is written takes 12 and 72, 4.3e-7
+// above 0 and 1.4e-6 below; x / (1 + e^{-2u}) takes 7 and 52, but 5.2e-7 above 0.  Infinities and NaN as x/2 (1 + tanh u) has them.
 __device__ __forceinline__ float gelu_tanh_f(float x) {
-  const float e = x * fmaf(-0.10294324f, x * x, -2.3022082f);   // -2 u log2 e
-  return x * rcp_f(1.0f + __builtin_amdgcn_exp2f(e));
+  const float a = fabsf(__builtin_amdgcn_fmed3f(x, -16.0f, 16.0f));   // nothing is taken off beyond, also of infinity
+  const float e = a * fmaf(0.10294324f, a * a, 2.3022082f);   // 2 |u| log2 e
+  const float t = rcp_f(1.0f + __builtin_amdgcn_exp2f(e));
+  return fmaf(-a, t, fmaf(0.5f, fabsf(x), 0.5f * x));
 }
 
 __device__ __forceinline__ float quick_gelu_f(float x) { return x * rcp_f(1.0f + __expf(-1.702f * x)); }

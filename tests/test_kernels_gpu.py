@@ -782,7 +782,7 @@ def test_mean_tokens(cuda, B, S, D):
 
 @pytest.mark.parametrize("act", ["gelu", "gelu_tanh"])
 def test_gelu_of_every_bf16(cuda, act):
-    """All 2^16 inputs.  One rounding to bf16 (half a unit in the last of 8 bits), and 6e-7 for the fp32 steps: 3.4e-7 (gelu) and 5.2e-7
+    """All 2^16 inputs.  One rounding to bf16 (half a unit in the last of 8 bits), and 6e-7 for the fp32 steps: 3.4e-7 (gelu) and 2.4e-7
     (gelu_tanh) at most over -12 .. 12, behind them the results are 0 and x.  NaN for NaN; -inf times 0 is one too."""
     x = torch.arange(65536, dtype=torch.int32, device=cuda).to(torch.int16).view(torch.bfloat16).view(256, 256)
     y, xd = ops.bias_act(x, act=act).double(), x.double()
@@ -794,3 +794,27 @@ def test_gelu_of_every_bf16(cuda, act):
     assert bool(((y - want).abs() <= want.abs() * 2 ** -8 + 6e-7)[num].all())
     assert bool(torch.isnan(y[torch.isnan(xd)]).all()) and bool((y[xd == torch.inf] == torch.inf).all())
     assert bool(torch.isnan(y[xd == -torch.inf]).all())
+
+
+@pytest.mark.parametrize("low,high", [(0.02, 1.0), (1.0, 2.5), (2.5, 5.0), (5.0, 12.0), (-6.0, -1.0), (-1.0, -0.02)])
+def test_gelu_tanh_in_32_bits(cuda, low, high):
+    """The fp32 steps of the epilogue alone: arguments (three bf16 values each, their sum is exact) whose result is within 2^-18 of a bf16 value, which a
+    residual takes off before the rounding to bf16: 2^-27 of the result is left of that.  Half a unit of the result's 24 bits, and 1e-7 for
+    what is taken off max(x, 0): at most 0.17, with a reciprocal, an exponential (2^-23 each) and the rounding of its exponent."""
+    torch.manual_seed(3)
+    z = torch.rand(8 << 20, device=cuda) * (high - low) + low
+    zd = z.double()
+    g = zd * torch.sigmoid(2 * (2 / torch.pi) ** 0.5 * (zd + 0.044715 * zd ** 3))
+    near = (g - g.bfloat16().double()).abs() <= 2 ** -18 * g.abs()
+    z, g = z[near][:8192], g[near][:8192]
+    assert len(z) > 1000
+    h = z.bfloat16()
+    m = (z - h.float()).bfloat16()
+    x = torch.zeros(len(z), 64, device=cuda, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1], x[:, 2] = h, m, (z - h.float() - m.float()).bfloat16()
+    assert torch.equal(x.double().sum(1), z.double())
+    r = -g.bfloat16()
+    out = torch.empty(len(z), 64, device=cuda, dtype=torch.bfloat16)
+    ops.gemm_into(x, torch.ones(64, 64, device=cuda, dtype=torch.bfloat16), out, act="gelu_tanh", residual=r[:, None].expand(-1, 64).contiguous())
+    err = (out.double() - (g + r.double())[:, None]).abs().amax(1)
+    assert bool((err <= g.abs() * (2 ** -24 + 2 ** -27) + 1e-7).all()), (err / (g.abs() * 2 ** -24 + 1e-7)).max().item()
