@@ -7,10 +7,12 @@
 //
 // 8 waves: wave w takes the 32 k of sub-step w % 4 and the row blocks of half w / 4; the four k-groups' sums meet in LDS and are
 // added in their order.  Rows past M or N and values past K are out of the buffers' range: zeros, no traffic.
-// A workgroup with all of K begins kTurn steps behind the one before it and goes round: begun together, all of them read the same columns of
-// W, rows of 2^n bytes apart, from a part of the memory's channels.  us in order -> turned, cold weights, 16 / 32 / 64 rows: 28672 x 4096 54.1 / 53.3 /
-// 56.1 -> 43.8 / 43.9 / 46.5, 32768 x 2048 35.9 / 34.3 / 36.7 -> 35.7 / 32.7 / 29.3, 17424 x 2048 19.0 / 19.7 / 22.3 -> 16.7 / 17.1 / 20.0, 8192 x 8192
-// 36.3 / 35.4 / 38.0 -> 26.3 / 26.0 / 31.8 (by one step 35.2, by three 29.9, by five 27.1); nothing is slower (5632 x 1024, 4096 x 4096).
+// Where a row of W is a multiple of 4 KB, a workgroup with all of K begins kTurn steps behind the one before it and goes round: begun together,
+// all of them read the same columns of W from a part of the memory's channels.  us in order -> turned, cold weights, 16 / 32 / 64 rows: 8192 x 8192
+// 34.6 / 40.0 / 38.9 -> 26.8 / 26.6 / 33.3, 17424 x 2048 19.1 / 19.6 / 21.9 -> 16.7 / 17.2 / 20.4, 32768 x 2048 35.1 / 33.5 / 37.3 -> 35.4 / 33.5 / 29.6,
+// 28672 x 4096 53.9 / 57.0 / 54.0 -> 50.6 / 50.8 / 53.0, 8192 x 14336 (112 steps, 16 beginnings) 48.4 / 51.6 / 63.5 -> 44.2 / 48.3 / 62.0, 8192 x 6144 23.2 /
+// 24.7 / 30.5 -> 20.9 / 22.7 / 29.5; 8192 x 8192 on 16 rows by one step 35.2, by three 29.9, by five 27.1.  Other rows gain nothing by it and took longer: 5632 x
+// 1024 5.8 / 6.1 / 6.9 -> 6.0 / 6.4 / 7.2, 9216 x 3072 13.9 / 15.8 / 20.5 -> 14.4 / 16.1 / 20.8, 8192 x 3584 13.4 / 14.6 / 18.9 -> 14.0 / 14.9 / 19.1.
 //
 // LDS rows are 256 bytes; chunk c (16 bytes) of row r is at c ^ (r & 15): no bank conflicts, and the DMA stays lane-linear because
 // the source address carries the permutation.
@@ -61,7 +63,7 @@ __global__ void __launch_bounds__(512) gemm_ring_kernel(const GemmArgs p) {
     steps = (int)((blockIdx.y + 1L) * all / p.splits) - first;
     C += (long)blockIdx.y * p.M * p.N;
   }
-  const int turn = p.splits > 1 ? 0 : (int)(blockIdx.x * kTurn % steps);   // the first step
+  const int turn = p.splits > 1 || p.K % 2048 != 0 ? 0 : (int)(blockIdx.x * kTurn % steps);   // the first step
   uint32_t off[HI];
   int col[HI];                                // first k of this lane's chunk within a stage
 #pragma unroll

@@ -37,6 +37,23 @@ def test_plain(cuda, M, N, K):
     assert bool((out[:, :8] == 3).all()) and bool((out[:, N + 8:] == 3).all())
 
 
+# workgroups that begin at different steps of K: 16, 32 and 112 of them, columns that end inside a workgroup, more than one round
+@pytest.mark.parametrize("M", [12, 16, 33, 64])
+@pytest.mark.parametrize("N,K", [(8200, 2048), (7180, 4096), (7172, 14336), (32772, 4096)])
+def test_turned(cuda, M, N, K):
+    a, w = _problem(M, N, K, cuda, spare=8)
+    assert _rel(lm.matmul(a, w, torch.float32), a.double() @ w.double().T) < 1e-5
+
+
+@pytest.mark.parametrize("M", [12, 64])
+@pytest.mark.parametrize("N,K", [(5632, 1024), (9216, 3072), (8192, 3584), (7168, 7168), (5632, 2112)])
+def test_in_order_where_rows_are_not_4_kb(cuda, M, N, K):
+    """There the turn is time lost: every workgroup adds K in the same order, so that columns of the same weights are the same bits."""
+    a, w = _problem(M, N, K, cuda)
+    y = lm.matmul(a, w[:1].expand(N, K).contiguous(), torch.float32)
+    assert torch.equal(y, y[:, :1].expand_as(y))
+
+
 @pytest.mark.parametrize("M", [1, 8, 31, 64])
 @pytest.mark.parametrize("N,K", [(512, 512), (2048, 4096), (2048, 12544), (2000, 4160), (1788, 8256), (768, 4160), (4096, 1024), (8192, 576)])
 def test_parts(cuda, M, N, K):
