@@ -1848,6 +1848,14 @@ void softmax_(const Tensor& x, double scale) {
   shai::launch_softmax(mptr(x), x.numel() / x.size(-1), x.size(-1), scale, stream());
 }
 
+std::string decode_attn_form(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t splits) {
+  switch (shai::decode_attn_form((int)B, (int)Hq, (int)Hkv, (int)D, (int)splits)) {
+    case shai::DecodeForm::kWaves: return "waves";
+    case shai::DecodeForm::kItems: return "items";
+    default: return "walk";
+  }
+}
+
 std::vector<std::string> gemm_tuning() { return gemm_tuning_table(); }
 
 // Export / import the autotuner cache ("key=cfg,splits") so later processes skip tuning.
@@ -2125,6 +2133,7 @@ TORCH_LIBRARY(shai, m) {
   m.def("set_halo_conv(int mode, int waves=-1) -> int", &set_halo_conv);
   m.def("set_flash128x2(int mode) -> int", [](int64_t mode) -> int64_t { return shai::set_flash128x2((int)mode); });
   m.def("set_decode_wb(int mode) -> int", [](int64_t mode) -> int64_t { return shai::set_decode_wb((int)mode); });
+  m.def("decode_attn_form(int B, int Hq, int Hkv, int D, int splits) -> str", &decode_attn_form);
 }
 
 TORCH_LIBRARY_IMPL(shai, CUDA, m) {

@@ -985,7 +985,9 @@ __global__ void decode_combine_kernel(const DecodeAttnArgs p) {
 // 250 21.4 -> 16.8, 256 x 132 49.1 -> 34.3 (4.0 TB/s).
 // SPLIT: a workgroup has one of a row's da_splits parts of at least four blocks, one for each wave, and leaves (m, l, o)
 // for decode_combine_kernel, as the split kernel does; against that one, both with their combine, us: 1 x 1000 in 16
-// (4 after da_splits) 19.0 -> 11.7, 1 x 6000 in 64 33.7 -> 27.3, 8 x 2000 in 8 29.0 -> 24.5, 32 x 1000 in 2 37.2 -> 31.4.
+// (4 after da_splits) 19.0 -> 11.9, 1 x 6000 in 64 33.8 -> 27.7, 1 x 127000 in 64 145.1 -> 137.7 (one KV head 119.0 ->
+// 66.4), 8 x 2000 in 8 29.2 -> 24.6, 8 x 32000 in 8 208 -> 196, 32 x 1000 in 2 36.9 -> 32.2, 32 x 16000 in 2 392 -> 364; one
+// of 64000 beside one of 300 107 -> 95.  Faster at all 120 measured, 1 to 64 rows of 1000 to 127000 keys, 1, 2 and 8 KV heads.
 // SHAI_DECODE_WB=0 / set_decode_wb(0) routes these launches back to the split kernel (A/B).
 constexpr int kWbG = 4;
 constexpr size_t kWbLds = (size_t)kWbG * 64 * 128 * 2 + (size_t)kWbG * 128 * 2;
@@ -1326,26 +1328,39 @@ size_t decode_attn_workspace(int B, int Hq, int D, int num_splits) {
   return (size_t)B * Hq * num_splits * (D + 2) * sizeof(float);
 }
 
-void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t s) {
-  const int G = a.Hq / a.Hkv;
-  static const int width = [] {  // two workgroups per CU (70 KB of LDS each)
+static int decode_width() {  // two workgroups per CU (70 KB of LDS each)
+  static const int width = [] {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
       cus = 256;
     return 2 * cus;
   }();
-  // short-context batches (<= 8 splits: every item does work) keep one workgroup per item; the persistent walk is
-  // for the raised split factors of long contexts.  SHAI_DECODE_PERSIST=0 / 1 forces either form (A/B).
+  return width;
+}
+
+DecodeForm decode_attn_form(int B, int Hq, int Hkv, int D, int num_splits) {
+  // SHAI_DECODE_PERSIST=0 / 1 forces either form of the split kernel where there are splits (A/B).
   static const int force = [] {
     const char* e = getenv("SHAI_DECODE_PERSIST");
     return e ? (e[0] == '1' ? 1 : 0) : -1;
   }();
-  const long items = (long)a.B * a.Hkv * a.num_splits;
   // Wave-per-block kernel: unsplit, or up to two rounds of workgroups, which is what a split count made to fill the chip
-  // gives (faster at every one measured, 250 to 6,000 keys and 1 to 32 rows).  Beyond stands a count raised for one long
-  // row, and most workgroups have none of a short row's parts: the persistent walk of the split kernel is for those.
-  if (a.D == 128 && G == kWbG && decode_wb_mode() && (a.num_splits == 1 || items <= 2 * width)) {
+  // gives (SPLIT above).  Beyond stands a count raised for one long row, and most workgroups have none of a short row's
+  // parts: the persistent walk of the split kernel is for those.
+  if (D == 128 && Hq == kWbG * Hkv && decode_wb_mode() &&
+      (num_splits == 1 || (force < 0 && (long)B * Hkv * num_splits <= 2 * decode_width())))
+    return DecodeForm::kWaves;
+  // short-context batches (<= 8 splits: every item does work) keep one workgroup per item; the persistent walk is
+  // for the raised split factors of long contexts.
+  return (force >= 0 ? force == 1 : num_splits > 8) ? DecodeForm::kWalk : DecodeForm::kItems;
+}
+
+void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t s) {
+  const int G = a.Hq / a.Hkv;
+  const long items = (long)a.B * a.Hkv * a.num_splits;
+  const DecodeForm form = decode_attn_form(a.B, a.Hq, a.Hkv, a.D, a.num_splits);
+  if (form == DecodeForm::kWaves) {
     auto go = [&](auto split) {
       constexpr bool SPLIT = decltype(split)::value;
       const dim3 grid((unsigned)items);
@@ -1361,8 +1376,7 @@ void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t s) {
     }
     return;
   }
-  const bool persist = force >= 0 ? force == 1 : a.num_splits > 8;
-  dim3 grid((unsigned)(persist ? std::min<long>(items, width) : items));
+  dim3 grid((unsigned)(form == DecodeForm::kWalk ? std::min<long>(items, decode_width()) : items));
   const size_t lds = (size_t)4 * 64 * a.D * sizeof(bf16_t) + (size_t)8 * a.D * 4 + 8 * 64 * 4;
   // NI = wave DMA instructions per block per wave = (2 * 64 * D * 2 / 1024) / G
 #define DA(D_, NI_) decode_attn_kernel<D_, NI_><<<grid, G * 64, lds, s>>>(a)

@@ -338,7 +338,10 @@ struct DecodeAttnArgs {
   float qkv_eps;
 };
 void launch_decode_attn(const DecodeAttnArgs& a, hipStream_t s);
-// decode routing (D 128, GQA 4, one split or at most four workgroups per CU -> the wave-per-block kernel); SHAI_DECODE_WB=0 / mode 0: split kernel
+// a wave takes blocks of its own (D 128, GQA 4); the split kernel with a workgroup per (sequence, KV head, split), or with a persistent walk over them
+enum class DecodeForm { kWaves, kItems, kWalk };
+DecodeForm decode_attn_form(int B, int Hq, int Hkv, int D, int num_splits);
+// SHAI_DECODE_WB=0 / mode 0: never the wave-per-block kernel
 int decode_wb_mode();
 int set_decode_wb(int mode);   // -1 keeps the mode; returns the previous one
 size_t decode_attn_workspace(int B, int Hq, int D, int num_splits);

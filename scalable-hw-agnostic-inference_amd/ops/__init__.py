@@ -501,8 +501,9 @@ def bmm(a: torch.Tensor, w: torch.Tensor, alpha: float = 1.0) -> torch.Tensor:
 
 
 def set_decode_wb(mode: int = -1) -> int:
-    """Decode attention routing at D 128 / GQA 4 / one split: 1 = the wave-per-block short-context kernel (default),
-    0 = the split kernel (``SHAI_DECODE_WB=0``); -1 keeps the mode.  Returns the previous mode (A/B in one process)."""
+    """Decode attention routing at D 128 / GQA 4: 1 = the wave-per-block kernel (default) for one split, or for splits of up to
+    four (sequence, KV head, split) workgroups per CU unless ``SHAI_DECODE_PERSIST`` names a form of the split kernel; 0 = the
+    split kernel (``SHAI_DECODE_WB=0``); -1 keeps the mode.  Returns the previous mode (A/B in one process)."""
     return int(_K().set_decode_wb(int(mode)))
 
 
