@@ -22,9 +22,10 @@ def test_sched_step_rows_kernel(cuda):
         assert torch.equal(got[1], lat[1]) and torch.equal(got[4], lat[4])
 
 
-def test_step_batcher_gpu_matches_generate(cuda):
-    from shai_amd.engines.diffusion import SDConfig, StableDiffusionEngine, StepBatcher
-    eng = StableDiffusionEngine(SDConfig.tiny(), device="cuda")
+def _batched(eng):
+    """Two requests of a batch, one joined in mid-flight, beside the images of generate()."""
+    from shai_amd.engines.diffusion import StepBatcher
+    eng._graphs.clear()
     sb = StepBatcher(eng, max_batch=4)
     assert sb.warmup() == 4
     a = sb.add("a red fox", 6, seed=1)
@@ -33,10 +34,24 @@ def test_step_batcher_gpu_matches_generate(cuda):
         b = sb.add("a blue hen", 4, seed=2)
         while sb.has_work():
             sb.step()
-        for r, p, n, s in ((a, "a red fox", 6, 1), (b, "a blue hen", 4, 2)):
-            want = eng.generate([p], n, seed=s)[0]
-            # the batched bucket runs other GEMM configurations (per-shape autotune; the device debug build's
-            # timings pick others again), so bf16 rounding differs: uint8 pixels agree to a level or two
-            d = (r.image.float() - want.float()).abs()
-            assert d.mean() < 2.0 and (d <= 2).float().mean() > 0.9, (d.mean(), (d <= 2).float().mean())
-    assert sb.stats["joined_mid_batch"] == 1
+        assert sb.stats["joined_mid_batch"] == 1
+        return [(r.image, eng.generate([p], n, seed=s)[0]) for r, p, n, s in ((a, "a red fox", 6, 1), (b, "a blue hen", 4, 2))]
+
+
+def test_step_batcher_gpu_matches_generate(cuda):
+    """With one form for every product, the same in a batch and alone, the same image.  The forms that the tuner picks by time differ between
+    row counts, and so does the order of fp32 sums: this tiny model of random weights, 7.5 times the difference of two nearly equal outputs a
+    step, carries a rounding to bf16 as far as 18 to 20 of 255 levels from its fp32 form.  Two images of it then differ by a tenth of that
+    at most: 0.3 to 1.7 levels in the mean over 50 sets of forms picked at random."""
+    from shai_amd import ops
+    from shai_amd.engines.diffusion import SDConfig, StableDiffusionEngine
+    eng = StableDiffusionEngine(SDConfig.tiny(), device="cuda")
+    for got, want in _batched(eng):
+        assert (got.float() - want.float()).abs().mean() < 2.0
+    table = list(ops._K().gemm_tuning_export())     # with an entry for every product of this model now
+    try:
+        ops._K().gemm_tuning_import([e.rsplit("=", 1)[0] + "=4,1" for e in table])
+        for got, want in _batched(eng):
+            assert torch.equal(got, want)
+    finally:
+        ops._K().gemm_tuning_import(table)
