@@ -462,10 +462,16 @@ def test_skinny_turned(cuda, M, N, K, ld, cfg, rms):
     assert _rel(out, want) < 2.4e-3
 
 
-def test_skinny_turned_fp8(cuda):
-    M, N, K = 3, 16400, 4096
+@pytest.mark.parametrize("M", [3, 64])
+@pytest.mark.parametrize("N,K", [(16400, 4096), (16384, 8192), (16390, 4080)])
+def test_skinny_turned_fp8(cuda, M, N, K):
+    """All of K in a workgroup, rows of 4 or 8 KB; with 4080 columns of them K ends inside a step."""
     torch.manual_seed(5)
     x = torch.randn(M, K, device=cuda).bfloat16()
-    w8, scale = ops.quantize_fp8_rows(torch.randn(N, K, device=cuda) / K ** 0.5)
+    ld = (K + 4095) // 4096 * 4096
+    w8, scale = ops.quantize_fp8_rows(torch.randn(N, ld, device=cuda) / K ** 0.5)
+    w8 = w8[:, :K]
+    out = torch.empty(M, N, device=cuda, dtype=torch.bfloat16)
+    ops.gemm_into(x, w8, out, w_scale=scale, force_cfg=SKINNY + 1)
     want = x.double() @ (w8.double() * scale.double()[:, None]).t()
-    assert _rel(ops.linear(x, w8, w_scale=scale), want) < 2.4e-3
+    assert _rel(out, want) < 2.4e-3
