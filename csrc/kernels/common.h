@@ -82,20 +82,6 @@ __device__ __forceinline__ float rcp_f(float x) { return __builtin_amdgcn_rcpf(x
 
 __device__ __forceinline__ float silu_f(float x) { return x * rcp_f(1.0f + __expf(-x)); }
 
-// erf via Abramowitz-Stegun 7.1.26 (|error| <= 1.5e-7, far below bf16 resolution): one exp, one
-// reciprocal and a degree-5 Horner chain instead of the libm erff polynomial + branches, which
-// made GEGLU epilogues VALU-bound.
-__device__ __forceinline__ float erf_fast(float x) {
-  const float ax = fabsf(x);
-  const float t = rcp_f(fmaf(0.3275911f, ax, 1.0f));
-  float y = fmaf(1.061405429f, t, -1.453152027f);
-  y = fmaf(y, t, 1.421413741f);
-  y = fmaf(y, t, -0.284496736f);
-  y = fmaf(y, t, 0.254829592f);
-  y = 1.0f - y * t * __expf(-ax * ax);
-  return copysignf(y, x);
-}
-
 // gelu(x) = x/2 + |x| (1/2 - Phi(-|x|)).  log2 Phi(-a) is smooth: a polynomial of degree 8, minimax on 0 .. 6.5 with the weight Phi(-a) that its
 // error enters the result with, and falling everywhere behind.  12 VALU, one of them transcendental (a quarter of the rate): 60 clocks a
 // wave.  Before, the erf of Abramowitz and Stegun 7.1.26, 13 with two: 76.  Against 64 bits over -12 .. 12: at most 3.4e-7 and 1.9e-8 in the
