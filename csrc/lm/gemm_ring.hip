@@ -18,8 +18,8 @@
 // the source address carries the permutation.
 //
 // Replays of a HIP graph over weights larger than the caches, us (streaming kernel -> here; N x K, 64 rows): 17424 x 2048
-// 24.0 -> 19.3, 32768 x 2048 40.7 -> 34.7, 24576 x 4096 63.7 -> 44.7, 8256 x 2048 17.5 -> 12.6, 4096 x 2048 10.3 -> 7.9, partial
-// sums of 2048 x 12544 21.6 (4 parts) -> 14.5 (8 parts).  17424 x 2048 is 71 MB: 3.7 TB/s.  What is left is the start (launch, the
+// 26.2 -> 20.5, 32768 x 2048 42.3 -> 29.7, 24576 x 4096 69.3 -> 42.1, 8256 x 2048 18.0 -> 14.5, 4096 x 2048 11.0 -> 10.0, partial
+// sums of 2048 x 12544 21.6 (4 parts) -> 14.5 (8 parts).  17424 x 2048 is 71 MB: 3.5 TB/s.  What is left is the start (launch, the
 // first stage's latency) and the joining of the sums, about 5 us, and the memory's rate in between.
 #include "lm_device.h"
 #include "lm.h"
@@ -151,7 +151,8 @@ void launch_blocks(const GemmArgs& a, int nt, hipStream_t s) {
 
 // Columns of a workgroup, in blocks of 16: one workgroup per CU, or as few rounds of them as 128 columns allow.  Up to 32 rows a
 // stage is short, and beyond one round of 112 columns two workgroups of 48 per CU, each other's prologue and end hidden, are
-// faster (50176 x 4096, 32 rows: 91 us; one of 128: 95; 32768 x 2048: 32.9 and 34.1).
+// faster (50176 x 4096, 32 rows: 88.9 us; one of 128: 91.8).  That was so of all before workgroups began at different steps of K; since
+// then 32768 x 2048 is 33.1 us in 48 columns and 28.2 in 128, x 3072 45.7 and 40.2, x 4096 56.3 and 56.0.
 constexpr long kRound = 256 * 112;
 static int ring_blocks(const GemmArgs& a) {
   const long cols = (long)a.N * (a.splits > 1 ? a.splits : 1), rounds = (cols + 256 * 128 - 1) / (256 * 128);
@@ -160,18 +161,21 @@ static int ring_blocks(const GemmArgs& a) {
   return nt < 2 ? 2 : nt > 6 ? 8 : nt;
 }
 
-// Where the ring is no slower than the streaming kernel, whose 16-column workgroups read few rows of A from few cache lines, start
+// Where the ring was no slower than the streaming kernel, whose 16-column workgroups read few rows of A from few cache lines, start
 // faster, and have no sums to join.  Replays of a HIP graph, cold weights, N x K (streaming -> ring, us):
-//   from 4097 columns on, which are more 16-column workgroups than CUs: 9 rows (5120 x 2048: 0.87 of the time), from 7169 on 12 (8192 x
-//     8192: 9 rows 1.05, 12 1.04, 16 0.94; 17424 x 2048: 9 rows 0.96, 16 0.86);
-//   below: 33 rows from 2049 columns on (2304 x 4096, 64 rows: 24.2 -> 15.5; 2048 x 2048 8.5 -> 9.4), and 17 to 32 rows where M K >=
-//     24 * 1024 (2048 x 2048, 32 rows: 8.4 -> 7.5; 4096 x 1024: 17 rows 1.03 of the time, 24 rows 0.99);
+//   from 4097 columns on, which are more 16-column workgroups than CUs: 9 rows, from 7169 on 12.  These lines were drawn when all workgroups
+//     began at column 0 (8192 x 8192: 9 rows 1.05 of the time, 12 1.04, 16 0.94).  Now the ring is ahead on both sides of them: 5120 x 2048, 1 row
+//     0.87, 9 0.80; 8192 x 8192, 1 0.91, 9 0.83, 12 0.77, 16 0.70; 17424 x 2048, 1 0.96, 9 0.86, 16 0.74; 9216 x 3072, 1 0.82, 12 0.71; 14336 x 5120, 1 0.93,
+//     12 0.70; 28672 x 4096 alone 1 1.29, 9 1.08, 12 0.99.  Up to eleven rows they stand where they were: in whole steps only 1 row was
+//     timed with the ring, where most of such products are normed_gemm's, without a gain;
+//   below: 33 rows from 2049 columns on (2304 x 4096, 64 rows: 23.9 -> 15.3; 2048 x 2048 8.4 -> 9.4), and 17 to 32 rows where M K >=
+//     24 * 1024 (2048 x 2048, 32 rows: 8.3 -> 7.6; 4096 x 1024: 17 rows 1.04 of the time, 24 rows 1.00);
 //   partial sums: more than 16 rows (512 x 8448 in 8 parts, 17 rows: 6.8 -> 5.8); up to 16 of a K of 4096, from 2049 columns on, or
 //     where 32-column workgroups of all parts fill 7 of 8 CUs and either 9 rows or a K of 8192 are there: 2048 x 8448 in 4 parts,
 //     1 row 10.2 -> 9.4, 16 rows 11.4 -> 9.3; x 6144, 9 rows 8.1 -> 7.5; 1024 x 12544 in 8, 1 row 8.0 ->
 //     7.9, 16 rows 9.1 -> 7.8; with half of the CUs the streaming kernel's 16 columns are faster: 512 x 8448 in 8, 1 row 4.8 -> 5.3.
-//   Up to 32 rows more columns than one round of 112 (ring_blocks) take a K, or part of one, of 3072: 32768 x 1024, 32 rows 1.09 of
-//     the time, x 4096 0.98; 8192 x 2048 in 4 parts, 8 rows 15.6 -> 19.0.
+//   Up to 32 rows more columns than one round of 112 (ring_blocks) take a K, or part of one, of 3072: 32768 x 1024, 32 rows 1.14 of
+//     the time, x 2048 0.99, x 4096 0.89; 8192 x 2048 in 4 parts, 8 rows 15.6 -> 19.0.
 // Products per head, grouped by expert or longer than a buffer's range stay with the streaming kernel.
 bool gemm_ring_fits(const GemmArgs& a) {
   const long lim = 0x7fffffffL, splits = a.splits > 1 ? a.splits : 1;

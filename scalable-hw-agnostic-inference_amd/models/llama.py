@@ -252,7 +252,8 @@ class LlamaForCausalLM(nn.Module):
         (decode_attn_wb_kernel), and the launch that joins splits is saved, in an engine whose longest context is that short
         (``LLMEngine.decode_splits`` goes by ``max_model_len``): Mistral-7B, 8 layers, one step in parts and whole, at 616 cached
         tokens 834 and 803 us (batch 1), 884 and 839 (8); at 996 837 and 820, 898 and 875.  Attention alone at 1,600: 13.5 and 15.7
-        us (batch 1), 22.5 and 22.8 (8), 28.7 and 26.7 (16)."""
+        us (batch 1), 22.5 and 22.8 (8), 28.7 and 26.7 (16); with one KV head, as on a rank of eight, at 600 9.9 and 9.9, at 1,000 10.5
+        and 11.6."""
         a = self.layers[0].self_attn
         return 1, 16 if a.hd == 128 and a.h == 4 * a.hk else 0
 
